@@ -64,6 +64,7 @@
 #define EH_F_CHANGE_T (1 << 25) /* RFCA CHANGE_T: EH_D_TOFF whole RF periods taken out of t and s */
 #define EH_F_CHT_SELF (1 << 26) /* CHANGE_T with each particle as its own beam: the offset from its own time */
 #define EH_F_LEND (1 << 27)    /* KQUAD LEFFECTIVE: exact drifts of EH_D_LEND around the body */
+#define EH_F_WIDE (1 << 29)    /* with EH_F_FAST: a substep angle of 2^-6 or more */
 #define EH_F_FIRSTPASS (1 << 28) /* before the RECIRC point: tracked on pass 0 only (do_tracking.c:459-465) */
 
 /* Aperture shapes other than the closed rectangle, packed in one int32:
@@ -158,12 +159,12 @@ typedef struct {
 #define EH_D_BDSH 20      /* [8]: s * driftFrac[j] */
 #define EH_D_BDSHR 28     /* [8]: (s * driftFrac[j]) / rho0 */
 #define EH_D_BDS 36       /* [8]: s * kickFrac[j] */
-#define EH_D_BKF 44       /* [8]: kickFrac[j] (0 ends the slice) */
 #define EH_D_RHOA_SGN 52  /* +1 or -1: the sign of rho_actual (t / rho_actual for t = +-0 or NaN) */
 #define EH_D_RRHO0 53     /* 1 / rho0 rounded to nearest: the quotients by rho0 use em_div */
 #define EH_D_RRHOA 54     /* 1 / rho_actual rounded to nearest */
 #define EH_D_FIELD 55     /* [<= 28]: field coefficients in the order the sums read them (eh_bend_field.h) */
 #define EH_D_FIELD_MAX 28 /* expansion order 6: K1..K4 and XKICK */
+#define EH_D_ZLIM 44      /* with EH_F_FAST: phi^2 below this keeps every |substep angle + phi| below 2^-5 */
 #define EH_D_ET 83        /* [5]: ETILT exit offsets of x, x', y, y', s (eh_bend_etilt.h) */
 
 /* ---- RFCA ---- */

@@ -72,14 +72,15 @@
 #define EM_TWO_OVER_PI 0x1.45f306dc9c883p-1
 #define EM_SHIFT 0x1.8p+52
 
-/* A polynomial coefficient at its point of use.  On the device the empty
- * volatile asm keeps each 64-bit constant a scalar-register operand
- * materialized where it is used; without it the compiler hoists every
- * coefficient of every inlined polynomial into vector registers for the
- * whole kernel, which costs occupancy.  The value is unchanged. */
+/* A polynomial coefficient as a scalar-register operand.  The empty asm hides
+ * the value from the compiler, which otherwise hoists every coefficient of
+ * every inlined polynomial into vector registers for the whole kernel (that
+ * costs occupancy).  Not volatile: equal coefficients may share a register
+ * pair over a loop, which took 72 of 108 scalar instructions out of a slice of
+ * the bend's common path (a wave alone on its SIMD issues them one by one). */
 #if defined(__HIP_DEVICE_COMPILE__)
 EM_FN double em_k(double c) {
-  asm volatile("" : "=s"(c) : "0"(c));
+  asm("" : "=s"(c) : "0"(c));
   return c;
 }
 #else
@@ -176,9 +177,11 @@ EM_FN double em_sin_small(double x, double z) {
  * (k_cos.c) uses. */
 EM_FN double em_cos_small(double x, double z) {
   double r = z * z * em_cos_r_small(z);
-  double hz = 0.5 * z;
-  double w = 1.0 - hz;
-  return w + (((1.0 - w) - hz) + r);
+  /* z/2 is exact or, when subnormal, vanishes against w and rounds as the
+   * product would against 1 - w = 0, so the FMAs give the bits of 1 - z/2
+   * and of (1 - w) - z/2 */
+  double w = __builtin_fma(-0.5, z, 1.0);
+  return w + (__builtin_fma(-0.5, z, 1.0 - w) + r);
 }
 
 /* ---- double-double arithmetic ---- */
@@ -754,6 +757,45 @@ EM_FN double em_sqrt_mid(double x) {
   return __builtin_fma(d, h, g);
 #else
   return __builtin_sqrt(x);
+#endif
+}
+
+/* em_sqrt_mid(x) = g and em_recip(g) from one v_rsq_f64, 2^-128 <= x <= 2^128:
+ * after the iteration h is 1/(2 sqrt(x)) to about an ulp, so 2h stands in for
+ * v_rcp_f64 (four times the issue cycles of an FMA) and the first of em_recip's
+ * two Newton steps. */
+EM_FN double em_sqrt_recip_mid(double x, double *y) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  double r = __builtin_amdgcn_rsq(x);
+  double g = x * r, h = r * 0.5;
+  double e = __builtin_fma(-h, g, 0.5);
+  g = __builtin_fma(g, e, g);
+  double d = __builtin_fma(-g, g, x);
+  h = __builtin_fma(h, e, h);
+  g = __builtin_fma(d, h, g);
+  d = __builtin_fma(-g, g, x);
+  g = __builtin_fma(d, h, g);
+  h = h + h;
+  e = __builtin_fma(-g, h, 1.0);
+  *y = __builtin_fma(h, e, h);
+  return g;
+#else
+  double g = __builtin_sqrt(x);
+  *y = 1.0 / g;
+  return g;
+#endif
+}
+
+/* em_recip(c) of a cosine c = em_cos_small(a, z), z = a*a < 2^-10: the secant's
+ * series 1 + z/2 + 5 z^2/24 (next term below 2^-33) and one Newton step */
+EM_FN double em_recip_cos_small(double c, double z) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  double y = __builtin_fma(z, __builtin_fma(z, em_k(0x1.aaaaaaaaaaaabp-3), 0.5), 1.0);
+  double e = __builtin_fma(-c, y, 1.0);
+  return __builtin_fma(y, e, y);
+#else
+  (void)z;
+  return 1.0 / c;
 #endif
 }
 

@@ -688,21 +688,27 @@ static int compile_csbend(const eh_element *e, const EH_MAXAMP *maxamp, eh_op *o
       op->d[EH_D_BDSH + j] = dsh;
       op->d[EH_D_BDSHR + j] = dsh / rho0;
       op->d[EH_D_BDS + j] = s * kf[j];
-      op->d[EH_D_BKF + j] = kf[j];
     }
   }
   /* the branch-free common path of the kernel needs positive radii within
-   * the shared-reciprocal range, substep angles that are 0 or moderate and
-   * below 2^-5, and kick lengths that are 0 or moderate */
+   * the shared-reciprocal range, moderate substep angles below 2^-5, and kick
+   * lengths that are 0 or moderate */
   if (rho0 > 0 && rho_actual > 0 && em_recip_ok(rho0) && em_recip_ok(rho_actual) && !(op->flags & EH_F_FIELD)) {
     int fast = 1;
+    double amax = 0;
     for (int j = 0; j < nsub; j++) {
       double a = fabs(op->d[EH_D_BDSHR + j]), k = fabs(op->d[EH_D_BDS + j]);
-      if (!(a == 0 || (a >= 0x1.0p-700 && a < 0x1.0p-5)) || !(k == 0 || em_recip_ok(k)))
+      if (!(a >= 0x1.0p-300 && a < 0x1.0p-5) || !(k == 0 || em_recip_ok(k)))
         fast = 0;
+      amax = a > amax ? a : amax;
     }
-    if (fast)
+    if (fast) {
+      /* |phi| <= sqrt(zlim) (1 + 2^-52) leaves |a + phi| below 2^-5 after its rounding */
       op->flags |= EH_F_FAST;
+      op->d[EH_D_ZLIM] = sqr(0x1.0p-5 - amax) * (1 - 0x1.0p-40);
+      if (amax >= 0x1.0p-6)
+        op->flags |= EH_F_WIDE;
+    }
   }
   set_in_aperture(op, -tilt, maxamp);
   return EH_OK;

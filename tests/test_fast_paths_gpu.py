@@ -1,0 +1,83 @@
+"""The kernels' branch-free common paths at the edges of the ranges that
+select them, against the checker bit for bit."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from elegant_amd import _abi as A
+from elegant_amd import elements as E
+from oracle import oracle_ctypes as O
+from tests.helpers import assert_rows_bitwise
+from tests.test_elements_gpu import PO, assert_same_survivors, csbend_edge_rows, rows_ptr
+
+pytestmark = pytest.mark.gpu
+
+
+def near_midpoint_squares(n, rng):
+    """doubles whose square roots lie as close to a midpoint between two
+    doubles as any: N = M^2 + M + d, |d| small, with N a multiple of 2^52
+    (Hensel lifting of M^2 + M = -d modulo 2^52, d even)"""
+    out = []
+    for _ in range(n):
+        d = 2 * int(rng.integers(-64, 64))
+        m = int(rng.integers(0, 2))
+        for k in range(1, 52):
+            if (m * m + m + d) >> k & 1:
+                m += 1 << k
+        m |= 1 << 52
+        N = m * m + m + d
+        if N & ((1 << 52) - 1) == 0 and N >> 52 < 1 << 53:
+            out.append(float(N >> 52) * 2.0 ** 2)  # sqrt's exponent parity is that of 2^52 (even)
+        if len(out) >= n:
+            break
+    return np.array(out)
+
+
+@pytest.mark.parametrize("fn", ["sqrt", "quotient", "by_cosine"])
+def test_reciprocal_sequences_match_ieee(tracker, fn):
+    """sqrt with its reciprocal, quotients by it, and quotients by a cosine
+    on the narrow band: correctly rounded on 2^21 operands, the hard cases of
+    the square root among them"""
+    rng = np.random.default_rng(31)
+    n = 1 << 21
+    a = rng.uniform(1, 2, n) * np.exp2(rng.integers(-600, 600, n)) * rng.choice([-1.0, 1.0], n)
+    a[::5] = 0.0
+    if fn == "by_cosine":
+        b = rng.uniform(-1, 1, n) * np.exp2(-5.0 - 8 * rng.random(n))
+        c = O.math_eval(1, b, b, mode="emath")
+        gpu = tracker.math_probe(13, a, b)
+        cpu = a / c
+    else:
+        b = rng.uniform(1, 2, n) * np.exp2(rng.integers(-128, 128, n))
+        b[: n // 4] = 1 + rng.random(n // 4) * 2.0 ** -rng.integers(1, 60, n // 4)
+        hard = near_midpoint_squares(2000, rng)
+        b[: hard.size] = hard
+        root = np.sqrt(b)
+        q = n // 2
+        mid = root[q:] * rng.uniform(1, 2, n - q)
+        a[q:] = mid  # quotients that come near representable values
+        gpu = tracker.math_probe(11 if fn == "sqrt" else 12, a, b)
+        cpu = root if fn == "sqrt" else a / root
+    assert (gpu == cpu).all(), (fn, int((gpu != cpu).sum()))
+
+
+# substep angles just below and above 2^-6 (both squares watched from there
+# on) and 2^-5 (the general code from there on); 0.6756 of a slice is the
+# fourth-order integrator's longest substep, 0.5 the second-order one's
+@pytest.mark.parametrize("angle,order", [(0.3699, 4), (0.3701, 4), (0.7399, 4), (0.7402, 4), (0.01, 2), (0.9, 2),
+                                         (0.05, 6), (0.4, 6)])
+def test_csbend_substep_angles(tracker, angle, order):
+    b = E.CSBEND(L=1.0, ANGLE=angle, N_KICKS=16, INTEGRATION_ORDER=order).p.csbend
+    ap = A.EH_MAXAMP(0.05, 0.04, 0, 2, 2, 0)
+    r = csbend_edge_rows(1500, 41)
+    r[700::3, 3] = 0.0
+    r[701::3, 3] = -0.0
+    r[702::3, 5] = 0.0
+    r[1100::2, 1] *= 60.0  # slopes up to the band's edge on both sides
+    g, c = r.copy(), r.copy()
+    ng = tracker.track_through_csbend(g, b, PO, 3.0, ap)
+    ptr, keep = rows_ptr(c)
+    nc = O.lib("emath").or_track_through_csbend(ptr, c.shape[0], C.byref(b), PO, 3.0, C.byref(ap))
+    assert_same_survivors(r, g, ng, c, nc)
+    assert_rows_bitwise(g[:, :7], c[:, :7], "csbend angle %g order %d" % (angle, order))
