@@ -9,7 +9,7 @@ from elegant_amd import _abi as A
 from elegant_amd import elements as E
 from oracle import oracle_ctypes as O
 from tests.helpers import assert_rows_bitwise
-from tests.test_elements_gpu import PO, assert_same_survivors, csbend_edge_rows, rows_ptr
+from tests.test_elements_gpu import PO, assert_same_survivors, beam, csbend_edge_rows, rows_ptr
 
 pytestmark = pytest.mark.gpu
 
@@ -81,3 +81,37 @@ def test_csbend_substep_angles(tracker, angle, order):
     nc = O.lib("emath").or_track_through_csbend(ptr, c.shape[0], C.byref(b), PO, 3.0, C.byref(ap))
     assert_same_survivors(r, g, ng, c, nc)
     assert_rows_bitwise(g[:, :7], c[:, :7], "csbend angle %g order %d" % (angle, order))
+
+
+# strong kicks that carry slopes past the bound of the common path (2) and
+# past the end of the slope range, kicks so weak that momenta go below its
+# smallest dividend, thin elements, several orders at once, each integrator
+@pytest.mark.parametrize("make", [
+    lambda: E.KQUAD(L=0.5, K1=400.0, N_KICKS=4), lambda: E.KQUAD(L=0.5, K1=1e-300, N_KICKS=16),
+    lambda: E.KSEXT(L=0.2, K2=4e5, N_KICKS=4), lambda: E.KSEXT(L=0.3, K2=-30.0, K1=0.4, J1=0.1, N_KICKS=8),
+    lambda: E.KQUAD(L=0.4, K1=1.8, N_KICKS=5, INTEGRATION_ORDER=2, HKICK=1e-3, VKICK=-2e-3),
+    lambda: E.KOCT(L=0.1, K3=4e4, N_KICKS=12, INTEGRATION_ORDER=6, DX=1e-4, DY=-2e-4, DZ=1e-3, TILT=0.2),
+    lambda: E.KQUAD(L=0.0, K1=3.0, N_KICKS=4), lambda: E.KQUAD(L=0.4, K1=0.0, N_KICKS=4),
+])
+def test_multipole_common_path_bounds(tracker, make):
+    e = make()
+    # within the entry limits: a row beyond them is lost with the path length
+    # that the row before it reached, as the reference leaves that variable
+    r = beam(1500, 43, halo=0.0)
+    r[600:700, 1] = np.linspace(-1.0, 1.0, 100)
+    r[700:800, 3] = np.linspace(-1.0, 1.0, 100)
+    r[800:900, 0] = np.linspace(-0.05, 0.05, 100)
+    r[900:920, 5] = np.linspace(-0.9999, -0.98, 20)
+    r[920:940, 5] = 10.0 ** np.arange(20)
+    r[940:990, 0] = 10.0 ** -np.linspace(250, 320, 50)
+    r[990:1000, 1] = 10.0 ** -np.linspace(170, 190, 10)
+    r[1000:1010, :4] = 0.0
+    r[1010:1020, :4] = -0.0
+    for ap in (A.EH_MAXAMP(0.05, 0.04, 0, 2, 2, 0), None):
+        g, c = r.copy(), r.copy()
+        ng = tracker.multipole_tracking2(g, e, PO, 12.5, ap)
+        ptr, keep = rows_ptr(c)
+        nc = O.lib("emath").or_multipole_tracking2(ptr, c.shape[0], C.byref(e), PO, 12.5,
+                                                    C.byref(ap) if ap is not None else None)
+        assert ng == nc
+        assert_rows_bitwise(g[:, :7], c[:, :7], "multipole bounds")
