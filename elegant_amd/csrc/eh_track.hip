@@ -418,8 +418,13 @@ DEV int multipole_body(double &x, double &xp, double &y, double &yp, double &s, 
  *
  * One v_rsq_f64 per kick, and none per drift: den = sqrt(opd^2 - q^2) and its
  * reciprocal r come from one iteration, and with slopes q/den the drift's
- * sqrt(1 + x'^2 + y'^2) is opd r to a few ulps, with den/(2 opd) for half its
- * reciprocal, which the two residual corrections of em_sqrt_mid then round.
+ * sqrt(1 + x'^2 + y'^2) is opd r to a few ulps, with h = den/(2 opd) for half
+ * its reciprocal, which two residual corrections g + (t - g^2) h round.  With
+ * u = 2^-52 and t in [1, 4), a root that lies between g and g + u rounds
+ * wrongly only if t - g^2 = g u + m u^2 with |m| u/g below h's relative error,
+ * which is under 2 u (two products, a reciprocal and a root rounded once
+ * each); t being a double, m is even, and 0 only for t = 1 + u, whose lanes
+ * take the general code.
  * The slopes at the exit are those after the last kick, as the momenta have
  * not changed since.  A slice of four substeps of a quadrupole takes 182 VALU
  * instructions, 3 of them transcendental (276 with 16 before).  FODO ring, 10^4
@@ -429,9 +434,9 @@ DEV int multipole_body(double &x, double &xp, double &y, double &yp, double &s, 
  *  - the entry and exit limits of the integrator and the aperture at every
  *    slice hold (a NaN in the row or the momenta reaches one of them);
  *  - opd in [2^-64, 2^64], the received slopes are 0 or >= 2^-600;
- *  - opd^2 - qx^2 - qy^2 >= opd^2/4 at every conversion to slopes, tested
+ *  - opd^2 - qx^2 - qy^2 >= 0.26 opd^2 at every conversion to slopes, tested
  *    after the round trip, which moves it by a few ulps: no slope loss on
- *    either side of it, the root in range, slopes below 2;
+ *    either side of it, the roots in range, t < 4;
  *  - after the kicks qx and qy are 0 or >= 2^-700 in magnitude (binary
  *    exponent >= -699), so every dividend is 0 or within [2^-900, 2^900].
  * Arithmetic is otherwise the general code's, operation for operation. */
@@ -469,6 +474,7 @@ DEV bool multipole_fast(const particle &p, double &x, double &xp, double &y, dou
         x += xp * dsh;
         y += yp * dsh;
         const double t = 1 + sq(xp) + sq(yp), h = den * hr;
+        good = good && t != 0x1.0000000000001p+0;
         double g = opd * r;
         g = __builtin_fma(__builtin_fma(-g, g, t), h, g);
         g = __builtin_fma(__builtin_fma(-g, g, t), h, g);
@@ -503,7 +509,7 @@ DEV bool multipole_fast(const particle &p, double &x, double &xp, double &y, dou
       yp = em_div_pos(qy, den, r);
     }
   }
-  return good && emin >= -699 && dmin >= 0.25 * o2 && in_rect(x + dxa, y + dya, op) &&
+  return good && emin >= -699 && dmin >= 0.26 * o2 && in_rect(x + dxa, y + dya, op) &&
          __builtin_fabs(x) <= EH_COORD_LIMIT && __builtin_fabs(y) <= EH_COORD_LIMIT &&
          __builtin_fabs(xp) <= EH_SLOPE_LIMIT && __builtin_fabs(yp) <= EH_SLOPE_LIMIT;
 }

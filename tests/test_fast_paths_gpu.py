@@ -115,3 +115,22 @@ def test_multipole_common_path_bounds(tracker, make):
                                                     C.byref(ap) if ap is not None else None)
         assert ng == nc
         assert_rows_bitwise(g[:, :7], c[:, :7], "multipole bounds")
+
+
+@pytest.mark.parametrize("make", [lambda: E.KQUAD(L=0.3, K1=1.1, N_KICKS=4), lambda: E.KSEXT(L=0.2, K2=40.0),
+                                  lambda: E.KOCT(L=0.1, K3=200.0)])
+def test_slopes_of_a_few_ulps(tracker, make):
+    """1 + x'^2 + y'^2 of one or a few ulps above 1, where the root lies within
+    2^-55 of a midpoint between doubles: the path length decides its rounding"""
+    e = make()
+    rng = np.random.default_rng(47)
+    r = beam(60000, 47, halo=0.0)
+    r[:, 1] = rng.choice([-1.0, 1.0], 60000) * 10.0 ** rng.uniform(-8.5, -6.5, 60000)
+    r[:, 3] = rng.choice([-1.0, 1.0, 0.0], 60000) * 10.0 ** rng.uniform(-8.5, -6.5, 60000)
+    r[:, [0, 2]] *= 1e-6
+    r[::3, 5] = 0.0
+    g, c = r.copy(), r.copy()
+    ng = tracker.multipole_tracking2(g, e, PO, 12.5)
+    ptr, keep = rows_ptr(c)
+    assert ng == O.lib("emath").or_multipole_tracking2(ptr, c.shape[0], C.byref(e), PO, 12.5, None)
+    assert_rows_bitwise(g[:, :7], c[:, :7], "small slopes")
