@@ -9,11 +9,13 @@
  * per-particle arithmetic.  The kernel reads records with wave-uniform
  * indices, which the compiler turns into scalar-cache loads.
  *
- * Layout: 16 int32 + 97 doubles = 840 bytes per record.
+ * Layout: 16 int32 + 100 doubles = 864 bytes per record.
  */
 #ifndef ELEGANT_AMD_EH_PROGRAM_H
 #define ELEGANT_AMD_EH_PROGRAM_H
 
+#include <float.h>
+#include <math.h>
 #include <stdint.h>
 
 /* op codes */
@@ -95,9 +97,42 @@ typedef struct {
   double ap_xmax, ap_ymax;      /* post-element rectangle (0 = open in that plane) */
   double in_xmax, in_ymax;      /* in-element rectangle */
   double in_cs0, in_cs1;        /* cos/sin of the aperture's reverse tilt */
+  double chk_x, chk_y;          /* |x| <= chk_x and |y| <= chk_y: no check after the element fires (eh_op_bounds) */
+  double in_bx, in_by;          /* the same for the check inside it */
   /* element specific, indexed by the EH_D_* names below */
   double d[88];
 } eh_op;
+
+/* Half-widths inside which an element's checks cannot fire, so that the
+ * kernel tests one pair of compares and leaves everything else to the general
+ * code: the rectangle itself (where open, the largest finite number, as the
+ * checks after an element remove infinities; nothing is removed in a
+ * single-element call), and for a (super-)ellipse the box of 0.7 of its
+ * half-axes, as 0.7^2 + 0.7^2 < 1.  Tiny half-axes whose powers leave the
+ * normal range get no box. */
+static inline void eh_op_bounds(eh_op *op) {
+  op->in_bx = op->in_by = op->chk_x = op->chk_y = HUGE_VAL;
+  if (op->flags & EH_F_INAP) {
+    const double c = op->in_code & EH_AP_ELL ? 0.7 : 1.0;
+    if (op->in_xmax > 0)
+      op->in_bx = c * op->in_xmax;
+    if (op->in_ymax > 0)
+      op->in_by = c * op->in_ymax;
+  }
+  if (op->flags & EH_F_ALONE)
+    return;
+  op->chk_x = op->chk_y = DBL_MAX;
+  if (op->flags & EH_F_AP) {
+    const double c = op->ap_code & EH_AP_ELL ? 0.7 : 1.0;
+    if (op->ap_xmax > 0)
+      op->chk_x = fmin(c * op->ap_xmax, DBL_MAX);
+    if (op->ap_ymax > 0)
+      op->chk_y = fmin(c * op->ap_ymax, DBL_MAX);
+    if ((op->ap_code & EH_AP_ELL) &&
+        !(pow(op->ap_xmax, EH_AP_XE(op->ap_code)) >= 1e-280 && pow(op->ap_ymax, EH_AP_YE(op->ap_code)) >= 1e-280))
+      op->chk_x = op->chk_y = -1;
+  }
+}
 
 /* ---- MULT ---- */
 #define EH_D_DX 0
@@ -165,6 +200,8 @@ typedef struct {
 #define EH_D_FIELD 55     /* [<= 28]: field coefficients in the order the sums read them (eh_bend_field.h) */
 #define EH_D_FIELD_MAX 28 /* expansion order 6: K1..K4 and XKICK */
 #define EH_D_ZLIM 44      /* with EH_F_FAST: phi^2 below this keeps every |substep angle + phi| below 2^-5 */
+#define EH_D_TE1 45       /* with EH_F_FAST, unless EH_F_PSI1/2: em_tan of the edge angles */
+#define EH_D_TE2 46
 #define EH_D_ET 83        /* [5]: ETILT exit offsets of x, x', y, y', s (eh_bend_etilt.h) */
 
 /* ---- RFCA ---- */

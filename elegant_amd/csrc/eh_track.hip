@@ -31,10 +31,14 @@
 
 DEV double sq(double v) { return v * v; }
 
-/* A wave-uniform read of the element program through the constant address
- * space: the records are read-only while a kernel runs, so a uniform address
- * becomes a scalar load instead of a vector load and wait. */
-DEV double opc(const double *p) { return *(const __attribute__((address_space(4))) double *)p; }
+/* Element records and positions are read-only while a kernel runs and every
+ * lane of a wave reads the same ones: in the constant address space a uniform
+ * address is a scalar load instead of a vector load and wait. */
+#define EH_CONST const __attribute__((address_space(4)))
+typedef EH_CONST eh_op eh_opc;
+typedef EH_CONST double eh_zc;
+
+DEV double opc(EH_CONST double *p) { return *p; }
 
 struct particle {
   double x, xp, y, yp, s, dp;
@@ -76,14 +80,12 @@ DEV void aperture_loss(particle &p, double xmax, double ymax, int is_out, bool e
 
 /* the two checks that follow every element (do_tracking.c:2459-2477, 2628-2637).
  * Returns 0 if the particle survives, else stage + 1 with the row frozen.
- * In the SH instance an element with a shaped MAXAMP (ap_code != 0) takes
- * elimit_amplitudes or the open-sided limit_amplitudes instead of the
- * rectangle. */
-template <bool SH>
-DEV int post_element_checks(particle &p, const eh_op &op, const double *z) {
+ * A shaped MAXAMP (ap_code != 0) takes elimit_amplitudes or the open-sided
+ * limit_amplitudes instead of the rectangle. */
+DEV int post_element_checks(particle &p, eh_opc &op, eh_zc *z) {
   if (op.flags & EH_F_ALONE)
     return 0;
-  if (SH && (op.flags & EH_F_AP) && op.ap_code) {
+  if ((op.flags & EH_F_AP) && op.ap_code) {
     if (ap_maxamp_shaped(p.x, p.xp, p.y, p.yp, p.s, p.dp, op.ap_xmax, op.ap_ymax, op.ap_code,
                          (op.flags & EH_F_EXTRAP) != 0, opc(&z[1]), op.Po))
       return EH_STAGE_MAXAMP + 1;
@@ -207,7 +209,7 @@ DEV void drift1(particle &p, double L) {
 
 /* track_particles with a first-order matrix (matrix.c:430-458): each
  * coordinate is C[i] plus R[i][j] x[j] added from j = 5 down to 0 */
-DEV void matrix1(particle &p, const double *m) {
+DEV void matrix1(particle &p, EH_CONST double *m) {
   const double x[6] = {p.x, p.xp, p.y, p.yp, p.s, p.dp};
   double o[6];
 #pragma unroll
@@ -255,9 +257,8 @@ DEV void rotate(particle &p, double c, double s) {
 /* ---- multipoles ---- */
 
 
-/* checkMultAperture (multipole.c:1786-1833) for the closed rectangle: the
- * only shape the branch-free bodies see */
-DEV bool in_rect(double x, double y, const eh_op &op) {
+/* checkMultAperture (multipole.c:1786-1833) */
+DEV bool in_aperture(double x, double y, eh_opc &op) {
   if (!(op.flags & EH_F_INAP))
     return true;
   if (op.flags & EH_F_INTILT) {
@@ -265,27 +266,20 @@ DEV bool in_rect(double x, double y, const eh_op &op) {
     x = x0 * op.in_cs0 + y0 * op.in_cs1;
     y = -x0 * op.in_cs1 + y0 * op.in_cs0;
   }
-  if ((op.in_xmax > 0 && __builtin_fabs(x) > op.in_xmax) || (op.in_ymax > 0 && __builtin_fabs(y) > op.in_ymax))
-    return false;
-  return true;
+  if (op.in_code)
+    return ap_inside_shaped(x, y, op.in_xmax, op.in_ymax, op.in_code);
+  return !((op.in_xmax > 0 && __builtin_fabs(x) > op.in_xmax) || (op.in_ymax > 0 && __builtin_fabs(y) > op.in_ymax));
 }
 
-/* checkMultAperture for any MAXAMP shape (in_code != 0: ellipse or open
- * side).  SH: the kernel instance built for programs with such shapes; the
- * other instance keeps the closed rectangle only, so the code of the common
- * case is the same as without them. */
-template <bool SH>
-DEV bool in_aperture(double x, double y, const eh_op &op) {
-  if (!SH || !op.in_code)
-    return in_rect(x, y, op);
-  if (!(op.flags & EH_F_INAP))
-    return true;
+/* surely inside it (the host's bounds, eh_op_bounds): two compares without
+ * a branch for the common paths, whose lanes outside take the general code */
+DEV bool in_bounds(double x, double y, eh_opc &op) {
   if (op.flags & EH_F_INTILT) {
     double x0 = x, y0 = y;
     x = x0 * op.in_cs0 + y0 * op.in_cs1;
     y = -x0 * op.in_cs1 + y0 * op.in_cs0;
   }
-  return ap_inside_shaped(x, y, op.in_xmax, op.in_ymax, op.in_code);
+  return __builtin_fabs(x) <= op.in_bx && __builtin_fabs(y) <= op.in_by;
 }
 
 /* 1 + delta and its reciprocal for the IEEE quotients of emath.h, fixed for
@@ -360,16 +354,15 @@ DEV void apply_kick(double &qx, double &qy, int order, int skew, double KnL, dou
  * loads of the element record).
  * Returns 0, or the loss kind: 1 aperture (x, y hold the loss point),
  * 2 slopes (the row is left as received). */
-template <bool SH>
 DEV int multipole_body(double &x, double &xp, double &y, double &yp, double &s, double &qx, double &qy,
-                       double &dzLoss, const double dp, const bool expand, const opd_recip &o, const eh_op &op) {
+                       double &dzLoss, const double dp, const bool expand, const opd_recip &o, eh_opc &op) {
   const int nsub = op.nsub;
   const int flags = op.flags;
   const double dxa = op.d[EH_D_DX], dya = op.d[EH_D_DY];
   const bool has_drift = op.d[EH_D_DRIFT] != 0;
   const int nko = op.nkick_orders;
   for (int ik = 0; ik < op.nslices; ik++) {
-    if (!in_aperture<SH>(x + dxa, y + dya, op))
+    if (!in_aperture(x + dxa, y + dya, op))
       return 1;
     for (int step = 0; step < nsub; step++) {
       if (has_drift) {
@@ -418,13 +411,15 @@ DEV int multipole_body(double &x, double &xp, double &y, double &yp, double &s, 
  *
  * One v_rsq_f64 per kick, and none per drift: den = sqrt(opd^2 - q^2) and its
  * reciprocal r come from one iteration, and with slopes q/den the drift's
- * sqrt(1 + x'^2 + y'^2) is opd r to a few ulps, with h = den/(2 opd) for half
- * its reciprocal, which two residual corrections g + (t - g^2) h round.  With
- * u = 2^-52 and t in [1, 4), a root that lies between g and g + u rounds
- * wrongly only if t - g^2 = g u + m u^2 with |m| u/g below h's relative error,
- * which is under 2 u (two products, a reciprocal and a root rounded once
- * each); t being a double, m is even, and 0 only for t = 1 + u, whose lanes
- * take the general code.
+ * root of t = 1 + x'^2 + y'^2 is opd r and half its reciprocal den/(2 opd), both
+ * to within 3 u (u = 2^-52).  Two residual corrections g + (t - g^2) h round
+ * it.  Both estimates are taken 4 u low: then the first correction gives the
+ * root rounded, less a relative 2^-97 before rounding, so a root just below
+ * a midpoint of two doubles (t = 1 + (2k + 1) u for small slopes) goes down as
+ * it must, and the second one keeps it.  A root just above the midpoint g + u/2
+ * has t = (g + u/2)^2 + (m - 1/4) u^2 with m even as t is a double, and comes
+ * out wrong only for m <= 10: nine doubles below 4, the least of them 1.1525,
+ * which the bound on the slopes (t < 1.137) leaves out.
  * The slopes at the exit are those after the last kick, as the momenta have
  * not changed since.  A slice of four substeps of a quadrupole takes 182 VALU
  * instructions, 3 of them transcendental (276 with 16 before).  FODO ring, 10^4
@@ -434,21 +429,21 @@ DEV int multipole_body(double &x, double &xp, double &y, double &yp, double &s, 
  *  - the entry and exit limits of the integrator and the aperture at every
  *    slice hold (a NaN in the row or the momenta reaches one of them);
  *  - opd in [2^-64, 2^64], the received slopes are 0 or >= 2^-600;
- *  - opd^2 - qx^2 - qy^2 >= 0.26 opd^2 at every conversion to slopes, tested
+ *  - opd^2 - qx^2 - qy^2 >= 0.88 opd^2 at every conversion to slopes, tested
  *    after the round trip, which moves it by a few ulps: no slope loss on
- *    either side of it, the roots in range, t < 4;
+ *    either side of it, the roots in range, t < 1.137;
  *  - after the kicks qx and qy are 0 or >= 2^-700 in magnitude (binary
  *    exponent >= -699), so every dividend is 0 or within [2^-900, 2^900].
  * Arithmetic is otherwise the general code's, operation for operation. */
 template <int ORD, int NSUB>
 DEV bool multipole_fast(const particle &p, double &x, double &xp, double &y, double &yp, double &s,
-                        const opd_recip &o, const eh_op &op) {
+                        const opd_recip &o, eh_opc &op) {
   const int nsub = NSUB ? NSUB : op.nsub;
   const int flags = op.flags;
   const double dxa = op.d[EH_D_DX], dya = op.d[EH_D_DY];
   const bool has_drift = ORD > 0 || op.d[EH_D_DRIFT] != 0;
   const int nko = op.nkick_orders;
-  const double opd = o.v, o2 = sq(opd), hr = 0.5 * o.r;
+  const double opd = o.v, o2 = sq(opd), hr = (0.5 - 0x1.0p-51) * o.r;
   x = p.x;
   y = p.y;
   xp = p.xp;
@@ -466,7 +461,7 @@ DEV bool multipole_fast(const particle &p, double &x, double &xp, double &y, dou
   yp = em_div_pos(qy, den, r);
   int emin = 0;
   for (int ik = 0; ik < op.nslices; ik++) {
-    good = good && in_rect(x + dxa, y + dya, op);
+    good = good && in_bounds(x + dxa, y + dya, op);
 #pragma unroll
     for (int step = 0; step < nsub; step++) {
       if (has_drift) {
@@ -474,8 +469,7 @@ DEV bool multipole_fast(const particle &p, double &x, double &xp, double &y, dou
         x += xp * dsh;
         y += yp * dsh;
         const double t = 1 + sq(xp) + sq(yp), h = den * hr;
-        good = good && t != 0x1.0000000000001p+0;
-        double g = opd * r;
+        double g = __builtin_fma(opd, r, -0x1.0p-50);
         g = __builtin_fma(__builtin_fma(-g, g, t), h, g);
         g = __builtin_fma(__builtin_fma(-g, g, t), h, g);
         s += dsh * g;
@@ -509,7 +503,7 @@ DEV bool multipole_fast(const particle &p, double &x, double &xp, double &y, dou
       yp = em_div_pos(qy, den, r);
     }
   }
-  return good && emin >= -699 && dmin >= 0.26 * o2 && in_rect(x + dxa, y + dya, op) &&
+  return good && emin >= -699 && dmin >= 0.88 * o2 && in_bounds(x + dxa, y + dya, op) &&
          __builtin_fabs(x) <= EH_COORD_LIMIT && __builtin_fabs(y) <= EH_COORD_LIMIT &&
          __builtin_fabs(xp) <= EH_SLOPE_LIMIT && __builtin_fabs(yp) <= EH_SLOPE_LIMIT;
 }
@@ -517,7 +511,7 @@ DEV bool multipole_fast(const particle &p, double &x, double &xp, double &y, dou
 /* the integrator's entry (multipole.c:1176-1205): limits, slopes to
  * momenta and back.  Returns 0, or 2 for a slope loss (dzLoss set). */
 DEV int multipole_entry(const particle &p, double &xp, double &yp, double &qx, double &qy, double &dzLoss,
-                        const bool expand, const opd_recip &o, const eh_op &op) {
+                        const bool expand, const opd_recip &o, eh_opc &op) {
   const double dp = p.dp;
   xp = p.xp;
   yp = p.yp;
@@ -545,17 +539,16 @@ DEV int multipole_entry(const particle &p, double &xp, double &yp, double &qx, d
 /* the integrator of integrate_kick_multipole_ordn (multipole.c:1122-1410) on
  * one particle by the general code.  Returns 0, or the loss kind with the
  * row frozen. */
-template <bool SH>
-DEV int multipole_general(particle &p, const bool expand, const opd_recip &o, const eh_op &op, const double *z) {
+DEV int multipole_general(particle &p, const bool expand, const opd_recip &o, eh_opc &op, eh_zc *z) {
   const double dp = p.dp;
   double x = p.x, xp = 0, y = p.y, yp = 0, s = 0, qx = 0, qy = 0, dzLoss = 0;
   const double dxa = op.d[EH_D_DX], dya = op.d[EH_D_DY];
   /* 1: aperture (x, y written), 2: slopes (nothing written), 3: final limits */
   int lost = multipole_entry(p, xp, yp, qx, qy, dzLoss, expand, o, op);
   if (!lost)
-    lost = multipole_body<SH>(x, xp, y, yp, s, qx, qy, dzLoss, dp, expand, o, op);
+    lost = multipole_body(x, xp, y, yp, s, qx, qy, dzLoss, dp, expand, o, op);
   if (!lost) {
-    if (!in_aperture<SH>(x + dxa, y + dya, op))
+    if (!in_aperture(x + dxa, y + dya, op))
       lost = 1;
     else if (!momenta_to_slopes(xp, yp, qx, qy, dp, expand, o))
       lost = 2;
@@ -584,60 +577,70 @@ DEV int multipole_general(particle &p, const bool expand, const opd_recip &o, co
   return lost;
 }
 
-/* multipole_tracking2 per particle: entry misalignment, the integrator of
- * integrate_kick_multipole_ordn (multipole.c:1122-1410), exit misalignment.
- * Returns 0 if alive, EH_STAGE_ELEMENT + 1 if lost (row frozen). */
-template <bool SH>
-DEV int track_multipole(particle &p, const eh_op &op, const double *z) {
+/* entry and exit of multipole_tracking2: misalignment, roll and the exact
+ * drifts of KQUAD LEFFECTIVE around the body (multipole.c:1028-1030), the
+ * exit ones applied to lost rows too (multipole.c:1098-1104) */
+DEV void multipole_in(particle &p, eh_opc &op) {
   const int flags = op.flags;
-  const bool expand = (flags & EH_F_EXPAND) != 0;
   if (flags & EH_F_OFFSET)
     offset(p, op.d[EH_D_DX], op.d[EH_D_DY], op.d[EH_D_DZ]);
   if (flags & EH_F_ROTATE)
     rotate(p, op.d[EH_D_COS_IN], op.d[EH_D_SIN_IN]);
-  /* KQUAD LEFFECTIVE: an exact drift before the body (multipole.c:1028-1030) */
   if (flags & EH_F_LEND)
     exact_drift(p, op.d[EH_D_LEND]);
+}
 
-  /* the row as the integrator receives it stays in p until the end */
-  const opd_recip o = make_opd(p.dp);
-  int lost = 0;
-  bool done = false;
-  if (!expand && !(SH && op.in_code)) {
-    /* the common thick element with one normal multipole and no steering
-     * gets a body specialised to its order: the kick is straight-line code */
-    const int ord = (op.nkick_orders == 1 && !op.skew0 && !(flags & (EH_F_XKICK | EH_F_YKICK)) &&
-                     op.d[EH_D_DRIFT] != 0 && op.nsub == 4)
-                        ? op.order0
-                        : 0;
-    double x, xp, y, yp, s;
-    if (ord == 1)
-      done = multipole_fast<1, 4>(p, x, xp, y, yp, s, o, op);
-    else if (ord == 2)
-      done = multipole_fast<2, 4>(p, x, xp, y, yp, s, o, op);
-    else if (ord == 3)
-      done = multipole_fast<3, 4>(p, x, xp, y, yp, s, o, op);
-    else
-      done = multipole_fast<0, 0>(p, x, xp, y, yp, s, o, op);
-    if (done) {
-      p.x = x;
-      p.xp = xp;
-      p.y = y;
-      p.yp = yp;
-      p.s += s;
-    }
-  }
-  if (!ALL_LANES(done) && !done)
-    lost = multipole_general<SH>(p, expand, o, op, z);
-  /* the exit drift of LEFFECTIVE and the exit misalignment, applied to
-   * lost rows too (multipole.c:1098-1104) */
+DEV void multipole_out(particle &p, eh_opc &op) {
+  const int flags = op.flags;
   if (flags & EH_F_LEND)
     exact_drift(p, op.d[EH_D_LEND]);
   if (flags & EH_F_ROTATE)
     rotate(p, op.d[EH_D_COS_OUT], op.d[EH_D_SIN_OUT]);
   if (flags & EH_F_OFFSET)
     offset(p, -op.d[EH_D_DX], -op.d[EH_D_DY], -op.d[EH_D_DZ]);
+}
+
+/* multipole_tracking2 per particle by the general code.  Returns 0 if
+ * alive, EH_STAGE_ELEMENT + 1 if lost (row frozen). */
+DEV int track_multipole(particle &p, eh_opc &op, eh_zc *z) {
+  multipole_in(p, op);
+  const opd_recip o = make_opd(p.dp);
+  const int lost = multipole_general(p, (op.flags & EH_F_EXPAND) != 0, o, op, z);
+  multipole_out(p, op);
   return lost ? EH_STAGE_ELEMENT + 1 : 0;
+}
+
+/* the same on the common path; false: p is not to be used */
+DEV bool track_multipole_fast(particle &p, eh_opc &op) {
+  if (op.flags & EH_F_EXPAND)
+    return false;
+  multipole_in(p, op);
+  opd_recip o;
+  o.v = 1 + p.dp;
+  o.r = em_recip(o.v);
+  /* the common thick element with one normal multipole and no steering gets
+   * a body specialised to its order: the kick is straight-line code */
+  const int ord = (op.nkick_orders == 1 && !op.skew0 && !(op.flags & (EH_F_XKICK | EH_F_YKICK)) &&
+                   op.d[EH_D_DRIFT] != 0 && op.nsub == 4)
+                      ? op.order0
+                      : 0;
+  double x, xp, y, yp, s;
+  bool done;
+  if (ord == 1)
+    done = multipole_fast<1, 4>(p, x, xp, y, yp, s, o, op);
+  else if (ord == 2)
+    done = multipole_fast<2, 4>(p, x, xp, y, yp, s, o, op);
+  else if (ord == 3)
+    done = multipole_fast<3, 4>(p, x, xp, y, yp, s, o, op);
+  else
+    done = multipole_fast<0, 0>(p, x, xp, y, yp, s, o, op);
+  p.x = x;
+  p.xp = xp;
+  p.y = y;
+  p.yp = yp;
+  p.s += s;
+  multipole_out(p, op);
+  return done;
 }
 
 /* ---- CSBEND ---- */
@@ -651,7 +654,7 @@ DEV int track_multipole(particle &p, const eh_op &op, const double *z) {
  * coefficients in the order eh_bend_field_flatten lays them out, each term
  * (F x^i) y^j with the powers of y built by repeated multiplication as the
  * reference's table of powers is */
-DEV void bend_fields(const eh_op &op, double x, double y, double &Fx, double &Fy) {
+DEV void bend_fields(eh_opc &op, double x, double y, double &Fx, double &Fy) {
   const int n1 = op.nfield;
   double sumFx = 0, sumFy = 0, xt = 1;
   int k = 0;
@@ -676,9 +679,8 @@ DEV void bend_fields(const eh_op &op, double x, double y, double &Fx, double &Fy
   Fy = sumFy;
 }
 
-template <bool SH>
 DEV bool csbend_body(double &X, double &QX, double &Y, double &QY, const double DP, double &dist, double &dz_lost,
-                     const eh_op &op) {
+                     eh_opc &op) {
   const double rho0 = op.d[EH_D_RHO0], rhoa = op.d[EH_D_RHOA], rsgn = op.d[EH_D_RHOA_SGN];
   const double opd = 1 + DP;
   const int nsub = op.nsub;
@@ -688,7 +690,7 @@ DEV bool csbend_body(double &X, double &QX, double &Y, double &QY, const double 
   const int ok_opd = em_recip_ok(opd);
   const int ok_rho = (op.flags & EH_F_RCP) != 0;
   for (int i = 0; i < op.nslices; i++) {
-    if (!in_aperture<SH>(X, Y, op))
+    if (!in_aperture(X, Y, op))
       return true;
     for (int j = 0; j < nsub; j++) {
       double f = sq(opd) - sq(QY);
@@ -783,12 +785,10 @@ DEV bool csbend_body(double &X, double &QX, double &Y, double &QY, const double 
  *  - the aperture holds at every slice; dz_lost only matters for a loss.
  * Arithmetic is otherwise csbend_body's, operation for operation. */
 template <int NSUB, bool WIDE>
-DEV bool csbend_body_fast(double &X, double &QX, double &Y, double &QY, const double DP, double &dist,
-                          const eh_op &op) {
+DEV bool csbend_body_fast(double &X, double &QX, double &Y, double &QY, const double opd, const double r_opd,
+                          double &dist, eh_opc &op) {
   const double rho0 = op.d[EH_D_RHO0], rhoa = op.d[EH_D_RHOA];
-  const double opd = 1 + DP;
   const int nsub = NSUB ? NSUB : op.nsub;
-  const double r_opd = em_recip(opd);
   bool good = opd >= 0x1.0p-64 && opd <= 0x1.0p+64 && em_bits(QY) != 0x8000000000000000ULL &&
               (__builtin_fabs(X) + __builtin_fabs(QX)) + __builtin_fabs(QY) <= 0x1.0p+600 &&
               imin3(__builtin_amdgcn_frexp_exp(X), __builtin_amdgcn_frexp_exp(QX), __builtin_amdgcn_frexp_exp(QY)) >=
@@ -802,7 +802,7 @@ DEV bool csbend_body_fast(double &X, double &QX, double &Y, double &QY, const do
   const double f1 = em_sqrt_recip_mid(fin1, &r_f1);
   double acc = 0, zmax = 0;
   for (int i = 0; i < op.nslices; i++) {
-    good = good && in_rect(X, Y, op);
+    good = good && in_bounds(X, Y, op);
     acc += __builtin_fabs(X) + __builtin_fabs(QX);
 #pragma unroll
     for (int j = 0; j < nsub; j++) {
@@ -841,8 +841,7 @@ DEV bool csbend_body_fast(double &X, double &QX, double &Y, double &QY, const do
   return good && acc <= 0x1.0p+600 && zmax < (WIDE ? EM_SMALL_Z : op.d[EH_D_ZLIM]);
 }
 
-template <bool SH>
-DEV int track_csbend(particle &p, const eh_op &op, const double *z) {
+DEV int track_csbend(particle &p, eh_opc &op, eh_zc *z) {
   const int flags = op.flags;
   const double ct = op.d[EH_D_CT], st = op.d[EH_D_ST];
   const double rho0 = op.d[EH_D_RHO0], rhoa = op.d[EH_D_RHOA];
@@ -873,29 +872,12 @@ DEV int track_csbend(particle &p, const eh_op &op, const double *z) {
     QX = xp * f;
     QY = yp * f;
   }
-  /* integrate_csbend_ordn (csbend.c:1434-1693), Fx = 0, Fy = 1 */
+  /* integrate_csbend_ordn (csbend.c:1434-1693) */
   double dist = 0, dz_lost = 0;
-  bool lost = false, done = false;
-  if ((flags & EH_F_FAST) && !(SH && op.in_code)) {
-    const double X0 = X, QX0 = QX, Y0 = Y, QY0 = QY;
-    /* the 4th-order integrator's four substeps of a slice unrolled (NSUB =
-     * 4): the substep coefficients load once per slice and the scheduler
-     * overlaps neighbouring substeps */
-    done = op.nsub == 4 && !(flags & EH_F_WIDE) ? csbend_body_fast<4, false>(X, QX, Y, QY, DP, dist, op)
-                                                : csbend_body_fast<0, true>(X, QX, Y, QY, DP, dist, op);
-    if (!ALL_LANES(done) && !done) {
-      X = X0;
-      QX = QX0;
-      Y = Y0;
-      QY = QY0;
-      dist = 0;
-    }
-  }
-  if (!ALL_LANES(done) && !done)
-    lost = csbend_body<SH>(X, QX, Y, QY, DP, dist, dz_lost, op);
+  bool lost = csbend_body(X, QX, Y, QY, DP, dist, dz_lost, op);
   if (!lost) {
     dz_lost = op.d[EH_D_NS];
-    if (!in_aperture<SH>(X, Y, op))
+    if (!in_aperture(X, Y, op))
       lost = true;
     else
       S += dist;
@@ -959,6 +941,106 @@ DEV int track_csbend(particle &p, const eh_op &op, const double *z) {
   return 0;
 }
 
+/* tan of a fringe field's edge angle, which depends on the particle */
+static __device__ __attribute__((noinline)) double edge_tan(double a) { return em_tan(a); }
+
+/* track_through_csbend on the common path: the general code's operations
+ * with the unscaled quotients and roots; false: p is not to be used.  Beside
+ * csbend_body_fast's conditions the slopes, the path and the momentum are
+ * moderate, and the host has checked the edges (EH_F_FAST).  1 + delta, the
+ * edges' radius and the velocity are the same at both ends (nothing changes
+ * delta here), so each has one reciprocal. */
+DEV bool track_csbend_fast(particle &p, eh_opc &op) {
+  const int flags = op.flags;
+  if (!(flags & EH_F_FAST))
+    return false;
+  const double ct = op.d[EH_D_CT], st = op.d[EH_D_ST];
+  const double rhoa = op.d[EH_D_RHOA], dzi = op.d[EH_D_DZI], dzf = op.d[EH_D_DZF];
+  const double dp = p.dp, opd = 1 + dp, r_opd = em_recip(opd);
+  bool good = __builtin_fabs(p.xp) + __builtin_fabs(p.yp) <= 0x1.0p+60 && __builtin_fabs(p.s) <= 0x1.0p+500 &&
+              __builtin_amdgcn_frexp_exp(p.s) >= -500;
+  p.s += dzi != 0 ? dzi * em_sqrt_mid(1 + sq(p.xp) + sq(p.yp)) : dzi;
+  p.x = p.x + op.d[EH_D_DXI] + dzi * p.xp;
+  p.y = p.y + op.d[EH_D_DYI] + dzi * p.yp;
+  double x = p.x * ct + p.y * st;
+  double y = -p.x * st + p.y * ct;
+  double xp = p.xp * ct + p.yp * st;
+  double yp = -p.xp * st + p.yp * ct;
+  double rho = 1.0, r_rho = 1.0;
+  if (flags & (EH_F_EDGE1 | EH_F_EDGE2)) {
+    rho = opd * rhoa;
+    r_rho = em_recip(rho);
+    good = good && rho >= 0x1.0p-64 && rho <= 0x1.0p+64;
+  }
+  if (flags & EH_F_EDGE1) {
+    double delta_xp = em_div_pos(op.d[EH_D_TANE1], rho, r_rho) * x;
+    if ((flags & EH_F_KLIM1) && __builtin_fabs(delta_xp) > op.d[EH_D_KLIM1])
+      delta_xp = (delta_xp > 0 ? 1 : -1) * op.d[EH_D_KLIM1];
+    xp += delta_xp;
+    double te = op.d[EH_D_TE1];
+    if (flags & EH_F_PSI1)
+      te = edge_tan(op.d[EH_D_E1] - em_div_pos(op.d[EH_D_PSI1], opd, r_opd));
+    yp -= em_div_pos(te, rho, r_rho) * y;
+  }
+  double X = x, Y = y, dist = 0, r, g = em_sqrt_recip_mid(1 + sq(xp) + sq(yp), &r);
+  const double f = em_div_pos(opd, g, r);
+  double QX = xp * f, QY = yp * f;
+  good = good && __builtin_fabs(xp) + __builtin_fabs(yp) <= 0x1.0p+60;
+  /* the 4th-order integrator's four substeps of a slice unrolled (NSUB = 4):
+   * the scheduler overlaps neighbouring substeps */
+  if (op.nsub == 4 && !(flags & EH_F_WIDE))
+    good = csbend_body_fast<4, false>(X, QX, Y, QY, opd, r_opd, dist, op) && good;
+  else
+    good = csbend_body_fast<0, true>(X, QX, Y, QY, opd, r_opd, dist, op) && good;
+  good = good && in_bounds(X, Y, op);
+  {
+    const double den2 = sq(opd) - sq(QX) - sq(QY);
+    good = good && den2 >= 0x1.0p-128;
+    g = em_sqrt_recip_mid(den2, &r);
+    const double q = em_div_pos(1.0, g, r);
+    QX *= q;
+    QY *= q;
+  }
+  /* velocity rescaling of s: beta1 = beta0 */
+  const double p0 = op.Po * opd;
+  good = good && p0 >= 0x1.0p-60 && p0 <= 0x1.0p+60;
+  g = em_sqrt_recip_mid(sq(p0) + 1, &r);
+  const double beta0 = em_div_pos(p0, g, r);
+  const double s = em_div_pos(beta0 * p.s, beta0, em_recip(beta0)) + dist;
+  x = X;
+  xp = QX;
+  y = Y;
+  yp = QY;
+  if (flags & EH_F_EDGE2) {
+    double delta_xp = em_div_pos(op.d[EH_D_TANE2], rho, r_rho) * x;
+    if ((flags & EH_F_KLIM2) && __builtin_fabs(delta_xp) > op.d[EH_D_KLIM2])
+      delta_xp = (delta_xp > 0 ? 1 : -1) * op.d[EH_D_KLIM2];
+    xp += delta_xp;
+    double te = op.d[EH_D_TE2];
+    if (flags & EH_F_PSI2)
+      te = edge_tan(op.d[EH_D_E2] - em_div_pos(op.d[EH_D_PSI2], opd, r_opd));
+    yp -= em_div_pos(te, rho, r_rho) * y;
+  }
+  double o0 = 0.0, o1 = 0.0, o2 = 0.0, o3 = 0.0, o4 = 0.0;
+  if (flags & EH_F_ETILT) {
+    o0 = op.d[EH_D_ET];
+    o1 = op.d[EH_D_ET + 1];
+    o2 = op.d[EH_D_ET + 2];
+    o3 = op.d[EH_D_ET + 3];
+    o4 = op.d[EH_D_ET + 4];
+  }
+  p.x = x * ct - y * st + o0;
+  p.y = x * st + y * ct + o2;
+  p.xp = xp * ct - yp * st + o1;
+  p.yp = xp * st + yp * ct + o3;
+  p.s = s + o4;
+  p.x += op.d[EH_D_DXF] + dzf * p.xp;
+  p.y += op.d[EH_D_DYF] + dzf * p.yp;
+  good = good && __builtin_fabs(p.xp) + __builtin_fabs(p.yp) <= 0x1.0p+60;
+  p.s += dzf != 0 ? dzf * em_sqrt_mid(1 + sq(p.xp) + sq(p.yp)) : dzf;
+  return good;
+}
+
 /* ---- RFCA ---- */
 
 /* add_to_particle_energy (simple_rfca.c:987-1007) */
@@ -980,7 +1062,7 @@ DEV void add_energy(particle &p, double tof, double Po, double dgamma) {
 
 /* trackRfCavityWithWakes for one particle, forward tracking, no wakes
  * (simple_rfca.c:557-984) followed by removeInvalidParticles (:975) */
-DEV int track_rfca(particle &p, const eh_op &op, const double *z) {
+DEV int track_rfca(particle &p, eh_opc &op, eh_zc *z) {
   const double Po = op.Po;
   const double volt = op.d[EH_D_VOLT], omega = op.d[EH_D_OMEGA], phase = op.d[EH_D_PHASE];
   const double length = op.d[EH_D_LENGTH], dtLight = op.d[EH_D_DTLIGHT];
@@ -1095,7 +1177,7 @@ DEV int track_rfca(particle &p, const eh_op &op, const double *z) {
 
 /* offset_beam (do_tracking.c:3243-3306) for one particle, on pass ON_PASS
  * or, with -1, every pass (do_tracking.c:1818-1822) */
-DEV void track_malign(particle &p, const eh_op &op, int64_t pass) {
+DEV void track_malign(particle &p, eh_opc &op, int64_t pass) {
   const int32_t on_pass = op.nkicks_rf;
   if (!(on_pass == -1 || on_pass == pass))
     return;
@@ -1132,7 +1214,7 @@ DEV void track_malign(particle &p, const eh_op &op, int64_t pass) {
  * lost outside the half-widths (an open side may spare it) or with a
  * non-finite x or y, INVERT swapping the verdict; the loss at the
  * element's start */
-DEV int track_rcol_in(particle &p, const eh_op &op, const double *z) {
+DEV int track_rcol_in(particle &p, eh_opc &op, eh_zc *z) {
   const double xsize = op.d[EH_D_RC_XMAX], ysize = op.d[EH_D_RC_YMAX];
   const double dx = p.x - op.d[EH_D_RC_DX], dy = p.y - op.d[EH_D_RC_DY];
   const int open = op.order1;
@@ -1154,7 +1236,7 @@ DEV int track_rcol_in(particle &p, const eh_op &op, const double *z) {
 /* the collimator's drift and exit check: a particle outside at the exit
  * is lost where its straight orbit met the jaw (no open side), a
  * non-finite exit position at the exit; survivors take the drift */
-DEV int track_rcol_body(particle &p, const eh_op &op, const double *z) {
+DEV int track_rcol_body(particle &p, eh_opc &op, eh_zc *z) {
   const double length = op.d[EH_D_RC_LEN];
   const double xsize = op.d[EH_D_RC_XMAX], ysize = op.d[EH_D_RC_YMAX];
   const double xc = op.d[EH_D_RC_DX], yc = op.d[EH_D_RC_DY];
@@ -1197,12 +1279,81 @@ DEV int track_rcol_body(particle &p, const eh_op &op, const double *z) {
   return 0;
 }
 
+/* The general code, out of line: it decides for the lanes that a common path
+ * hands on, and for element kinds met once a turn or less.  Inlined, its
+ * polynomials and branches took the registers of the common paths (11,500
+ * instructions with scalar values spilled to vector lanes around every
+ * element; 4,600 now).  FODO ring, 10^4 particles, 64 turns: 54.9 -> 44.9 ms;
+ * storage ring, 10^6, 10 turns: 258 -> 242 ms. */
+struct step_out {
+  particle p;
+  int lost;
+};
+#define SLOW static __device__ __attribute__((noinline)) step_out
+
+/* a pointer that every lane holds alike, back in scalar registers */
+template <class T> DEV T *uniform(T *p) {
+  const uint64_t u = (uint64_t)p;
+  return (T *)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(u >> 32)) << 32) |
+               (uint32_t)__builtin_amdgcn_readfirstlane((int)u));
+}
+
+SLOW slow_multipole(particle p, eh_opc *op, eh_zc *z) {
+  step_out o;
+  o.lost = track_multipole(p, *uniform(op), uniform(z));
+  o.p = p;
+  return o;
+}
+
+SLOW slow_csbend(particle p, eh_opc *op, eh_zc *z) {
+  step_out o;
+  o.lost = track_csbend(p, *uniform(op), uniform(z));
+  o.p = p;
+  return o;
+}
+
+SLOW slow_rfca(particle p, eh_opc *op, eh_zc *z) {
+  step_out o;
+  o.lost = track_rfca(p, *uniform(op), uniform(z));
+  o.p = p;
+  return o;
+}
+
+/* the rare kinds: MALIGN, RCOL */
+SLOW slow_other(particle p, eh_opc *op, eh_zc *z, int64_t pass) {
+  step_out o;
+  eh_opc &u = *uniform(op);
+  eh_zc *zu = uniform(z);
+  o.lost = 0;
+  if (u.op == EH_OP_MALIGN)
+    track_malign(p, u, pass);
+  else
+    o.lost = u.op == EH_OP_RCOL_IN ? track_rcol_in(p, u, zu) : track_rcol_body(p, u, zu);
+  o.p = p;
+  return o;
+}
+
+SLOW slow_drift2(particle p, double L, double hL) {
+  step_out o;
+  drift2_exact(p, L, hL);
+  o.lost = 0;
+  o.p = p;
+  return o;
+}
+
+SLOW slow_checks(particle p, eh_opc *op, eh_zc *z) {
+  step_out o;
+  o.lost = post_element_checks(p, *uniform(op), uniform(z));
+  o.p = p;
+  return o;
+}
+
 /* One element on one particle.  z points at the element's (z_start, z_end),
  * which only the loss paths read: in the element record itself, or in the
  * position table of a program whose repeated cells share one record. */
-template <bool SH>
-DEV int run_op(particle &p, const eh_op &op, const double *z, int64_t pass) {
-  int lost = 0;
+DEV int run_op(particle &p, eh_opc &op, eh_zc *z, int64_t pass) {
+  step_out o;
+  o.lost = 0;
   /* elements before the recirculation point act on pass 0 only */
   if ((op.flags & EH_F_FIRSTPASS) && pass != 0)
     return 0;
@@ -1211,7 +1362,7 @@ DEV int run_op(particle &p, const eh_op &op, const double *z, int64_t pass) {
     if ((op.flags & EH_F_DFAST) && ALL_LANES(drift2_ok(p)))
       drift2(p, op.d[0], op.d[1]);
     else
-      drift2_exact(p, op.d[0], op.d[1]);
+      p = slow_drift2(p, op.d[0], op.d[1]).p;
     break;
   case EH_OP_DRIFT1:
     drift1(p, op.d[0]);
@@ -1222,23 +1373,41 @@ DEV int run_op(particle &p, const eh_op &op, const double *z, int64_t pass) {
   case EH_OP_MATRIX1:
     matrix1(p, op.d);
     break;
-  case EH_OP_MULT:
-    lost = track_multipole<SH>(p, op, z);
+  case EH_OP_MULT: {
+    particle q = p;
+    const bool done = track_multipole_fast(q, op);
+    if (ALL_LANES(done))
+      p = q;
+    else if (done)
+      p = q;
+    else {
+      o = slow_multipole(p, &op, z);
+      p = o.p;
+    }
     break;
-  case EH_OP_CSBEND:
-    lost = track_csbend<SH>(p, op, z);
+  }
+  case EH_OP_CSBEND: {
+    particle q = p;
+    const bool done = track_csbend_fast(q, op);
+    if (ALL_LANES(done))
+      p = q;
+    else if (done)
+      p = q;
+    else {
+      o = slow_csbend(p, &op, z);
+      p = o.p;
+    }
     break;
+  }
   case EH_OP_RFCA:
-    lost = track_rfca(p, op, z);
+    o = slow_rfca(p, &op, z);
+    p = o.p;
     break;
   case EH_OP_MALIGN:
-    track_malign(p, op, pass);
-    break;
   case EH_OP_RCOL_IN:
-    lost = track_rcol_in(p, op, z);
-    break;
   case EH_OP_RCOL_BODY:
-    lost = track_rcol_body(p, op, z);
+    o = slow_other(p, &op, z, pass);
+    p = o.p;
     break;
   case EH_OP_RFCA_DRIFT:
     /* VOLT=0: a drift when the cavity has length, else nothing (simple_rfca.c:389-402) */
@@ -1251,25 +1420,26 @@ DEV int run_op(particle &p, const eh_op &op, const double *z, int64_t pass) {
   default:
     break;
   }
-  if (lost)
-    return lost;
-  return post_element_checks<SH>(p, op, z);
+  if (o.lost)
+    return o.lost;
+  /* inside these bounds none of the checks after the element can fire */
+  const bool inside = __builtin_fabs(p.x) <= op.chk_x && __builtin_fabs(p.y) <= op.chk_y;
+  if (!ALL_LANES(inside) && !inside) {
+    o = slow_checks(p, &op, z);
+    p = o.p;
+  }
+  return o.lost;
 }
 
-/* Four waves per SIMD (up to 128 VGPRs): the branch-free bend body needs
- * about 111 registers in this kernel; squeezing it into five or six waves
- * spills to scratch or parks state in LDS, and measured no faster on the
- * storage ring (29.0-29.3 M against 29.4 M particle-turns/s).
- * SH: built with the elliptical / open-sided MAXAMP checks; launched only for
- * programs that have such an aperture, so the rectangle-only instance keeps
- * the registers and schedule of the common case.
+/* Four waves per SIMD (up to 128 VGPRs).  The bound reaches the general code's
+ * functions only if every kernel that calls them states it: the batch kernel
+ * does too (without it they took 148 VGPRs, three waves).
  * The beamline of nflat elements arrives as runs (eh_run): a body of
  * records executed reps times in a row, so a ring of identical cells keeps
  * one cell's records hot in the scalar cache instead of streaming every
  * element's record through it each pass.  Loss codes and op_first/op_last
  * count positions in the flat beamline; zpos holds (z_start, z_end) for
  * each of them. */
-template <bool SH>
 __global__ void __launch_bounds__(256, 4) eh_track_kernel(eh_state st, const eh_op *__restrict__ ops,
                                                        const eh_run *__restrict__ runs, int32_t nruns,
                                                        const double *__restrict__ zpos, int64_t pass0,
@@ -1287,6 +1457,8 @@ __global__ void __launch_bounds__(256, 4) eh_track_kernel(eh_state st, const eh_
   p.yp = st.yp[i];
   p.s = st.s[i];
   p.dp = st.dp[i];
+  eh_opc *cops = (eh_opc *)ops;
+  eh_zc *zs = (eh_zc *)zpos;
   int lost = 0, lost_op = 0;
   int64_t lost_pass = 0;
   for (int32_t ip = 0; ip < npasses && !lost; ip++) {
@@ -1304,7 +1476,7 @@ __global__ void __launch_bounds__(256, 4) eh_track_kernel(eh_state st, const eh_
       const int32_t f1 = fe < oe ? fe : oe;
       int32_t k = (f - fs) % len;
       for (; f < f1; f++) {
-        lost = run_op<SH>(p, ops[first + k], zpos + 2 * f, pass0 + ip);
+        lost = run_op(p, cops[first + k], zs + 2 * f, pass0 + ip);
         if (lost) {
           lost_op = f;
           lost_pass = pass0 + ip;
@@ -1331,9 +1503,9 @@ __global__ void __launch_bounds__(256, 4) eh_track_kernel(eh_state st, const eh_
  * of its particles) from a queue until it is empty; every lane tracks PPL
  * particles of the chunk through the variant's program.  The chunk queue is
  * ordered by variant so that workgroups resident at the same time share a few
- * programs in L2.  SH as for eh_track_kernel. */
-template <int PPL, bool SH>
-__global__ void __launch_bounds__(256) eh_batch_kernel(eh_state st, const eh_op *__restrict__ ops,
+ * programs in L2. */
+template <int PPL>
+__global__ void __launch_bounds__(256, 4) eh_batch_kernel(eh_state st, const eh_op *__restrict__ ops,
                                                        const eh_vdesc *__restrict__ vars,
                                                        const eh_chunk *__restrict__ chunks,
                                                        const int32_t *__restrict__ nchunks_p,
@@ -1351,7 +1523,7 @@ __global__ void __launch_bounds__(256) eh_batch_kernel(eh_state st, const eh_op 
       return;
     const eh_chunk ch = chunks[c];
     const eh_vdesc vd = vars[ch.variant];
-    const eh_op *vops = ops + vd.op_offset;
+    eh_opc *vops = (eh_opc *)ops + vd.op_offset;
     const int32_t nops = vd.nops;
     particle p[PPL];
     int lost[PPL], lost_op[PPL];
@@ -1381,11 +1553,11 @@ __global__ void __launch_bounds__(256) eh_batch_kernel(eh_state st, const eh_op 
       if (!any)
         break;
       for (int32_t io = 0; io < nops; io++) {
-        const eh_op &op = vops[io];
+        eh_opc &op = vops[io];
         for (int k = 0; k < PPL; k++) {
           if (!live[k])
             continue;
-          int l = run_op<SH>(p[k], op, &op.z_start, pass0 + ip);
+          int l = run_op(p[k], op, &op.z_start, pass0 + ip);
           if (l) {
             live[k] = false;
             lost[k] = l;
@@ -1584,8 +1756,6 @@ int ehd_get_sdp(ehd_dev *d, double *s, double *dp, int32_t *loss_pass, int64_t n
   return ehd_get_state(d, NULL, NULL, NULL, NULL, s, dp, loss_pass, NULL, n);
 }
 
-static int tops_shaped(const eh_op *op) { return op->ap_code || op->in_code; }
-
 int ehd_put_ops(ehd_dev *d, const eh_op *ops, int32_t nops) {
   HIPCHK(d, hipSetDevice(d->device));
   if (nops > d->ops_cap) {
@@ -1599,12 +1769,6 @@ int ehd_put_ops(ehd_dev *d, const eh_op *ops, int32_t nops) {
     HIPCHK(d, hipMemcpyAsync(d->ops, ops, sizeof(eh_op) * nops, hipMemcpyHostToDevice, d->stream));
   HIPCHK(d, hipStreamSynchronize(d->stream));
   d->nops = nops;
-  /* programs with an elliptical or open-sided MAXAMP run on the kernel
-   * instance that evaluates those shapes */
-  d->shaped = 0;
-  for (int32_t k = 0; k < nops; k++)
-    if (tops_shaped(&ops[k]))
-      d->shaped = 1;
   return EH_OK;
 }
 
@@ -1672,10 +1836,6 @@ static int upload_program(ehd_dev *d) {
   }
   d->nruns = nr;
   d->ntops = nb;
-  d->tshaped = 0;
-  for (int32_t f = 0; f < n; f++)
-    if (tops_shaped(&d->host_prog[f]))
-      d->tshaped = 1;
   return EH_OK;
 }
 
@@ -1692,6 +1852,8 @@ int ehd_put_program(ehd_dev *d, const eh_op *ops, int32_t nops) {
   }
   if (nops > 0)
     memcpy(d->host_prog, ops, sizeof(eh_op) * (size_t)nops);
+  for (int32_t f = 0; f < nops; f++)
+    eh_op_bounds(&d->host_prog[f]);
   d->nflat = nops;
   return upload_program(d);
 }
@@ -1701,6 +1863,7 @@ int ehd_patch_op(ehd_dev *d, int32_t index, const eh_op *op) {
     return EH_ERR_INVALID;
   HIPCHK(d, hipSetDevice(d->device));
   d->host_prog[index] = *op;
+  eh_op_bounds(&d->host_prog[index]);
   return upload_program(d);
 }
 
@@ -1743,12 +1906,8 @@ int ehd_track(ehd_dev *d, int64_t pass0, int32_t npasses, int32_t op_first, int3
   }
   const int64_t grid = (d->n + block - 1) / block;
   HIPCHK(d, hipEventRecord(d->ev0, d->stream));
-  if (d->tshaped)
-    hipLaunchKernelGGL(eh_track_kernel<true>, dim3((unsigned)grid), dim3(block), 0, d->stream, st, d->tops, d->runs,
-                       d->nruns, d->zpos, pass0, npasses, op_first, op_last, d->nflat);
-  else
-    hipLaunchKernelGGL(eh_track_kernel<false>, dim3((unsigned)grid), dim3(block), 0, d->stream, st, d->tops, d->runs,
-                       d->nruns, d->zpos, pass0, npasses, op_first, op_last, d->nflat);
+  hipLaunchKernelGGL(eh_track_kernel, dim3((unsigned)grid), dim3(block), 0, d->stream, st, d->tops, d->runs, d->nruns,
+                     d->zpos, pass0, npasses, op_first, op_last, d->nflat);
   HIPCHK(d, hipGetLastError());
   HIPCHK(d, hipEventRecord(d->ev1, d->stream));
   HIPCHK(d, hipEventSynchronize(d->ev1));
@@ -2082,18 +2241,12 @@ static int batch_launch(ehd_dev *d, eh_state st, int64_t pass0, int32_t npasses,
                         int grid) {
   hipLaunchKernelGGL(eh_queue_reset, dim3(1), dim3(1), 0, d->stream, d->queue);
   const int32_t *perm = d->use_perm ? d->perm : (const int32_t *)NULL;
-  if (ppl == 2 && d->shaped)
-    hipLaunchKernelGGL((eh_batch_kernel<2, true>), dim3(grid), dim3(block), 0, d->stream, st, d->ops, d->vdesc,
-                       d->chunks, d->dev_nchunks, perm, pass0, npasses, d->queue);
-  else if (ppl == 2)
-    hipLaunchKernelGGL((eh_batch_kernel<2, false>), dim3(grid), dim3(block), 0, d->stream, st, d->ops, d->vdesc,
-                       d->chunks, d->dev_nchunks, perm, pass0, npasses, d->queue);
-  else if (d->shaped)
-    hipLaunchKernelGGL((eh_batch_kernel<1, true>), dim3(grid), dim3(block), 0, d->stream, st, d->ops, d->vdesc,
-                       d->chunks, d->dev_nchunks, perm, pass0, npasses, d->queue);
+  if (ppl == 2)
+    hipLaunchKernelGGL(eh_batch_kernel<2>, dim3(grid), dim3(block), 0, d->stream, st, d->ops, d->vdesc, d->chunks,
+                       d->dev_nchunks, perm, pass0, npasses, d->queue);
   else
-    hipLaunchKernelGGL((eh_batch_kernel<1, false>), dim3(grid), dim3(block), 0, d->stream, st, d->ops, d->vdesc,
-                       d->chunks, d->dev_nchunks, perm, pass0, npasses, d->queue);
+    hipLaunchKernelGGL(eh_batch_kernel<1>, dim3(grid), dim3(block), 0, d->stream, st, d->ops, d->vdesc, d->chunks,
+                       d->dev_nchunks, perm, pass0, npasses, d->queue);
   return EH_OK;
 }
 
@@ -2123,14 +2276,10 @@ int ehd_batch_track(ehd_dev *d, int64_t pass0, int32_t npasses, int32_t passes_p
   st.loss_code = d->loss_code;
   st.n = d->n;
   int per_cu = 0;
-  if (ppl == 2 && d->shaped)
-    HIPCHK(d, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, eh_batch_kernel<2, true>, block, 0));
-  else if (ppl == 2)
-    HIPCHK(d, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, eh_batch_kernel<2, false>, block, 0));
-  else if (d->shaped)
-    HIPCHK(d, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, eh_batch_kernel<1, true>, block, 0));
+  if (ppl == 2)
+    HIPCHK(d, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, eh_batch_kernel<2>, block, 0));
   else
-    HIPCHK(d, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, eh_batch_kernel<1, false>, block, 0));
+    HIPCHK(d, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, eh_batch_kernel<1>, block, 0));
   if (per_cu < 1)
     per_cu = 1;
   int grid = d->num_cu * per_cu;

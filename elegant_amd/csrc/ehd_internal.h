@@ -40,7 +40,6 @@ struct ehd_dev {
   eh_run *runs;
   double *zpos;        /* (z_start, z_end) of each flat position */
   int32_t ntops, nruns, tops_cap, runs_cap, zpos_cap;
-  int tshaped;         /* the tracking program has an elliptical or open-sided MAXAMP */
   int32_t block;
   unsigned long long *counter;
   double track_ms, coll_ms;
@@ -64,7 +63,6 @@ struct ehd_dev {
   int32_t *tile_sum;    /* device compaction: tile prefix sums, then per-variant info */
   int64_t tile_cap;
   int32_t vinfo_cap;
-  int shaped; /* the loaded program has an elliptical or open-sided MAXAMP */
   double *snap[6];
   int32_t *snap_lp, *snap_lc;
   int64_t snap_cap;

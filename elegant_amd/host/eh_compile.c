@@ -702,7 +702,18 @@ static int compile_csbend(const eh_element *e, const EH_MAXAMP *maxamp, eh_op *o
         fast = 0;
       amax = a > amax ? a : amax;
     }
+    /* the edges' quotients: tan E and the fringe angle 0 or moderate */
+    const double e[4] = {op->d[EH_D_TANE1], op->d[EH_D_TANE2], psi1, psi2};
+    for (int j = 0; j < 4; j++)
+      if (!(e[j] == 0 || (fabs(e[j]) >= 0x1.0p-500 && fabs(e[j]) <= 0x1.0p+500)))
+        fast = 0;
     if (fast) {
+      if (psi1)
+        op->flags |= EH_F_PSI1;
+      if (psi2)
+        op->flags |= EH_F_PSI2;
+      op->d[EH_D_TE1] = em_tan(e1 - psi1);
+      op->d[EH_D_TE2] = em_tan(e2 - psi2);
       /* |phi| <= sqrt(zlim) (1 + 2^-52) leaves |a + phi| below 2^-5 after its rounding */
       op->flags |= EH_F_FAST;
       op->d[EH_D_ZLIM] = sqr(0x1.0p-5 - amax) * (1 - 0x1.0p-40);

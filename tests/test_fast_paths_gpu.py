@@ -134,3 +134,26 @@ def test_slopes_of_a_few_ulps(tracker, make):
     ptr, keep = rows_ptr(c)
     assert ng == O.lib("emath").or_multipole_tracking2(ptr, c.shape[0], C.byref(e), PO, 12.5, None)
     assert_rows_bitwise(g[:, :7], c[:, :7], "small slopes")
+
+
+# edges, fringe angles (a tangent per particle), kick limits, error tilt,
+# misalignment with DZ, a bore along the aperture's edge
+@pytest.mark.parametrize("kw", [
+    dict(E1=0.03, E2=-0.02), dict(E1=0.02, E2=0.03, HGAP=0.02), dict(E1=0.02, E2=0.03, HGAP=0.02, FINT=0.4, FSE=2e-3),
+    dict(E1=0.05, E2=0.05, EDGE1_KICK_LIMIT=1e-5, EDGE2_KICK_LIMIT=2e-5), dict(EDGE1_EFFECTS=0, EDGE2_EFFECTS=0),
+    dict(E1=0.01, ETILT=1e-3, TILT=0.3, DX=1e-4, DY=-2e-4, DZ=3e-4), dict(TILT=1.5707963267948966),
+])
+def test_csbend_whole_element_common_path(tracker, kw):
+    b = E.CSBEND(L=1.0, ANGLE=0.08, N_KICKS=16, **kw).p.csbend
+    r = csbend_edge_rows(1500, 45)
+    r[800:850, 0] = np.linspace(-0.0062, 0.0062, 50)
+    r[850:900, 4] = 10.0 ** -np.linspace(100, 300, 50)
+    r[900:950, 5] = np.linspace(-1.0, 1.0, 50)
+    for ap in (A.EH_MAXAMP(0.006, 0.004, 0, 2, 2, 0), A.EH_MAXAMP(0.006, 0.004, 1, 2, 4, 0),
+               A.EH_MAXAMP(0.006, 0.004, 0, 2, 2, A.EH_OPEN_PLUS_X)):
+        g, c = r.copy(), r.copy()
+        ng = tracker.track_through_csbend(g, b, PO, 3.0, ap)
+        ptr, keep = rows_ptr(c)
+        nc = O.lib("emath").or_track_through_csbend(ptr, c.shape[0], C.byref(b), PO, 3.0, C.byref(ap))
+        assert_same_survivors(r, g, ng, c, nc)
+        assert_rows_bitwise(g[:, :7], c[:, :7], "csbend whole element")
