@@ -9,7 +9,11 @@
  * per-particle arithmetic.  The kernel reads records with wave-uniform
  * indices, which the compiler turns into scalar-cache loads.
  *
- * Layout: 16 int32 + 100 doubles = 864 bytes per record.
+ * Layout: 18 lines of 64 bytes (the scalar cache's line).  The first is the
+ * header, the next two hold what the common path of a multipole, a drift or
+ * a bend's substeps reads, the two after them the rest of a bend's common path
+ * (eh_op_finish copies both from the general fields); everything else is
+ * read by the general code only.
  */
 #ifndef ELEGANT_AMD_EH_PROGRAM_H
 #define ELEGANT_AMD_EH_PROGRAM_H
@@ -87,52 +91,57 @@
 #define EH_STAGE_NAN 2      /* limit_amplitudes(DBL_MAX): NaN/Inf cull */
 
 typedef struct {
-  int32_t op, elem, flags, nslices;
-  int32_t nsub, nkick_orders, order0, order1;
-  int32_t order2, skew0, skew1, skew2;
-  int32_t nkicks_rf, ap_code, in_code; /* ap_code, in_code: EH_AP_* shape of the two checks, 0 = rectangle */
-  int32_t nfield;                       /* CSBEND: expansion order + 1 of the field sums (EH_F_FIELD) */
+  int32_t op, flags, nslices;   /* these four the kernel reads an element ahead */
+  int32_t nfield;               /* CSBEND: expansion order + 1 of the field sums (EH_F_FIELD); MULT: the order whose
+                                   body the common path takes, 0 the generic one */
+  int32_t elem, nsub, nkick_orders, order0;
+  int32_t order1, order2, skew0, skew1;
+  int32_t skew2, nkicks_rf, ap_code, in_code; /* ap_code, in_code: EH_AP_* shape of the two checks, 0 = rectangle */
+  double hot[16];               /* EH_H_* */
+  double bend[16];              /* EH_B_* */
   /* common */
   double z_start, z_end, Po;
   double ap_xmax, ap_ymax;      /* post-element rectangle (0 = open in that plane) */
   double in_xmax, in_ymax;      /* in-element rectangle */
   double in_cs0, in_cs1;        /* cos/sin of the aperture's reverse tilt */
-  double chk_x, chk_y;          /* |x| <= chk_x and |y| <= chk_y: no check after the element fires (eh_op_bounds) */
-  double in_bx, in_by;          /* the same for the check inside it */
   /* element specific, indexed by the EH_D_* names below */
-  double d[88];
+  double d[95];
 } eh_op;
 
-/* Half-widths inside which an element's checks cannot fire, so that the
- * kernel tests one pair of compares and leaves everything else to the general
- * code: the rectangle itself (where open, the largest finite number, as the
- * checks after an element remove infinities; nothing is removed in a
- * single-element call), and for a (super-)ellipse the box of 0.7 of its
- * half-axes, as 0.7^2 + 0.7^2 < 1.  Tiny half-axes whose powers leave the
- * normal range get no box. */
-static inline void eh_op_bounds(eh_op *op) {
-  op->in_bx = op->in_by = op->chk_x = op->chk_y = HUGE_VAL;
-  if (op->flags & EH_F_INAP) {
-    const double c = op->in_code & EH_AP_ELL ? 0.7 : 1.0;
-    if (op->in_xmax > 0)
-      op->in_bx = c * op->in_xmax;
-    if (op->in_ymax > 0)
-      op->in_by = c * op->in_ymax;
-  }
-  if (op->flags & EH_F_ALONE)
-    return;
-  op->chk_x = op->chk_y = DBL_MAX;
-  if (op->flags & EH_F_AP) {
-    const double c = op->ap_code & EH_AP_ELL ? 0.7 : 1.0;
-    if (op->ap_xmax > 0)
-      op->chk_x = fmin(c * op->ap_xmax, DBL_MAX);
-    if (op->ap_ymax > 0)
-      op->chk_y = fmin(c * op->ap_ymax, DBL_MAX);
-    if ((op->ap_code & EH_AP_ELL) &&
-        !(pow(op->ap_xmax, EH_AP_XE(op->ap_code)) >= 1e-280 && pow(op->ap_ymax, EH_AP_YE(op->ap_code)) >= 1e-280))
-      op->chk_x = op->chk_y = -1;
-  }
-}
+/* ---- hot: common to all ---- */
+#define EH_H_CHKX 0 /* |x| <= and |y| <=: no check after the element fires */
+#define EH_H_CHKY 1
+#define EH_H_INBX 2 /* the same for the check inside it */
+#define EH_H_INBY 3
+/* DRIFT2: L and L/2 */
+#define EH_H_L 4
+/* MULT, 4th order: the drifts, the first multipole's kicks, DX and DY */
+#define EH_H_DSH 4
+#define EH_H_KICK 8
+#define EH_H_DXA 11
+#define EH_H_DYA 12
+/* CSBEND, 4th order */
+#define EH_H_RHO0 4
+#define EH_H_RHOA 5
+#define EH_H_RRHO0 6
+#define EH_H_RRHOA 7
+#define EH_H_BDSHR 8
+#define EH_H_BDS 12
+#define EH_H_ZLIM 15
+/* ---- bend: the common path of a CSBEND around its substeps ---- */
+#define EH_B_DXI 0
+#define EH_B_DYI 1
+#define EH_B_DZI 2
+#define EH_B_CT 3
+#define EH_B_ST 4
+#define EH_B_TANE1 5
+#define EH_B_TE1 6
+#define EH_B_PO 8
+#define EH_B_DXF 9
+#define EH_B_DYF 10
+#define EH_B_DZF 11
+#define EH_B_TANE2 12
+#define EH_B_TE2 13
 
 /* ---- MULT ---- */
 #define EH_D_DX 0
@@ -216,6 +225,81 @@ static inline void eh_op_bounds(eh_op *op) {
 #define EH_D_RFLEN_TOTAL 8 /* element length (VOLT=0 drift) */
 #define EH_D_TOFF 9       /* CHANGE_T timeOffset (set by the host from the beam's first row) */
 #define EH_D_TO 10        /* RF period 2 pi / omega */
+
+/* The part of a finished record that the common paths read.  The bounds are
+ * half-widths inside which an element's checks cannot fire, so that the
+ * kernel tests one pair of compares and leaves everything else to the general
+ * code: the rectangle itself (where open, the largest finite number, as the
+ * checks after an element remove infinities; nothing is removed in a
+ * single-element call), and for a (super-)ellipse the box of 0.7 of its
+ * half-axes, as 0.7^2 + 0.7^2 < 1.  Tiny half-axes whose powers leave the
+ * normal range get no box. */
+static inline void eh_op_finish(eh_op *op) {
+  double *h = op->hot, *b = op->bend;
+  const double *d = op->d;
+  for (int k = 0; k < 16; k++)
+    h[k] = b[k] = 0;
+  h[EH_H_CHKX] = h[EH_H_CHKY] = h[EH_H_INBX] = h[EH_H_INBY] = HUGE_VAL;
+  if (op->flags & EH_F_INAP) {
+    const double c = op->in_code & EH_AP_ELL ? 0.7 : 1.0;
+    if (op->in_xmax > 0)
+      h[EH_H_INBX] = c * op->in_xmax;
+    if (op->in_ymax > 0)
+      h[EH_H_INBY] = c * op->in_ymax;
+  }
+  if (!(op->flags & EH_F_ALONE)) {
+    h[EH_H_CHKX] = h[EH_H_CHKY] = DBL_MAX;
+    if (op->flags & EH_F_AP) {
+      const double c = op->ap_code & EH_AP_ELL ? 0.7 : 1.0;
+      if (op->ap_xmax > 0)
+        h[EH_H_CHKX] = fmin(c * op->ap_xmax, DBL_MAX);
+      if (op->ap_ymax > 0)
+        h[EH_H_CHKY] = fmin(c * op->ap_ymax, DBL_MAX);
+      if ((op->ap_code & EH_AP_ELL) &&
+          !(pow(op->ap_xmax, EH_AP_XE(op->ap_code)) >= 1e-280 && pow(op->ap_ymax, EH_AP_YE(op->ap_code)) >= 1e-280))
+        h[EH_H_CHKX] = h[EH_H_CHKY] = -1;
+    }
+  }
+  if (op->op == EH_OP_DRIFT2) {
+    h[EH_H_L] = d[0];
+    h[EH_H_L + 1] = d[1];
+  } else if (op->op == EH_OP_MULT) {
+    for (int k = 0; k < 4; k++)
+      h[EH_H_DSH + k] = d[EH_D_DSH + k];
+    for (int k = 0; k < 3; k++)
+      h[EH_H_KICK + k] = d[EH_D_KICK + k];
+    h[EH_H_DXA] = d[EH_D_DX];
+    h[EH_H_DYA] = d[EH_D_DY];
+    /* one normal multipole, no steering, thick, 4th order: the order */
+    op->nfield = (op->nkick_orders == 1 && !op->skew0 && !(op->flags & (EH_F_XKICK | EH_F_YKICK)) &&
+                d[EH_D_DRIFT] != 0 && op->nsub == 4)
+                   ? op->order0
+                   : 0;
+  } else if (op->op == EH_OP_CSBEND) {
+    h[EH_H_RHO0] = d[EH_D_RHO0];
+    h[EH_H_RHOA] = d[EH_D_RHOA];
+    h[EH_H_RRHO0] = d[EH_D_RRHO0];
+    h[EH_H_RRHOA] = d[EH_D_RRHOA];
+    for (int k = 0; k < 4; k++)
+      h[EH_H_BDSHR + k] = d[EH_D_BDSHR + k];
+    for (int k = 0; k < 3; k++)
+      h[EH_H_BDS + k] = d[EH_D_BDS + k];
+    h[EH_H_ZLIM] = d[EH_D_ZLIM];
+    b[EH_B_DXI] = d[EH_D_DXI];
+    b[EH_B_DYI] = d[EH_D_DYI];
+    b[EH_B_DZI] = d[EH_D_DZI];
+    b[EH_B_CT] = d[EH_D_CT];
+    b[EH_B_ST] = d[EH_D_ST];
+    b[EH_B_TANE1] = d[EH_D_TANE1];
+    b[EH_B_TE1] = d[EH_D_TE1];
+    b[EH_B_PO] = op->Po;
+    b[EH_B_DXF] = d[EH_D_DXF];
+    b[EH_B_DYF] = d[EH_D_DYF];
+    b[EH_B_DZF] = d[EH_D_DZF];
+    b[EH_B_TANE2] = d[EH_D_TANE2];
+    b[EH_B_TE2] = d[EH_D_TE2];
+  }
+}
 
 /* A run of the tracking kernel's program: records [first, first + len) of
  * the run table's record array, executed reps times in a row, standing for

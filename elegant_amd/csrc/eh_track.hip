@@ -40,6 +40,81 @@ typedef EH_CONST double eh_zc;
 
 DEV double opc(EH_CONST double *p) { return *p; }
 
+/* What a common path reads of a record, in scalar registers: the header, read
+ * an element ahead, and the element's hot values.  The empty asm makes one
+ * group of loads and one wait of them: left to itself the compiler loads each
+ * field where it is first used, and a wave alone on its SIMD waits for every
+ * one (37 % of its cycles on the FODO ring). */
+typedef int hdr_t __attribute__((ext_vector_type(4)));
+#define HD_OP(h) ((h).x)
+#define HD_FLAGS(h) ((h).y)
+#define HD_NSLICES(h) ((h).z)
+#define HD_BODY(h) ((h).w)
+
+DEV hdr_t load_hdr(eh_opc *op) { return *(EH_CONST hdr_t *)op; }
+
+struct bounds_t {
+  double chk_x, chk_y, in_x, in_y;
+};
+struct mult_t {
+  bounds_t b;
+  double dsh[4], kick[3], dx, dy;
+};
+struct bendc_t { /* the substeps of a bend */
+  bounds_t b;
+  double rho0, rhoa, rrho0, rrhoa, dshr[4], ds[3], zlim;
+};
+struct bend_t { /* around them */
+  double dxi, dyi, dzi, ct, st, tane1, te1, po, dxf, dyf, dzf, tane2, te2;
+};
+
+#define PIN4(a, b, c, d) asm volatile("" : "+s"(a), "+s"(b), "+s"(c), "+s"(d))
+
+DEV bounds_t load_bounds(eh_opc &op) {
+  bounds_t b = {op.hot[EH_H_CHKX], op.hot[EH_H_CHKY], op.hot[EH_H_INBX], op.hot[EH_H_INBY]};
+  return b;
+}
+
+DEV mult_t load_mult(eh_opc &op, hdr_t next) {
+  mult_t m;
+  m.b = load_bounds(op);
+  for (int k = 0; k < 4; k++)
+    m.dsh[k] = op.hot[EH_H_DSH + k];
+  for (int k = 0; k < 3; k++)
+    m.kick[k] = op.hot[EH_H_KICK + k];
+  m.dx = op.hot[EH_H_DXA];
+  m.dy = op.hot[EH_H_DYA];
+  asm volatile(""
+               : "+s"(m.b.chk_x), "+s"(m.b.chk_y), "+s"(m.b.in_x), "+s"(m.b.in_y), "+s"(m.dsh[0]), "+s"(m.dsh[1]),
+                 "+s"(m.dsh[2]), "+s"(m.dsh[3]), "+s"(m.kick[0]), "+s"(m.kick[1]), "+s"(m.kick[2]), "+s"(m.dx),
+                 "+s"(m.dy)
+               : "s"(next));
+  return m;
+}
+
+DEV bendc_t load_bendc(eh_opc &op, hdr_t next) {
+  bendc_t m;
+  m.b = load_bounds(op);
+  m.rho0 = op.hot[EH_H_RHO0];
+  m.rhoa = op.hot[EH_H_RHOA];
+  m.rrho0 = op.hot[EH_H_RRHO0];
+  m.rrhoa = op.hot[EH_H_RRHOA];
+  for (int k = 0; k < 4; k++)
+    m.dshr[k] = op.hot[EH_H_BDSHR + k];
+  for (int k = 0; k < 3; k++)
+    m.ds[k] = op.hot[EH_H_BDS + k];
+  m.zlim = op.hot[EH_H_ZLIM];
+  asm volatile("" ::"s"(next));
+  return m;
+}
+
+DEV bend_t load_bend(eh_opc &op) {
+  bend_t b = {op.bend[EH_B_DXI], op.bend[EH_B_DYI], op.bend[EH_B_DZI],   op.bend[EH_B_CT],   op.bend[EH_B_ST],
+              op.bend[EH_B_TANE1], op.bend[EH_B_TE1], op.bend[EH_B_PO],  op.bend[EH_B_DXF],  op.bend[EH_B_DYF],
+              op.bend[EH_B_DZF], op.bend[EH_B_TANE2], op.bend[EH_B_TE2]};
+  return b;
+}
+
 struct particle {
   double x, xp, y, yp, s, dp;
 };
@@ -273,13 +348,13 @@ DEV bool in_aperture(double x, double y, eh_opc &op) {
 
 /* surely inside it (the host's bounds, eh_op_bounds): two compares without
  * a branch for the common paths, whose lanes outside take the general code */
-DEV bool in_bounds(double x, double y, eh_opc &op) {
-  if (op.flags & EH_F_INTILT) {
+DEV bool in_bounds(double x, double y, const bounds_t &b, int flags, eh_opc &op) {
+  if (flags & EH_F_INTILT) {
     double x0 = x, y0 = y;
     x = x0 * op.in_cs0 + y0 * op.in_cs1;
     y = -x0 * op.in_cs1 + y0 * op.in_cs0;
   }
-  return __builtin_fabs(x) <= op.in_bx && __builtin_fabs(y) <= op.in_by;
+  return (__builtin_fabs(x) <= b.in_x) & (__builtin_fabs(y) <= b.in_y);
 }
 
 /* 1 + delta and its reciprocal for the IEEE quotients of emath.h, fixed for
@@ -435,24 +510,24 @@ DEV int multipole_body(double &x, double &xp, double &y, double &yp, double &s, 
  *  - after the kicks qx and qy are 0 or >= 2^-700 in magnitude (binary
  *    exponent >= -699), so every dividend is 0 or within [2^-900, 2^900].
  * Arithmetic is otherwise the general code's, operation for operation. */
-template <int ORD, int NSUB>
+template <int ORD>
 DEV bool multipole_fast(const particle &p, double &x, double &xp, double &y, double &yp, double &s,
-                        const opd_recip &o, eh_opc &op) {
-  const int nsub = NSUB ? NSUB : op.nsub;
-  const int flags = op.flags;
-  const double dxa = op.d[EH_D_DX], dya = op.d[EH_D_DY];
+                        const opd_recip &o, const hdr_t H, const mult_t &m, eh_opc &op) {
+  const int nsub = ORD ? 4 : op.nsub;
+  const int flags = HD_FLAGS(H);
+  const double dxa = m.dx, dya = m.dy;
   const bool has_drift = ORD > 0 || op.d[EH_D_DRIFT] != 0;
-  const int nko = op.nkick_orders;
   const double opd = o.v, o2 = sq(opd), hr = (0.5 - 0x1.0p-51) * o.r;
   x = p.x;
   y = p.y;
   xp = p.xp;
   yp = p.yp;
   s = 0;
-  bool good = opd >= 0x1.0p-64 && opd <= 0x1.0p+64 && __builtin_fabs(x) <= EH_COORD_LIMIT &&
-              __builtin_fabs(y) <= EH_COORD_LIMIT && __builtin_fabs(xp) <= EH_SLOPE_LIMIT &&
-              __builtin_fabs(yp) <= EH_SLOPE_LIMIT &&
-              imin3(__builtin_amdgcn_frexp_exp(xp), __builtin_amdgcn_frexp_exp(yp), 0) >= -599;
+  /* & instead of &&: no lane skips the rest of a test that all lanes pass */
+  bool good = (opd >= 0x1.0p-64) & (opd <= 0x1.0p+64) & (__builtin_fabs(x) <= EH_COORD_LIMIT) &
+              (__builtin_fabs(y) <= EH_COORD_LIMIT) & (__builtin_fabs(xp) <= EH_SLOPE_LIMIT) &
+              (__builtin_fabs(yp) <= EH_SLOPE_LIMIT) &
+              (imin3(__builtin_amdgcn_frexp_exp(xp), __builtin_amdgcn_frexp_exp(yp), 0) >= -599);
   double r, den = em_sqrt_recip_mid(1 + sq(xp) + sq(yp), &r);
   double qx = em_div_pos(opd * xp, den, r), qy = em_div_pos(opd * yp, den, r);
   double den2 = o2 - sq(qx) - sq(qy), dmin = den2;
@@ -460,12 +535,12 @@ DEV bool multipole_fast(const particle &p, double &x, double &xp, double &y, dou
   xp = em_div_pos(qx, den, r);
   yp = em_div_pos(qy, den, r);
   int emin = 0;
-  for (int ik = 0; ik < op.nslices; ik++) {
-    good = good && in_bounds(x + dxa, y + dya, op);
+  for (int ik = 0; ik < HD_NSLICES(H); ik++) {
+    good &= in_bounds(x + dxa, y + dya, m.b, flags, op);
 #pragma unroll
     for (int step = 0; step < nsub; step++) {
       if (has_drift) {
-        const double dsh = opc(&op.d[EH_D_DSH + step]);
+        const double dsh = ORD ? m.dsh[step & 3] : opc(&op.d[EH_D_DSH + step]);
         x += xp * dsh;
         y += yp * dsh;
         const double t = 1 + sq(xp) + sq(yp), h = den * hr;
@@ -477,8 +552,9 @@ DEV bool multipole_fast(const particle &p, double &x, double &xp, double &y, dou
       if (step == nsub - 1)
         break; /* kickFrac[last] == 0 */
       if (ORD > 0) {
-        apply_kick(qx, qy, ORD, 0, opc(&op.d[EH_D_KICK + step]), x, y);
+        apply_kick(qx, qy, ORD, 0, m.kick[step % 3], x, y);
       } else {
+        const int nko = op.nkick_orders;
         if (nko > 0)
           apply_kick(qx, qy, op.order0, op.skew0, opc(&op.d[EH_D_KICK + step]), x, y);
         if (nko > 1)
@@ -503,9 +579,9 @@ DEV bool multipole_fast(const particle &p, double &x, double &xp, double &y, dou
       yp = em_div_pos(qy, den, r);
     }
   }
-  return good && emin >= -699 && dmin >= 0.88 * o2 && in_bounds(x + dxa, y + dya, op) &&
-         __builtin_fabs(x) <= EH_COORD_LIMIT && __builtin_fabs(y) <= EH_COORD_LIMIT &&
-         __builtin_fabs(xp) <= EH_SLOPE_LIMIT && __builtin_fabs(yp) <= EH_SLOPE_LIMIT;
+  return good & (emin >= -699) & (dmin >= 0.88 * o2) & in_bounds(x + dxa, y + dya, m.b, flags, op) &
+         (__builtin_fabs(x) <= EH_COORD_LIMIT) & (__builtin_fabs(y) <= EH_COORD_LIMIT) &
+         (__builtin_fabs(xp) <= EH_SLOPE_LIMIT) & (__builtin_fabs(yp) <= EH_SLOPE_LIMIT);
 }
 
 /* the integrator's entry (multipole.c:1176-1205): limits, slopes to
@@ -611,35 +687,35 @@ DEV int track_multipole(particle &p, eh_opc &op, eh_zc *z) {
 }
 
 /* the same on the common path; false: p is not to be used */
-DEV bool track_multipole_fast(particle &p, eh_opc &op) {
-  if (op.flags & EH_F_EXPAND)
+DEV bool track_multipole_fast(particle &p, const hdr_t H, const mult_t &m, eh_opc &op) {
+  const int flags = HD_FLAGS(H);
+  if (flags & EH_F_EXPAND)
     return false;
-  multipole_in(p, op);
+  if (flags & (EH_F_OFFSET | EH_F_ROTATE | EH_F_LEND))
+    multipole_in(p, op);
   opd_recip o;
   o.v = 1 + p.dp;
   o.r = em_recip(o.v);
   /* the common thick element with one normal multipole and no steering gets
    * a body specialised to its order: the kick is straight-line code */
-  const int ord = (op.nkick_orders == 1 && !op.skew0 && !(op.flags & (EH_F_XKICK | EH_F_YKICK)) &&
-                   op.d[EH_D_DRIFT] != 0 && op.nsub == 4)
-                      ? op.order0
-                      : 0;
+  const int body = HD_BODY(H);
   double x, xp, y, yp, s;
   bool done;
-  if (ord == 1)
-    done = multipole_fast<1, 4>(p, x, xp, y, yp, s, o, op);
-  else if (ord == 2)
-    done = multipole_fast<2, 4>(p, x, xp, y, yp, s, o, op);
-  else if (ord == 3)
-    done = multipole_fast<3, 4>(p, x, xp, y, yp, s, o, op);
+  if (body == 1)
+    done = multipole_fast<1>(p, x, xp, y, yp, s, o, H, m, op);
+  else if (body == 2)
+    done = multipole_fast<2>(p, x, xp, y, yp, s, o, H, m, op);
+  else if (body == 3)
+    done = multipole_fast<3>(p, x, xp, y, yp, s, o, H, m, op);
   else
-    done = multipole_fast<0, 0>(p, x, xp, y, yp, s, o, op);
+    done = multipole_fast<0>(p, x, xp, y, yp, s, o, H, m, op);
   p.x = x;
   p.xp = xp;
   p.y = y;
   p.yp = yp;
   p.s += s;
-  multipole_out(p, op);
+  if (flags & (EH_F_OFFSET | EH_F_ROTATE | EH_F_LEND))
+    multipole_out(p, op);
   return done;
 }
 
@@ -786,50 +862,51 @@ DEV bool csbend_body(double &X, double &QX, double &Y, double &QY, const double 
  * Arithmetic is otherwise csbend_body's, operation for operation. */
 template <int NSUB, bool WIDE>
 DEV bool csbend_body_fast(double &X, double &QX, double &Y, double &QY, const double opd, const double r_opd,
-                          double &dist, eh_opc &op) {
-  const double rho0 = op.d[EH_D_RHO0], rhoa = op.d[EH_D_RHOA];
+                          double &dist, const hdr_t H, const bendc_t &m, eh_opc &op) {
+  const double rho0 = m.rho0, rhoa = m.rhoa;
   const int nsub = NSUB ? NSUB : op.nsub;
-  bool good = opd >= 0x1.0p-64 && opd <= 0x1.0p+64 && em_bits(QY) != 0x8000000000000000ULL &&
-              (__builtin_fabs(X) + __builtin_fabs(QX)) + __builtin_fabs(QY) <= 0x1.0p+600 &&
-              imin3(__builtin_amdgcn_frexp_exp(X), __builtin_amdgcn_frexp_exp(QX), __builtin_amdgcn_frexp_exp(QY)) >=
-                  -699;
+  bool good = (opd >= 0x1.0p-64) & (opd <= 0x1.0p+64) & (em_bits(QY) != 0x8000000000000000ULL) &
+              ((__builtin_fabs(X) + __builtin_fabs(QX)) + __builtin_fabs(QY) <= 0x1.0p+600) &
+              (imin3(__builtin_amdgcn_frexp_exp(X), __builtin_amdgcn_frexp_exp(QX), __builtin_amdgcn_frexp_exp(QY)) >=
+               -699);
   const double q1 = em_div_pos(QY, opd, r_opd) * opd;
-  good = good && em_div_pos(q1, opd, r_opd) * opd == q1;
+  good &= em_div_pos(q1, opd, r_opd) * opd == q1;
   const double fin = sq(opd) - sq(QY), fin1 = sq(opd) - sq(q1);
-  good = good && __builtin_fmin(fin, fin1) >= 0x1.0p-128;
+  good &= __builtin_fmin(fin, fin1) >= 0x1.0p-128;
   double r_f, r_f1;
   double f = em_sqrt_recip_mid(fin, &r_f);
   const double f1 = em_sqrt_recip_mid(fin1, &r_f1);
   double acc = 0, zmax = 0;
-  for (int i = 0; i < op.nslices; i++) {
-    good = good && in_bounds(X, Y, op);
+  const em_small_k K = em_small_coefs();
+  for (int i = 0; i < HD_NSLICES(H); i++) {
+    good &= in_bounds(X, Y, m.b, HD_FLAGS(H), op);
     acc += __builtin_fabs(X) + __builtin_fabs(QX);
 #pragma unroll
     for (int j = 0; j < nsub; j++) {
       double sin_phi = em_div_pos(QX, f, r_f);
-      double phi = em_asin_small(sin_phi, sin_phi * sin_phi);
-      const double ang = opc(&op.d[EH_D_BDSHR + j]) + phi;
+      double phi = em_asin_small_c(sin_phi, sin_phi * sin_phi, &K);
+      const double ang = (NSUB ? m.dshr[j & 3] : opc(&op.d[EH_D_BDSHR + j])) + phi;
       const double za = ang * ang, zp = phi * phi;
       zmax = __builtin_fmax(zmax, zp);
       if (WIDE)
         zmax = __builtin_fmax(zmax, za);
-      double sine = em_sin_small(ang, za), cosi = em_cos_small(ang, za);
-      const double r_c = em_recip_cos_small(cosi, za);
+      double sine = em_sin_small_c(ang, za, &K), cosi = em_cos_small_c(za, &K);
+      const double r_c = em_recip_cos_small(cosi, za, &K);
       double tang = em_div_pos(sine, cosi, r_c);
-      double cos_phi = em_cos_small(phi, zp);
+      double cos_phi = em_cos_small_c(zp, &K);
       QX = f * sine;
       double factor = em_div_pos((rho0 + X) * cos_phi, f, r_f) *
-                      (tang - em_div_pos(sin_phi, cos_phi, em_recip_cos_small(cos_phi, zp)));
+                      (tang - em_div_pos(sin_phi, cos_phi, em_recip_cos_small(cos_phi, zp, &K)));
       Y += QY * factor;
       dist += factor * opd;
       const double fc = em_div_pos(cos_phi, cosi, r_c);
       X = rho0 * (fc - 1) + fc * X;
       if (j == nsub - 1)
         break; /* kickFrac[last] == 0 */
-      double ds = opc(&op.d[EH_D_BDS + j]);
-      double g = 1 + em_div_pos(X, rho0, opc(&op.d[EH_D_RRHO0]));
+      double ds = NSUB ? m.ds[j % 3] : opc(&op.d[EH_D_BDS + j]);
+      double g = 1 + em_div_pos(X, rho0, m.rrho0);
       /* (-ds) g 1.0 = -(ds g): the general code's bits, one product fewer */
-      QX += em_div_pos(-(ds * g), rhoa, opc(&op.d[EH_D_RRHOA]));
+      QX += em_div_pos(-(ds * g), rhoa, m.rrhoa);
       QX = em_div_pos(QX, opd, r_opd);
       QX *= opd;
       QY = q1;
@@ -838,7 +915,7 @@ DEV bool csbend_body_fast(double &X, double &QX, double &Y, double &QY, const do
     }
   }
   acc += __builtin_fabs(X) + __builtin_fabs(QX);
-  return good && acc <= 0x1.0p+600 && zmax < (WIDE ? EM_SMALL_Z : op.d[EH_D_ZLIM]);
+  return good & (acc <= 0x1.0p+600) & (zmax < (WIDE ? EM_SMALL_Z : m.zlim));
 }
 
 DEV int track_csbend(particle &p, eh_opc &op, eh_zc *z) {
@@ -950,34 +1027,35 @@ static __device__ __attribute__((noinline)) double edge_tan(double a) { return e
  * moderate, and the host has checked the edges (EH_F_FAST).  1 + delta, the
  * edges' radius and the velocity are the same at both ends (nothing changes
  * delta here), so each has one reciprocal. */
-DEV bool track_csbend_fast(particle &p, eh_opc &op) {
-  const int flags = op.flags;
+DEV bool track_csbend_fast(particle &p, const hdr_t H, hdr_t next, eh_opc &op) {
+  const int flags = HD_FLAGS(H);
   if (!(flags & EH_F_FAST))
     return false;
-  const double ct = op.d[EH_D_CT], st = op.d[EH_D_ST];
-  const double rhoa = op.d[EH_D_RHOA], dzi = op.d[EH_D_DZI], dzf = op.d[EH_D_DZF];
+  const bendc_t m = load_bendc(op, next);
+  const bend_t B = load_bend(op);
+  const double rhoa = m.rhoa, dzi = B.dzi, dzf = B.dzf;
   const double dp = p.dp, opd = 1 + dp, r_opd = em_recip(opd);
-  bool good = __builtin_fabs(p.xp) + __builtin_fabs(p.yp) <= 0x1.0p+60 && __builtin_fabs(p.s) <= 0x1.0p+500 &&
-              __builtin_amdgcn_frexp_exp(p.s) >= -500;
+  bool good = (__builtin_fabs(p.xp) + __builtin_fabs(p.yp) <= 0x1.0p+60) & (__builtin_fabs(p.s) <= 0x1.0p+500) &
+              (__builtin_amdgcn_frexp_exp(p.s) >= -500);
   p.s += dzi != 0 ? dzi * em_sqrt_mid(1 + sq(p.xp) + sq(p.yp)) : dzi;
-  p.x = p.x + op.d[EH_D_DXI] + dzi * p.xp;
-  p.y = p.y + op.d[EH_D_DYI] + dzi * p.yp;
-  double x = p.x * ct + p.y * st;
-  double y = -p.x * st + p.y * ct;
-  double xp = p.xp * ct + p.yp * st;
-  double yp = -p.xp * st + p.yp * ct;
+  p.x = p.x + B.dxi + dzi * p.xp;
+  p.y = p.y + B.dyi + dzi * p.yp;
+  double x = p.x * B.ct + p.y * B.st;
+  double y = -p.x * B.st + p.y * B.ct;
+  double xp = p.xp * B.ct + p.yp * B.st;
+  double yp = -p.xp * B.st + p.yp * B.ct;
   double rho = 1.0, r_rho = 1.0;
   if (flags & (EH_F_EDGE1 | EH_F_EDGE2)) {
     rho = opd * rhoa;
     r_rho = em_recip(rho);
-    good = good && rho >= 0x1.0p-64 && rho <= 0x1.0p+64;
+    good &= (rho >= 0x1.0p-64) & (rho <= 0x1.0p+64);
   }
   if (flags & EH_F_EDGE1) {
-    double delta_xp = em_div_pos(op.d[EH_D_TANE1], rho, r_rho) * x;
+    double delta_xp = em_div_pos(B.tane1, rho, r_rho) * x;
     if ((flags & EH_F_KLIM1) && __builtin_fabs(delta_xp) > op.d[EH_D_KLIM1])
       delta_xp = (delta_xp > 0 ? 1 : -1) * op.d[EH_D_KLIM1];
     xp += delta_xp;
-    double te = op.d[EH_D_TE1];
+    double te = B.te1;
     if (flags & EH_F_PSI1)
       te = edge_tan(op.d[EH_D_E1] - em_div_pos(op.d[EH_D_PSI1], opd, r_opd));
     yp -= em_div_pos(te, rho, r_rho) * y;
@@ -985,25 +1063,25 @@ DEV bool track_csbend_fast(particle &p, eh_opc &op) {
   double X = x, Y = y, dist = 0, r, g = em_sqrt_recip_mid(1 + sq(xp) + sq(yp), &r);
   const double f = em_div_pos(opd, g, r);
   double QX = xp * f, QY = yp * f;
-  good = good && __builtin_fabs(xp) + __builtin_fabs(yp) <= 0x1.0p+60;
+  good &= __builtin_fabs(xp) + __builtin_fabs(yp) <= 0x1.0p+60;
   /* the 4th-order integrator's four substeps of a slice unrolled (NSUB = 4):
    * the scheduler overlaps neighbouring substeps */
   if (op.nsub == 4 && !(flags & EH_F_WIDE))
-    good = csbend_body_fast<4, false>(X, QX, Y, QY, opd, r_opd, dist, op) && good;
+    good &= csbend_body_fast<4, false>(X, QX, Y, QY, opd, r_opd, dist, H, m, op);
   else
-    good = csbend_body_fast<0, true>(X, QX, Y, QY, opd, r_opd, dist, op) && good;
-  good = good && in_bounds(X, Y, op);
+    good &= csbend_body_fast<0, true>(X, QX, Y, QY, opd, r_opd, dist, H, m, op);
+  good &= in_bounds(X, Y, m.b, flags, op);
   {
     const double den2 = sq(opd) - sq(QX) - sq(QY);
-    good = good && den2 >= 0x1.0p-128;
+    good &= den2 >= 0x1.0p-128;
     g = em_sqrt_recip_mid(den2, &r);
     const double q = em_div_pos(1.0, g, r);
     QX *= q;
     QY *= q;
   }
   /* velocity rescaling of s: beta1 = beta0 */
-  const double p0 = op.Po * opd;
-  good = good && p0 >= 0x1.0p-60 && p0 <= 0x1.0p+60;
+  const double p0 = B.po * opd;
+  good &= (p0 >= 0x1.0p-60) & (p0 <= 0x1.0p+60);
   g = em_sqrt_recip_mid(sq(p0) + 1, &r);
   const double beta0 = em_div_pos(p0, g, r);
   const double s = em_div_pos(beta0 * p.s, beta0, em_recip(beta0)) + dist;
@@ -1012,11 +1090,11 @@ DEV bool track_csbend_fast(particle &p, eh_opc &op) {
   y = Y;
   yp = QY;
   if (flags & EH_F_EDGE2) {
-    double delta_xp = em_div_pos(op.d[EH_D_TANE2], rho, r_rho) * x;
+    double delta_xp = em_div_pos(B.tane2, rho, r_rho) * x;
     if ((flags & EH_F_KLIM2) && __builtin_fabs(delta_xp) > op.d[EH_D_KLIM2])
       delta_xp = (delta_xp > 0 ? 1 : -1) * op.d[EH_D_KLIM2];
     xp += delta_xp;
-    double te = op.d[EH_D_TE2];
+    double te = B.te2;
     if (flags & EH_F_PSI2)
       te = edge_tan(op.d[EH_D_E2] - em_div_pos(op.d[EH_D_PSI2], opd, r_opd));
     yp -= em_div_pos(te, rho, r_rho) * y;
@@ -1029,14 +1107,15 @@ DEV bool track_csbend_fast(particle &p, eh_opc &op) {
     o3 = op.d[EH_D_ET + 3];
     o4 = op.d[EH_D_ET + 4];
   }
+  const double ct = B.ct, st = B.st;
   p.x = x * ct - y * st + o0;
   p.y = x * st + y * ct + o2;
   p.xp = xp * ct - yp * st + o1;
   p.yp = xp * st + yp * ct + o3;
   p.s = s + o4;
-  p.x += op.d[EH_D_DXF] + dzf * p.xp;
-  p.y += op.d[EH_D_DYF] + dzf * p.yp;
-  good = good && __builtin_fabs(p.xp) + __builtin_fabs(p.yp) <= 0x1.0p+60;
+  p.x += B.dxf + dzf * p.xp;
+  p.y += B.dyf + dzf * p.yp;
+  good &= __builtin_fabs(p.xp) + __builtin_fabs(p.yp) <= 0x1.0p+60;
   p.s += dzf != 0 ? dzf * em_sqrt_mid(1 + sq(p.xp) + sq(p.yp)) : dzf;
   return good;
 }
@@ -1351,31 +1430,17 @@ SLOW slow_checks(particle p, eh_opc *op, eh_zc *z) {
 /* One element on one particle.  z points at the element's (z_start, z_end),
  * which only the loss paths read: in the element record itself, or in the
  * position table of a program whose repeated cells share one record. */
-DEV int run_op(particle &p, eh_opc &op, eh_zc *z, int64_t pass) {
+DEV int run_op(particle &p, const hdr_t H, hdr_t next, eh_opc &op, eh_zc *z, int64_t pass) {
+  const int code = HD_OP(H);
   step_out o;
   o.lost = 0;
   /* elements before the recirculation point act on pass 0 only */
-  if ((op.flags & EH_F_FIRSTPASS) && pass != 0)
+  if ((HD_FLAGS(H) & EH_F_FIRSTPASS) && pass != 0)
     return 0;
-  switch (op.op) {
-  case EH_OP_DRIFT2:
-    if ((op.flags & EH_F_DFAST) && ALL_LANES(drift2_ok(p)))
-      drift2(p, op.d[0], op.d[1]);
-    else
-      p = slow_drift2(p, op.d[0], op.d[1]).p;
-    break;
-  case EH_OP_DRIFT1:
-    drift1(p, op.d[0]);
-    break;
-  case EH_OP_EXACT_DRIFT:
-    exact_drift(p, op.d[0]);
-    break;
-  case EH_OP_MATRIX1:
-    matrix1(p, op.d);
-    break;
-  case EH_OP_MULT: {
+  if (code == EH_OP_MULT) {
     particle q = p;
-    const bool done = track_multipole_fast(q, op);
+    const mult_t m = load_mult(op, next);
+    const bool done = track_multipole_fast(q, H, m, op);
     if (ALL_LANES(done))
       p = q;
     else if (done)
@@ -1384,11 +1449,16 @@ DEV int run_op(particle &p, eh_opc &op, eh_zc *z, int64_t pass) {
       o = slow_multipole(p, &op, z);
       p = o.p;
     }
-    break;
-  }
-  case EH_OP_CSBEND: {
+  } else if (code == EH_OP_DRIFT2) {
+    double L = op.hot[EH_H_L], hL = op.hot[EH_H_L + 1];
+    asm volatile("" : "+s"(L), "+s"(hL) : "s"(next));
+    if ((HD_FLAGS(H) & EH_F_DFAST) && ALL_LANES(drift2_ok(p)))
+      drift2(p, L, hL);
+    else
+      p = slow_drift2(p, L, hL).p;
+  } else if (code == EH_OP_CSBEND) {
     particle q = p;
-    const bool done = track_csbend_fast(q, op);
+    const bool done = track_csbend_fast(q, H, next, op);
     if (ALL_LANES(done))
       p = q;
     else if (done)
@@ -1397,33 +1467,43 @@ DEV int run_op(particle &p, eh_opc &op, eh_zc *z, int64_t pass) {
       o = slow_csbend(p, &op, z);
       p = o.p;
     }
-    break;
-  }
-  case EH_OP_RFCA:
-    o = slow_rfca(p, &op, z);
-    p = o.p;
-    break;
-  case EH_OP_MALIGN:
-  case EH_OP_RCOL_IN:
-  case EH_OP_RCOL_BODY:
-    o = slow_other(p, &op, z, pass);
-    p = o.p;
-    break;
-  case EH_OP_RFCA_DRIFT:
-    /* VOLT=0: a drift when the cavity has length, else nothing (simple_rfca.c:389-402) */
-    if (op.d[EH_D_RFLEN_TOTAL] != 0) {
-      p.x += p.xp * op.d[EH_D_RFLEN_TOTAL];
-      p.y += p.yp * op.d[EH_D_RFLEN_TOTAL];
-      p.s += op.d[EH_D_RFLEN_TOTAL] * em_sqrt(1 + sq(p.xp) + sq(p.yp));
+  } else {
+    switch (code) {
+    case EH_OP_DRIFT1:
+      drift1(p, op.d[0]);
+      break;
+    case EH_OP_EXACT_DRIFT:
+      exact_drift(p, op.d[0]);
+      break;
+    case EH_OP_MATRIX1:
+      matrix1(p, op.d);
+      break;
+    case EH_OP_RFCA:
+      o = slow_rfca(p, &op, z);
+      p = o.p;
+      break;
+    case EH_OP_MALIGN:
+    case EH_OP_RCOL_IN:
+    case EH_OP_RCOL_BODY:
+      o = slow_other(p, &op, z, pass);
+      p = o.p;
+      break;
+    case EH_OP_RFCA_DRIFT:
+      /* VOLT=0: a drift when the cavity has length, else nothing (simple_rfca.c:389-402) */
+      if (op.d[EH_D_RFLEN_TOTAL] != 0) {
+        p.x += p.xp * op.d[EH_D_RFLEN_TOTAL];
+        p.y += p.yp * op.d[EH_D_RFLEN_TOTAL];
+        p.s += op.d[EH_D_RFLEN_TOTAL] * em_sqrt(1 + sq(p.xp) + sq(p.yp));
+      }
+      break;
+    default:
+      break;
     }
-    break;
-  default:
-    break;
   }
   if (o.lost)
     return o.lost;
   /* inside these bounds none of the checks after the element can fire */
-  const bool inside = __builtin_fabs(p.x) <= op.chk_x && __builtin_fabs(p.y) <= op.chk_y;
+  const bool inside = (__builtin_fabs(p.x) <= op.hot[EH_H_CHKX]) & (__builtin_fabs(p.y) <= op.hot[EH_H_CHKY]);
   if (!ALL_LANES(inside) && !inside) {
     o = slow_checks(p, &op, z);
     p = o.p;
@@ -1459,31 +1539,39 @@ __global__ void __launch_bounds__(256, 4) eh_track_kernel(eh_state st, const eh_
   p.dp = st.dp[i];
   eh_opc *cops = (eh_opc *)ops;
   eh_zc *zs = (eh_zc *)zpos;
-  int lost = 0, lost_op = 0;
-  int64_t lost_pass = 0;
-  for (int32_t ip = 0; ip < npasses && !lost; ip++) {
+  EH_CONST eh_run *cruns = (EH_CONST eh_run *)runs;
+  /* the loops are the same for all lanes; a lost lane sits out (its mask would
+   * otherwise be kept at every loop level) */
+  int lost = 0, lost_op = 0, lost_pass = 0;
+  for (int32_t ip = 0; ip < npasses; ip++) {
     /* element positions [ob, oe) of the flat beamline in this pass */
     const int32_t ob = (ip == 0) ? op_first : 0;
     const int32_t oe = (ip == npasses - 1) ? op_last : nflat;
-    for (int32_t r = 0; r < nruns && !lost; r++) {
-      const int32_t fs = runs[r].flat, len = runs[r].len, first = runs[r].first;
-      const int32_t fe = fs + len * runs[r].reps;
+    if (ALL_LANES(lost))
+      break;
+    for (int32_t r = 0; r < nruns; r++) {
+      const int32_t fs = cruns[r].flat, len = cruns[r].len, first = cruns[r].first;
+      const int32_t fe = fs + len * cruns[r].reps;
       if (fe <= ob)
         continue;
       if (fs >= oe)
         break;
       int32_t f = fs > ob ? fs : ob;
       const int32_t f1 = fe < oe ? fe : oe;
-      int32_t k = (f - fs) % len;
+      eh_opc *op0 = cops + first, *op1 = op0 + len, *op = op0 + (f - fs) % len;
+      hdr_t h = load_hdr(op);
       for (; f < f1; f++) {
-        lost = run_op(p, cops[first + k], zs + 2 * f, pass0 + ip);
-        if (lost) {
-          lost_op = f;
-          lost_pass = pass0 + ip;
-          break;
+        eh_opc *nxt = op + 1 == op1 ? op0 : op + 1;
+        hdr_t hn = load_hdr(nxt);
+        if (!lost) {
+          lost = run_op(p, h, hn, *op, zs + 2 * f, pass0 + ip);
+          if (lost) {
+            lost_op = f;
+            lost_pass = ip;
+          }
         }
-        if (++k == len)
-          k = 0;
+        op = nxt;
+        h = hn;
       }
     }
   }
@@ -1494,7 +1582,7 @@ __global__ void __launch_bounds__(256, 4) eh_track_kernel(eh_state st, const eh_
   st.s[i] = p.s;
   st.dp[i] = p.dp;
   if (lost) {
-    st.loss_pass[i] = (int32_t)lost_pass;
+    st.loss_pass[i] = (int32_t)(pass0 + lost_pass);
     st.loss_code[i] = 4 * lost_op + (lost - 1);
   }
 }
@@ -1552,12 +1640,15 @@ __global__ void __launch_bounds__(256, 4) eh_batch_kernel(eh_state st, const eh_
         any |= live[k];
       if (!any)
         break;
+      hdr_t h = load_hdr(vops);
       for (int32_t io = 0; io < nops; io++) {
         eh_opc &op = vops[io];
+        const hdr_t hcur = h;
+        h = load_hdr(vops + (io + 1 < nops ? io + 1 : 0));
         for (int k = 0; k < PPL; k++) {
           if (!live[k])
             continue;
-          int l = run_op(p[k], op, &op.z_start, pass0 + ip);
+          int l = run_op(p[k], hcur, h, op, &op.z_start, pass0 + ip);
           if (l) {
             live[k] = false;
             lost[k] = l;
@@ -1853,7 +1944,7 @@ int ehd_put_program(ehd_dev *d, const eh_op *ops, int32_t nops) {
   if (nops > 0)
     memcpy(d->host_prog, ops, sizeof(eh_op) * (size_t)nops);
   for (int32_t f = 0; f < nops; f++)
-    eh_op_bounds(&d->host_prog[f]);
+    eh_op_finish(&d->host_prog[f]);
   d->nflat = nops;
   return upload_program(d);
 }
@@ -1863,7 +1954,7 @@ int ehd_patch_op(ehd_dev *d, int32_t index, const eh_op *op) {
     return EH_ERR_INVALID;
   HIPCHK(d, hipSetDevice(d->device));
   d->host_prog[index] = *op;
-  eh_op_bounds(&d->host_prog[index]);
+  eh_op_finish(&d->host_prog[index]);
   return upload_program(d);
 }
 
@@ -2440,7 +2531,8 @@ __global__ void eh_math_probe_kernel(int32_t fn, const double *in, const double 
   }
   case 13: { /* in / cos(in2), |in2| < 2^-5 */
     const double z = in2[i] * in2[i], c = em_cos_small(in2[i], z);
-    r = em_div_pos(v, c, em_recip_cos_small(c, z));
+    const em_small_k k = em_small_coefs();
+    r = em_div_pos(v, c, em_recip_cos_small(c, z, &k));
     break;
   }
   default:

@@ -72,15 +72,14 @@
 #define EM_TWO_OVER_PI 0x1.45f306dc9c883p-1
 #define EM_SHIFT 0x1.8p+52
 
-/* A polynomial coefficient as a scalar-register operand.  The empty asm hides
- * the value from the compiler, which otherwise hoists every coefficient of
- * every inlined polynomial into vector registers for the whole kernel (that
- * costs occupancy).  Not volatile: equal coefficients may share a register
- * pair over a loop, which took 72 of 108 scalar instructions out of a slice of
- * the bend's common path (a wave alone on its SIMD issues them one by one). */
+/* A polynomial coefficient at its point of use.  On the device the empty
+ * volatile asm keeps each 64-bit constant a scalar-register operand
+ * materialized where it is used; without it the compiler hoists every
+ * coefficient of every inlined polynomial into registers for the whole
+ * kernel, which costs occupancy.  The value is unchanged. */
 #if defined(__HIP_DEVICE_COMPILE__)
 EM_FN double em_k(double c) {
-  asm("" : "=s"(c) : "0"(c));
+  asm volatile("" : "=s"(c) : "0"(c));
   return c;
 }
 #else
@@ -786,15 +785,61 @@ EM_FN double em_sqrt_recip_mid(double x, double *y) {
 #endif
 }
 
-/* em_recip(c) of a cosine c = em_cos_small(a, z), z = a*a < 2^-10: the secant's
+/* The narrow bands with their coefficients held in registers, for a loop that
+ * evaluates them often: em_small_coefs() before the loop takes the scalar
+ * instructions that load them (108 of a bend slice's 600) out of it.  Same
+ * operations as em_sin_small, em_cos_small and em_asin_small. */
+typedef struct {
+  double s1, s2, s3, s4, c2, c3, c4, a1, a2, a3, a4, a5, sec;
+} em_small_k;
+
+EM_FN em_small_k em_small_coefs(void) {
+  em_small_k k;
+  k.s1 = em_k(EM_S1);
+  k.s2 = em_k(0x1.1111111111111p-7);
+  k.s3 = em_k(-0x1.a01a01a01a01ap-13);
+  k.s4 = em_k(0x1.71de3a556c734p-19);
+  k.c2 = em_k(0x1.5555555555555p-5);
+  k.c3 = em_k(-0x1.6c16c16c16c17p-10);
+  k.c4 = em_k(0x1.a01a01a01a01ap-16);
+  k.a1 = em_k(0x1.5555555555555p-3);
+  k.a2 = em_k(0x1.3333333333333p-4);
+  k.a3 = em_k(0x1.6db6db6db6db7p-5);
+  k.a4 = em_k(0x1.f1c71c71c71c7p-6);
+  k.a5 = em_k(0x1.6e8ba2e8ba2e9p-6);
+  k.sec = em_k(0x1.aaaaaaaaaaaabp-3); /* 5/24 */
+  return k;
+}
+
+EM_FN double em_sin_small_c(double x, double z, const em_small_k *k) {
+  const double r = __builtin_fma(z, __builtin_fma(z, k->s4, k->s3), k->s2);
+  return x + (z * x) * __builtin_fma(z, r, k->s1);
+}
+
+EM_FN double em_cos_small_c(double z, const em_small_k *k) {
+  double r = z * z * __builtin_fma(z, __builtin_fma(z, k->c4, k->c3), k->c2);
+  double w = __builtin_fma(-0.5, z, 1.0);
+  return w + (__builtin_fma(-0.5, z, 1.0 - w) + r);
+}
+
+EM_FN double em_asin_small_c(double x, double z, const em_small_k *k) {
+  double p = __builtin_fma(z, k->a5, k->a4);
+  p = __builtin_fma(z, p, k->a3);
+  p = __builtin_fma(z, p, k->a2);
+  p = __builtin_fma(z, p, k->a1);
+  return __builtin_fma(x, z * p, x);
+}
+
+/* em_recip(c) of a cosine c = em_cos_small_c(z, k), z < 2^-10: the secant's
  * series 1 + z/2 + 5 z^2/24 (next term below 2^-33) and one Newton step */
-EM_FN double em_recip_cos_small(double c, double z) {
+EM_FN double em_recip_cos_small(double c, double z, const em_small_k *k) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  double y = __builtin_fma(z, __builtin_fma(z, em_k(0x1.aaaaaaaaaaaabp-3), 0.5), 1.0);
+  double y = __builtin_fma(z, __builtin_fma(z, k->sec, 0.5), 1.0);
   double e = __builtin_fma(-c, y, 1.0);
   return __builtin_fma(y, e, y);
 #else
   (void)z;
+  (void)k;
   return 1.0 / c;
 #endif
 }

@@ -220,7 +220,7 @@ int eh_batch_add_variant(eh_batch *b, const eh_element *elems, int64_t n_elems, 
   }
   memcpy(b->ops + b->nops, b->prog->ops, sizeof(eh_op) * b->prog->nops);
   for (int k = 0; k < b->prog->nops; k++)
-    eh_op_bounds(&b->ops[b->nops + k]);
+    eh_op_finish(&b->ops[b->nops + k]);
   b->var[b->nvar].op_offset = (int32_t)b->nops;
   b->var[b->nvar].nops = b->prog->nops;
   b->var[b->nvar].first = b->n;
