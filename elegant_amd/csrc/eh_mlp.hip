@@ -200,6 +200,434 @@ __global__ void adam_k(float *w, const float *g, float *m, float *v, int64_t n, 
   w[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
 }
 
+/* ---- the fused path: hidden <= 256, inputs <= 256 ----
+ *
+ * A training step is three kernels: mlp_rows takes 16 samples per workgroup
+ * through all layers and back (activations stay in LDS; they and the layers'
+ * gradients are also written out), mlp_wgrad contracts those over the batch
+ * into partial weight gradients, mlp_update sums the partials in order and
+ * applies Adam.  The products run on the matrix cores in FP32
+ * (v_mfma_f32_16x16x4f32: FP32 multiplies and sums, as the LDS-tiled gemm_f32
+ * has, which stays for larger nets).  What bounds it: 3.3 GFLOP per step of 4096
+ * samples is 22 us at the 150 TFLOP/s of a large FP32 product; the step was 35
+ * launches and 470 us, and takes @S@ us.
+ *
+ * Layouts.  HS = hidden rounded up to 64, XS = inputs rounded up to 64; padded
+ * weights are zero, so padded activations and gradients are zero.  A
+ * contraction is cut into chunks of 16; lane l of a wave holds elements
+ * 4 (l / 16) .. + 3 of the chunk for row (or column) l % 16 as one 16-byte
+ * load, and product m of four takes element m of each, in both operands.
+ * Weights are kept in that order, one 1 KB block per tile of 16 outputs and
+ * chunk: wf for the forward products, wb for the ones going back. */
+typedef float f4 __attribute__((ext_vector_type(4)));
+
+struct mlp_net {
+  const float *wf[3], *wb[3]; /* wb[0] unused */
+  const float *bias[3], *w4, *b4;
+  int nin, hidden, xc, xs;    /* xc: input chunks of 16 */
+};
+
+struct mlp_batch {
+  const float *X, *y;
+  const int32_t *perm;        /* sample indices, or NULL */
+  float *xb, *h[3], *dz[3];   /* [rows][xs] and [rows][HS] */
+  float *vec;                 /* per workgroup: bias gradients of 3 layers, last weights', last bias', loss */
+  float *prob;                /* prediction */
+  int rows;
+};
+
+/* acc[mt][t] += rows of a (LDS, stride lda) x tile wave + 4 t of wt, kc
+ * chunks; the weights of the next two chunks are in flight (a workgroup is
+ * alone on its CU, one wave per SIMD) */
+template <int NT, int MT>
+static __device__ __forceinline__ void rows_mm(const float *a, int lda, const float *__restrict__ wt, int kc,
+                                               f4 (&acc)[MT][NT]) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const float *ar = a + (lane & 15) * lda + 4 * (lane >> 4);
+  const float *w0 = wt + (size_t)wave * kc * 256 + 4 * lane;
+  f4 b0[NT], b1[NT];
+#pragma unroll
+  for (int t = 0; t < NT; t++) {
+    b0[t] = *(const f4 *)(w0 + (size_t)4 * t * kc * 256);
+    b1[t] = *(const f4 *)(w0 + (size_t)4 * t * kc * 256 + (kc > 1 ? 256 : 0));
+  }
+  for (int c = 0; c < kc; c++) {
+    f4 b2[NT], av[MT];
+    const int cn = c + 2 < kc ? c + 2 : kc - 1;
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+      b2[t] = *(const f4 *)(w0 + ((size_t)4 * t * kc + cn) * 256);
+#pragma unroll
+    for (int m = 0; m < MT; m++)
+      av[m] = *(const f4 *)(ar + 16 * m * lda + 16 * c);
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+#pragma unroll
+      for (int m = 0; m < MT; m++)
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+          acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[m][k], b0[t][k], acc[m][t], 0, 0, 0);
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+      b0[t] = b1[t];
+      b1[t] = b2[t];
+    }
+  }
+}
+
+/* rows [0, 16 MT) of an LDS buffer to global rows r0.. of width HS, as far as
+ * rows exist */
+template <int HS>
+static __device__ __forceinline__ void rows_out(const float *a, int lda, float *g, int r0, int nr, int rows) {
+  for (int e = threadIdx.x; e < nr * (HS / 4); e += 256) {
+    const int r = e / (HS / 4), c = e % (HS / 4) * 4;
+    if (r0 + r < rows)
+      *(f4 *)(g + (size_t)(r0 + r) * HS + c) = *(const f4 *)(a + r * lda + c);
+  }
+}
+
+/* TRAIN: forward, loss, backward of 16 rows at a time (MT = 1); else the
+ * probabilities of 16 MT rows.  Workgroups stride over the batch. */
+template <int NT, int MT, bool TRAIN>
+__global__ void __launch_bounds__(256) mlp_rows(mlp_net N, mlp_batch Q) {
+  constexpr int HS = 64 * NT, R = 16 * MT, LD = HS + 4, LX = 260;
+  __shared__ float sx[TRAIN ? R * LX : R * (LX > LD ? LX : LD)];
+  __shared__ float sh[TRAIN ? 3 : 1][R * LD];
+  __shared__ float sz[R], sd[R];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  float vs[4] = {0, 0, 0, 0}, vb4 = 0, vloss = 0;
+  for (int r0 = blockIdx.x * R; r0 < Q.rows; r0 += gridDim.x * R) {
+    /* the rows' inputs, zero beyond the net's and beyond the batch */
+    const int xw = TRAIN ? N.xs : 16 * N.xc;
+    for (int e = tid; e < R * xw; e += 256) {
+      const int r = e / xw, k = e % xw;
+      float v = 0.f;
+      if (r0 + r < Q.rows && k < N.nin) {
+        const int64_t j = Q.perm ? Q.perm[r0 + r] : r0 + r;
+        v = Q.X[j * N.nin + k];
+      }
+      sx[r * LX + k] = v;
+      if (TRAIN && r0 + r < Q.rows)
+        Q.xb[(size_t)(r0 + r) * N.xs + k] = v;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int l = 0; l < 3; l++) {
+      /* prediction alternates between two buffers */
+      const float *in = l == 0 ? sx : (TRAIN ? sh[l - 1] : (l == 1 ? sh[0] : sx));
+      float *out = TRAIN ? sh[l] : (l == 1 ? sx : sh[0]);
+      const int lin = l == 0 ? LX : LD;
+      f4 acc[MT][NT];
+#pragma unroll
+      for (int m = 0; m < MT; m++)
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+          acc[m][t] = (f4){0.f, 0.f, 0.f, 0.f};
+      rows_mm<NT, MT>(in, lin, N.wf[l], l == 0 ? N.xc : HS / 16, acc);
+#pragma unroll
+      for (int t = 0; t < NT; t++) {
+        const int c = 16 * (wave + 4 * t) + (lane & 15);
+        const float b = c < N.hidden ? N.bias[l][c] : 0.f;
+#pragma unroll
+        for (int m = 0; m < MT; m++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            const float v = acc[m][t][i] + b;
+            out[(16 * m + 4 * (lane >> 4) + i) * LD + c] = v > 0.f ? v : 0.f;
+          }
+      }
+      __syncthreads();
+      if (TRAIN)
+        rows_out<HS>(sh[l], LD, Q.h[l], r0, R, Q.rows);
+    }
+    /* the last layer: 256 / R threads per row */
+    const float *h3 = TRAIN ? sh[2] : sh[0];
+    {
+      constexpr int P = 256 / R;
+      const int r = tid / P, q = tid % P;
+      float v = 0.f;
+      for (int c = q; c < N.hidden; c += P)
+        v = fmaf(h3[r * LD + c], N.w4[c], v);
+#pragma unroll
+      for (int o = P / 2; o > 0; o >>= 1)
+        v += __shfl_xor(v, o);
+      if (q == 0) {
+        const float z = v + N.b4[0];
+        if (!TRAIN) {
+          if (r0 + r < Q.rows)
+            Q.prob[r0 + r] = 1.f / (1.f + expf(-z));
+        } else {
+          float l = 0.f, d = 0.f;
+          if (r0 + r < Q.rows) {
+            const float yi = Q.y[Q.perm ? Q.perm[r0 + r] : r0 + r];
+            const float sp = z > 0 ? z + log1pf(expf(-z)) : log1pf(expf(z)); /* softplus */
+            l = sp - yi * z;
+            d = (1.f / (1.f + expf(-z)) - yi) / (float)Q.rows;
+          }
+          sz[r] = l;
+          sd[r] = d;
+        }
+      }
+    }
+    __syncthreads();
+    if (TRAIN) {
+      if (tid < HS) {
+        float s = 0.f;
+        for (int r = 0; r < R; r++)
+          s = fmaf(sd[r], sh[2][r * LD + tid], s);
+        vs[3] += s;
+      }
+      if (tid == 0) {
+        float s = 0.f, d = 0.f;
+        for (int r = 0; r < R; r++) {
+          s += sz[r];
+          d += sd[r];
+        }
+        vloss += s;
+        vb4 += d;
+      }
+      __syncthreads();
+      /* dz3 in place of h3, then dz2 in place of h2, dz1 of h1 */
+      for (int e = tid; e < R * HS; e += 256) {
+        const int r = e / HS, c = e % HS;
+        const float w = c < N.hidden ? N.w4[c] : 0.f;
+        sh[2][r * LD + c] = sh[2][r * LD + c] > 0.f ? sd[r] * w : 0.f;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int l = 2; l >= 0; l--) {
+        rows_out<HS>(sh[l], LD, Q.dz[l], r0, R, Q.rows);
+        if (tid < HS) {
+          float s = 0.f;
+          for (int r = 0; r < R; r++)
+            s += sh[l][r * LD + tid];
+          vs[l] += s;
+        }
+        if (l > 0) {
+          f4 acc[MT][NT];
+#pragma unroll
+          for (int m = 0; m < MT; m++)
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+              acc[m][t] = (f4){0.f, 0.f, 0.f, 0.f};
+          rows_mm<NT, MT>(sh[l], LD, N.wb[l], HS / 16, acc);
+#pragma unroll
+          for (int t = 0; t < NT; t++) {
+            const int c = 16 * (wave + 4 * t) + (lane & 15);
+#pragma unroll
+            for (int m = 0; m < MT; m++)
+#pragma unroll
+              for (int i = 0; i < 4; i++) {
+                float *h = &sh[l - 1][(16 * m + 4 * (lane >> 4) + i) * LD + c];
+                *h = *h > 0.f ? acc[m][t][i] : 0.f;
+              }
+          }
+          __syncthreads();
+        }
+      }
+    }
+    __syncthreads();
+  }
+  if (TRAIN) {
+    float *v = Q.vec + (size_t)blockIdx.x * (4 * HS + 2);
+    if (tid < HS)
+      for (int l = 0; l < 4; l++)
+        v[l * HS + tid] = vs[l];
+    if (tid == 0) {
+      v[4 * HS] = vb4;
+      v[4 * HS + 1] = vloss;
+    }
+  }
+}
+
+/* Partial weight gradients dW[n][k] = sum over a slice of the batch of
+ * dz[b][n] in[b][k]: a wave takes a tile of 64 x 64 (16 products of 16 x 16)
+ * and four rows of the batch per step, its operands straight from memory, one
+ * 16-byte load each: tile row 4 i + rt is row i of product rt, so a lane's four
+ * elements feed four products.  The tiles of one slice read the same rows, so
+ * a slice stays on one XCD (workgroups go round the 8 of them). */
+__global__ void __launch_bounds__(256) mlp_wgrad(mlp_batch Q, int hs, int xs, int nslice, int slice_rows, float *part) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int ht = hs / 64, t0 = ht * (xs / 64), tiles = t0 + 2 * ht * ht, wgs = (tiles + 3) / 4;
+  const int xcd = blockIdx.x % 8, j = blockIdx.x / 8;
+  const int slice = xcd + 8 * (j / wgs), tile = 4 * (j % wgs) + wave;
+  if (slice >= nslice || tile >= tiles)
+    return;
+  int l = 0, t = tile, ks = xs;
+  const float *in = Q.xb;
+  size_t off = 0;
+  if (tile >= t0) {
+    l = 1 + (tile - t0) / (ht * ht);
+    t = (tile - t0) % (ht * ht);
+    ks = hs;
+    in = Q.h[l - 1];
+    off = (size_t)hs * xs + (size_t)(l - 1) * hs * hs;
+  }
+  const int n0 = t / (ks / 64) * 64, k0 = t % (ks / 64) * 64;
+  const int b0 = slice * slice_rows, b1 = b0 + slice_rows < Q.rows ? b0 + slice_rows : Q.rows;
+  const int g = lane >> 4, c = 4 * (lane & 15);
+  const float *pa = Q.dz[l] + n0 + c, *pb = in + k0 + c;
+  f4 acc[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+      acc[i][k] = (f4){0.f, 0.f, 0.f, 0.f};
+  /* three steps' operands in flight; rows past the slice count as zero */
+  f4 av[3], bv[3];
+#pragma unroll
+  for (int u = 0; u < 3; u++) {
+    const int r = b0 + 4 * u + g, rc = r < b1 ? r : b0;
+    av[u] = *(const f4 *)(pa + (size_t)rc * hs);
+    bv[u] = *(const f4 *)(pb + (size_t)rc * ks);
+  }
+  for (int b = b0; b < b1; b += 12) {
+#pragma unroll
+    for (int u = 0; u < 3; u++) {
+      f4 a = av[u], v = bv[u];
+      if (b + 4 * u + g >= b1)
+        a = (f4){0.f, 0.f, 0.f, 0.f};
+      const int r = b + 12 + 4 * u + g, rc = r < b1 ? r : b0;
+      av[u] = *(const f4 *)(pa + (size_t)rc * hs);
+      bv[u] = *(const f4 *)(pb + (size_t)rc * ks);
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+          acc[i][k] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], v[k], acc[i][k], 0, 0, 0);
+    }
+  }
+  float *o = part + (size_t)slice * ((size_t)hs * xs + 2 * (size_t)hs * hs) + off;
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const f4 v = {acc[i][0][r], acc[i][1][r], acc[i][2][r], acc[i][3][r]};
+      *(f4 *)(o + (size_t)(n0 + 4 * (4 * g + r) + i) * ks + k0 + c) = v;
+    }
+}
+
+struct mlp_param {
+  float *w, *g, *m, *v;       /* parameters, gradients out (or NULL), Adam moments */
+  float *wf[3], *wb[3];
+  int64_t woff[4], boff[4];
+  int nin, hidden, hs, xs, xc;
+  float lr, b1, b2, eps, c1, c2;
+};
+
+/* where weight (n, k) of layer l lies in the tiled copies */
+static __device__ __forceinline__ void mlp_tiles(const mlp_param &P, int l, int n, int k, float w) {
+  const int kc = l == 0 ? P.xc : P.hs / 16;
+  P.wf[l][((size_t)(n / 16) * kc + k / 16) * 256 + 4 * ((n % 16) + 16 * (k % 16 / 4)) + k % 4] = w;
+  if (l > 0)
+    P.wb[l][((size_t)(k / 16) * (P.hs / 16) + n / 16) * 256 + 4 * ((k % 16) + 16 * (n % 16 / 4)) + n % 4] = w;
+}
+
+static __device__ __forceinline__ float mlp_step(const mlp_param &P, int64_t p, float gi) {
+  const float mi = P.b1 * P.m[p] + (1.f - P.b1) * gi;
+  const float vi = P.b2 * P.v[p] + (1.f - P.b2) * gi * gi;
+  P.m[p] = mi;
+  P.v[p] = vi;
+  const float w = P.w[p] - P.lr * (mi / P.c1) / (sqrtf(vi / P.c2) + P.eps);
+  P.w[p] = w;
+  return w;
+}
+
+/* layer, row and column of weight i of the three tiled layers */
+static __device__ __forceinline__ int mlp_where(const mlp_param &P, int64_t i, int &n, int &k) {
+  const int64_t w0 = (int64_t)P.hidden * P.nin, w1 = (int64_t)P.hidden * P.hidden;
+  const int l = i < w0 ? 0 : (i < w0 + w1 ? 1 : 2), in = l ? P.hidden : P.nin;
+  const int q = (int)(i - (l == 0 ? 0 : (l == 1 ? w0 : w0 + w1)));
+  n = q / in;
+  k = q % in;
+  return l;
+}
+
+/* the tiled copies from the parameters (their padding is zeroed before) */
+__global__ void __launch_bounds__(256) mlp_retile(mlp_param P, int64_t nw) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= nw)
+    return;
+  int n, k;
+  const int l = mlp_where(P, i, n, k);
+  mlp_tiles(P, l, n, k, P.w[P.woff[l] + (int64_t)n * (l ? P.hidden : P.nin) + k]);
+}
+
+__global__ void mlp_zero(float *p, int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n)
+    p[i] = 0.f;
+}
+
+/* The partial gradients summed in order, then Adam (or, with P.g, the
+ * gradients themselves): the first nwb workgroups take the weights of the
+ * tiled layers, the others 64 entries of the per-workgroup vectors each, in
+ * four interleaved sums.  The loss is added to *loss. */
+__global__ void __launch_bounds__(256) mlp_update(mlp_param P, const float *__restrict__ part, int nslice,
+                                                  const float *__restrict__ vec, int nvec, int64_t nw, int nwb,
+                                                  float *loss, float rows) {
+  if ((int)blockIdx.x < nwb) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= nw)
+      return;
+    int n, k;
+    const int l = mlp_where(P, i, n, k);
+    const int ks = l ? P.hs : P.xs;
+    const size_t all = (size_t)P.hs * P.xs + 2 * (size_t)P.hs * P.hs;
+    const float *q = part + (l ? (size_t)P.hs * P.xs + (size_t)(l - 1) * P.hs * P.hs : 0) + (size_t)n * ks + k;
+    float s = 0.f;
+    int u = 0;
+    for (; u + 8 <= nslice; u += 8) {
+      float t[8];
+#pragma unroll
+      for (int e = 0; e < 8; e++)
+        t[e] = q[(size_t)(u + e) * all];
+#pragma unroll
+      for (int e = 0; e < 8; e++)
+        s += t[e];
+    }
+    for (; u < nslice; u++)
+      s += q[(size_t)u * all];
+    const int64_t p = P.woff[l] + (int64_t)n * (l ? P.hidden : P.nin) + k;
+    if (P.g)
+      P.g[p] = s;
+    else
+      mlp_tiles(P, l, n, k, mlp_step(P, p, s));
+    return;
+  }
+  __shared__ float red[4][64];
+  const int V = 4 * P.hs + 2;
+  const int c = ((int)blockIdx.x - nwb) * 64 + (threadIdx.x & 63), q = threadIdx.x >> 6;
+  float s = 0.f;
+  if (c < V) {
+#pragma unroll 8
+    for (int u = q; u < nvec; u += 4)
+      s += vec[(size_t)u * V + c];
+  }
+  red[q][threadIdx.x & 63] = s;
+  __syncthreads();
+  if (q || c >= V)
+    return;
+  s = ((red[0][threadIdx.x] + red[1][threadIdx.x]) + red[2][threadIdx.x]) + red[3][threadIdx.x];
+  if (c == V - 1) {
+    *loss += s / rows;
+    return;
+  }
+  int64_t p;
+  if (c == V - 2)
+    p = P.boff[3];
+  else {
+    const int l = c / P.hs, e = c % P.hs;
+    if (e >= P.hidden)
+      return;
+    p = (l < 3 ? P.boff[l] : P.woff[3]) + e;
+  }
+  if (P.g)
+    P.g[p] = s;
+  else
+    mlp_step(P, p, s);
+}
+
 /* ------------------------------------------------------------ host side */
 
 #define MLP_LAYERS 4
@@ -221,8 +649,28 @@ struct ehd_mlp {
   int32_t *permd;        /* its sample order, epochs x n */
   float *eloss;          /* per-epoch loss sums */
   int64_t data_cap, y_cap, perm_cap, eloss_cap;
+  /* the fused path */
+  int fused, hs, xs, xc;
+  int tiles_stale;       /* the parameters were set: wf, wb to be filled */
+  float *tiles;          /* wf[0], wf[1], wb[1], wf[2], wb[2] */
+  float *fbuf;           /* xb, h[3], dz[3] for fcap rows */
+  int64_t fcap;
+  float *fvec, *fpart;   /* per-workgroup vectors, weight-gradient slices */
+  float *floss;
+  float *pin[2], *pout[2]; /* prediction: two chunks of inputs and of probabilities */
+  hipStream_t pstream;   /* their copies */
+  hipEvent_t pev[4];
   char msg[256];
 };
+
+/* two row tiles per workgroup (half the weight reads) once one each fills
+ * the device twice */
+template <int NT> static void rows_predict(hipStream_t st, const mlp_net &N, const mlp_batch &Q) {
+  if (Q.rows > 16 * 512)
+    hipLaunchKernelGGL((mlp_rows<NT, 2, false>), dim3((Q.rows + 31) / 32), dim3(256), 0, st, N, Q);
+  else
+    hipLaunchKernelGGL((mlp_rows<NT, 1, false>), dim3((Q.rows + 15) / 16), dim3(256), 0, st, N, Q);
+}
 
 extern "C" {
 
@@ -314,6 +762,11 @@ static int ensure_batch(ehd_mlp *m, int32_t B) {
 
 void ehd_mlp_destroy(ehd_mlp *m);
 
+#define FUSED_WGS 512     /* most workgroups of mlp_rows in training */
+#define FUSED_SLICES 24   /* most batch slices of mlp_wgrad: 36 tiles of a 256-wide net times 24 fill 864 of 1,024 SIMDs */
+
+static size_t tiles_len(const ehd_mlp *m) { return (size_t)m->hs * 16 * m->xc + 4 * (size_t)m->hs * m->hs; }
+
 int ehd_mlp_create(ehd_dev *d, int32_t nin, int32_t hidden, const float *init, ehd_mlp **out) {
   ehd_mlp *m = (ehd_mlp *)calloc(1, sizeof(ehd_mlp));
   if (!m)
@@ -344,6 +797,21 @@ int ehd_mlp_create(ehd_dev *d, int32_t nin, int32_t hidden, const float *init, e
     ehd_mlp_destroy(m);
     return EH_ERR_HIP;
   }
+  if ((hidden + 63) / 64 <= 4 && (nin + 63) / 64 <= 4) {
+    m->fused = 1;
+    m->hs = (hidden + 63) / 64 * 64;
+    m->xs = (nin + 63) / 64 * 64;
+    m->xc = (nin + 15) / 16;
+    m->tiles_stale = 1;
+    const size_t all = (size_t)m->hs * m->xs + 2 * (size_t)m->hs * m->hs;
+    if (hipMalloc((void **)&m->tiles, sizeof(float) * tiles_len(m)) != hipSuccess ||
+        hipMalloc((void **)&m->fvec, sizeof(float) * FUSED_WGS * (4 * (size_t)m->hs + 2)) != hipSuccess ||
+        hipMalloc((void **)&m->fpart, sizeof(float) * FUSED_SLICES * all) != hipSuccess ||
+        hipMalloc((void **)&m->floss, sizeof(float)) != hipSuccess) {
+      ehd_mlp_destroy(m);
+      return EH_ERR_NOMEM;
+    }
+  }
   *out = m;
   return EH_OK;
 }
@@ -356,8 +824,16 @@ void ehd_mlp_destroy(ehd_mlp *m) {
     return;
   (void)hipSetDevice(m->d->device);
   (void)hipStreamSynchronize(m->d->stream);
-  void *bufs[9] = {m->params, m->grads, m->adam_m, m->adam_v, m->part, m->Xd, m->yd, m->permd, m->eloss};
-  for (int k = 0; k < 9; k++)
+  if (m->pstream) {
+    (void)hipStreamSynchronize(m->pstream);
+    (void)hipStreamDestroy(m->pstream);
+  }
+  for (int k = 0; k < 4; k++)
+    if (m->pev[k])
+      (void)hipEventDestroy(m->pev[k]);
+  void *bufs[18] = {m->params, m->grads, m->adam_m, m->adam_v, m->part,   m->Xd,     m->yd,     m->permd,  m->eloss,
+                    m->tiles,  m->fbuf,  m->fvec,   m->fpart,  m->floss,  m->pin[0], m->pin[1], m->pout[0], m->pout[1]};
+  for (int k = 0; k < 18; k++)
     if (bufs[k])
       (void)hipFree(bufs[k]);
   for (int l = 0; l <= MLP_LAYERS; l++) {
@@ -434,9 +910,125 @@ static int backward(ehd_mlp *m, int B, float *loss, float *loss_acc) {
   return EH_OK;
 }
 
+static mlp_net fused_net(const ehd_mlp *m) {
+  mlp_net N;
+  const size_t w0 = (size_t)m->hs * 16 * m->xc, w1 = (size_t)m->hs * m->hs;
+  N.wf[0] = m->tiles;
+  N.wf[1] = m->tiles + w0;
+  N.wb[1] = m->tiles + w0 + w1;
+  N.wf[2] = m->tiles + w0 + 2 * w1;
+  N.wb[2] = m->tiles + w0 + 3 * w1;
+  N.wb[0] = NULL;
+  for (int l = 0; l < 3; l++)
+    N.bias[l] = m->params + m->boff[l];
+  N.w4 = m->params + m->woff[3];
+  N.b4 = m->params + m->boff[3];
+  N.nin = m->nin;
+  N.hidden = m->hidden;
+  N.xc = m->xc;
+  N.xs = m->xs;
+  return N;
+}
+
+static mlp_param fused_param(const ehd_mlp *m) {
+  mlp_param P;
+  const mlp_net N = fused_net(m);
+  memset(&P, 0, sizeof P);
+  P.w = m->params;
+  P.m = m->adam_m;
+  P.v = m->adam_v;
+  for (int l = 0; l < 3; l++) {
+    P.wf[l] = (float *)N.wf[l];
+    P.wb[l] = (float *)N.wb[l];
+  }
+  for (int l = 0; l < MLP_LAYERS; l++) {
+    P.woff[l] = m->woff[l];
+    P.boff[l] = m->boff[l];
+  }
+  P.nin = m->nin;
+  P.hidden = m->hidden;
+  P.hs = m->hs;
+  P.xs = m->xs;
+  P.xc = m->xc;
+  return P;
+}
+
+static int64_t fused_weights(const ehd_mlp *m) { return (int64_t)m->hidden * m->nin + 2 * (int64_t)m->hidden * m->hidden; }
+
+/* the tiled weights, filled after the parameters were set from outside */
+static void fused_tiles(ehd_mlp *m) {
+  if (!m->tiles_stale)
+    return;
+  const int64_t len = (int64_t)tiles_len(m), nw = fused_weights(m);
+  hipLaunchKernelGGL(mlp_zero, dim3((unsigned)((len + 255) / 256)), dim3(256), 0, m->d->stream, m->tiles, len);
+  hipLaunchKernelGGL(mlp_retile, dim3((unsigned)((nw + 255) / 256)), dim3(256), 0, m->d->stream, fused_param(m), nw);
+  m->tiles_stale = 0;
+}
+
+/* buffers for batches of B rows, and the batch that uses them */
+static int fused_batch(ehd_mlp *m, int32_t B, mlp_batch *Q) {
+  if (B > m->fcap) {
+    if (m->fbuf)
+      MCHK(hipFree(m->fbuf));
+    m->fbuf = NULL;
+    m->fcap = 0;
+    MCHK(hipMalloc((void **)&m->fbuf, sizeof(float) * (size_t)B * (m->xs + 6 * (size_t)m->hs)));
+    m->fcap = B;
+  }
+  memset(Q, 0, sizeof *Q);
+  Q->xb = m->fbuf;
+  for (int l = 0; l < 3; l++) {
+    Q->h[l] = m->fbuf + (size_t)B * (m->xs + (size_t)l * m->hs);
+    Q->dz[l] = m->fbuf + (size_t)B * (m->xs + (size_t)(3 + l) * m->hs);
+  }
+  Q->vec = m->fvec;
+  Q->rows = B;
+  return EH_OK;
+}
+
+/* one batch: gradients to P.g, or an Adam step; its loss is added to *loss */
+static void fused_step(ehd_mlp *m, const mlp_param &P, const mlp_batch &Q, float *loss) {
+  const mlp_net N = fused_net(m);
+  hipStream_t st = m->d->stream;
+  int wgs = (Q.rows + 15) / 16;
+  if (wgs > FUSED_WGS)
+    wgs = FUSED_WGS;
+  switch (m->hs / 64) {
+  case 1:
+    hipLaunchKernelGGL((mlp_rows<1, 1, true>), dim3(wgs), dim3(256), 0, st, N, Q);
+    break;
+  case 2:
+    hipLaunchKernelGGL((mlp_rows<2, 1, true>), dim3(wgs), dim3(256), 0, st, N, Q);
+    break;
+  case 3:
+    hipLaunchKernelGGL((mlp_rows<3, 1, true>), dim3(wgs), dim3(256), 0, st, N, Q);
+    break;
+  default:
+    hipLaunchKernelGGL((mlp_rows<4, 1, true>), dim3(wgs), dim3(256), 0, st, N, Q);
+  }
+  /* slices of at least 64 rows, a multiple of the step of 12 */
+  int ns = (Q.rows + 63) / 64;
+  if (ns > FUSED_SLICES)
+    ns = FUSED_SLICES;
+  const int rows = ((Q.rows + ns - 1) / ns + 11) / 12 * 12;
+  ns = (Q.rows + rows - 1) / rows;
+  const int ht = m->hs / 64, tiles = ht * (m->xs / 64) + 2 * ht * ht, per = (tiles + 3) / 4;
+  hipLaunchKernelGGL(mlp_wgrad, dim3(8 * per * ((ns + 7) / 8)), dim3(256), 0, st, Q, m->hs, m->xs, ns, rows, m->fpart);
+  const int64_t nw = fused_weights(m);
+  const int nwb = (int)((nw + 255) / 256), nvb = (4 * m->hs + 2 + 63) / 64;
+  hipLaunchKernelGGL(mlp_update, dim3(nwb + nvb), dim3(256), 0, st, P, m->fpart, ns, m->fvec, wgs, nw, nwb, loss,
+                     (float)Q.rows);
+}
+
+static int fused_grad(ehd_mlp *m, const float *X, const float *y, int32_t B, float *grad, float *loss);
+static int fused_predict(ehd_mlp *m, const float *X, int64_t n, float *prob);
+static int grow_dev(ehd_mlp *m, void **p, int64_t *cap, int64_t count, size_t sz);
+
 int ehd_mlp_grad(ehd_mlp *m, const float *X, const float *y, int32_t B, float *grad, float *loss) {
   int rc;
   MCHK(hipSetDevice(m->d->device));
+  if (m->fused)
+    return fused_grad(m, X, y, B, grad, loss);
   if ((rc = ensure_batch(m, B)))
     return rc;
   MCHK(hipMemcpyAsync(m->act[0], X, sizeof(float) * (size_t)B * m->nin, hipMemcpyHostToDevice, m->d->stream));
@@ -463,6 +1055,96 @@ static int grow_dev(ehd_mlp *m, void **p, int64_t *cap, int64_t count, size_t sz
   return EH_OK;
 }
 
+static int fused_grad(ehd_mlp *m, const float *X, const float *y, int32_t B, float *grad, float *loss) {
+  mlp_batch Q;
+  float h = 0;
+  int rc = fused_batch(m, B, &Q);
+  if (!rc)
+    rc = grow_dev(m, (void **)&m->Xd, &m->data_cap, (int64_t)B * m->nin, sizeof(float));
+  if (!rc)
+    rc = grow_dev(m, (void **)&m->yd, &m->y_cap, B, sizeof(float));
+  if (rc)
+    return rc;
+  Q.X = m->Xd;
+  Q.y = m->yd;
+  mlp_param P = fused_param(m);
+  P.g = m->grads;
+  MCHK(hipMemcpyAsync(m->Xd, X, sizeof(float) * (size_t)B * m->nin, hipMemcpyHostToDevice, m->d->stream));
+  MCHK(hipMemcpyAsync(m->yd, y, sizeof(float) * B, hipMemcpyHostToDevice, m->d->stream));
+  fused_tiles(m);
+  hipLaunchKernelGGL(mlp_zero, dim3(1), dim3(64), 0, m->d->stream, m->floss, (int64_t)1);
+  fused_step(m, P, Q, m->floss);
+  MCHK(hipGetLastError());
+  MCHK(hipMemcpyAsync(&h, m->floss, sizeof(float), hipMemcpyDeviceToHost, m->d->stream));
+  MCHK(hipMemcpyAsync(grad, m->grads, sizeof(float) * m->nparams, hipMemcpyDeviceToHost, m->d->stream));
+  MCHK(hipStreamSynchronize(m->d->stream));
+  if (loss)
+    *loss = h;
+  return EH_OK;
+}
+
+/* chunks of rows: the copies of the next chunk's inputs and the last one's
+ * probabilities run beside a chunk's kernel */
+#define PRED_ROWS 32768
+static int fused_predict(ehd_mlp *m, const float *X, int64_t n, float *prob) {
+  hipStream_t st = m->d->stream;
+  fused_tiles(m);
+  const mlp_net N = fused_net(m);
+  if (!m->pstream) {
+    MCHK(hipStreamCreateWithFlags(&m->pstream, hipStreamNonBlocking));
+    for (int k = 0; k < 4; k++)
+      MCHK(hipEventCreateWithFlags(&m->pev[k], hipEventDisableTiming));
+    for (int k = 0; k < 2; k++) {
+      MCHK(hipMalloc((void **)&m->pin[k], sizeof(float) * (size_t)PRED_ROWS * m->nin));
+      MCHK(hipMalloc((void **)&m->pout[k], sizeof(float) * PRED_ROWS));
+    }
+  }
+  int64_t done = 0; /* probabilities copied out */
+  int c = 0;
+  for (int64_t s0 = 0; s0 < n; s0 += PRED_ROWS, c++) {
+    const int b = (int)(n - s0 < PRED_ROWS ? n - s0 : PRED_ROWS), k = c & 1;
+    mlp_batch Q;
+    memset(&Q, 0, sizeof Q);
+    Q.X = m->pin[k];
+    Q.prob = m->pout[k];
+    Q.rows = b;
+    /* chunk c - 2's kernel is done with this buffer (its results were copied) */
+    MCHK(hipMemcpyAsync(m->pin[k], X + (size_t)s0 * m->nin, sizeof(float) * (size_t)b * m->nin, hipMemcpyHostToDevice,
+                        m->pstream));
+    MCHK(hipEventRecord(m->pev[k], m->pstream));
+    MCHK(hipStreamWaitEvent(st, m->pev[k], 0));
+    switch (m->hs / 64) {
+    case 1:
+      rows_predict<1>(st, N, Q);
+      break;
+    case 2:
+      rows_predict<2>(st, N, Q);
+      break;
+    case 3:
+      rows_predict<3>(st, N, Q);
+      break;
+    default:
+      rows_predict<4>(st, N, Q);
+    }
+    MCHK(hipGetLastError());
+    MCHK(hipEventRecord(m->pev[2 + k], st));
+    if (c > 0) {
+      const int64_t p0 = done;
+      MCHK(hipStreamWaitEvent(m->pstream, m->pev[2 + (k ^ 1)], 0));
+      MCHK(hipMemcpyAsync(prob + p0, m->pout[k ^ 1], sizeof(float) * PRED_ROWS, hipMemcpyDeviceToHost, m->pstream));
+      done = s0;
+    }
+  }
+  if (n > 0) {
+    MCHK(hipStreamWaitEvent(m->pstream, m->pev[2 + ((c - 1) & 1)], 0));
+    MCHK(hipMemcpyAsync(prob + done, m->pout[(c - 1) & 1], sizeof(float) * (size_t)(n - done), hipMemcpyDeviceToHost,
+                        m->pstream));
+  }
+  MCHK(hipStreamSynchronize(m->pstream));
+  MCHK(hipStreamSynchronize(st));
+  return EH_OK;
+}
+
 /* minibatch Adam over n samples (X row-major [n, nin]) for the given epochs;
  * the sample order per epoch is the given permutation table (epochs x n).
  * The training set and the order are copied to the device once; each step
@@ -475,7 +1157,8 @@ int ehd_mlp_train(ehd_mlp *m, const float *X, const float *y, int64_t n, const i
   MCHK(hipSetDevice(m->d->device));
   if (n > 0x7fffffff)
     return EH_ERR_INVALID;
-  if ((rc = ensure_batch(m, B)))
+  mlp_batch Q;
+  if ((rc = m->fused ? fused_batch(m, B, &Q) : ensure_batch(m, B)))
     return rc;
   if ((rc = grow_dev(m, (void **)&m->Xd, &m->data_cap, n * m->nin, sizeof(float))) ||
       (rc = grow_dev(m, (void **)&m->yd, &m->y_cap, n, sizeof(float))) ||
@@ -498,7 +1181,25 @@ int ehd_mlp_train(ehd_mlp *m, const float *X, const float *y, int64_t n, const i
   if (epochs > 0)
     hipLaunchKernelGGL(reduce_slices, dim3((unsigned)((epochs + 255) / 256)), dim3(256), 0, m->d->stream, m->eloss,
                        0, (int64_t)epochs, m->eloss); /* zero the per-epoch sums (a kernel, no memset) */
-  for (int ep = 0; ep < epochs; ep++) {
+  if (m->fused) {
+    mlp_param P = fused_param(m);
+    P.lr = lr;
+    P.b1 = 0.9f;
+    P.b2 = 0.999f;
+    P.eps = 1e-8f;
+    Q.X = m->Xd;
+    Q.y = m->yd;
+    fused_tiles(m);
+    for (int ep = 0; ep < epochs; ep++)
+      for (int64_t st = 0; st < nsteps; st++) {
+        Q.perm = m->permd + (int64_t)ep * n + st * B;
+        m->step++;
+        P.c1 = 1.f - powf(0.9f, (float)m->step);
+        P.c2 = 1.f - powf(0.999f, (float)m->step);
+        fused_step(m, P, Q, m->eloss + ep);
+      }
+  }
+  for (int ep = 0; ep < epochs && !m->fused; ep++) {
     for (int64_t st = 0; st < nsteps; st++) {
       const int64_t e = (int64_t)B * m->nin;
       hipLaunchKernelGGL(gather_batch, dim3((unsigned)((e + 255) / 256)), dim3(256), 0, m->d->stream, m->Xd, m->yd,
@@ -527,6 +1228,8 @@ int ehd_mlp_predict(ehd_mlp *m, const float *X, int64_t n, float *prob) {
   int rc;
   const int32_t B = 8192;
   MCHK(hipSetDevice(m->d->device));
+  if (m->fused)
+    return fused_predict(m, X, n, prob);
   if ((rc = ensure_batch(m, B)))
     return rc;
   for (int64_t s0 = 0; s0 < n; s0 += B) {
@@ -544,6 +1247,8 @@ int ehd_mlp_predict(ehd_mlp *m, const float *X, int64_t n, float *prob) {
 
 int ehd_mlp_params(ehd_mlp *m, float *buf, int set) {
   MCHK(hipSetDevice(m->d->device));
+  if (set)
+    m->tiles_stale = 1;
   if (set)
     MCHK(hipMemcpy(m->params, buf, sizeof(float) * m->nparams, hipMemcpyHostToDevice));
   else
