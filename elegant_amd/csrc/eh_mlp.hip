@@ -210,7 +210,7 @@ __global__ void adam_k(float *w, const float *g, float *m, float *v, int64_t n, 
  * (v_mfma_f32_16x16x4f32: FP32 multiplies and sums, as the LDS-tiled gemm_f32
  * has, which stays for larger nets).  What bounds it: 3.3 GFLOP per step of 4096
  * samples is 22 us at the 150 TFLOP/s of a large FP32 product; the step was 35
- * launches and 470 us, and takes @S@ us.
+ * launches and 470 us, and takes 67 (36 + 23 + 8).
  *
  * Layouts.  HS = hidden rounded up to 64, XS = inputs rounded up to 64; padded
  * weights are zero, so padded activations and gradients are zero.  A
@@ -236,41 +236,56 @@ struct mlp_batch {
   int rows;
 };
 
-/* acc[mt][t] += rows of a (LDS, stride lda) x tile wave + 4 t of wt, kc
- * chunks; the weights of the next two chunks are in flight (a workgroup is
- * alone on its CU, one wave per SIMD) */
-template <int NT, int MT>
+/* acc[mt][t] += rows of a (LDS, stride lda) x tile wave + 4 t of wt, over kc
+ * chunks.  A workgroup is alone on its CU, one wave per SIMD, so D chunks of
+ * weights are in flight; and the workgroups of an XCD (every eighth) start at
+ * different chunks, so that each finds most of its weights already in the
+ * XCD's L2 instead of all of them waiting for the same lines at once. */
+template <int NT, int MT, int D>
 static __device__ __forceinline__ void rows_mm(const float *a, int lda, const float *__restrict__ wt, int kc,
                                                f4 (&acc)[MT][NT]) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  /* opaque: the addresses of every layer's chunks are otherwise computed ahead
+   * of the loop over rows and spilled */
+  asm volatile("" : "+v"(lane));
   const float *ar = a + (lane & 15) * lda + 4 * (lane >> 4);
   const float *w0 = wt + (size_t)wave * kc * 256 + 4 * lane;
-  f4 b0[NT], b1[NT];
+  int first = (int)((blockIdx.x >> 3) % (unsigned)kc), cl = first, ca = first; /* chunks to load and to use */
+  f4 b[D][NT];
 #pragma unroll
-  for (int t = 0; t < NT; t++) {
-    b0[t] = *(const f4 *)(w0 + (size_t)4 * t * kc * 256);
-    b1[t] = *(const f4 *)(w0 + (size_t)4 * t * kc * 256 + (kc > 1 ? 256 : 0));
-  }
-  for (int c = 0; c < kc; c++) {
-    f4 b2[NT], av[MT];
-    const int cn = c + 2 < kc ? c + 2 : kc - 1;
+  for (int u = 0; u < D; u++) {
 #pragma unroll
     for (int t = 0; t < NT; t++)
-      b2[t] = *(const f4 *)(w0 + ((size_t)4 * t * kc + cn) * 256);
+      b[u][t] = *(const f4 *)(w0 + ((size_t)4 * t * kc + cl) * 256);
+    cl = cl + 1 < kc ? cl + 1 : 0;
+  }
+  f4 av[2][MT]; /* the next chunk's rows are read while a chunk's products run */
 #pragma unroll
-    for (int m = 0; m < MT; m++)
-      av[m] = *(const f4 *)(ar + 16 * m * lda + 16 * c);
+  for (int m = 0; m < MT; m++)
+    av[0][m] = *(const f4 *)(ar + 16 * m * lda + 16 * ca);
+  for (int c = 0; c < kc; c += D) {
 #pragma unroll
-    for (int k = 0; k < 4; k++)
+    for (int u = 0; u < D; u++) {
+      ca = ca + 1 < kc ? ca + 1 : 0;
 #pragma unroll
       for (int m = 0; m < MT; m++)
+        av[D > 1 ? (u + 1) & 1 : 1][m] = *(const f4 *)(ar + 16 * m * lda + 16 * ca);
 #pragma unroll
-        for (int t = 0; t < NT; t++)
-          acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[m][k], b0[t][k], acc[m][t], 0, 0, 0);
+      for (int k = 0; k < 4; k++)
 #pragma unroll
-    for (int t = 0; t < NT; t++) {
-      b0[t] = b1[t];
-      b1[t] = b2[t];
+        for (int m = 0; m < MT; m++)
+#pragma unroll
+          for (int t = 0; t < NT; t++)
+            acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[D > 1 ? u & 1 : 0][m][k], b[u][t][k], acc[m][t], 0, 0, 0);
+#pragma unroll
+      for (int t = 0; t < NT; t++)
+        b[u][t] = *(const f4 *)(w0 + ((size_t)4 * t * kc + cl) * 256);
+      cl = cl + 1 < kc ? cl + 1 : 0;
+      if (D == 1)
+#pragma unroll
+        for (int m = 0; m < MT; m++)
+          av[0][m] = av[1][m];
     }
   }
 }
@@ -289,26 +304,76 @@ static __device__ __forceinline__ void rows_out(const float *a, int lda, float *
 /* TRAIN: forward, loss, backward of 16 rows at a time (MT = 1); else the
  * probabilities of 16 MT rows.  Workgroups stride over the batch. */
 template <int NT, int MT, bool TRAIN>
-__global__ void __launch_bounds__(256) mlp_rows(mlp_net N, mlp_batch Q) {
+__global__ void __launch_bounds__(256, TRAIN ? 1 : 2) mlp_rows(mlp_net N, mlp_batch Q) {
   constexpr int HS = 64 * NT, R = 16 * MT, LD = HS + 4, LX = 260;
   __shared__ float sx[TRAIN ? R * LX : R * (LX > LD ? LX : LD)];
   __shared__ float sh[TRAIN ? 3 : 1][R * LD];
-  __shared__ float sz[R], sd[R];
+  __shared__ float sz[R], sd[R], sy[R];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   float vs[4] = {0, 0, 0, 0}, vb4 = 0, vloss = 0;
+  /* biases and the last layer's weights, loaded once and together (indices
+   * clamped, no load behind a branch): each would cost a trip to L2 where it
+   * is used */
+  constexpr int P = 256 / R; /* threads per row in the last layer */
+  float bias[3][NT], w4[HS / P];
+#pragma unroll
+  for (int l = 0; l < 3; l++)
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+      const int c = 16 * (wave + 4 * t) + (lane & 15);
+      bias[l][t] = N.bias[l][c < N.hidden ? c : 0];
+    }
+#pragma unroll
+  for (int u = 0; u < HS / P; u++)
+    w4[u] = N.w4[tid % P + P * u < N.hidden ? tid % P + P * u : 0];
+  float b4 = N.b4[0], w4c = N.w4[tid < N.hidden ? tid : 0];
+  w4c = tid < N.hidden ? w4c : 0.f;
+#pragma unroll
+  for (int u = 0; u < HS / P; u++)
+    w4[u] = tid % P + P * u < N.hidden ? w4[u] : 0.f;
+#pragma unroll
+  for (int l = 0; l < 3; l++)
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+      bias[l][t] = 16 * (wave + 4 * t) + (lane & 15) < N.hidden ? bias[l][t] : 0.f;
   for (int r0 = blockIdx.x * R; r0 < Q.rows; r0 += gridDim.x * R) {
-    /* the rows' inputs, zero beyond the net's and beyond the batch */
-    const int xw = TRAIN ? N.xs : 16 * N.xc;
-    for (int e = tid; e < R * xw; e += 256) {
-      const int r = e / xw, k = e % xw;
-      float v = 0.f;
-      if (r0 + r < Q.rows && k < N.nin) {
-        const int64_t j = Q.perm ? Q.perm[r0 + r] : r0 + r;
-        v = Q.X[j * N.nin + k];
+    /* the rows' inputs, zero beyond the net's and beyond the batch: 16 threads
+     * per row, the sample's index first, then its inputs together */
+    {
+      const int q = tid & 15, xw = TRAIN ? N.xs : 16 * N.xc;
+      int64_t j[MT];
+#pragma unroll
+      for (int m = 0; m < MT; m++) {
+        const int r = r0 + 16 * m + (tid >> 4), rc = r < Q.rows ? r : Q.rows - 1;
+        j[m] = Q.perm ? Q.perm[rc] : rc;
       }
-      sx[r * LX + k] = v;
-      if (TRAIN && r0 + r < Q.rows)
-        Q.xb[(size_t)(r0 + r) * N.xs + k] = v;
+      float yv = 0.f;
+      if (TRAIN)
+        yv = Q.y[j[0]];
+      for (int k0 = 0; k0 < xw; k0 += 64) {
+        float v[MT][4];
+#pragma unroll
+        for (int m = 0; m < MT; m++)
+#pragma unroll
+          for (int u = 0; u < 4; u++) {
+            const int k = k0 + q + 16 * u;
+            v[m][u] = Q.X[j[m] * N.nin + (k < N.nin ? k : N.nin - 1)];
+          }
+#pragma unroll
+        for (int m = 0; m < MT; m++)
+#pragma unroll
+          for (int u = 0; u < 4; u++) {
+            const int k = k0 + q + 16 * u, r = 16 * m + (tid >> 4);
+            const bool on = r0 + r < Q.rows && k < N.nin;
+            if (k < xw) {
+              sx[r * LX + k] = on ? v[m][u] : 0.f;
+              if (TRAIN && r0 + r < Q.rows)
+                Q.xb[(size_t)(r0 + r) * N.xs + k] = on ? v[m][u] : 0.f;
+            }
+          }
+      }
+      if (TRAIN && q == 0)
+        sy[tid >> 4] = yv;
     }
     __syncthreads();
 #pragma unroll
@@ -323,11 +388,14 @@ __global__ void __launch_bounds__(256) mlp_rows(mlp_net N, mlp_batch Q) {
 #pragma unroll
         for (int t = 0; t < NT; t++)
           acc[m][t] = (f4){0.f, 0.f, 0.f, 0.f};
-      rows_mm<NT, MT>(in, lin, N.wf[l], l == 0 ? N.xc : HS / 16, acc);
+      if (l == 0)
+        rows_mm<NT, MT, 1>(in, lin, N.wf[l], N.xc, acc);
+      else
+        rows_mm<NT, MT, 4>(in, lin, N.wf[l], HS / 16, acc);
 #pragma unroll
       for (int t = 0; t < NT; t++) {
         const int c = 16 * (wave + 4 * t) + (lane & 15);
-        const float b = c < N.hidden ? N.bias[l][c] : 0.f;
+        const float b = bias[l][t];
 #pragma unroll
         for (int m = 0; m < MT; m++)
 #pragma unroll
@@ -343,23 +411,23 @@ __global__ void __launch_bounds__(256) mlp_rows(mlp_net N, mlp_batch Q) {
     /* the last layer: 256 / R threads per row */
     const float *h3 = TRAIN ? sh[2] : sh[0];
     {
-      constexpr int P = 256 / R;
       const int r = tid / P, q = tid % P;
       float v = 0.f;
-      for (int c = q; c < N.hidden; c += P)
-        v = fmaf(h3[r * LD + c], N.w4[c], v);
+#pragma unroll
+      for (int u = 0; u < HS / P; u++)
+        v = fmaf(h3[r * LD + q + P * u], w4[u], v);
 #pragma unroll
       for (int o = P / 2; o > 0; o >>= 1)
         v += __shfl_xor(v, o);
       if (q == 0) {
-        const float z = v + N.b4[0];
+        const float z = v + b4;
         if (!TRAIN) {
           if (r0 + r < Q.rows)
             Q.prob[r0 + r] = 1.f / (1.f + expf(-z));
         } else {
           float l = 0.f, d = 0.f;
           if (r0 + r < Q.rows) {
-            const float yi = Q.y[Q.perm ? Q.perm[r0 + r] : r0 + r];
+            const float yi = sy[r];
             const float sp = z > 0 ? z + log1pf(expf(-z)) : log1pf(expf(z)); /* softplus */
             l = sp - yi * z;
             d = (1.f / (1.f + expf(-z)) - yi) / (float)Q.rows;
@@ -373,6 +441,7 @@ __global__ void __launch_bounds__(256) mlp_rows(mlp_net N, mlp_batch Q) {
     if (TRAIN) {
       if (tid < HS) {
         float s = 0.f;
+#pragma unroll
         for (int r = 0; r < R; r++)
           s = fmaf(sd[r], sh[2][r * LD + tid], s);
         vs[3] += s;
@@ -388,17 +457,17 @@ __global__ void __launch_bounds__(256) mlp_rows(mlp_net N, mlp_batch Q) {
       }
       __syncthreads();
       /* dz3 in place of h3, then dz2 in place of h2, dz1 of h1 */
-      for (int e = tid; e < R * HS; e += 256) {
-        const int r = e / HS, c = e % HS;
-        const float w = c < N.hidden ? N.w4[c] : 0.f;
-        sh[2][r * LD + c] = sh[2][r * LD + c] > 0.f ? sd[r] * w : 0.f;
-      }
+      if (tid < HS)
+#pragma unroll
+        for (int r = 0; r < R; r++)
+          sh[2][r * LD + tid] = sh[2][r * LD + tid] > 0.f ? sd[r] * w4c : 0.f;
       __syncthreads();
 #pragma unroll
       for (int l = 2; l >= 0; l--) {
         rows_out<HS>(sh[l], LD, Q.dz[l], r0, R, Q.rows);
         if (tid < HS) {
           float s = 0.f;
+#pragma unroll
           for (int r = 0; r < R; r++)
             s += sh[l][r * LD + tid];
           vs[l] += s;
@@ -410,7 +479,7 @@ __global__ void __launch_bounds__(256) mlp_rows(mlp_net N, mlp_batch Q) {
 #pragma unroll
             for (int t = 0; t < NT; t++)
               acc[m][t] = (f4){0.f, 0.f, 0.f, 0.f};
-          rows_mm<NT, MT>(sh[l], LD, N.wb[l], HS / 16, acc);
+          rows_mm<NT, MT, 4>(sh[l], LD, N.wb[l], HS / 16, acc);
 #pragma unroll
           for (int t = 0; t < NT; t++) {
             const int c = 16 * (wave + 4 * t) + (lane & 15);
@@ -446,7 +515,8 @@ __global__ void __launch_bounds__(256) mlp_rows(mlp_net N, mlp_batch Q) {
  * 16-byte load each: tile row 4 i + rt is row i of product rt, so a lane's four
  * elements feed four products.  The tiles of one slice read the same rows, so
  * a slice stays on one XCD (workgroups go round the 8 of them). */
-__global__ void __launch_bounds__(256) mlp_wgrad(mlp_batch Q, int hs, int xs, int nslice, int slice_rows, float *part) {
+#define WG_D 6
+__global__ void __launch_bounds__(256, 1) mlp_wgrad(mlp_batch Q, int hs, int xs, int nslice, int slice_rows, float *part) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int ht = hs / 64, t0 = ht * (xs / 64), tiles = t0 + 2 * ht * ht, wgs = (tiles + 3) / 4;
   const int xcd = blockIdx.x % 8, j = blockIdx.x / 8;
@@ -473,21 +543,21 @@ __global__ void __launch_bounds__(256) mlp_wgrad(mlp_batch Q, int hs, int xs, in
 #pragma unroll
     for (int k = 0; k < 4; k++)
       acc[i][k] = (f4){0.f, 0.f, 0.f, 0.f};
-  /* three steps' operands in flight; rows past the slice count as zero */
-  f4 av[3], bv[3];
+  /* WG_D steps' operands in flight; rows past the slice count as zero */
+  f4 av[WG_D], bv[WG_D];
 #pragma unroll
-  for (int u = 0; u < 3; u++) {
+  for (int u = 0; u < WG_D; u++) {
     const int r = b0 + 4 * u + g, rc = r < b1 ? r : b0;
     av[u] = *(const f4 *)(pa + (size_t)rc * hs);
     bv[u] = *(const f4 *)(pb + (size_t)rc * ks);
   }
-  for (int b = b0; b < b1; b += 12) {
+  for (int b = b0; b < b1; b += 4 * WG_D) {
 #pragma unroll
-    for (int u = 0; u < 3; u++) {
+    for (int u = 0; u < WG_D; u++) {
       f4 a = av[u], v = bv[u];
       if (b + 4 * u + g >= b1)
         a = (f4){0.f, 0.f, 0.f, 0.f};
-      const int r = b + 12 + 4 * u + g, rc = r < b1 ? r : b0;
+      const int r = b + 4 * WG_D + 4 * u + g, rc = r < b1 ? r : b0;
       av[u] = *(const f4 *)(pa + (size_t)rc * hs);
       bv[u] = *(const f4 *)(pb + (size_t)rc * ks);
 #pragma unroll
@@ -1006,11 +1076,11 @@ static void fused_step(ehd_mlp *m, const mlp_param &P, const mlp_batch &Q, float
   default:
     hipLaunchKernelGGL((mlp_rows<4, 1, true>), dim3(wgs), dim3(256), 0, st, N, Q);
   }
-  /* slices of at least 64 rows, a multiple of the step of 12 */
+  /* slices of at least 64 rows, a multiple of the step */
   int ns = (Q.rows + 63) / 64;
   if (ns > FUSED_SLICES)
     ns = FUSED_SLICES;
-  const int rows = ((Q.rows + ns - 1) / ns + 11) / 12 * 12;
+  const int rows = ((Q.rows + ns - 1) / ns + 4 * WG_D - 1) / (4 * WG_D) * (4 * WG_D);
   ns = (Q.rows + rows - 1) / rows;
   const int ht = m->hs / 64, tiles = ht * (m->xs / 64) + 2 * ht * ht, per = (tiles + 3) / 4;
   hipLaunchKernelGGL(mlp_wgrad, dim3(8 * per * ((ns + 7) / 8)), dim3(256), 0, st, Q, m->hs, m->xs, ns, rows, m->fpart);
