@@ -1019,38 +1019,70 @@ void ehd_free_collective(ehd_dev *d) {
   d->bunch_cap = 0;
 }
 
+/* the tables go through the stream the steps run on, behind the steps that
+ * still read the old ones */
+static int put_table(ehd_dev *d, double *dst, const double *src, int64_t count) {
+  CHK(hipMemcpyAsync(dst, src, sizeof(double) * (size_t)count, hipMemcpyHostToDevice, d->stream));
+  return EH_OK;
+}
+
 int ehd_put_wake(ehd_dev *d, int32_t slot, const double *W, int64_t npoints) {
   if (slot < 0 || slot >= EHD_MAX_COLL || npoints < 2)
     return EH_ERR_INVALID;
   ehd_coll_slot *sl = &d->slot[slot];
   CHK(hipSetDevice(d->device));
-  if (sl->W)
-    CHK(hipFree(sl->W));
-  sl->W = NULL;
-  CHK(hipMalloc((void **)&sl->W, sizeof(double) * npoints));
-  CHK(hipMemcpy(sl->W, W, sizeof(double) * npoints, hipMemcpyHostToDevice));
+  if (npoints > sl->W_cap) {
+    if (sl->W)
+      CHK(hipFree(sl->W));
+    sl->W = NULL;
+    sl->W_cap = 0;
+    CHK(hipMalloc((void **)&sl->W, sizeof(double) * npoints));
+    sl->W_cap = npoints;
+  }
+  int rc = put_table(d, sl->W, W, npoints);
+  if (rc)
+    return rc;
+  CHK(hipStreamSynchronize(d->stream));
   sl->wpoints = npoints;
   return EH_OK;
+}
+
+int32_t ehd_twiddle_bins(const ehd_dev *d, int32_t slot) {
+  return slot >= 0 && slot < EHD_MAX_COLL ? d->slot[slot].tw_nb : 0;
 }
 
 int ehd_put_zlongit(ehd_dev *d, int32_t slot, const double *Z, const double *tc, const double *ts, int32_t nb) {
   if (slot < 0 || slot >= EHD_MAX_COLL || nb < 4 || nb > EHD_ZL_MAX_BINS || (nb & (nb - 1)))
     return EH_ERR_INVALID;
   ehd_coll_slot *sl = &d->slot[slot];
+  if ((!tc || !ts) && sl->tw_nb != nb)
+    return EH_ERR_STATE;
   CHK(hipSetDevice(d->device));
-  if (sl->Z)
-    CHK(hipFree(sl->Z));
-  if (sl->tc)
-    CHK(hipFree(sl->tc));
-  if (sl->ts)
-    CHK(hipFree(sl->ts));
-  sl->Z = sl->tc = sl->ts = NULL;
-  CHK(hipMalloc((void **)&sl->Z, sizeof(double) * nb));
-  CHK(hipMalloc((void **)&sl->tc, sizeof(double) * (nb / 2 + 1)));
-  CHK(hipMalloc((void **)&sl->ts, sizeof(double) * (nb / 2 + 1)));
-  CHK(hipMemcpy(sl->Z, Z, sizeof(double) * nb, hipMemcpyHostToDevice));
-  CHK(hipMemcpy(sl->tc, tc, sizeof(double) * (nb / 2 + 1), hipMemcpyHostToDevice));
-  CHK(hipMemcpy(sl->ts, ts, sizeof(double) * (nb / 2 + 1), hipMemcpyHostToDevice));
+  int rc = EH_OK;
+  if (nb > sl->Z_cap) {
+    double **buf[3] = {&sl->Z, &sl->tc, &sl->ts};
+    sl->Z_cap = 0;
+    sl->tw_nb = 0;
+    for (int k = 0; k < 3; k++) {
+      if (*buf[k])
+        CHK(hipFree(*buf[k]));
+      *buf[k] = NULL;
+      CHK(hipMalloc((void **)buf[k], sizeof(double) * (k ? nb / 2 + 1 : nb)));
+    }
+    sl->Z_cap = nb;
+  }
+  rc = put_table(d, sl->Z, Z, nb);
+  if (tc && ts) {
+    sl->tw_nb = 0;
+    if (!rc)
+      rc = put_table(d, sl->tc, tc, nb / 2 + 1);
+    if (!rc)
+      rc = put_table(d, sl->ts, ts, nb / 2 + 1);
+  }
+  if (rc)
+    return rc;
+  CHK(hipStreamSynchronize(d->stream));
+  sl->tw_nb = nb;
   sl->nb = nb;
   return EH_OK;
 }

@@ -30,6 +30,28 @@ int ehd_get_state(ehd_dev *d, double *x, double *xp, double *y, double *yp, doub
 int ehd_get_sdp(ehd_dev *d, double *s, double *dp, int32_t *loss_pass, int64_t n);
 int64_t ehd_state_n(const ehd_dev *d);
 
+/* Rows (AoS, as the caller holds them) moved whole and turned into columns on
+ * the device.  ehd_put_rows copies n rows of w columns, sets the loss records
+ * (with cull, rows with a NaN or infinite x or y are lost before the first
+ * element, do_tracking.c:468-473) and keeps the rows; the copy may still run
+ * when it returns.  ehd_get_rows brings back rows of 8 columns in the given
+ * order (NULL: as uploaded) with column 7 = pass of loss.  ehd_rows_back
+ * writes columns 0..5 into the kept rows, ehd_fetch_rows copies the kept rows
+ * out in the given order. */
+int ehd_put_rows(ehd_dev *d, const double *rows, int64_t n, int32_t w, int cull, double Po);
+int ehd_get_rows(ehd_dev *d, double *out, int64_t n, const int32_t *order);
+int ehd_rows_back(ehd_dev *d);
+int ehd_fetch_rows(ehd_dev *d, double *out, const int32_t *order);
+/* the same for few rows, with their loss records, in one copy into a pinned
+ * buffer of the context (valid until its next call): NULL rows if they do not fit */
+int ehd_fetch_small(ehd_dev *d, const double **rows, const int32_t **loss_pass, const int32_t **loss_code);
+/* arrival times (s + ahead) / (c beta) of all slots, as simple_rfca.c:198-204 forms them */
+int ehd_fiducial_times(ehd_dev *d, double Po, double ahead, double *t);
+/* sums over the particles not lost before pass0: passes completed and those alive */
+int ehd_effort(ehd_dev *d, int64_t pass0, int64_t end, int64_t *effort, int64_t *left);
+/* one pass of one element, without timing events */
+int ehd_track_single(ehd_dev *d, int64_t pass);
+
 /* program: ehd_put_ops loads the flat record array the batch kernel reads
  * (eh_vdesc offsets into it); ehd_put_program loads the tracking kernel's
  * program, folded into runs of repeated cells (eh_fold_runs), and
@@ -99,6 +121,8 @@ typedef struct {
 
 /* WAKE Green function samples; ZLONGIT impedance Z[nb] and twiddles */
 int ehd_put_wake(ehd_dev *d, int32_t slot, const double *W, int64_t npoints);
+/* tc, ts NULL: the slot's twiddles are for nb bins already */
+int32_t ehd_twiddle_bins(const ehd_dev *d, int32_t slot);
 int ehd_put_zlongit(ehd_dev *d, int32_t slot, const double *Z, const double *tc, const double *ts, int32_t nb);
 /* one WAKE or ZLONGIT step on all alive particles.  Returns EH_ERR_LONGBEAM if the
  * bunch is longer than allowed.  hist/volt (optional, may be NULL) receive the

@@ -1681,6 +1681,129 @@ __global__ void __launch_bounds__(256, 4) eh_batch_kernel(eh_state st, const eh_
 
 __global__ void eh_queue_reset(unsigned int *queue) { *queue = 0u; }
 
+/* ---- rows <-> columns ----
+ * One thread a row: both sides are streamed once (128 B a row, about 30 us for
+ * 10^6 rows), against 6 ms for the copies to and from the host around them,
+ * so nothing is staged through LDS. */
+
+/* columns from rows; the loss records start here, and with cull rows with a
+ * NaN or infinite x or y are lost before the first element */
+__global__ void __launch_bounds__(256) rows_in(const double *__restrict__ rows, int64_t n, int32_t w, int32_t cull,
+                                               double Po, eh_state st, double *ids) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n)
+    return;
+  const double *r = rows + i * w;
+  double v[7];
+#pragma unroll
+  for (int k = 0; k < 7; k++)
+    v[k] = r[k];
+  const bool bad = cull && (__builtin_isinf(v[0]) || __builtin_isinf(v[2]) || __builtin_isnan(v[0]) ||
+                            __builtin_isnan(v[2]));
+  if (bad) {
+    /* limit_amplitudes(DBL_MAX) at z = 0: s = 0, delta = Po(1+delta) */
+    v[4] = 0.0;
+    v[5] = Po * (1 + v[5]);
+  }
+  st.x[i] = v[0];
+  st.xp[i] = v[1];
+  st.y[i] = v[2];
+  st.yp[i] = v[3];
+  st.s[i] = v[4];
+  st.dp[i] = v[5];
+  ids[i] = v[6];
+  st.loss_pass[i] = bad ? 0 : -1;
+  st.loss_code[i] = bad ? -1 : 0;
+}
+
+/* columns 0..5 back into the rows, the loss records behind the last row */
+__global__ void __launch_bounds__(256) rows_back(double *rows, int32_t w, eh_state st) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= st.n)
+    return;
+  double *r = rows + i * w;
+  int32_t *rec = (int32_t *)(rows + st.n * w);
+  r[0] = st.x[i];
+  r[1] = st.xp[i];
+  r[2] = st.y[i];
+  r[3] = st.yp[i];
+  r[4] = st.s[i];
+  r[5] = st.dp[i];
+  rec[i] = st.loss_pass[i];
+  rec[st.n + i] = st.loss_code[i];
+}
+
+/* rows of 8 columns in the given order, column 7 = pass of loss */
+__global__ void __launch_bounds__(256) rows_out(double *__restrict__ out, eh_state st, const double *__restrict__ ids,
+                                                const int32_t *__restrict__ order) {
+  const int64_t j = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (j >= st.n)
+    return;
+  const int64_t i = order ? order[j] : j;
+  double *r = out + 8 * j;
+  r[0] = st.x[i];
+  r[1] = st.xp[i];
+  r[2] = st.y[i];
+  r[3] = st.yp[i];
+  r[4] = st.s[i];
+  r[5] = st.dp[i];
+  r[6] = ids[i];
+  r[7] = st.loss_pass[i] >= 0 ? (double)st.loss_pass[i] : -1.0;
+}
+
+/* whole rows in the given order */
+__global__ void __launch_bounds__(256) rows_gather(const double *__restrict__ in, double *__restrict__ out, int64_t n,
+                                                   int32_t w, const int32_t *__restrict__ order) {
+  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (e >= n * w)
+    return;
+  out[e] = in[(int64_t)order[e / w] * w + e % w];
+}
+
+__global__ void __launch_bounds__(256) fiducial_times(eh_state st, double Po, double ahead, double *t) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= st.n)
+    return;
+  const double p = Po * (1 + st.dp[i]);
+  const double beta = p / __builtin_sqrt(p * p + 1);
+  t[i] = (st.s[i] + ahead) / (EH_C_MKS * beta);
+}
+
+/* out[0] += passes completed from pass0 on, out[1] += particles alive.  One
+ * pair of atomics per workgroup: with a pair per wave, all on one line, 10^6
+ * records took 102 us */
+__global__ void __launch_bounds__(256) effort_sum(const int32_t *__restrict__ lp, int64_t n, int64_t pass0, int64_t end,
+                                                  unsigned long long *out) {
+  __shared__ unsigned long long we[4], wa[4];
+  unsigned long long e = 0, a = 0;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+    const int64_t l = lp[i];
+    if (l < 0) {
+      e += (unsigned long long)(end - pass0);
+      a++;
+    } else if (l >= pass0)
+      e += (unsigned long long)(l - pass0);
+  }
+  for (int off = 32; off > 0; off >>= 1) {
+    e += __shfl_xor(e, off);
+    a += __shfl_xor(a, off);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    we[threadIdx.x >> 6] = e;
+    wa[threadIdx.x >> 6] = a;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    atomicAdd(&out[0], we[0] + we[1] + we[2] + we[3]);
+    atomicAdd(&out[1], wa[0] + wa[1] + wa[2] + wa[3]);
+  }
+}
+
+__global__ void clear_counters(unsigned long long *c) {
+  if (threadIdx.x < 2)
+    c[threadIdx.x] = 0;
+}
+
 /* ------------------------------------------------------------ host side */
 
 extern "C" {
@@ -1727,6 +1850,8 @@ int ehd_create(int device, ehd_dev **out, char *msg, int msglen) {
     e = hipEventCreate(&d->cev0);
   if (e == hipSuccess)
     e = hipEventCreate(&d->cev1);
+  if (e == hipSuccess)
+    e = hipEventCreateWithFlags(&d->pev, hipEventDisableTiming);
   if (e != hipSuccess) {
     if (msg && msglen > 0)
       snprintf(msg, msglen, "HIP set-up failed: %s", hipGetErrorString(e));
@@ -1755,12 +1880,17 @@ void ehd_destroy(ehd_dev *d) {
   void *bufs[] = {d->coord[0], d->coord[1], d->coord[2], d->coord[3], d->coord[4], d->coord[5],
                   d->loss_pass, d->loss_code, d->ops, d->counter, d->vdesc, d->chunks, d->perm, d->queue,
                   d->snap[0], d->snap[1], d->snap[2], d->snap[3], d->snap[4], d->snap[5], d->snap_lp, d->snap_lc,
-                  d->tile_sum, d->tops, d->runs, d->zpos};
+                  d->tile_sum, d->pbuf, d->ids, d->rows, d->rows2, d->order};
   for (size_t k = 0; k < sizeof(bufs) / sizeof(bufs[0]); k++)
     if (bufs[k])
       (void)hipFree(bufs[k]);
   ehd_free_collective(d);
   free(d->host_prog);
+  if (d->pstage)
+    (void)hipHostFree(d->pstage);
+  if (d->pin)
+    (void)hipHostFree(d->pin);
+  (void)hipEventDestroy(d->pev);
   (void)hipEventDestroy(d->ev0);
   (void)hipEventDestroy(d->ev1);
   (void)hipEventDestroy(d->cev0);
@@ -1781,12 +1911,16 @@ int ehd_alloc_state(ehd_dev *d, int64_t n) {
       HIPCHK(d, hipFree(d->loss_pass));
     if (d->loss_code)
       HIPCHK(d, hipFree(d->loss_code));
+    if (d->ids)
+      HIPCHK(d, hipFree(d->ids));
     d->loss_pass = d->loss_code = NULL;
+    d->ids = NULL;
     d->cap = 0;
     for (int k = 0; k < 6; k++)
       HIPCHK(d, hipMalloc((void **)&d->coord[k], sizeof(double) * (n > 0 ? n : 1)));
     HIPCHK(d, hipMalloc((void **)&d->loss_pass, sizeof(int32_t) * (n > 0 ? n : 1)));
     HIPCHK(d, hipMalloc((void **)&d->loss_code, sizeof(int32_t) * (n > 0 ? n : 1)));
+    HIPCHK(d, hipMalloc((void **)&d->ids, sizeof(double) * (n > 0 ? n : 1)));
     d->cap = n;
   }
   if (!d->counter)
@@ -1847,6 +1981,150 @@ int ehd_get_sdp(ehd_dev *d, double *s, double *dp, int32_t *loss_pass, int64_t n
   return ehd_get_state(d, NULL, NULL, NULL, NULL, s, dp, loss_pass, NULL, n);
 }
 
+static eh_state state_of(const ehd_dev *d) {
+  eh_state st;
+  st.x = d->coord[0];
+  st.xp = d->coord[1];
+  st.y = d->coord[2];
+  st.yp = d->coord[3];
+  st.s = d->coord[4];
+  st.dp = d->coord[5];
+  st.loss_pass = d->loss_pass;
+  st.loss_code = d->loss_code;
+  st.n = d->n;
+  return st;
+}
+
+static int grow_rows(ehd_dev *d, double **p, int64_t *cap, int64_t count) {
+  if (count <= *cap)
+    return EH_OK;
+  if (*p)
+    HIPCHK(d, hipFree(*p));
+  *p = NULL;
+  *cap = 0;
+  HIPCHK(d, hipMalloc((void **)p, sizeof(double) * (size_t)count));
+  *cap = count;
+  return EH_OK;
+}
+
+#define ROW_GRID(n) dim3((unsigned)(((n) + 255) / 256))
+
+int ehd_put_rows(ehd_dev *d, const double *rows, int64_t n, int32_t w, int cull, double Po) {
+  int rc = ehd_alloc_state(d, n);
+  if (rc || n == 0)
+    return rc;
+  rc = grow_rows(d, &d->rows, &d->rows_cap, n * (w + 1)); /* and the loss records behind them */
+  if (rc)
+    return rc;
+  d->rows_w = w;
+  HIPCHK(d, hipMemcpyAsync(d->rows, rows, sizeof(double) * (size_t)(n * w), hipMemcpyHostToDevice, d->stream));
+  hipLaunchKernelGGL(rows_in, ROW_GRID(n), dim3(256), 0, d->stream, d->rows, n, w, cull, Po, state_of(d), d->ids);
+  HIPCHK(d, hipGetLastError());
+  return EH_OK;
+}
+
+static int put_order(ehd_dev *d, const int32_t *order, int64_t n) {
+  if (n > d->order_cap) {
+    if (d->order)
+      HIPCHK(d, hipFree(d->order));
+    d->order = NULL;
+    d->order_cap = 0;
+    HIPCHK(d, hipMalloc((void **)&d->order, sizeof(int32_t) * (size_t)n));
+    d->order_cap = n;
+  }
+  HIPCHK(d, hipMemcpyAsync(d->order, order, sizeof(int32_t) * (size_t)n, hipMemcpyHostToDevice, d->stream));
+  return EH_OK;
+}
+
+int ehd_get_rows(ehd_dev *d, double *out, int64_t n, const int32_t *order) {
+  if (n != d->n)
+    return EH_ERR_STATE;
+  if (n == 0)
+    return EH_OK;
+  HIPCHK(d, hipSetDevice(d->device));
+  int rc = grow_rows(d, &d->rows2, &d->rows2_cap, 8 * n);
+  if (!rc && order)
+    rc = put_order(d, order, n);
+  if (rc)
+    return rc;
+  hipLaunchKernelGGL(rows_out, ROW_GRID(n), dim3(256), 0, d->stream, d->rows2, state_of(d), d->ids,
+                     order ? d->order : (const int32_t *)NULL);
+  HIPCHK(d, hipGetLastError());
+  HIPCHK(d, hipMemcpyAsync(out, d->rows2, sizeof(double) * 8 * (size_t)n, hipMemcpyDeviceToHost, d->stream));
+  HIPCHK(d, hipStreamSynchronize(d->stream));
+  return EH_OK;
+}
+
+int ehd_rows_back(ehd_dev *d) {
+  HIPCHK(d, hipSetDevice(d->device));
+  hipLaunchKernelGGL(rows_back, ROW_GRID(d->n), dim3(256), 0, d->stream, d->rows, d->rows_w, state_of(d));
+  HIPCHK(d, hipGetLastError());
+  return EH_OK;
+}
+
+int ehd_fetch_rows(ehd_dev *d, double *out, const int32_t *order) {
+  const int64_t n = d->n, w = d->rows_w;
+  const double *src = d->rows;
+  HIPCHK(d, hipSetDevice(d->device));
+  if (order) {
+    int rc = grow_rows(d, &d->rows2, &d->rows2_cap, n * w);
+    if (!rc)
+      rc = put_order(d, order, n);
+    if (rc)
+      return rc;
+    hipLaunchKernelGGL(rows_gather, ROW_GRID(n * w), dim3(256), 0, d->stream, d->rows, d->rows2, n, (int32_t)w,
+                       d->order);
+    HIPCHK(d, hipGetLastError());
+    src = d->rows2;
+  }
+  HIPCHK(d, hipMemcpyAsync(out, src, sizeof(double) * (size_t)(n * w), hipMemcpyDeviceToHost, d->stream));
+  HIPCHK(d, hipStreamSynchronize(d->stream));
+  return EH_OK;
+}
+
+int ehd_fetch_small(ehd_dev *d, const double **rows, const int32_t **loss_pass, const int32_t **loss_code) {
+  const size_t b = sizeof(double) * (size_t)(d->n * (d->rows_w + 1));
+  *rows = NULL;
+  if (b > EHD_PIN_BYTES)
+    return EH_OK;
+  HIPCHK(d, hipSetDevice(d->device));
+  if (!d->pin)
+    HIPCHK(d, hipHostMalloc(&d->pin, EHD_PIN_BYTES, hipHostMallocDefault));
+  HIPCHK(d, hipMemcpyAsync(d->pin, d->rows, b, hipMemcpyDeviceToHost, d->stream));
+  HIPCHK(d, hipStreamSynchronize(d->stream));
+  *rows = (const double *)d->pin;
+  *loss_pass = (const int32_t *)(*rows + d->n * d->rows_w);
+  *loss_code = *loss_pass + d->n;
+  return EH_OK;
+}
+
+int ehd_fiducial_times(ehd_dev *d, double Po, double ahead, double *t) {
+  HIPCHK(d, hipSetDevice(d->device));
+  int rc = grow_rows(d, &d->rows2, &d->rows2_cap, d->n);
+  if (rc)
+    return rc;
+  hipLaunchKernelGGL(fiducial_times, ROW_GRID(d->n), dim3(256), 0, d->stream, state_of(d), Po, ahead, d->rows2);
+  HIPCHK(d, hipGetLastError());
+  HIPCHK(d, hipMemcpyAsync(t, d->rows2, sizeof(double) * (size_t)d->n, hipMemcpyDeviceToHost, d->stream));
+  HIPCHK(d, hipStreamSynchronize(d->stream));
+  return EH_OK;
+}
+
+int ehd_effort(ehd_dev *d, int64_t pass0, int64_t end, int64_t *effort, int64_t *left) {
+  unsigned long long h[2];
+  HIPCHK(d, hipSetDevice(d->device));
+  const int64_t g = (d->n + 255) / 256;
+  hipLaunchKernelGGL(clear_counters, dim3(1), dim3(64), 0, d->stream, d->counter);
+  hipLaunchKernelGGL(effort_sum, dim3((unsigned)(g < 256 ? g : 256)), dim3(256), 0, d->stream, d->loss_pass, d->n,
+                     pass0, end, d->counter);
+  HIPCHK(d, hipGetLastError());
+  HIPCHK(d, hipMemcpyAsync(h, d->counter, sizeof h, hipMemcpyDeviceToHost, d->stream));
+  HIPCHK(d, hipStreamSynchronize(d->stream));
+  *effort = (int64_t)h[0];
+  *left = (int64_t)h[1];
+  return EH_OK;
+}
+
 int ehd_put_ops(ehd_dev *d, const eh_op *ops, int32_t nops) {
   HIPCHK(d, hipSetDevice(d->device));
   if (nops > d->ops_cap) {
@@ -1863,63 +2141,67 @@ int ehd_put_ops(ehd_dev *d, const eh_op *ops, int32_t nops) {
   return EH_OK;
 }
 
-/* grows a device buffer to hold n elements of size sz (contents dropped) */
-static int grow(ehd_dev *d, void **buf, int32_t *cap, int32_t n, size_t sz) {
-  if (n <= *cap)
-    return EH_OK;
-  if (*buf)
-    HIPCHK(d, hipFree(*buf));
-  *buf = NULL;
-  *cap = 0;
-  HIPCHK(d, hipMalloc(buf, sz * (size_t)(n > 0 ? n : 1)));
-  *cap = n;
-  return EH_OK;
-}
+static size_t up256(size_t b) { return (b + 255) / 256 * 256; }
 
-/* folds the host copy into runs and uploads bodies, runs and positions */
+/* folds the host copy into runs and uploads bodies, runs and positions, laid
+ * out in pinned memory, as one copy that nothing waits for (a single-element
+ * call spent three copies and a wait here) */
 static int upload_program(ehd_dev *d) {
   const int32_t n = d->nflat;
   const size_t m = (size_t)(n > 0 ? n : 1);
   eh_run *runs = (eh_run *)malloc(sizeof(eh_run) * m);
   int32_t *body = (int32_t *)malloc(sizeof(int32_t) * m);
-  eh_op *tops = (eh_op *)malloc(sizeof(eh_op) * m);
-  double *zpos = (double *)malloc(sizeof(double) * 2 * m);
   int32_t nb = 0, nr = -1;
   int rc = EH_OK;
-  if (runs && body && tops && zpos)
+  if (runs && body)
     nr = eh_fold_runs(d->host_prog, n, EH_RUN_MAX_LEN, runs, body, &nb);
   if (nr < 0) {
     rc = EH_ERR_NOMEM;
     snprintf(d->msg, sizeof d->msg, "out of host memory folding the program");
   }
-  if (!rc) {
+  const size_t o_runs = up256(sizeof(eh_op) * (size_t)nb), o_z = o_runs + up256(sizeof(eh_run) * (size_t)(nr > 0 ? nr : 0)),
+               bytes = o_z + sizeof(double) * 2 * m;
+  hipError_t e = hipSuccess;
+  if (!rc)
+    e = hipEventSynchronize(d->pev); /* the last copy has left pstage */
+  if (!rc && !e && bytes > d->pbuf_cap) {
+    /* kernels in flight may still read the old buffer */
+    e = hipStreamSynchronize(d->stream);
+    if (!e && d->pbuf)
+      e = hipFree(d->pbuf);
+    if (!e && d->pstage)
+      e = hipHostFree(d->pstage);
+    if (!e) {
+      d->pbuf = d->pstage = NULL;
+      d->pbuf_cap = 0;
+      e = hipMalloc(&d->pbuf, bytes);
+    }
+    if (!e)
+      e = hipHostMalloc(&d->pstage, bytes, hipHostMallocDefault);
+    if (!e)
+      d->pbuf_cap = bytes;
+  }
+  if (!rc && !e) {
+    char *h = (char *)d->pstage, *g = (char *)d->pbuf;
+    d->tops = (eh_op *)g;
+    d->runs = (eh_run *)(g + o_runs);
+    d->zpos = (double *)(g + o_z);
+    double *zpos = (double *)(h + o_z);
     for (int32_t j = 0; j < nb; j++)
-      tops[j] = d->host_prog[body[j]];
+      memcpy(h + sizeof(eh_op) * (size_t)j, &d->host_prog[body[j]], sizeof(eh_op));
+    memcpy(h + o_runs, runs, sizeof(eh_run) * (size_t)nr);
     for (int32_t f = 0; f < n; f++) {
       zpos[2 * f] = d->host_prog[f].z_start;
       zpos[2 * f + 1] = d->host_prog[f].z_end;
     }
-    rc = grow(d, (void **)&d->tops, &d->tops_cap, nb, sizeof(eh_op));
+    e = hipMemcpyAsync(d->pbuf, d->pstage, bytes, hipMemcpyHostToDevice, d->stream);
+    if (!e)
+      e = hipEventRecord(d->pev, d->stream);
   }
-  if (!rc)
-    rc = grow(d, (void **)&d->runs, &d->runs_cap, nr, sizeof(eh_run));
-  if (!rc)
-    rc = grow(d, (void **)&d->zpos, &d->zpos_cap, 2 * n, sizeof(double));
-  hipError_t e = hipSuccess;
-  if (!rc && nb > 0)
-    e = hipMemcpyAsync(d->tops, tops, sizeof(eh_op) * nb, hipMemcpyHostToDevice, d->stream);
-  if (!rc && !e && nr > 0)
-    e = hipMemcpyAsync(d->runs, runs, sizeof(eh_run) * nr, hipMemcpyHostToDevice, d->stream);
-  if (!rc && !e && n > 0)
-    e = hipMemcpyAsync(d->zpos, zpos, sizeof(double) * 2 * n, hipMemcpyHostToDevice, d->stream);
-  /* the host buffers are the copies' sources: wait before freeing them */
-  hipError_t es = hipStreamSynchronize(d->stream);
-  if (!rc && (e || es))
-    rc = hip_fail(d, e ? e : es, "uploading the tracking program");
+  if (!rc && e)
+    rc = hip_fail(d, e, "uploading the tracking program");
   free(runs);
   free(body);
-  free(tops);
-  free(zpos);
   if (rc) {
     d->nruns = d->ntops = 0;
     d->nflat = 0;
@@ -1966,7 +2248,7 @@ void ehd_set_block(ehd_dev *d, int32_t block) {
     d->block = block;
 }
 
-int ehd_track(ehd_dev *d, int64_t pass0, int32_t npasses, int32_t op_first, int32_t op_last) {
+static int track_launch(ehd_dev *d, int64_t pass0, int32_t npasses, int32_t op_first, int32_t op_last, int timed) {
   if (npasses <= 0 || d->n == 0)
     return EH_OK;
   if (op_first < 0 || op_last > d->nflat || op_first > d->nflat || (npasses == 1 && op_first > op_last))
@@ -1996,10 +2278,13 @@ int ehd_track(ehd_dev *d, int64_t pass0, int32_t npasses, int32_t op_first, int3
     block = d->n <= (int64_t)d->num_cu * 256 ? 64 : 256;
   }
   const int64_t grid = (d->n + block - 1) / block;
-  HIPCHK(d, hipEventRecord(d->ev0, d->stream));
+  if (timed)
+    HIPCHK(d, hipEventRecord(d->ev0, d->stream));
   hipLaunchKernelGGL(eh_track_kernel, dim3((unsigned)grid), dim3(block), 0, d->stream, st, d->tops, d->runs, d->nruns,
                      d->zpos, pass0, npasses, op_first, op_last, d->nflat);
   HIPCHK(d, hipGetLastError());
+  if (!timed)
+    return EH_OK;
   HIPCHK(d, hipEventRecord(d->ev1, d->stream));
   HIPCHK(d, hipEventSynchronize(d->ev1));
   float ms = 0;
@@ -2008,6 +2293,12 @@ int ehd_track(ehd_dev *d, int64_t pass0, int32_t npasses, int32_t op_first, int3
   d->track_launches += 1;
   return EH_OK;
 }
+
+int ehd_track(ehd_dev *d, int64_t pass0, int32_t npasses, int32_t op_first, int32_t op_last) {
+  return track_launch(d, pass0, npasses, op_first, op_last, 1);
+}
+
+int ehd_track_single(ehd_dev *d, int64_t pass) { return track_launch(d, pass, 1, 0, 1, 0); }
 
 /* do_match_energy's re-expression of delta against the new central
  * momentum, delta = dp + delta dr, on the particles still in the beam

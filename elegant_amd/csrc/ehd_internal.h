@@ -14,6 +14,7 @@
  * static scratch (plan 128 B + histogram and voltage for EHD_NOALLOC_BINS + 16
  * bins + 1,025 fixed-point partials, rounded up) */
 #define EHD_ZL_MAX_BINS (1 << 20) /* ZLONGIT bins: the bin optimiser's default cap (ztransverse.c:672-759) */
+#define EHD_PIN_BYTES (1 << 20) /* small results come back through pinned memory */
 #define EHD_NOALLOC_BINS 16384
 #define EHD_NOALLOC_BYTES (256 * 1024)
 
@@ -22,6 +23,8 @@ typedef struct {
   int64_t wpoints;
   double *Z, *tc, *ts; /* ZLONGIT impedance and FFT twiddles */
   int32_t nb;
+  int64_t W_cap, Z_cap; /* points the buffers hold: kept between uploads */
+  int32_t tw_nb;        /* bins the twiddles are for, 0: none yet */
 } ehd_coll_slot;
 
 struct ehd_dev {
@@ -30,16 +33,28 @@ struct ehd_dev {
   hipEvent_t ev0, ev1, cev0, cev1;
   double *coord[6];
   int32_t *loss_pass, *loss_code;
+  double *ids;         /* particle IDs (column 6 of the rows) */
   int64_t n, cap;
+  /* rows as the caller holds them, on their way to or from the columns
+   * above: kept between calls, freed with the context */
+  double *rows, *rows2;
+  int64_t rows_cap, rows2_cap;   /* doubles */
+  int32_t rows_w;                /* columns per row of the last upload */
+  int32_t *order;
+  int64_t order_cap;
+  void *pin;           /* pinned host buffer of EHD_PIN_BYTES */
   eh_op *ops;          /* flat records of the batch kernel's programs */
   int32_t nops, ops_cap;
   /* the tracking kernel's program (ehd_put_program) */
   eh_op *host_prog;    /* flat copy on the host: patches refold it */
   int32_t nflat, host_prog_cap;
+  void *pbuf, *pstage; /* the three arrays below in one buffer, and its pinned host copy */
+  size_t pbuf_cap;
+  hipEvent_t pev;      /* the last copy out of pstage */
   eh_op *tops;         /* run bodies */
   eh_run *runs;
   double *zpos;        /* (z_start, z_end) of each flat position */
-  int32_t ntops, nruns, tops_cap, runs_cap, zpos_cap;
+  int32_t ntops, nruns;
   int32_t block;
   unsigned long long *counter;
   double track_ms, coll_ms;

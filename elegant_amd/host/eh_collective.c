@@ -31,7 +31,7 @@ int eh_ctx_bucket_mean(eh_ctx *c, int64_t pass, int32_t code_lim, long b, double
 const char *ehd_message(const ehd_dev *d);
 int eh_upload(eh_ctx *c, double **coord, int64_t n, int32_t nprops);
 int eh_upload_rows(eh_ctx *c, double **coord, int64_t n, int32_t nprops, int cull);
-int eh_download(eh_ctx *c, double **coord, int64_t n, int32_t nprops, int64_t *nLeft);
+int eh_ctx_writeback(eh_ctx *c, double **rows, int64_t n, int64_t *nLeft);
 
 static double sqr(double x) { return x * x; }
 
@@ -109,18 +109,22 @@ static int wake_setup(eh_ctx *c, int slot, const EH_WAKE *w, double *dt, double 
  * table the CPU checker builds) to the device slot */
 static int zlongit_upload(eh_ctx *c, int slot, const double *Z, long n_bins, double bin_size) {
   ehd_dev *d = eh_ctx_dev(c);
-  double *tc = (double *)malloc(sizeof(double) * (n_bins / 2 + 1));
-  double *ts = (double *)malloc(sizeof(double) * (n_bins / 2 + 1));
+  double *tc = NULL, *ts = NULL;
   int rc;
-  if (!tc || !ts) {
-    free(tc);
-    free(ts);
-    return EH_ERR_NOMEM;
-  }
-  for (long k = 0; k <= n_bins / 2; k++) {
-    double a = EH_PIx2 * k / n_bins;
-    tc[k] = cos(a);
-    ts[k] = sin(a);
+  /* twiddles depend on the bin count alone: the slot keeps its last ones */
+  if (ehd_twiddle_bins(d, slot) != (int32_t)n_bins) {
+    tc = (double *)malloc(sizeof(double) * (n_bins / 2 + 1));
+    ts = (double *)malloc(sizeof(double) * (n_bins / 2 + 1));
+    if (!tc || !ts) {
+      free(tc);
+      free(ts);
+      return EH_ERR_NOMEM;
+    }
+    for (long k = 0; k <= n_bins / 2; k++) {
+      double a = EH_PIx2 * k / n_bins;
+      tc[k] = cos(a);
+      ts[k] = sin(a);
+    }
   }
   rc = ehd_put_zlongit(d, slot, Z, tc, ts, (int32_t)n_bins);
   free(tc);
@@ -391,24 +395,7 @@ int eh_collective_probe(eh_ctx *c, double **part, int64_t np, const eh_element *
   rc = collective_run(c, 0, e, &prog->ops[0], 0, i_pass, macro, EHD_COLL_NOCHECKS, hist, volt, nb, tmin);
   if (rc)
     return rc;
-  {
-    double **tmp = (double **)malloc(sizeof(double *) * (np > 0 ? np : 1));
-    double *buf = (double *)malloc(sizeof(double) * 8 * (np > 0 ? np : 1));
-    if (!tmp || !buf) {
-      free(tmp);
-      free(buf);
-      return EH_ERR_NOMEM;
-    }
-    for (int64_t i = 0; i < np; i++)
-      tmp[i] = buf + 8 * i;
-    rc = eh_download(c, tmp, np, 8, &nLeft);
-    if (!rc)
-      for (int64_t i = 0; i < np; i++)
-        memcpy(part[i], tmp[i], sizeof(double) * 7);
-    free(tmp);
-    free(buf);
-  }
-  return rc;
+  return np > 0 ? eh_ctx_writeback(c, part, np, &nLeft) : EH_OK;
 }
 
 int64_t eh_track_through_wake(eh_ctx *c, double **part, int64_t np, const EH_WAKE *wake, double Po, int64_t i_pass,

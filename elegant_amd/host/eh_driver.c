@@ -35,12 +35,17 @@ struct eh_ctx {
   int loaded;
   /* particles */
   int64_t n;
-  double *ids;
+  /* host arrays of cap_n slots, kept from one upload to the next; order, pos
+   * and applied are filled in once a particle is lost (have_order) */
+  int64_t cap_n;
   int64_t *order, *pos, *scratch;
+  int have_order;
   int64_t n_alive_ref;
   uint8_t *applied;
-  int32_t *h_pass, *h_code;
+  int32_t *h_pass, *h_code, *order32;
   double *h_s, *h_dp;
+  double *hrows; /* rows gathered from callers whose rows are not one block */
+  int64_t hrows_cap;
   /* per-program state (reference element-struct state) */
   int fid_seen[EH_MAX_RFCA];
   double phase_fid[EH_MAX_RFCA];
@@ -205,7 +210,6 @@ int eh_set_particle_properties(eh_ctx *c, int32_t nprops) {
 }
 
 static void free_particles(eh_ctx *c) {
-  free(c->ids);
   free(c->order);
   free(c->pos);
   free(c->scratch);
@@ -214,10 +218,14 @@ static void free_particles(eh_ctx *c) {
   free(c->h_code);
   free(c->h_s);
   free(c->h_dp);
+  free(c->order32);
+  free(c->hrows);
   free(c->extra);
   c->extra = NULL;
   c->extra_w = 0;
-  c->ids = NULL;
+  c->order32 = NULL;
+  c->hrows = NULL;
+  c->cap_n = c->hrows_cap = 0;
   c->order = c->pos = c->scratch = NULL;
   c->applied = NULL;
   c->h_pass = c->h_code = NULL;
@@ -299,37 +307,79 @@ int eh_load_program(eh_ctx *c, const eh_element *elems, int64_t n_elems, double 
 /* ------------------------------------------------------- particle state */
 
 static int alloc_particles(eh_ctx *c, int64_t n) {
-  free_particles(c);
-  c->ids = (double *)malloc(sizeof(double) * (n + 1));
-  c->order = (int64_t *)malloc(sizeof(int64_t) * (n + 1));
-  c->pos = (int64_t *)malloc(sizeof(int64_t) * (n + 1));
-  c->scratch = (int64_t *)malloc(sizeof(int64_t) * (n + 1));
-  c->applied = (uint8_t *)calloc(n + 1, 1);
-  c->h_pass = (int32_t *)malloc(sizeof(int32_t) * (n + 1));
-  c->h_code = (int32_t *)malloc(sizeof(int32_t) * (n + 1));
-  c->h_s = (double *)malloc(sizeof(double) * (n + 1));
-  c->h_dp = (double *)malloc(sizeof(double) * (n + 1));
-  if (!c->ids || !c->order || !c->pos || !c->scratch || !c->applied || !c->h_pass || !c->h_code || !c->h_s ||
-      !c->h_dp) {
+  free(c->extra);
+  c->extra = NULL;
+  c->extra_w = 0;
+  c->n = 0;
+  if (n >= c->cap_n) {
     free_particles(c);
-    return EH_ERR_NOMEM;
+    c->order = (int64_t *)malloc(sizeof(int64_t) * (n + 1));
+    c->pos = (int64_t *)malloc(sizeof(int64_t) * (n + 1));
+    c->scratch = (int64_t *)malloc(sizeof(int64_t) * (n + 1));
+    c->applied = (uint8_t *)malloc(n + 1);
+    c->h_pass = (int32_t *)malloc(sizeof(int32_t) * (n + 1));
+    c->h_code = (int32_t *)malloc(sizeof(int32_t) * (n + 1));
+    c->order32 = (int32_t *)malloc(sizeof(int32_t) * (n + 1));
+    c->h_s = (double *)malloc(sizeof(double) * (n + 1));
+    c->h_dp = (double *)malloc(sizeof(double) * (n + 1));
+    if (!c->order || !c->pos || !c->scratch || !c->applied || !c->h_pass || !c->h_code || !c->order32 || !c->h_s ||
+        !c->h_dp) {
+      free_particles(c);
+      return EH_ERR_NOMEM;
+    }
+    c->cap_n = n + 1;
   }
   c->n = n;
-  for (int64_t i = 0; i < n; i++) {
-    c->order[i] = i;
-    c->pos[i] = i;
-  }
+  c->have_order = 0;
   c->n_alive_ref = n;
   return EH_OK;
 }
 
-/* AoS rows -> SoA, with do_tracking's initial NaN/Inf cull (do_tracking.c:468-473)
- * when cull is set: such rows are recorded as lost on pass 0 before the first
+/* the reference row order, the upload's until a particle is lost */
+static void make_order(eh_ctx *c) {
+  if (c->have_order)
+    return;
+  for (int64_t i = 0; i < c->n; i++) {
+    c->order[i] = i;
+    c->pos[i] = i;
+  }
+  memset(c->applied, 0, (size_t)c->n);
+  c->have_order = 1;
+}
+
+static int64_t slot_at(const eh_ctx *c, int64_t j) { return c->have_order ? c->order[j] : j; }
+
+/* the caller's rows as one block of n x w doubles, or NULL where they are
+ * not exactly adjacent (a gap may belong to someone else) */
+static double *one_block(double **rows, int64_t n, int32_t w) {
+  for (int64_t i = 1; i < n; i++)
+    if ((uintptr_t)rows[i] != (uintptr_t)rows[0] + (uintptr_t)i * sizeof(double) * (uintptr_t)w)
+      return NULL;
+  return rows[0];
+}
+
+static double *host_rows(eh_ctx *c, int64_t count) {
+  if (count > c->hrows_cap) {
+    free(c->hrows);
+    c->hrows = (double *)malloc(sizeof(double) * (size_t)count);
+    c->hrows_cap = c->hrows ? count : 0;
+  }
+  return c->hrows;
+}
+
+/* The rows go to the device whole, as one copy, and are turned into columns
+ * there, with do_tracking's initial NaN/Inf cull (do_tracking.c:468-473) when
+ * cull is set: such rows are recorded as lost on pass 0 before the first
  * element.  The single-element entry points upload without it, as the
- * element routines leave such rows to their caller. */
-int eh_upload_rows(eh_ctx *c, double **coord, int64_t n, int32_t nprops, int cull) {
+ * element routines leave such rows to their caller.  Splitting rows into
+ * columns and back on the host, with the loss records and row order of every
+ * call, was 27 ms of a 233 ms run (10^6 rows, 10 passes) and 180 of the 219 us
+ * of one quadrupole over 100 rows; moved whole, what is left of it is the
+ * pageable copies (64 MB each way at 30 and 18 GB/s).
+ */
+static int upload_rows(eh_ctx *c, double **coord, int64_t n, int32_t nprops, int cull) {
   int rc;
-  double *soa;
+  double *block;
   if (!c || (!coord && n > 0) || n < 0 || nprops < 7)
     return fail(c, EH_ERR_INVALID, "eh_upload: bad arguments");
   if (n > 0x7fffffff)
@@ -337,48 +387,37 @@ int eh_upload_rows(eh_ctx *c, double **coord, int64_t n, int32_t nprops, int cul
   rc = alloc_particles(c, n);
   if (rc)
     return rc;
-  soa = (double *)malloc(sizeof(double) * 6 * (n + 1));
-  if (!soa)
-    return EH_ERR_NOMEM;
   c->bunch_on_device = 0;
+  block = n > 0 ? one_block(coord, n, nprops) : NULL;
+  if (n > 0 && !block) {
+    block = host_rows(c, n * nprops);
+    if (!block)
+      return EH_ERR_NOMEM;
+    for (int64_t i = 0; i < n; i++)
+      memcpy(block + nprops * i, coord[i], sizeof(double) * nprops);
+  }
+  rc = ehd_put_rows(c->dev, block, n, nprops, cull, c->Po);
+  return rc ? devfail(c, rc) : EH_OK;
+}
+
+int eh_upload_rows(eh_ctx *c, double **coord, int64_t n, int32_t nprops, int cull) {
+  int rc = upload_rows(c, coord, n, nprops, cull);
+  if (rc)
+    return rc;
   if (nprops > 8) {
     c->extra_w = nprops - 8;
     c->extra = (double *)malloc(sizeof(double) * c->extra_w * (n + 1));
     if (!c->extra) {
-      free(soa);
+      c->extra_w = 0;
+      ehd_sync(c->dev);
       return EH_ERR_NOMEM;
     }
     for (int64_t i = 0; i < n; i++)
       memcpy(c->extra + c->extra_w * i, coord[i] + 8, sizeof(double) * c->extra_w);
   }
-  {
-    int64_t nlost = 0;
-    for (int64_t i = 0; i < n; i++) {
-      double *r = coord[i];
-      for (int k = 0; k < 6; k++)
-        soa[k * n + i] = r[k];
-      c->ids[i] = r[6];
-      c->h_pass[i] = -1;
-      c->h_code[i] = 0;
-      if (cull && (isinf(r[0]) || isinf(r[2]) || isnan(r[0]) || isnan(r[2]))) {
-        /* limit_amplitudes(DBL_MAX) at z = 0: s = 0, delta = Po(1+delta) */
-        soa[4 * n + i] = 0.0;
-        soa[5 * n + i] = c->Po * (1 + r[5]);
-        c->h_pass[i] = 0;
-        c->h_code[i] = -1;
-        nlost++;
-      }
-    }
-    (void)nlost;
-  }
-  rc = ehd_alloc_state(c->dev, n);
-  if (!rc)
-    rc = ehd_put_state(c->dev, soa, soa + n, soa + 2 * n, soa + 3 * n, soa + 4 * n, soa + 5 * n, c->h_pass, c->h_code,
-                       n);
-  free(soa);
-  if (rc)
-    return devfail(c, rc);
-  return EH_OK;
+  /* the rows are the caller's again */
+  rc = ehd_sync(c->dev);
+  return rc ? devfail(c, rc) : EH_OK;
 }
 
 int eh_upload(eh_ctx *c, double **coord, int64_t n, int32_t nprops) { return eh_upload_rows(c, coord, n, nprops, 1); }
@@ -444,6 +483,7 @@ static int cmp_ev(const void *a, const void *b) {
 static int replay_until(eh_ctx *c, int64_t pass_lim, int32_t code_lim) {
   int64_t m = 0;
   loss_ev *ev;
+  make_order(c);
   for (int64_t i = 0; i < c->n; i++)
     if (c->h_pass[i] >= 0 && !c->applied[i])
       m++;
@@ -497,12 +537,29 @@ static int refresh_losses(eh_ctx *c) {
   return rc ? devfail(c, rc) : EH_OK;
 }
 
+/* the row order as of (pass_lim, code_lim): while no particle of the upload
+ * has been lost, which the device counts, it is the upload's and no record
+ * is read back */
+static int order_until(eh_ctx *c, int64_t pass_lim, int32_t code_lim) {
+  int64_t effort, left;
+  int rc;
+  if (!c->n)
+    return EH_OK;
+  rc = ehd_effort(c->dev, 0, 0, &effort, &left);
+  if (rc)
+    return devfail(c, rc);
+  if (left == c->n)
+    return EH_OK;
+  rc = refresh_losses(c);
+  return rc ? rc : replay_until(c, pass_lim, code_lim);
+}
+
 /* ------------------------------------------------------------ tracking */
 
 /* RFCA TMEAN fiducial on the first pass: KahanPlus mean of arrival times over
  * the particles in reference row order (simple_rfca.c:179-210, kahan.c:27-36) */
 static double kahan_plus(double oldSum, double b, double *error) {
-  volatile double sum, Y;
+  double sum, Y; /* IEEE double arithmetic, nothing contracted or reassociated */
   Y = b + *error;
   sum = oldSum + Y;
   *error = Y - (sum - oldSum);
@@ -521,17 +578,14 @@ static int rfca_fiducial(eh_ctx *c, int k, int64_t pass) {
     nKicks = 1;
   length /= nKicks;
   sOffset = length / 2;
-  rc = ehd_get_state(c->dev, NULL, NULL, NULL, NULL, c->h_s, c->h_dp, c->h_pass, c->h_code, c->n);
-  if (rc)
-    return devfail(c, rc);
-  rc = replay_until(c, pass, 4 * opi);
+  rc = order_until(c, pass, 4 * opi);
   if (rc)
     return rc;
+  rc = ehd_fiducial_times(c->dev, c->Po, sOffset, c->h_s);
+  if (rc)
+    return devfail(c, rc);
   for (int64_t j = 0; j < c->n_alive_ref; j++) {
-    int64_t i = c->order[j];
-    double p = c->Po * (1 + c->h_dp[i]);
-    double beta = p / sqrt(p * p + 1);
-    tsum = kahan_plus(tsum, (c->h_s[i] + sOffset) / (EH_C_MKS * beta), &error);
+    tsum = kahan_plus(tsum, c->h_s[slot_at(c, j)], &error);
     nsum++;
   }
   if (nsum <= 0)
@@ -572,7 +626,7 @@ static int rfca_time_offset(eh_ctx *c, int k, int64_t pass) {
   int32_t lp = 0;
   int rc;
   if (c->n_alive_ref > 0) {
-    rc = ehd_get_one(c->dev, c->order[0], NULL, NULL, &lp);
+    rc = ehd_get_one(c->dev, slot_at(c, 0), NULL, NULL, &lp);
     if (rc)
       return devfail(c, rc);
   }
@@ -584,7 +638,7 @@ static int rfca_time_offset(eh_ctx *c, int k, int64_t pass) {
       return rc;
   }
   if (c->n_alive_ref > 0) {
-    rc = ehd_get_one(c->dev, c->order[0], &s, &dp, NULL);
+    rc = ehd_get_one(c->dev, slot_at(c, 0), &s, &dp, NULL);
     if (rc)
       return devfail(c, rc);
     toff = eh_rfca_time_offset(op, c->Po, s, dp);
@@ -640,16 +694,16 @@ static int recompile_program(eh_ctx *c) {
  * EH_OP_MATCH_P0 step. */
 static int match_energy(eh_ctx *c, int32_t opi, int64_t pass, int recompile) {
   double P_average = 0, error = 0;
-  int rc = ehd_get_state(c->dev, NULL, NULL, NULL, NULL, NULL, c->h_dp, c->h_pass, c->h_code, c->n);
-  if (rc)
-    return devfail(c, rc);
-  rc = replay_until(c, pass, 4 * opi);
+  int rc = order_until(c, pass, 4 * opi);
   if (rc)
     return rc;
   if (c->n_alive_ref <= 0)
     return EH_OK;
+  rc = ehd_get_state(c->dev, NULL, NULL, NULL, NULL, NULL, c->h_dp, NULL, NULL, c->n);
+  if (rc)
+    return devfail(c, rc);
   for (int64_t j = 0; j < c->n_alive_ref; j++)
-    P_average = kahan_plus(P_average, c->Po * (1 + c->h_dp[c->order[j]]), &error);
+    P_average = kahan_plus(P_average, c->Po * (1 + c->h_dp[slot_at(c, j)]), &error);
   P_average /= c->n_alive_ref;
   if (fabs(P_average - c->Po) / c->Po > 1e-14) {
     const double dp = (c->Po - P_average) / P_average, dr = c->Po / P_average;
@@ -745,7 +799,7 @@ static int64_t alive_at(const eh_ctx *c, int64_t q) {
 
 int eh_track(eh_ctx *c, int64_t pass0, int64_t npasses, double *P_central, eh_stats *stats) {
   int rc;
-  int64_t n_alive0 = 0, done_end;
+  int64_t done_end;
   if (!c || !P_central || npasses < 0)
     return fail(c, EH_ERR_INVALID, "eh_track: bad arguments");
   if (!c->loaded)
@@ -758,12 +812,6 @@ int eh_track(eh_ctx *c, int64_t pass0, int64_t npasses, double *P_central, eh_st
     return EH_OK;
   }
   ehd_timing_reset(c->dev);
-  rc = refresh_losses(c);
-  if (rc)
-    return rc;
-  for (int64_t i = 0; i < c->n; i++)
-    if (c->h_pass[i] < 0 || c->h_pass[i] >= pass0)
-      n_alive0++;
   {
     int64_t pass = pass0, end = pass0 + npasses;
     while (pass < end) {
@@ -869,21 +917,11 @@ int eh_track(eh_ctx *c, int64_t pass0, int64_t npasses, double *P_central, eh_st
     }
     done_end = pass;
   }
-  rc = refresh_losses(c);
-  if (rc)
-    return rc;
   if (stats) {
-    int64_t effort = 0, left = 0;
-    for (int64_t i = 0; i < c->n; i++) {
-      int64_t lp = c->h_pass[i];
-      if (lp >= 0 && lp < pass0)
-        continue;
-      if (lp < 0) {
-        effort += done_end - pass0;
-        left++;
-      } else
-        effort += lp - pass0;
-    }
+    int64_t effort, left;
+    rc = ehd_effort(c->dev, pass0, done_end, &effort, &left);
+    if (rc)
+      return devfail(c, rc);
     memset(stats, 0, sizeof(*stats));
     stats->effort = effort;
     stats->n_left = left;
@@ -891,7 +929,6 @@ int eh_track(eh_ctx *c, int64_t pass0, int64_t npasses, double *P_central, eh_st
     ehd_timing(c->dev, &stats->kernel_launches, &stats->track_ms);
     ehd_collective_timing(c->dev, &left, &stats->collective_ms);
   }
-  (void)n_alive0;
   *P_central = c->Po; /* moved by CHANGE_P0 cavities, as do_tracking's *P_central */
   return EH_OK;
 }
@@ -902,40 +939,47 @@ int eh_last_kernel_timing(const eh_ctx *c, int64_t *launches, double *total_ms) 
   return ehd_timing(c->dev, launches, total_ms);
 }
 
+static const int32_t *order_for_device(eh_ctx *c) {
+  if (!c->have_order)
+    return NULL;
+  for (int64_t j = 0; j < c->n; j++)
+    c->order32[j] = (int32_t)c->order[j];
+  return c->order32;
+}
+
 /* rows in reference order: survivors, then lost rows (tail order of the
  * compactions), column 7 = pass of loss (-1 for survivors) */
 int eh_download(eh_ctx *c, double **coord, int64_t n, int32_t nprops, int64_t *nLeft) {
-  double *soa;
+  double *block;
   int rc;
   if (!c || (!coord && n > 0) || nprops < 8 || n != c->n)
     return fail(c, EH_ERR_INVALID, "eh_download: bad arguments");
-  soa = (double *)malloc(sizeof(double) * 6 * (n + 1));
-  if (!soa)
-    return EH_ERR_NOMEM;
-  rc = ehd_get_state(c->dev, soa, soa + n, soa + 2 * n, soa + 3 * n, soa + 4 * n, soa + 5 * n, c->h_pass, c->h_code,
-                     n);
-  if (rc) {
-    free(soa);
-    return devfail(c, rc);
+  if (n == 0) {
+    if (nLeft)
+      *nLeft = c->n_alive_ref;
+    return EH_OK;
   }
-  rc = replay_until(c, INT64_MAX, INT32_MAX);
-  if (rc) {
-    free(soa);
+  rc = order_until(c, INT64_MAX, INT32_MAX);
+  if (rc)
     return rc;
+  block = nprops == 8 ? one_block(coord, n, 8) : NULL;
+  const int direct = block != NULL;
+  if (!direct) {
+    block = host_rows(c, 8 * n);
+    if (!block)
+      return EH_ERR_NOMEM;
   }
-  for (int64_t j = 0; j < n; j++) {
-    int64_t i = c->order[j];
+  rc = ehd_get_rows(c->dev, block, n, order_for_device(c));
+  if (rc)
+    return devfail(c, rc);
+  for (int64_t j = 0; !direct && j < n; j++) {
     double *r = coord[j];
-    for (int k = 0; k < 6; k++)
-      r[k] = soa[k * n + i];
-    r[6] = c->ids[i];
-    r[7] = c->h_pass[i] >= 0 ? (double)c->h_pass[i] : -1.0;
+    memcpy(r, block + 8 * j, sizeof(double) * 8);
     for (int k = 8; k < nprops && k - 8 < c->extra_w; k++)
-      r[k] = c->extra[c->extra_w * i + k - 8];
+      r[k] = c->extra[c->extra_w * slot_at(c, j) + k - 8];
   }
   if (nLeft)
     *nLeft = c->n_alive_ref;
-  free(soa);
   return EH_OK;
 }
 
@@ -971,7 +1015,7 @@ int64_t eh_do_tracking(eh_ctx *c, double **coord, int64_t nOriginal, int64_t *ef
     rc = eh_download(c, coord, nOriginal, (int32_t)W, &nLeft);
   if (!rc && initial)
     for (int64_t j = 0; j < nOriginal; j++)
-      memcpy(accepted[j], initial + W * c->order[j], sizeof(double) * W);
+      memcpy(accepted[j], initial + W * slot_at(c, j), sizeof(double) * W);
   free(initial);
   if (rc)
     return rc;
@@ -991,39 +1035,74 @@ int64_t eh_do_tracking(eh_ctx *c, double **coord, int64_t nOriginal, int64_t *ef
  * order, so slot i is row i. */
 static int writeback_rows(eh_ctx *c, double **rows, int64_t n, double **accepted, int64_t *nLeft) {
   const int64_t W = c->row_props;
-  double **tmp = (double **)malloc(sizeof(double *) * n);
-  double *buf = (double *)malloc(sizeof(double) * 8 * n);
-  double *keep = (double *)malloc(sizeof(double) * W * n);
-  double *acc = accepted ? (double *)malloc(sizeof(double) * W * n) : NULL;
-  int rc;
-  if (!tmp || !buf || !keep || (accepted && !acc)) {
-    free(tmp);
-    free(buf);
-    free(keep);
+  const double *src = NULL;
+  const int32_t *lp = NULL, *lc = NULL;
+  double *block = NULL;
+  int rc = ehd_rows_back(c->dev);
+  if (!rc)
+    rc = ehd_fetch_small(c->dev, &src, &lp, &lc);
+  if (rc)
+    return devfail(c, rc);
+  if (src) { /* rows and loss records came in one copy, ordered here */
+    int lost = 0;
+    for (int64_t i = 0; i < n; i++)
+      lost |= lp[i] >= 0;
+    if (lost) {
+      memcpy(c->h_pass, lp, sizeof(int32_t) * n);
+      memcpy(c->h_code, lc, sizeof(int32_t) * n);
+      rc = replay_until(c, INT64_MAX, INT32_MAX);
+    }
+  } else {
+    rc = order_until(c, INT64_MAX, INT32_MAX);
+    block = one_block(rows, n, (int32_t)W);
+    src = block;
+    if (!rc && !block) {
+      src = block = host_rows(c, n * W);
+      if (!block)
+        rc = EH_ERR_NOMEM;
+    } else
+      src = NULL;
+    if (!rc) {
+      rc = ehd_fetch_rows(c->dev, block, order_for_device(c));
+      if (rc)
+        devfail(c, rc);
+    }
+  }
+  double *acc = NULL;
+  if (!rc && accepted && c->have_order) {
+    acc = (double *)malloc(sizeof(double) * W * n);
+    if (!acc)
+      rc = EH_ERR_NOMEM;
+  }
+  if (rc)
+    return rc;
+  for (int64_t j = 0; src && j < n; j++)
+    memcpy(rows[j], src + W * (block ? j : slot_at(c, j)), sizeof(double) * W);
+  if (acc) {
+    for (int64_t i = 0; i < n; i++)
+      memcpy(acc + W * i, accepted[i], sizeof(double) * W);
+    for (int64_t j = 0; j < n; j++)
+      memcpy(accepted[j], acc + W * c->order[j], sizeof(double) * W);
     free(acc);
-    return EH_ERR_NOMEM;
   }
-  for (int64_t i = 0; i < n; i++)
-    tmp[i] = buf + 8 * i;
-  rc = eh_download(c, tmp, n, 8, nLeft);
-  if (!rc) {
-    for (int64_t i = 0; i < n; i++) {
-      memcpy(keep + W * i, rows[i], sizeof(double) * W);
-      if (acc)
-        memcpy(acc + W * i, accepted[i], sizeof(double) * W);
-    }
-    for (int64_t j = 0; j < n; j++) {
-      const int64_t src = c->order[j];
-      memcpy(rows[j], tmp[j], sizeof(double) * 7);
-      memcpy(rows[j] + 7, keep + W * src + 7, sizeof(double) * (W - 7));
-      if (acc)
-        memcpy(accepted[j], acc + W * src, sizeof(double) * W);
-    }
+  *nLeft = c->n_alive_ref;
+  return EH_OK;
+}
+
+int eh_ctx_writeback(eh_ctx *c, double **rows, int64_t n, int64_t *nLeft) {
+  return writeback_rows(c, rows, n, NULL, nLeft);
+}
+
+/* one pass of the loaded one-element program over the caller's rows */
+static int track_single(eh_ctx *c, double **rows, int64_t n, int64_t pass) {
+  int rc = upload_rows(c, rows, n, c->row_props, 0);
+  if (rc)
+    return rc;
+  rc = ehd_track_single(c->dev, pass);
+  if (rc) {
+    devfail(c, rc);
+    ehd_sync(c->dev); /* the rows are the caller's again */
   }
-  free(tmp);
-  free(buf);
-  free(keep);
-  free(acc);
   return rc;
 }
 
@@ -1034,7 +1113,6 @@ static int64_t run_single(eh_ctx *c, double **rows, int64_t n, double **accepted
   eh_element bl[2];
   int nb = 0, rc;
   int64_t nLeft = 0;
-  eh_stats st;
   if (n <= 0)
     return 0;
   if (maxamp) {
@@ -1060,16 +1138,11 @@ static int64_t run_single(eh_ctx *c, double **rows, int64_t n, double **accepted
   rc = ehd_put_program(c->dev, c->prog->ops, 1);
   if (rc)
     return devfail(c, rc);
-  rc = eh_upload_rows(c, rows, n, 8, 0);
+  rc = track_single(c, rows, n, pass);
+  if (!rc)
+    rc = writeback_rows(c, rows, n, accepted, &nLeft);
   if (rc)
     return rc;
-  rc = ehd_track(c->dev, pass, 1, 0, 1);
-  if (rc)
-    return devfail(c, rc);
-  rc = writeback_rows(c, rows, n, accepted, &nLeft);
-  if (rc)
-    return rc;
-  (void)st;
   return nLeft;
 }
 
@@ -1155,12 +1228,9 @@ int64_t eh_simple_rf_cavity(eh_ctx *c, double **part, int64_t np, const EH_RFCA 
     rc = ehd_put_program(c->dev, c->prog->ops, 1);
     if (rc)
       return devfail(c, rc);
-    rc = eh_upload_rows(c, part, np, 8, 0);
+    rc = track_single(c, part, np, 0);
     if (rc)
       return rc;
-    rc = ehd_track(c->dev, 0, 1, 0, 1);
-    if (rc)
-      return devfail(c, rc);
     if (c->prog->n_p0) {
       /* CHANGE_P0: the match step that follows the cavity's own culls */
       rc = match_energy(c, c->prog->p0_op[0], 0, 0);
@@ -1203,12 +1273,9 @@ static int64_t run_aperture(eh_ctx *c, double **coord, int64_t np, double **acce
   if (rc)
     return devfail(c, rc);
   /* NaN and infinite rows are the check's own to remove, at z */
-  rc = eh_upload_rows(c, coord, np, 8, 0);
+  rc = track_single(c, coord, np, 0);
   if (rc)
     return rc;
-  rc = ehd_track(c->dev, 0, 1, 0, 1);
-  if (rc)
-    return devfail(c, rc);
   rc = writeback_rows(c, coord, np, accepted, &nLeft);
   if (rc)
     return rc;

@@ -1,0 +1,90 @@
+"""Rows on their way to the device and back: adjacent rows (one copy) and
+rows that are not, few rows (ordered on the host) and many (on the device),
+with and without losses, wider rows, accepted rows."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from elegant_amd import _abi as A
+from elegant_amd import elements as E
+from elegant_amd import native
+from oracle import oracle_ctypes as O
+from tests.helpers import assert_rows_bitwise
+from tests.test_elements_gpu import PO, beam
+
+pytestmark = pytest.mark.gpu
+
+
+def pointers(block, w, adjacent):
+    """row pointers over block (n, w), or over the same rows two apart"""
+    if adjacent:
+        return A.rows_pointer(block) + (block,)
+    wide = np.full((2 * block.shape[0], w), 7.5)
+    wide[::2] = block
+    ptr, keep = A.rows_pointer(wide)
+    every = np.ascontiguousarray(keep[::2])
+    return every.ctypes.data_as(C.POINTER(C.POINTER(C.c_double))), every, wide
+
+
+def rows_of(holder, adjacent):
+    if adjacent:
+        return holder
+    assert (holder[1::2] == 7.5).all()  # what lies between the rows is not ours
+    return holder[::2]
+
+
+@pytest.mark.parametrize("adjacent", [True, False])
+@pytest.mark.parametrize("n,w,loss", [(1, 8, True), (255, 8, False), (257, 11, True), (14563, 8, True),
+                                      (14564, 8, False), (14564, 8, True), (20011, 10, True)])
+def test_element_rows(tracker, n, w, loss, adjacent):
+    """an aperture check over rows of w columns (14563 rows of 8 columns with
+    their loss records are the most that take the small copy): survivors and
+    order as the checker's, other columns and accepted rows follow"""
+    r = np.zeros((n, w))
+    r[:, :8] = beam(n, 5)[:, :8]
+    r[:, 7:] = np.arange(n)[:, None] + np.arange(w - 7) / 64
+    xmax, ymax = (0.004, 0.002) if loss else (10.0, 10.0)
+    c = r[:, :8].copy()
+    cp, keep = A.rows_pointer(c)
+    nc = O.lib("glibc").or_limit_amplitudes(cp, xmax, ymax, n, 9.0, PO, 1, 0)
+    assert (nc < n) == (loss and n > 1)
+    ptr, k1, held = pointers(r.copy(), w, adjacent)
+    acc, k2, aheld = pointers(-r, w, adjacent)
+    tracker.set_particle_properties(w)
+    try:
+        ng = native.lib().eh_limit_amplitudes(tracker._ctx, ptr, xmax, ymax, n, acc, 9.0, PO, 1, 0)
+    finally:
+        tracker.set_particle_properties(8)
+    g = rows_of(held, adjacent)
+    assert ng == nc
+    assert_rows_bitwise(np.ascontiguousarray(g[:, :7]), np.ascontiguousarray(c[:, :7]), "rows")
+    src = g[:, 6].astype(np.int64) - 1  # IDs are 1..n
+    assert_rows_bitwise(np.ascontiguousarray(g[:, 7:]), np.ascontiguousarray(r[src, 7:]), "other columns")
+    assert_rows_bitwise(np.ascontiguousarray(rows_of(aheld, adjacent)), np.ascontiguousarray(-r[src]), "accepted")
+
+
+@pytest.mark.parametrize("adjacent", [True, False])
+@pytest.mark.parametrize("n", [1, 256, 14565])
+def test_upload_track_download(tracker, n, adjacent):
+    """do_tracking's calls over both kinds of rows, with rows culled for NaN
+    and infinity before the first element, against the one-call entry"""
+    r = beam(n, 6)[:, :8].copy()
+    if n > 1:
+        r[n // 2, 0] = np.nan
+        r[n - 1, 2] = np.inf
+    bl = E.Beamline([E.MAXAMP(X_MAX=0.004, Y_MAX=0.003), E.DRIF(L=0.7), E.KQUAD(L=0.3, K1=0.9, N_KICKS=4)])
+    o = O.Oracle("emath")
+    c = r.copy()
+    o_left = o.do_tracking(c, bl, PO, 3)
+    tracker.load(bl, PO)
+    ptr, k1, held = pointers(r.copy(), 8, adjacent)
+    native.check(tracker._ctx, native.lib().eh_upload(tracker._ctx, ptr, n, 8))
+    tracker.n = n
+    held[:] = 7.5  # the rows are the caller's again once eh_upload returns
+    st = tracker.track(0, 3)
+    left = C.c_int64()
+    native.check(tracker._ctx, native.lib().eh_download(tracker._ctx, ptr, n, 8, C.byref(left)))
+    assert left.value == o_left == st.n_left
+    assert_rows_bitwise(np.ascontiguousarray(rows_of(held, adjacent)[:, :7]),
+                        np.ascontiguousarray(c[:, :7]), "tracked")
