@@ -845,14 +845,15 @@ DEV bool csbend_body(double &X, double &QX, double &Y, double &QY, const double 
  *  - at the entry X, QX, QY are 0 or within [2^-700, 2^600] in magnitude
  *    (QY not -0, whose sign the first kick could change), opd^2 - QY^2 >=
  *    2^-128, opd in [2^-64, 2^64]; the host has checked radii, substep
- *    angles c (2^-300 <= |c| < 2^-5) and kick lengths (EH_F_FAST);
+ *    angles c (2^-20 <= |c| < 2^-5) and kick lengths (EH_F_FAST);
  *  - phi^2 < zlim at every substep (a running maximum), where zlim keeps
  *    |phi| and |c + phi| below 2^-5 (in the WIDE instance, for substep
  *    angles of 2^-6 and more, both squares are watched).  |phi| >= |sin phi|
  *    as the series' terms have one sign, so that rules out |sin phi| > 1 and
- *    cos = 0, and cos phi / cos(c + phi) lies within 1 % of 1;
+ *    cos = 0, and cos phi / cos(c + phi) lies within 1 % of 1 (and is not
+ *    1 / (1 - 2^-53), as c is far above 2^-26);
  *  - the dividends stay 0 or >= 2^-718: c + phi is 0 or at least an ulp of
- *    2^-300, hence QX = f sin(c + phi) is 0 or >= 2^-420 after a drift, and
+ *    2^-20, hence QX = f sin(c + phi) is 0 or >= 2^-140 after a drift, and
  *    after a kick 0 or an ulp of such terms; X = rho0 (f - 1) + f X is its
  *    old value when f = 1 and otherwise has a term of at least 2^-117;
  *  - |X| + |QX| <= 2^600 at the start of every slice and at the end: X
@@ -876,6 +877,9 @@ DEV bool csbend_body_fast(double &X, double &QX, double &Y, double &QY, const do
   double r_f, r_f1;
   double f = em_sqrt_recip_mid(fin, &r_f);
   const double f1 = em_sqrt_recip_mid(fin1, &r_f1);
+  /* sin_phi = 2^-26 exactly over cos_phi = 1 - 2^-53 (em_recip_cos_small): a
+   * slope of sqrt(machine epsilon) at the entry, a usual finite-difference step */
+  good &= __builtin_fabs(QX) != 0x1.0p-26 * f;
   double acc = 0, zmax = 0;
   const em_small_k K = em_small_coefs();
   for (int i = 0; i < HD_NSLICES(H); i++) {

@@ -762,7 +762,10 @@ EM_FN double em_sqrt_mid(double x) {
 /* em_sqrt_mid(x) = g and em_recip(g) from one v_rsq_f64, 2^-128 <= x <= 2^128:
  * after the iteration h is 1/(2 sqrt(x)) to about an ulp, so 2h stands in for
  * v_rcp_f64 (four times the issue cycles of an FMA) and the first of em_recip's
- * two Newton steps. */
+ * two Newton steps.  It is doubled an ulp high: for g = 1 - 2^-53 (times a
+ * power of 2) h is 1/2, from 1 the Newton step ends on the tie 1 + 2^-53 and
+ * rounds down to 1, and quotients of powers of 2 by g would come out an ulp
+ * low; from 1 + 2^-52 it ends just above the tie, on 1/g rounded. */
 EM_FN double em_sqrt_recip_mid(double x, double *y) {
 #if defined(__HIP_DEVICE_COMPILE__)
   double r = __builtin_amdgcn_rsq(x);
@@ -774,7 +777,7 @@ EM_FN double em_sqrt_recip_mid(double x, double *y) {
   g = __builtin_fma(d, h, g);
   d = __builtin_fma(-g, g, x);
   g = __builtin_fma(d, h, g);
-  h = h + h;
+  h = h * 0x1.0000000000001p+1;
   e = __builtin_fma(-g, h, 1.0);
   *y = __builtin_fma(h, e, h);
   return g;
@@ -831,7 +834,9 @@ EM_FN double em_asin_small_c(double x, double z, const em_small_k *k) {
 }
 
 /* em_recip(c) of a cosine c = em_cos_small_c(z, k), z < 2^-10: the secant's
- * series 1 + z/2 + 5 z^2/24 (next term below 2^-33) and one Newton step */
+ * series 1 + z/2 + 5 z^2/24 (next term below 2^-33) and one Newton step.  For
+ * c = 1 - 2^-53 it may be 1, which only shows in quotients of powers of 2:
+ * callers keep those away from it */
 EM_FN double em_recip_cos_small(double c, double z, const em_small_k *k) {
 #if defined(__HIP_DEVICE_COMPILE__)
   double y = __builtin_fma(z, __builtin_fma(z, k->sec, 0.5), 1.0);

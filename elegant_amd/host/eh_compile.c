@@ -698,7 +698,7 @@ static int compile_csbend(const eh_element *e, const EH_MAXAMP *maxamp, eh_op *o
     double amax = 0;
     for (int j = 0; j < nsub; j++) {
       double a = fabs(op->d[EH_D_BDSHR + j]), k = fabs(op->d[EH_D_BDS + j]);
-      if (!(a >= 0x1.0p-300 && a < 0x1.0p-5) || !(k == 0 || em_recip_ok(k)))
+      if (!(a >= 0x1.0p-20 && a < 0x1.0p-5) || !(k == 0 || em_recip_ok(k)))
         fast = 0;
       amax = a > amax ? a : amax;
     }

@@ -157,3 +157,48 @@ def test_csbend_whole_element_common_path(tracker, kw):
         nc = O.lib("emath").or_track_through_csbend(ptr, c.shape[0], C.byref(b), PO, 3.0, C.byref(ap))
         assert_same_survivors(r, g, ng, c, nc)
         assert_rows_bitwise(g[:, :7], c[:, :7], "csbend whole element")
+
+
+def test_quotients_of_powers_of_two(tracker):
+    """divisors 1 - k 2^-53 (all mantissa bits set for k = 1) under powers of
+    two and their neighbours: the reciprocal that ends on a rounding tie"""
+    k = np.arange(1, 8193)
+    g = (1 - k * 2.0 ** -53)[None, :] * 2.0 ** np.array([-60, -1, 0, 1, 60])[:, None]
+    for a in (1.0, -(2.0 ** -26), 2.0 ** 500, 1 + 2.0 ** -52, 1.5, 2 - 2.0 ** -52):
+        b = np.concatenate([(g * g).ravel(), (2.0 ** np.array([-120, 0, 2, 120])[:, None] *
+                                              (1 - k * 2.0 ** -53)[None, :]).ravel()])
+        aa = np.full(b.size, a)
+        assert (tracker.math_probe(12, aa, b) == aa / np.sqrt(b)).all(), a
+
+
+@pytest.mark.parametrize("make", [
+    lambda: E.KQUAD(L=0.3, K1=1.1, N_KICKS=4), lambda: E.KOCT(L=0.1, K3=10.0, N_KICKS=4),
+    lambda: E.CSBEND(L=1.0, ANGLE=0.08, N_KICKS=16), lambda: E.CSBEND(L=0.3, ANGLE=4e-7, N_KICKS=4),
+    lambda: E.CSBEND(L=1.0, ANGLE=0.08, K1=0.3, NONLINEAR=0, N_KICKS=16)])
+def test_slopes_near_sqrt_epsilon(tracker, make):
+    """slopes of 2^-26 and around it on the reference energy, where momenta
+    are powers of two and roots 1 - 2^-53, and a scan that crosses such slopes
+    at a bend's exit"""
+    el = make()
+    h = 2.0 ** -26
+    r = np.zeros((6001, 8))
+    r[:, 6] = np.arange(1, 6002)
+    r[:, 1] = np.linspace(-1.5e-7, 1.5e-7, 6001)
+    edge = [(a, b) for a in (0, h, -h, h / 2, 2 * h, h * (1 + 2.0 ** -52)) for b in (0, h, -h, h / 2)]
+    for i, (a, b) in enumerate(edge):
+        r[10 * i:10 * i + 5, 1] = a
+        r[10 * i:10 * i + 5, 3] = b
+        r[10 * i + 1, 5] = 1.0
+        r[10 * i + 2, 5] = -0.5
+        r[10 * i + 3, 0] = 1e-3
+        r[10 * i + 4, 2] = 1e-9
+    g, c = r.copy(), r.copy()
+    ptr, keep = rows_ptr(c)
+    if el.type == A.EH_T_CSBEND:
+        ng = tracker.track_through_csbend(g, el.p.csbend, PO, 3.0)
+        nc = O.lib("emath").or_track_through_csbend(ptr, c.shape[0], C.byref(el.p.csbend), PO, 3.0, None)
+    else:
+        ng = tracker.multipole_tracking2(g, el, PO, 3.0)
+        nc = O.lib("emath").or_multipole_tracking2(ptr, c.shape[0], C.byref(el), PO, 3.0, None)
+    assert ng == nc == r.shape[0]
+    assert_rows_bitwise(g[:, :7], c[:, :7], "slopes near 2^-26")
