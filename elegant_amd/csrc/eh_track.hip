@@ -922,6 +922,100 @@ DEV bool csbend_body_fast(double &X, double &QX, double &Y, double &QY, const do
   return good & (acc <= 0x1.0p+600) & (zmax < (WIDE ? EM_SMALL_Z : m.zlim));
 }
 
+/* The slices of a combined-function bend with expansion order 4 (K1 and K2),
+ * four substeps a slice: csbend_body with FIELD, without branches.  Bound by
+ * the latency of the general code's 15 coefficient loads per kick, each used
+ * as it arrives; here they are loaded once per element, and the powers of x
+ * and y are shared by the terms they appear in (the same products: y^k is
+ * built from y^(k-1) in every sum of bend_fields).  Fx and Fy are summed in
+ * its order.  A bend of 16 slices over 20011 rows: 378 -> 287 us with the
+ * transfers.
+ *
+ * Against the dipole's conditions above: QY moves with the kicks, so f is
+ * taken anew after each (a running minimum keeps it >= 2^-64), the kicks'
+ * dividends and the momenta after them are 0 or >= 2^-700 by their running
+ * minimum exponent, and acc bounds the dividends from above and catches a NaN
+ * of either plane (in Y it reaches QX through Fy). */
+DEV void field5(const double *F, double x, double y, double &Fx, double &Fy) {
+  const double y2 = y * y, y3 = y2 * y, y4 = y3 * y, x2 = x * x, x3 = x2 * x, x4 = x3 * x;
+  Fx = 0.0 + F[0] * y;
+  Fx += F[1] * y3;
+  Fy = 0.0 + F[2];
+  Fy += F[3] * y2;
+  Fy += F[4] * y4;
+  Fx += F[5] * x * y;
+  Fx += F[6] * x * y3;
+  Fy += F[7] * x;
+  Fy += F[8] * x * y2;
+  Fx += F[9] * x2 * y;
+  Fy += F[10] * x2;
+  Fy += F[11] * x2 * y2;
+  Fx += F[12] * x3 * y;
+  Fy += F[13] * x3;
+  Fy += F[14] * x4;
+}
+
+DEV bool csbend_field_fast(double &X, double &QX, double &Y, double &QY, const double opd, const double r_opd,
+                           double &dist, const hdr_t H, const bendc_t &m, eh_opc &op) {
+  const double rho0 = m.rho0, rhoa = m.rhoa;
+  double F[15];
+  for (int k = 0; k < 15; k++)
+    F[k] = op.d[EH_D_FIELD + k];
+  bool good = (opd >= 0x1.0p-64) & (opd <= 0x1.0p+64) &
+              ((__builtin_fabs(X) + __builtin_fabs(QX)) + __builtin_fabs(QY) <= 0x1.0p+600) &
+              (imin3(__builtin_amdgcn_frexp_exp(X), __builtin_amdgcn_frexp_exp(QX), __builtin_amdgcn_frexp_exp(QY)) >=
+               -699);
+  const double o2 = sq(opd);
+  double f2 = o2 - sq(QY), fmin2 = f2, r_f, f = em_sqrt_recip_mid(f2, &r_f);
+  good &= __builtin_fabs(QX) != 0x1.0p-26 * f; /* as for the dipole */
+  double acc = 0, zmax = 0;
+  int emin = 0;
+  const em_small_k K = em_small_coefs();
+  for (int i = 0; i < HD_NSLICES(H); i++) {
+    good &= in_bounds(X, Y, m.b, HD_FLAGS(H), op);
+    acc += __builtin_fabs(X) + __builtin_fabs(QX);
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      double sin_phi = em_div_pos(QX, f, r_f);
+      double phi = em_asin_small_c(sin_phi, sin_phi * sin_phi, &K);
+      const double ang = m.dshr[j] + phi;
+      const double za = ang * ang, zp = phi * phi;
+      zmax = __builtin_fmax(zmax, __builtin_fmax(zp, za));
+      double sine = em_sin_small_c(ang, za, &K), cosi = em_cos_small_c(za, &K);
+      const double r_c = em_recip_cos_small(cosi, za, &K);
+      double tang = em_div_pos(sine, cosi, r_c);
+      double cos_phi = em_cos_small_c(zp, &K);
+      QX = f * sine;
+      double factor = em_div_pos((rho0 + X) * cos_phi, f, r_f) *
+                      (tang - em_div_pos(sin_phi, cos_phi, em_recip_cos_small(cos_phi, zp, &K)));
+      Y += QY * factor;
+      dist += factor * opd;
+      const double fc = em_div_pos(cos_phi, cosi, r_c);
+      X = rho0 * (fc - 1) + fc * X;
+      if (j == 3)
+        break; /* kickFrac[last] == 0 */
+      double Fx, Fy;
+      field5(F, X, Y, Fx, Fy);
+      /* (-ds g) Fy = -(ds g Fy) */
+      const double dg = m.ds[j] * (1 + em_div_pos(X, rho0, m.rrho0)), kx = -(dg * Fy), ky = dg * Fx;
+      QX += em_div_pos(kx, rhoa, m.rrhoa);
+      QY += em_div_pos(ky, rhoa, m.rrhoa);
+      acc += __builtin_fabs(kx) + __builtin_fabs(ky);
+      emin = imin3(emin, __builtin_amdgcn_frexp_exp(kx), __builtin_amdgcn_frexp_exp(ky));
+      emin = imin3(emin, __builtin_amdgcn_frexp_exp(QX), __builtin_amdgcn_frexp_exp(QY));
+      QX = em_div_pos(QX, opd, r_opd);
+      QY = em_div_pos(QY, opd, r_opd);
+      QX *= opd;
+      QY *= opd;
+      f2 = o2 - sq(QY);
+      fmin2 = __builtin_fmin(fmin2, f2);
+      f = em_sqrt_recip_mid(f2, &r_f);
+    }
+  }
+  acc += __builtin_fabs(X) + __builtin_fabs(QX) + __builtin_fabs(QY);
+  return good & (acc <= 0x1.0p+600) & (emin >= -699) & (fmin2 >= 0x1.0p-128) & (zmax < EM_SMALL_Z);
+}
+
 DEV int track_csbend(particle &p, eh_opc &op, eh_zc *z) {
   const int flags = op.flags;
   const double ct = op.d[EH_D_CT], st = op.d[EH_D_ST];
@@ -1031,9 +1125,9 @@ static __device__ __attribute__((noinline)) double edge_tan(double a) { return e
  * moderate, and the host has checked the edges (EH_F_FAST).  1 + delta, the
  * edges' radius and the velocity are the same at both ends (nothing changes
  * delta here), so each has one reciprocal. */
-DEV bool track_csbend_fast(particle &p, const hdr_t H, hdr_t next, eh_opc &op) {
+template <bool FIELD> DEV bool track_csbend_fast(particle &p, const hdr_t H, hdr_t next, eh_opc &op) {
   const int flags = HD_FLAGS(H);
-  if (!(flags & EH_F_FAST))
+  if (!(flags & EH_F_FAST) || (!FIELD && (flags & EH_F_FIELD)))
     return false;
   const bendc_t m = load_bendc(op, next);
   const bend_t B = load_bend(op);
@@ -1070,7 +1164,9 @@ DEV bool track_csbend_fast(particle &p, const hdr_t H, hdr_t next, eh_opc &op) {
   good &= __builtin_fabs(xp) + __builtin_fabs(yp) <= 0x1.0p+60;
   /* the 4th-order integrator's four substeps of a slice unrolled (NSUB = 4):
    * the scheduler overlaps neighbouring substeps */
-  if (op.nsub == 4 && !(flags & EH_F_WIDE))
+  if (FIELD)
+    good &= csbend_field_fast(X, QX, Y, QY, opd, r_opd, dist, H, m, op);
+  else if (op.nsub == 4 && !(flags & EH_F_WIDE))
     good &= csbend_body_fast<4, false>(X, QX, Y, QY, opd, r_opd, dist, H, m, op);
   else
     good &= csbend_body_fast<0, true>(X, QX, Y, QY, opd, r_opd, dist, H, m, op);
@@ -1395,6 +1491,23 @@ SLOW slow_csbend(particle p, eh_opc *op, eh_zc *z) {
   return o;
 }
 
+/* the same with the common path of combined-function bends, out of line with
+ * its registers.  Only the tracking kernel takes it: in the batch kernel the
+ * values kept across the call spill (27 VGPRs with two particles per lane),
+ * and an aperture study without such bends took 96 ms where it takes 83 */
+SLOW slow_csbend_field(particle p, eh_opc *op, eh_zc *z) {
+  step_out o;
+  eh_opc &u = *uniform(op);
+  const hdr_t H = load_hdr(&u);
+  o.p = p;
+  o.lost = 0;
+  if ((HD_FLAGS(H) & EH_F_FIELD) && track_csbend_fast<true>(o.p, H, H, u))
+    return o;
+  o.lost = track_csbend(p, u, uniform(z));
+  o.p = p;
+  return o;
+}
+
 SLOW slow_rfca(particle p, eh_opc *op, eh_zc *z) {
   step_out o;
   o.lost = track_rfca(p, *uniform(op), uniform(z));
@@ -1434,7 +1547,7 @@ SLOW slow_checks(particle p, eh_opc *op, eh_zc *z) {
 /* One element on one particle.  z points at the element's (z_start, z_end),
  * which only the loss paths read: in the element record itself, or in the
  * position table of a program whose repeated cells share one record. */
-DEV int run_op(particle &p, const hdr_t H, hdr_t next, eh_opc &op, eh_zc *z, int64_t pass) {
+template <bool FIELD> DEV int run_op(particle &p, const hdr_t H, hdr_t next, eh_opc &op, eh_zc *z, int64_t pass) {
   const int code = HD_OP(H);
   step_out o;
   o.lost = 0;
@@ -1462,13 +1575,13 @@ DEV int run_op(particle &p, const hdr_t H, hdr_t next, eh_opc &op, eh_zc *z, int
       p = slow_drift2(p, L, hL).p;
   } else if (code == EH_OP_CSBEND) {
     particle q = p;
-    const bool done = track_csbend_fast(q, H, next, op);
+    const bool done = track_csbend_fast<false>(q, H, next, op);
     if (ALL_LANES(done))
       p = q;
     else if (done)
       p = q;
     else {
-      o = slow_csbend(p, &op, z);
+      o = FIELD ? slow_csbend_field(p, &op, z) : slow_csbend(p, &op, z);
       p = o.p;
     }
   } else {
@@ -1568,7 +1681,7 @@ __global__ void __launch_bounds__(256, 4) eh_track_kernel(eh_state st, const eh_
         eh_opc *nxt = op + 1 == op1 ? op0 : op + 1;
         hdr_t hn = load_hdr(nxt);
         if (!lost) {
-          lost = run_op(p, h, hn, *op, zs + 2 * f, pass0 + ip);
+          lost = run_op<true>(p, h, hn, *op, zs + 2 * f, pass0 + ip);
           if (lost) {
             lost_op = f;
             lost_pass = ip;
@@ -1652,7 +1765,7 @@ __global__ void __launch_bounds__(256, 4) eh_batch_kernel(eh_state st, const eh_
         for (int k = 0; k < PPL; k++) {
           if (!live[k])
             continue;
-          int l = run_op(p[k], hcur, h, op, &op.z_start, pass0 + ip);
+          int l = run_op<false>(p[k], hcur, h, op, &op.z_start, pass0 + ip);
           if (l) {
             live[k] = false;
             lost[k] = l;

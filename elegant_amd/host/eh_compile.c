@@ -692,8 +692,11 @@ static int compile_csbend(const eh_element *e, const EH_MAXAMP *maxamp, eh_op *o
   }
   /* the branch-free common path of the kernel needs positive radii within
    * the shared-reciprocal range, moderate substep angles below 2^-5, and kick
-   * lengths that are 0 or moderate */
-  if (rho0 > 0 && rho_actual > 0 && em_recip_ok(rho0) && em_recip_ok(rho_actual) && !(op->flags & EH_F_FIELD)) {
+   * lengths that are 0 or moderate; with multipoles (EH_F_FIELD) the one
+   * expansion it is written for, order 4 (K1, K2 and XKICK), and the
+   * 4th-order integrator */
+  if (rho0 > 0 && rho_actual > 0 && em_recip_ok(rho0) && em_recip_ok(rho_actual) &&
+      (!(op->flags & EH_F_FIELD) || (op->nfield == 5 && nsub == 4))) {
     int fast = 1;
     double amax = 0;
     for (int j = 0; j < nsub; j++) {

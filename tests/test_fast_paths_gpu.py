@@ -202,3 +202,30 @@ def test_slopes_near_sqrt_epsilon(tracker, make):
         nc = O.lib("emath").or_multipole_tracking2(ptr, c.shape[0], C.byref(el), PO, 3.0, None)
     assert ng == nc == r.shape[0]
     assert_rows_bitwise(g[:, :7], c[:, :7], "slopes near 2^-26")
+
+
+# expansion order 4 with the 4th-order integrator (the common path), and next
+# to it what stays with the general code: orders 5 and 6, another integrator;
+# kicks so strong that slopes leave the bands, so weak that kicks fall below
+# the smallest dividend; wide substep angles; XKICK alone
+@pytest.mark.parametrize("kw", [
+    dict(K1=-0.4, K2=2.0), dict(K1=0.6, E1=0.02, E2=0.03, HGAP=0.02), dict(K2=200.0, ANGLE=-0.08), dict(XKICK=1e-4),
+    dict(K1=0.3, NONLINEAR=0), dict(K1=400.0), dict(K1=1e-250), dict(K1=-0.4, ANGLE=0.5), dict(K1=-0.4, FSE=1e-3,
+    ETILT=1e-3, DX=1e-4, DZ=2e-4), dict(K1=0.2, K3=30.0), dict(K4=900.0), dict(K1=-0.4, INTEGRATION_ORDER=2),
+    dict(K1=-0.4, INTEGRATION_ORDER=6)])
+def test_combined_function_bend(tracker, kw):
+    b = E.CSBEND(L=1.0, N_KICKS=16, **{"ANGLE": 0.08, **kw}).p.csbend
+    r = csbend_edge_rows(1500, 47)
+    r[700::3, 3] = 0.0
+    r[701::3, 3] = -0.0
+    r[800:850, 0] = np.linspace(-0.0062, 0.0062, 50)
+    r[850:900, 2] = 10.0 ** -np.linspace(100, 320, 50)
+    r[900:950, 5] = np.linspace(-1.0, 1.0, 50)
+    r[1100::2, 1] *= 60.0
+    for ap in (A.EH_MAXAMP(0.05, 0.04, 0, 2, 2, 0), A.EH_MAXAMP(0.006, 0.004, 1, 2, 4, 0)):
+        g, c = r.copy(), r.copy()
+        ng = tracker.track_through_csbend(g, b, PO, 3.0, ap)
+        ptr, keep = rows_ptr(c)
+        nc = O.lib("emath").or_track_through_csbend(ptr, c.shape[0], C.byref(b), PO, 3.0, C.byref(ap))
+        assert_same_survivors(r, g, ng, c, nc)
+        assert_rows_bitwise(g[:, :7], c[:, :7], "combined-function bend")
