@@ -346,7 +346,7 @@ DEV bool in_aperture(double x, double y, eh_opc &op) {
   return !((op.in_xmax > 0 && __builtin_fabs(x) > op.in_xmax) || (op.in_ymax > 0 && __builtin_fabs(y) > op.in_ymax));
 }
 
-/* surely inside it (the host's bounds, eh_op_bounds): two compares without
+/* surely inside it (bounds from eh_op_finish): two compares without
  * a branch for the common paths, whose lanes outside take the general code */
 DEV bool in_bounds(double x, double y, const bounds_t &b, int flags, eh_opc &op) {
   if (flags & EH_F_INTILT) {

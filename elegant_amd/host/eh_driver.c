@@ -543,6 +543,8 @@ static int refresh_losses(eh_ctx *c) {
 static int order_until(eh_ctx *c, int64_t pass_lim, int32_t code_lim) {
   int64_t effort, left;
   int rc;
+  if (ehd_state_n(c->dev) != c->n)
+    return devfail(c, EH_ERR_STATE);
   if (!c->n)
     return EH_OK;
   rc = ehd_effort(c->dev, 0, 0, &effort, &left);
@@ -811,6 +813,8 @@ int eh_track(eh_ctx *c, int64_t pass0, int64_t npasses, double *P_central, eh_st
       memset(stats, 0, sizeof(*stats));
     return EH_OK;
   }
+  if (ehd_state_n(c->dev) != c->n) /* a batch of the context holds the device's columns */
+    return devfail(c, EH_ERR_STATE);
   ehd_timing_reset(c->dev);
   {
     int64_t pass = pass0, end = pass0 + npasses;

@@ -88,3 +88,19 @@ def test_upload_track_download(tracker, n, adjacent):
     assert left.value == o_left == st.n_left
     assert_rows_bitwise(np.ascontiguousarray(rows_of(held, adjacent)[:, :7]),
                         np.ascontiguousarray(c[:, :7]), "tracked")
+
+
+def test_columns_taken_by_a_batch(tracker):
+    """a batch of the context leaves its own particles on the device: the
+    upload before it is refused, not read as if it were still there"""
+    bl = E.Beamline([E.DRIF(L=0.7)])
+    tracker.load(bl, PO)
+    tracker.upload(beam(300, 8))
+    b = native.Batch(tracker)
+    b.add_variant(bl, PO, beam(500, 9))
+    b.track(0, 1)
+    b.close()
+    for call in (lambda: tracker.track(0, 1), tracker.download):
+        with pytest.raises(native.EHError) as e:
+            call()
+        assert e.value.code == A.EH_ERR_STATE
