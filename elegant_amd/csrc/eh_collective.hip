@@ -70,8 +70,48 @@ typedef struct {
   int32_t pad[3];
 } coll_plan;
 
-/* after the min/max pass: the decisions of wake.c:120-182 and
+/* after the min/max pass, from its result in p->red: the decisions of wake.c:120-182 and
  * zlongit.c:195-236 that do not need the mean */
+DEV void plan_decide(coll_plan *p, int32_t kind, int32_t n_fixed, int32_t zl_nb, double dt, double wake_span,
+                     int32_t allow_long, int32_t nb_cap, int32_t mean_given, double mean) {
+  if (p->red[2] == 0) {
+    p->nb = 0;
+    return;
+  }
+  double tmin = key_value(p->red[0]), tmax = key_value(p->red[1]);
+  p->tmin = tmin;
+  p->tmax = tmax;
+  if (kind == EH_OP_ZLONGIT || n_fixed) {
+    double am = __builtin_fabs(tmin) > __builtin_fabs(tmax) ? __builtin_fabs(tmin) : __builtin_fabs(tmax);
+    p->e = eh_fsum_exponent(am);
+  }
+  if (kind == EH_OP_WAKE) {
+    if ((tmax - tmin) > wake_span && !allow_long) {
+      p->err = EH_ERR_LONGBEAM;
+      return;
+    }
+    if (n_fixed) {
+      p->nb = n_fixed; /* tmin set from the mean: the fixed-point one, or the host's */
+      if (mean_given) {
+        p->tmean = mean;
+        p->tmin = mean - dt * p->nb / 2.0;
+      }
+    } else {
+      int32_t nb = (int32_t)(int64_t)((tmax - tmin) / dt + 3);
+      p->tmin = tmin - dt;
+      p->nb = nb;
+    }
+  } else {
+    p->nb = zl_nb;
+    if ((tmax - tmin) * 2 > zl_nb * dt && !allow_long) {
+      p->err = EH_ERR_LONGBEAM;
+      return;
+    }
+  }
+  if (p->nb > nb_cap)
+    p->err = EH_ERR_LONGBEAM;
+}
+
 __global__ void __launch_bounds__(CB) coll_plan_minmax(coll_plan *plan, const unsigned long long *part,
                                                        int64_t nparts, int32_t kind, int32_t n_fixed, int32_t zl_nb,
                                                        double dt, double wake_span, int32_t allow_long,
@@ -114,42 +154,7 @@ __global__ void __launch_bounds__(CB) coll_plan_minmax(coll_plan *plan, const un
   p->red[2] = scnt[0];
   if (kind < 0)
     return; /* the time span only */
-  if (p->red[2] == 0) {
-    p->nb = 0;
-    return;
-  }
-  double tmin = key_value(p->red[0]), tmax = key_value(p->red[1]);
-  p->tmin = tmin;
-  p->tmax = tmax;
-  if (kind == EH_OP_ZLONGIT || n_fixed) {
-    double am = __builtin_fabs(tmin) > __builtin_fabs(tmax) ? __builtin_fabs(tmin) : __builtin_fabs(tmax);
-    p->e = eh_fsum_exponent(am);
-  }
-  if (kind == EH_OP_WAKE) {
-    if ((tmax - tmin) > wake_span && !allow_long) {
-      p->err = EH_ERR_LONGBEAM;
-      return;
-    }
-    if (n_fixed) {
-      p->nb = n_fixed; /* tmin set from the mean: the fixed-point one, or the host's */
-      if (mean_given) {
-        p->tmean = mean;
-        p->tmin = mean - dt * p->nb / 2.0;
-      }
-    } else {
-      int32_t nb = (int32_t)(int64_t)((tmax - tmin) / dt + 3);
-      p->tmin = tmin - dt;
-      p->nb = nb;
-    }
-  } else {
-    p->nb = zl_nb;
-    if ((tmax - tmin) * 2 > zl_nb * dt && !allow_long) {
-      p->err = EH_ERR_LONGBEAM;
-      return;
-    }
-  }
-  if (p->nb > nb_cap)
-    p->err = EH_ERR_LONGBEAM;
+  plan_decide(p, kind, n_fixed, zl_nb, dt, wake_span, allow_long, nb_cap, mean_given, mean);
 }
 
 /* per-workgroup (min key, max key, alive count) triples in red[3 k ..];
@@ -164,11 +169,14 @@ DEV bool in_step(const int32_t *__restrict__ lp, const int32_t *__restrict__ bun
 __global__ void __launch_bounds__(CB) time_minmax(const double *__restrict__ s, const double *__restrict__ dp,
                                                   const int32_t *__restrict__ lp, int64_t n, double Po,
                                                   unsigned long long *red, const int32_t *__restrict__ bunch,
-                                                  int32_t target) {
+                                                  int32_t target, unsigned int *hist, int32_t nclear) {
   __shared__ unsigned long long smin[CB / 64], smax[CB / 64], scnt[CB / 64];
   unsigned long long kmin = ~0ULL, kmax = 0, cnt = 0;
   const int64_t stride = (int64_t)gridDim.x * CB;
   int64_t i = (int64_t)blockIdx.x * CB + threadIdx.x;
+  /* where the histogram makes the plan itself, its counts are cleared here */
+  for (int64_t k = i; k < nclear; k += stride)
+    hist[k] = 0;
   /* SWEEP_U particles per lane per step, their loads issued together */
   for (; i + (SWEEP_U - 1) * stride < n; i += SWEEP_U * stride) {
     double S[SWEEP_U], D[SWEEP_U];
@@ -298,17 +306,67 @@ DEV int64_t bin_of(double t, double tmin, double dt, int round_half) {
  * atomic per bin per CU */
 #define HB 1024
 #define HIST_LDS_WORDS 16384 /* 64 KB of counts */
+#define HIST_PLAN_WORDS 128  /* at least this much LDS where the plan is made there: 16 triples and the plan */
 #define HIST_U 4 /* particles per lane per step of the histogram sweep (8 measured the same) */
 
 __global__ void __launch_bounds__(HB) histogram(const double *__restrict__ s, const double *__restrict__ dp,
                                                 const int32_t *__restrict__ lp, int64_t n, double Po,
-                                                const coll_plan *plan, double dt, int32_t round_half,
-                                                int32_t lds_bins, unsigned int *hist, const int32_t *__restrict__ bunch,
-                                                int32_t target) {
-  extern __shared__ unsigned int lh[];
-  const int32_t nb = plan->nb;
-  const double tmin = plan->tmin;
-  if (nb <= 0 || plan->err)
+                                                coll_plan *plan, double dt, int32_t round_half, int32_t lds_bins,
+                                                unsigned int *hist, const int32_t *__restrict__ bunch, int32_t target,
+                                                const unsigned long long *__restrict__ part, int64_t nparts,
+                                                double wake_span, int32_t allow_long, int32_t nb_cap) {
+  extern __shared__ __align__(16) unsigned int lh[];
+  coll_plan *p = plan;
+  if (part) {
+    /* a WAKE on its own bins needs nothing but the extremes for its plan:
+     * every workgroup combines them (a few KB from L2) and the first one
+     * stores the plan for the later kernels.  That costs it 2 us and saves
+     * the planning kernel, 5 us, and the gaps around it, 14 us: a step on
+     * 10^6 particles takes 89 us where it took 106 */
+    unsigned long long *sm = (unsigned long long *)lh;
+    unsigned long long kmin = ~0ULL, kmax = 0, cnt = 0;
+    for (int64_t k = threadIdx.x; k < nparts; k += HB) {
+      const unsigned long long a = part[3 * k], b = part[3 * k + 1];
+      kmin = a < kmin ? a : kmin;
+      kmax = b > kmax ? b : kmax;
+      cnt += part[3 * k + 2];
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+      const unsigned long long a = __shfl_xor(kmin, off), b = __shfl_xor(kmax, off);
+      kmin = a < kmin ? a : kmin;
+      kmax = b > kmax ? b : kmax;
+      cnt += __shfl_xor(cnt, off);
+    }
+    const int w = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 0) {
+      sm[3 * w] = kmin;
+      sm[3 * w + 1] = kmax;
+      sm[3 * w + 2] = cnt;
+    }
+    __syncthreads();
+    p = (coll_plan *)(sm + 3 * (HB / 64));
+    if (threadIdx.x == 0) {
+      for (int k = 1; k < HB / 64; k++) {
+        kmin = sm[3 * k] < kmin ? sm[3 * k] : kmin;
+        kmax = sm[3 * k + 1] > kmax ? sm[3 * k + 1] : kmax;
+        cnt += sm[3 * k + 2];
+      }
+      coll_plan q = {};
+      q.red[0] = kmin;
+      q.red[1] = kmax;
+      q.red[2] = cnt;
+      plan_decide(&q, EH_OP_WAKE, 0, 0, dt, wake_span, allow_long, nb_cap, 0, 0.0);
+      *p = q;
+      if (blockIdx.x == 0)
+        *plan = q;
+    }
+    __syncthreads();
+  }
+  const int32_t nb = p->nb, err = p->err;
+  const double tmin = p->tmin;
+  if (part)
+    __syncthreads(); /* the plan's place in LDS is the counts' */
+  if (nb <= 0 || err)
     return;
   /* counts in LDS: as many copies (a power of 2, at most one per wave) as
    * fit, the waves sharing them in turn (a bunch puts most particles in a
@@ -1146,12 +1204,14 @@ static int coll_launch(ehd_dev *d, const ehd_collective *c, double *const crd[6]
   const int32_t *bunch = c->use_bunch ? d->bunch : NULL;
   const int32_t target = c->bunch_target;
   const int32_t mean_given = kind == EH_OP_WAKE && fixed && c->mean_given;
+  const int own_bins = kind == EH_OP_WAKE && !fixed; /* no mean between the extremes and the plan */
   CHK(hipEventRecord(d->cev0, d->stream));
   hipLaunchKernelGGL(time_minmax, dim3((unsigned)rgrid), dim3(CB), 0, d->stream, crd[4], crd[5], lp, n, c->Po,
-                     (unsigned long long *)parts, bunch, target);
-  hipLaunchKernelGGL(coll_plan_minmax, dim3(1), dim3(CB), 0, d->stream, plan, (const unsigned long long *)parts, rgrid,
-                     kind, fixed, c->nb, c->dt, c->wake_span, c->allow_long_beam, (int32_t)nb_max, hist, nclear,
-                     mean_given, c->mean);
+                     (unsigned long long *)parts, bunch, target, hist, own_bins ? nclear : 0);
+  if (!own_bins)
+    hipLaunchKernelGGL(coll_plan_minmax, dim3(1), dim3(CB), 0, d->stream, plan, (const unsigned long long *)parts,
+                       rgrid, kind, fixed, c->nb, c->dt, c->wake_span, c->allow_long_beam, (int32_t)nb_max, hist,
+                       nclear, mean_given, c->mean);
   if ((kind == EH_OP_ZLONGIT || fixed) && !mean_given) {
     hipLaunchKernelGGL(time_fsum, dim3((unsigned)rgrid), dim3(CB), 0, d->stream, crd[4], crd[5], lp, n, c->Po, plan,
                        parts, bunch, target);
@@ -1175,8 +1235,11 @@ static int coll_launch(ehd_dev *d, const ehd_collective *c, double *const crd[6]
     /* room for one copy of the counts per wave, at most 64 KB of LDS */
     const int32_t lds_bins =
         nb_max * (HB / 64) < HIST_LDS_WORDS ? (int32_t)(nb_max * (HB / 64)) : HIST_LDS_WORDS;
-    hipLaunchKernelGGL(histogram, dim3(hgrid), dim3(HB), sizeof(unsigned int) * lds_bins, d->stream, crd[4], crd[5],
-                       lp, n, c->Po, plan, c->dt, kind == EH_OP_WAKE ? 1 : 0, lds_bins, hist, bunch, target);
+    const int32_t lds_words = lds_bins > HIST_PLAN_WORDS ? lds_bins : HIST_PLAN_WORDS;
+    hipLaunchKernelGGL(histogram, dim3(hgrid), dim3(HB), sizeof(unsigned int) * lds_words, d->stream, crd[4], crd[5],
+                       lp, n, c->Po, plan, c->dt, kind == EH_OP_WAKE ? 1 : 0, lds_bins, hist, bunch, target,
+                       own_bins ? (const unsigned long long *)parts : NULL, rgrid, c->wake_span, c->allow_long_beam,
+                       (int32_t)nb_max);
   }
   if (kind == EH_OP_WAKE) {
     hipLaunchKernelGGL(wake_convolve, dim3((unsigned)((nb_max + 1 + CONV_B - 1) / CONV_B)), dim3(CONV_B), 0, d->stream,
@@ -1326,7 +1389,7 @@ int ehd_time_span(ehd_dev *d, double Po, int32_t use_bunch, int32_t target, doub
   unsigned int *hist = (unsigned int *)((char *)d->cwork + PLAN_BYTES);
   unsigned long long *mm = (unsigned long long *)((char *)hist + hist_bytes(64) + 8 * (64 + 8));
   hipLaunchKernelGGL(time_minmax, dim3((unsigned)rgrid), dim3(CB), 0, d->stream, d->coord[4], d->coord[5],
-                     d->loss_pass, n, Po, mm, use_bunch ? d->bunch : NULL, target);
+                     d->loss_pass, n, Po, mm, use_bunch ? d->bunch : NULL, target, (unsigned int *)NULL, 0);
   hipLaunchKernelGGL(coll_plan_minmax, dim3(1), dim3(CB), 0, d->stream, plan, (const unsigned long long *)mm, rgrid,
                      -1, 0, 0, 1.0, 0.0, 0, 0, hist, 0, 0, 0.0);
   CHK(hipGetLastError());

@@ -189,3 +189,35 @@ def test_ring_with_wake_change_p0_bit_exact(tracker):
     assert rows.shape[0] - ng > 10
     assert tracker.P_central == o.P_central != Po
     assert_rows_identical(g, c, "ring with wake change_p0")
+
+
+@pytest.mark.parametrize("n,points,dt", [(1, 10, 1e-12), (2, 4, 1e-9), (255, 4, 2e-10), (1025, 300, 2e-12),
+                                         (4097, 8, 1e-10), (262145, 3000, 2e-13), (300000, 40000, 1e-14)])
+def test_wake_plan_from_the_histogram(tracker, n, points, dt):
+    """a WAKE on its own bins, whose plan the histogram's workgroups make: one
+    workgroup and many, one partial and the most, tables too small to hold the
+    partials' LDS otherwise, counts with and without copies in LDS; then a
+    window the bunch does not fit, refused each time and not remembered"""
+    rows = wake_bunch(n, 20e-12, seed=13)
+    table = Lt.resonator_wake(points=points, dt=dt)  # the element holds its address
+    w = E.WAKE(table)
+    q = 5e-9 / n
+    g, c = rows.copy(), rows.copy()
+    h, v, tmin = tracker.collective_probe(g, w, PO, 0, q)
+    o = O.Oracle("emath")
+    o.set_macro_charge(q)
+    o.wake(c, w.p.wake, PO, 0)
+    hc, vc, tminc, _ = o.last_hist()
+    assert tmin == tminc and np.array_equal(h, hc) and h.sum() == n and np.array_equal(v, vc)
+    assert_rows_identical(g, c, "wake kick")
+    if n > 2:
+        short_table = Lt.resonator_wake(points=points, dt=dt * 1e-3)
+        short = E.WAKE(short_table)
+        from elegant_amd import native
+        for _ in range(2):
+            with pytest.raises(native.EHError) as e:
+                tracker.collective_probe(rows.copy(), short, PO, 0, q)
+            assert e.value.code == A.EH_ERR_LONGBEAM
+        g = rows.copy()
+        assert np.array_equal(tracker.collective_probe(g, w, PO, 0, q)[0], hc)
+        assert_rows_identical(g, c, "wake kick after a refusal")
