@@ -146,6 +146,7 @@ int64_t ehd_noalloc_bins_max(void);
 int ehd_wake_step_noalloc(ehd_dev *d, const ehd_collective *c, double *const crd[6], int64_t n, const double *W,
                           int64_t wpoints);
 #define EHD_COLL_NOCHECKS (1 << 30) /* element entry points: no do_tracking checks after the step */
+#define EHD_COLL_UNTIMED (1 << 29)  /* nothing reads the time of this step: no events around it */
 
 /* tests: op 0 allocate *ptr, 1 free it, 2 copy host -> *ptr, 3 copy *ptr -> host */
 int ehd_test_buffer(ehd_dev *d, int32_t op, void **ptr, void *host, int64_t bytes);

@@ -62,6 +62,7 @@ struct ehd_dev {
   /* collective work buffers */
   ehd_coll_slot slot[EHD_MAX_COLL];
   void *cwork;       /* reductions, histogram, voltages */
+  void *host_plan;   /* a collective step's plan, pinned */
   int32_t *bunch;    /* bunch index per particle (bunched beams) */
   int64_t bunch_cap;
   void *noalloc;     /* device address of this GPU's static no-allocation scratch */

@@ -392,7 +392,7 @@ int eh_collective_probe(eh_ctx *c, double **part, int64_t np, const eh_element *
   rc = eh_upload_rows(c, part, np, eh_ctx_row_props(c), 0);
   if (rc)
     return rc;
-  rc = collective_run(c, 0, e, &prog->ops[0], 0, i_pass, macro, EHD_COLL_NOCHECKS, hist, volt, nb, tmin);
+  rc = collective_run(c, 0, e, &prog->ops[0], 0, i_pass, macro, EHD_COLL_NOCHECKS | EHD_COLL_UNTIMED, hist, volt, nb, tmin);
   if (rc)
     return rc;
   return np > 0 ? eh_ctx_writeback(c, part, np, &nLeft) : EH_OK;
@@ -471,7 +471,7 @@ int64_t eh_track_through_wake_noalloc(eh_ctx *c, double *const coord[6], int64_t
   cc.mc2 = 1e6 * eh_ctx_species(c)->massMV * eh_ctx_species(c)->relSign;
   cc.pass = i_pass;
   cc.Po = Po;
-  cc.flags = EHD_COLL_NOCHECKS;
+  cc.flags = EHD_COLL_NOCHECKS | EHD_COLL_UNTIMED;
   cc.dt = (tmax - tmin) / (wake->wakePoints - 1);
   cc.wake_span = wake->t[wake->wakePoints - 1] - wake->t[0];
   cc.interpolate = wake->interpolate;
