@@ -498,7 +498,7 @@ DEV int multipole_body(double &x, double &xp, double &y, double &yp, double &s, 
  * The slopes at the exit are those after the last kick, as the momenta have
  * not changed since.  A slice of four substeps of a quadrupole takes 182 VALU
  * instructions, 3 of them transcendental (276 with 16 before).  FODO ring, 10^4
- * particles, 64 turns: 84.1 -> 54.9 ms (36.2 with what came after it).
+ * particles, 64 turns: 84.1 -> 54.9 ms (37.1 with what came after it).
  *
  * What makes every step valid:
  *  - the entry and exit limits of the integrator and the aperture at every

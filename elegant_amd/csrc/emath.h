@@ -762,10 +762,12 @@ EM_FN double em_sqrt_mid(double x) {
 /* em_sqrt_mid(x) = g and em_recip(g) from one v_rsq_f64, 2^-128 <= x <= 2^128:
  * after the iteration h is 1/(2 sqrt(x)) to about an ulp, so 2h stands in for
  * v_rcp_f64 (four times the issue cycles of an FMA) and the first of em_recip's
- * two Newton steps.  It is doubled an ulp high: for g = 1 - 2^-53 (times a
- * power of 2) h is 1/2, from 1 the Newton step ends on the tie 1 + 2^-53 and
- * rounds down to 1, and quotients of powers of 2 by g would come out an ulp
- * low; from 1 + 2^-52 it ends just above the tie, on 1/g rounded. */
+ * two Newton steps.  Its last bit is set: for g = 1 - 2^-53 (times a power of
+ * 2) 2h is 1, from where the Newton step ends on the tie 1 + 2^-53 and rounds
+ * down to 1, and quotients of powers of 2 by g would come out an ulp low; from
+ * 1 + 2^-52 it ends just above the tie, on 1/g rounded.  (Doubling by
+ * 2 + 2^-51 instead holds a constant in scalar registers that the batch kernel
+ * does not have: 12 aperture grids took 95-105 ms where they take 88.) */
 EM_FN double em_sqrt_recip_mid(double x, double *y) {
 #if defined(__HIP_DEVICE_COMPILE__)
   double r = __builtin_amdgcn_rsq(x);
@@ -777,7 +779,7 @@ EM_FN double em_sqrt_recip_mid(double x, double *y) {
   g = __builtin_fma(d, h, g);
   d = __builtin_fma(-g, g, x);
   g = __builtin_fma(d, h, g);
-  h = h * 0x1.0000000000001p+1;
+  h = em_from_bits(em_bits(h + h) | 1);
   e = __builtin_fma(-g, h, 1.0);
   *y = __builtin_fma(h, e, h);
   return g;
