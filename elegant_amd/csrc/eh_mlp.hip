@@ -205,21 +205,35 @@ __global__ void adam_k(float *w, const float *g, float *m, float *v, int64_t n, 
  * A training step is three kernels: mlp_rows takes 16 samples per workgroup
  * through all layers and back (activations stay in LDS; they and the layers'
  * gradients are also written out), mlp_wgrad contracts those over the batch
- * into partial weight gradients, mlp_update sums the partials in order and
- * applies Adam.  The products run on the matrix cores in FP32
- * (v_mfma_f32_16x16x4f32: FP32 multiplies and sums, as the LDS-tiled gemm_f32
- * has, which stays for larger nets).  What bounds it: 3.3 GFLOP per step of 4096
- * samples is 22 us at the 150 TFLOP/s of a large FP32 product; the step was 35
- * launches and 470 us, and takes 67 (36 + 23 + 8).
+ * into partial gradients, mlp_update sums the partials in order and applies
+ * Adam.  The products run on the matrix cores in FP32 (v_mfma_f32_16x16x4f32).
+ *
+ * The results are the general path's bit for bit: one such instruction is
+ * four FMAs in the order of its contraction index, each rounded, so every sum
+ * is taken in the order that gemm_f32, col_sum_part, bce_grad and
+ * reduce_slices take it (ascending from zero, the batch in ksplit's slices,
+ * column sums in slices of 64 rows).  Adam divides by the root of the squared
+ * gradient, so another order of a sum shows in the weights: 1.4e-3 of their
+ * norm after 64 steps of 4096 samples.
+ *
+ * What bounds it: 3.3 GFLOP per step of 4096 samples is 22 us at the 150
+ * TFLOP/s of a large FP32 product; a step takes 65 us (38 + 19 + 8), the
+ * general path's 35 launches 470.  mlp_rows reads 1.3 MB of weights per
+ * workgroup from L2, all workgroups in the same order (with the order of the
+ * sums free it took 35).
  *
  * Layouts.  HS = hidden rounded up to 64, XS = inputs rounded up to 64; padded
  * weights are zero, so padded activations and gradients are zero.  A
- * contraction is cut into chunks of 16; lane l of a wave holds elements
- * 4 (l / 16) .. + 3 of the chunk for row (or column) l % 16 as one 16-byte
- * load, and product m of four takes element m of each, in both operands.
- * Weights are kept in that order, one 1 KB block per tile of 16 outputs and
- * chunk: wf for the forward products, wb for the ones going back. */
+ * contraction is cut into chunks of 16, product m of the four that a chunk
+ * takes has elements 4 m .. 4 m + 3 (element 4 m + g in the lanes l / 16 = g),
+ * and a lane loads its elements of all four products as one 16-byte load.  So
+ * element k of a chunk is kept at place mlp_place(k) of it: in the weights,
+ * one 1 KB block per tile of 16 outputs and chunk (wf for the forward
+ * products, wb for the ones going back), and in the rows of activations and
+ * gradients, in LDS and in memory. */
 typedef float f4 __attribute__((ext_vector_type(4)));
+
+static __host__ __device__ __forceinline__ int mlp_place(int k) { return (k & ~15) | (k & 3) << 2 | (k >> 2 & 3); } /* its own inverse */
 
 struct mlp_net {
   const float *wf[3], *wb[3]; /* wb[0] unused */
@@ -231,16 +245,14 @@ struct mlp_batch {
   const float *X, *y;
   const int32_t *perm;        /* sample indices, or NULL */
   float *xb, *h[3], *dz[3];   /* [rows][xs] and [rows][HS] */
-  float *vec;                 /* per workgroup: bias gradients of 3 layers, last weights', last bias', loss */
+  float *dz4, *lrow;          /* per row: the output's gradient and the loss */
   float *prob;                /* prediction */
   int rows;
 };
 
 /* acc[mt][t] += rows of a (LDS, stride lda) x tile wave + 4 t of wt, over kc
- * chunks.  A workgroup is alone on its CU, one wave per SIMD, so D chunks of
- * weights are in flight; and the workgroups of an XCD (every eighth) start at
- * different chunks, so that each finds most of its weights already in the
- * XCD's L2 instead of all of them waiting for the same lines at once. */
+ * chunks, D of them in flight: a workgroup is alone on its CU, one wave per
+ * SIMD. */
 template <int NT, int MT, int D>
 static __device__ __forceinline__ void rows_mm(const float *a, int lda, const float *__restrict__ wt, int kc,
                                                f4 (&acc)[MT][NT]) {
@@ -251,23 +263,20 @@ static __device__ __forceinline__ void rows_mm(const float *a, int lda, const fl
   asm volatile("" : "+v"(lane));
   const float *ar = a + (lane & 15) * lda + 4 * (lane >> 4);
   const float *w0 = wt + (size_t)wave * kc * 256 + 4 * lane;
-  int first = (int)((blockIdx.x >> 3) % (unsigned)kc), cl = first, ca = first; /* chunks to load and to use */
   f4 b[D][NT];
 #pragma unroll
-  for (int u = 0; u < D; u++) {
+  for (int u = 0; u < D; u++)
 #pragma unroll
     for (int t = 0; t < NT; t++)
-      b[u][t] = *(const f4 *)(w0 + ((size_t)4 * t * kc + cl) * 256);
-    cl = cl + 1 < kc ? cl + 1 : 0;
-  }
+      b[u][t] = *(const f4 *)(w0 + ((size_t)4 * t * kc + (u < kc ? u : 0)) * 256);
   f4 av[2][MT]; /* the next chunk's rows are read while a chunk's products run */
 #pragma unroll
   for (int m = 0; m < MT; m++)
-    av[0][m] = *(const f4 *)(ar + 16 * m * lda + 16 * ca);
+    av[0][m] = *(const f4 *)(ar + 16 * m * lda);
   for (int c = 0; c < kc; c += D) {
 #pragma unroll
     for (int u = 0; u < D; u++) {
-      ca = ca + 1 < kc ? ca + 1 : 0;
+      const int ca = c + u + 1 < kc ? c + u + 1 : 0, cl = c + u + D < kc ? c + u + D : 0; /* rows, weights to load */
 #pragma unroll
       for (int m = 0; m < MT; m++)
         av[D > 1 ? (u + 1) & 1 : 1][m] = *(const f4 *)(ar + 16 * m * lda + 16 * ca);
@@ -281,7 +290,6 @@ static __device__ __forceinline__ void rows_mm(const float *a, int lda, const fl
 #pragma unroll
       for (int t = 0; t < NT; t++)
         b[u][t] = *(const f4 *)(w0 + ((size_t)4 * t * kc + cl) * 256);
-      cl = cl + 1 < kc ? cl + 1 : 0;
       if (D == 1)
 #pragma unroll
         for (int m = 0; m < MT; m++)
@@ -308,14 +316,14 @@ __global__ void __launch_bounds__(256, TRAIN ? 1 : 2) mlp_rows(mlp_net N, mlp_ba
   constexpr int HS = 64 * NT, R = 16 * MT, LD = HS + 4, LX = 260;
   __shared__ float sx[TRAIN ? R * LX : R * (LX > LD ? LX : LD)];
   __shared__ float sh[TRAIN ? 3 : 1][R * LD];
-  __shared__ float sz[R], sd[R], sy[R];
+  __shared__ float sd[R], sy[R];
+  __shared__ __attribute__((aligned(16))) float sw[HS]; /* the last layer's weights, placed */
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  float vs[4] = {0, 0, 0, 0}, vb4 = 0, vloss = 0;
   /* biases and the last layer's weights, loaded once and together (indices
    * clamped, no load behind a branch): each would cost a trip to L2 where it
    * is used */
-  constexpr int P = 256 / R; /* threads per row in the last layer */
-  float bias[3][NT], w4[HS / P];
+  float bias[3][NT];
+  const int pt = mlp_place(tid), pc = mlp_place(lane & 15);
 #pragma unroll
   for (int l = 0; l < 3; l++)
 #pragma unroll
@@ -323,14 +331,10 @@ __global__ void __launch_bounds__(256, TRAIN ? 1 : 2) mlp_rows(mlp_net N, mlp_ba
       const int c = 16 * (wave + 4 * t) + (lane & 15);
       bias[l][t] = N.bias[l][c < N.hidden ? c : 0];
     }
-#pragma unroll
-  for (int u = 0; u < HS / P; u++)
-    w4[u] = N.w4[tid % P + P * u < N.hidden ? tid % P + P * u : 0];
-  float b4 = N.b4[0], w4c = N.w4[tid < N.hidden ? tid : 0];
-  w4c = tid < N.hidden ? w4c : 0.f;
-#pragma unroll
-  for (int u = 0; u < HS / P; u++)
-    w4[u] = tid % P + P * u < N.hidden ? w4[u] : 0.f;
+  float b4 = N.b4[0], w4c = N.w4[pt < N.hidden ? pt : 0];
+  w4c = pt < N.hidden ? w4c : 0.f;
+  if (tid < HS)
+    sw[tid] = w4c;
 #pragma unroll
   for (int l = 0; l < 3; l++)
 #pragma unroll
@@ -366,9 +370,9 @@ __global__ void __launch_bounds__(256, TRAIN ? 1 : 2) mlp_rows(mlp_net N, mlp_ba
             const int k = k0 + q + 16 * u, r = 16 * m + (tid >> 4);
             const bool on = r0 + r < Q.rows && k < N.nin;
             if (k < xw) {
-              sx[r * LX + k] = on ? v[m][u] : 0.f;
+              sx[r * LX + mlp_place(k)] = on ? v[m][u] : 0.f;
               if (TRAIN && r0 + r < Q.rows)
-                Q.xb[(size_t)(r0 + r) * N.xs + k] = on ? v[m][u] : 0.f;
+                Q.xb[(size_t)(r0 + r) * N.xs + mlp_place(k)] = on ? v[m][u] : 0.f;
             }
           }
       }
@@ -394,7 +398,7 @@ __global__ void __launch_bounds__(256, TRAIN ? 1 : 2) mlp_rows(mlp_net N, mlp_ba
         rows_mm<NT, MT, 4>(in, lin, N.wf[l], HS / 16, acc);
 #pragma unroll
       for (int t = 0; t < NT; t++) {
-        const int c = 16 * (wave + 4 * t) + (lane & 15);
+        const int c = 16 * (wave + 4 * t) + pc;
         const float b = bias[l][t];
 #pragma unroll
         for (int m = 0; m < MT; m++)
@@ -408,70 +412,51 @@ __global__ void __launch_bounds__(256, TRAIN ? 1 : 2) mlp_rows(mlp_net N, mlp_ba
       if (TRAIN)
         rows_out<HS>(sh[l], LD, Q.h[l], r0, R, Q.rows);
     }
-    /* the last layer: 256 / R threads per row */
+    /* the last layer: a thread per row, as its sum has one order */
     const float *h3 = TRAIN ? sh[2] : sh[0];
-    {
-      const int r = tid / P, q = tid % P;
+    if (tid < R) {
+      const float *h = h3 + tid * LD;
       float v = 0.f;
+#pragma unroll 2
+      for (int c = 0; c < HS; c += 16) {
+        f4 a[4], w[4];
 #pragma unroll
-      for (int u = 0; u < HS / P; u++)
-        v = fmaf(h3[r * LD + q + P * u], w4[u], v);
-#pragma unroll
-      for (int o = P / 2; o > 0; o >>= 1)
-        v += __shfl_xor(v, o);
-      if (q == 0) {
-        const float z = v + b4;
-        if (!TRAIN) {
-          if (r0 + r < Q.rows)
-            Q.prob[r0 + r] = 1.f / (1.f + expf(-z));
-        } else {
-          float l = 0.f, d = 0.f;
-          if (r0 + r < Q.rows) {
-            const float yi = sy[r];
-            const float sp = z > 0 ? z + log1pf(expf(-z)) : log1pf(expf(z)); /* softplus */
-            l = sp - yi * z;
-            d = (1.f / (1.f + expf(-z)) - yi) / (float)Q.rows;
-          }
-          sz[r] = l;
-          sd[r] = d;
+        for (int g = 0; g < 4; g++) {
+          a[g] = *(const f4 *)(h + c + 4 * g);
+          w[g] = *(const f4 *)(sw + c + 4 * g);
         }
+#pragma unroll
+        for (int k = 0; k < 16; k++)
+          v = fmaf(a[k & 3][k >> 2], w[k & 3][k >> 2], v);
+      }
+      const int r = r0 + tid;
+      const float z = v + b4;
+      if (!TRAIN) {
+        if (r < Q.rows)
+          Q.prob[r] = 1.f / (1.f + expf(-z));
+      } else {
+        float d = 0.f;
+        if (r < Q.rows) {
+          const float yi = sy[tid];
+          const float sp = z > 0 ? z + log1pf(expf(-z)) : log1pf(expf(z)); /* softplus */
+          Q.lrow[r] = sp - yi * z;
+          d = (1.f / (1.f + expf(-z)) - yi) / (float)Q.rows;
+          Q.dz4[r] = d;
+        }
+        sd[tid] = d;
       }
     }
     __syncthreads();
     if (TRAIN) {
-      if (tid < HS) {
-        float s = 0.f;
-#pragma unroll
-        for (int r = 0; r < R; r++)
-          s = fmaf(sd[r], sh[2][r * LD + tid], s);
-        vs[3] += s;
-      }
-      if (tid == 0) {
-        float s = 0.f, d = 0.f;
-        for (int r = 0; r < R; r++) {
-          s += sz[r];
-          d += sd[r];
-        }
-        vloss += s;
-        vb4 += d;
-      }
-      __syncthreads();
       /* dz3 in place of h3, then dz2 in place of h2, dz1 of h1 */
       if (tid < HS)
 #pragma unroll
         for (int r = 0; r < R; r++)
-          sh[2][r * LD + tid] = sh[2][r * LD + tid] > 0.f ? sd[r] * w4c : 0.f;
+          sh[2][r * LD + tid] = sh[2][r * LD + tid] > 0.f ? fmaf(sd[r], w4c, 0.f) : 0.f;
       __syncthreads();
 #pragma unroll
       for (int l = 2; l >= 0; l--) {
         rows_out<HS>(sh[l], LD, Q.dz[l], r0, R, Q.rows);
-        if (tid < HS) {
-          float s = 0.f;
-#pragma unroll
-          for (int r = 0; r < R; r++)
-            s += sh[l][r * LD + tid];
-          vs[l] += s;
-        }
         if (l > 0) {
           f4 acc[MT][NT];
 #pragma unroll
@@ -482,7 +467,7 @@ __global__ void __launch_bounds__(256, TRAIN ? 1 : 2) mlp_rows(mlp_net N, mlp_ba
           rows_mm<NT, MT, 4>(sh[l], LD, N.wb[l], HS / 16, acc);
 #pragma unroll
           for (int t = 0; t < NT; t++) {
-            const int c = 16 * (wave + 4 * t) + (lane & 15);
+            const int c = 16 * (wave + 4 * t) + pc;
 #pragma unroll
             for (int m = 0; m < MT; m++)
 #pragma unroll
@@ -497,84 +482,148 @@ __global__ void __launch_bounds__(256, TRAIN ? 1 : 2) mlp_rows(mlp_net N, mlp_ba
     }
     __syncthreads();
   }
-  if (TRAIN) {
-    float *v = Q.vec + (size_t)blockIdx.x * (4 * HS + 2);
-    if (tid < HS)
-      for (int l = 0; l < 4; l++)
-        v[l * HS + tid] = vs[l];
-    if (tid == 0) {
-      v[4 * HS] = vb4;
-      v[4 * HS + 1] = vloss;
-    }
-  }
 }
 
-/* Partial weight gradients dW[n][k] = sum over a slice of the batch of
- * dz[b][n] in[b][k]: a wave takes a tile of 64 x 64 (16 products of 16 x 16)
- * and four rows of the batch per step, its operands straight from memory, one
- * 16-byte load each: tile row 4 i + rt is row i of product rt, so a lane's four
- * elements feed four products.  The tiles of one slice read the same rows, so
- * a slice stays on one XCD (workgroups go round the 8 of them). */
-#define WG_D 6
-__global__ void __launch_bounds__(256, 1) mlp_wgrad(mlp_batch Q, int hs, int xs, int nslice, int slice_rows, float *part) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int ht = hs / 64, t0 = ht * (xs / 64), tiles = t0 + 2 * ht * ht, wgs = (tiles + 3) / 4;
-  const int xcd = blockIdx.x % 8, j = blockIdx.x / 8;
-  const int slice = xcd + 8 * (j / wgs), tile = 4 * (j % wgs) + wave;
-  if (slice >= nslice || tile >= tiles)
-    return;
-  int l = 0, t = tile, ks = xs;
-  const float *in = Q.xb;
-  size_t off = 0;
-  if (tile >= t0) {
-    l = 1 + (tile - t0) / (ht * ht);
-    t = (tile - t0) % (ht * ht);
-    ks = hs;
-    in = Q.h[l - 1];
-    off = (size_t)hs * xs + (size_t)(l - 1) * hs * hs;
-  }
-  const int n0 = t / (ks / 64) * 64, k0 = t % (ks / 64) * 64;
-  const int b0 = slice * slice_rows, b1 = b0 + slice_rows < Q.rows ? b0 + slice_rows : Q.rows;
-  const int g = lane >> 4, c = 4 * (lane & 15);
-  const float *pa = Q.dz[l] + n0 + c, *pb = in + k0 + c;
-  f4 acc[4][4];
+/* The partial gradients: how the batch is cut for each layer (as ksplit cuts
+ * it for the general path, the column sums in slices of 64 rows) and where the
+ * partials lie. */
+struct mlp_cut {
+  int hidden, nin, hs, xs;
+  int S[4], rows[4];          /* slices of the weights' contractions and their rows */
+  int rs, nb;                 /* slices of 64 rows; blocks of 256 rows of the loss */
+  float *pw[4];               /* [S][hs][xs or hs] of the tiled layers, [S][hs] of the last */
+  float *pb[4];               /* bias gradients [rs][hs], of the last layer [rs] */
+  float *loss;                /* [nb] */
+  int first[4], wgs[3];       /* first workgroup of the tiled layers' parts, and of what follows; workgroups per slice */
+  int nbias, nlast;           /* workgroups of the column sums and of the last layer's weights */
+};
+
+/* Workgroups [first[l], first[l + 1]) take layer 2 - l: partial weight
+ * gradients dW[n][k] = sum over a slice of the batch of dz[b][n] in[b][k].  A
+ * wave takes a tile of 64 x 32 (8 products of 16 x 16) and four rows of the
+ * batch per step, its operands straight from memory, 16 and 8 bytes per load:
+ * tile row 4 i + rt is row i of product rt, so a lane's elements feed as many
+ * products.  The 32 tiles and 16 slices of a layer of 256 make 512 waves, two
+ * such layers one per SIMD of the device (with tiles of 64 x 64 half of them
+ * would be idle).  The tiles of one slice read the same rows, so a slice stays
+ * on one XCD (workgroups go round the 8 of them).  The workgroups after them
+ * make the column sums, the last layer's weight gradients and the loss. */
+typedef float f2 __attribute__((ext_vector_type(2)));
+#define WG_D 8
+__global__ void __launch_bounds__(256, 2) mlp_wgrad(mlp_batch Q, mlp_cut C) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  int blk = (int)blockIdx.x;
+  if (blk < C.first[3]) {
+    const int l = blk < C.first[1] ? 2 : (blk < C.first[2] ? 1 : 0);
+    const int hs = C.hs, ks = l ? hs : C.xs, kn = ((l ? C.hidden : C.nin) + 31) / 32;
+    const int tiles = (C.hidden + 63) / 64 * kn;
+    blk -= C.first[2 - l];
+    const int j = blk / 8, slice = blk % 8 + 8 * (j / C.wgs[l]), tile = 4 * (j % C.wgs[l]) + wave;
+    if (slice >= C.S[l] || tile >= tiles)
+      return;
+    const int n0 = tile / kn * 64, k0 = tile % kn * 32;
+    const int b0 = slice * C.rows[l], b1 = b0 + C.rows[l] < Q.rows ? b0 + C.rows[l] : Q.rows;
+    const int g = lane >> 4, ca = 4 * (lane & 15), cb = 2 * (lane & 15), last = Q.rows - 1;
+    const float *pa = Q.dz[l] + n0 + ca, *pb = (l ? Q.h[l - 1] : Q.xb) + k0 + cb;
+    f4 acc[4][2];
 #pragma unroll
-  for (int i = 0; i < 4; i++)
+    for (int i = 0; i < 4; i++)
 #pragma unroll
-    for (int k = 0; k < 4; k++)
-      acc[i][k] = (f4){0.f, 0.f, 0.f, 0.f};
-  /* WG_D steps' operands in flight; rows past the slice count as zero */
-  f4 av[WG_D], bv[WG_D];
-#pragma unroll
-  for (int u = 0; u < WG_D; u++) {
-    const int r = b0 + 4 * u + g, rc = r < b1 ? r : b0;
-    av[u] = *(const f4 *)(pa + (size_t)rc * hs);
-    bv[u] = *(const f4 *)(pb + (size_t)rc * ks);
-  }
-  for (int b = b0; b < b1; b += 4 * WG_D) {
+      for (int k = 0; k < 2; k++)
+        acc[i][k] = (f4){0.f, 0.f, 0.f, 0.f};
+    /* WG_D steps' operands in flight; rows past the slice count as zero */
+    f4 av[WG_D];
+    f2 bv[WG_D];
 #pragma unroll
     for (int u = 0; u < WG_D; u++) {
-      f4 a = av[u], v = bv[u];
-      if (b + 4 * u + g >= b1)
-        a = (f4){0.f, 0.f, 0.f, 0.f};
-      const int r = b + 4 * WG_D + 4 * u + g, rc = r < b1 ? r : b0;
+      const int r = b0 + 4 * u + g, rc = r < last ? r : last;
       av[u] = *(const f4 *)(pa + (size_t)rc * hs);
-      bv[u] = *(const f4 *)(pb + (size_t)rc * ks);
-#pragma unroll
-      for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int k = 0; k < 4; k++)
-          acc[i][k] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], v[k], acc[i][k], 0, 0, 0);
+      bv[u] = *(const f2 *)(pb + (size_t)rc * ks);
     }
+    for (int b = b0; b < b1; b += 4 * WG_D) {
+#pragma unroll
+      for (int u = 0; u < WG_D; u++) {
+        f4 a = av[u];
+        f2 v = bv[u];
+        if (b + 4 * u + g >= b1) {
+          a = (f4){0.f, 0.f, 0.f, 0.f};
+          v = (f2){0.f, 0.f};
+        }
+        const int r = b + 4 * WG_D + 4 * u + g, rc = r < last ? r : last;
+        av[u] = *(const f4 *)(pa + (size_t)rc * hs);
+        bv[u] = *(const f2 *)(pb + (size_t)rc * ks);
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+          for (int k = 0; k < 2; k++)
+            acc[i][k] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], v[k], acc[i][k], 0, 0, 0);
+      }
+    }
+    float *o = C.pw[l] + (size_t)slice * hs * ks;
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const f2 v = {acc[i][0][r], acc[i][1][r]};
+        *(f2 *)(o + (size_t)(n0 + 4 * (4 * g + r) + i) * ks + k0 + cb) = v;
+      }
+    return;
   }
-  float *o = part + (size_t)slice * ((size_t)hs * xs + 2 * (size_t)hs * hs) + off;
-#pragma unroll
-  for (int i = 0; i < 4; i++)
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const f4 v = {acc[i][0][r], acc[i][1][r], acc[i][2][r], acc[i][3][r]};
-      *(f4 *)(o + (size_t)(n0 + 4 * (4 * g + r) + i) * ks + k0 + c) = v;
+  blk -= C.first[3];
+  __shared__ float red[256];
+  if (blk < C.nbias) {
+    /* column sums of 64 rows and 64 columns: four interleaved rows */
+    const int cg = C.hs / 64, slice = blk / (3 * cg), l = blk / cg % 3, c = blk % cg * 64 + lane;
+    const int r0 = slice * 64, r1 = r0 + 64 < Q.rows ? r0 + 64 : Q.rows;
+    const float *p = Q.dz[l] + c;
+    float s = 0.f;
+#pragma unroll 16
+    for (int r = r0 + wave; r < r1; r += 4)
+      s += p[(size_t)r * C.hs];
+    red[tid] = s;
+    __syncthreads();
+    if (wave == 0)
+      C.pb[l][(size_t)slice * C.hs + c] = ((red[lane] + red[64 + lane]) + red[128 + lane]) + red[192 + lane];
+    return;
+  }
+  blk -= C.nbias;
+  if (blk < C.nlast) {
+    const int r0 = blk * C.rows[3], r1 = r0 + C.rows[3] < Q.rows ? r0 + C.rows[3] : Q.rows;
+    if (tid >= C.hs)
+      return;
+    const float *p = Q.h[2] + tid;
+    float s = 0.f;
+#pragma unroll 8
+    for (int r = r0; r < r1; r++)
+      s = fmaf(Q.dz4[r], p[(size_t)r * C.hs], s);
+    C.pw[3][(size_t)blk * C.hs + tid] = s;
+    return;
+  }
+  blk -= C.nlast;
+  if (blk < C.nb) {
+    /* the loss of 256 rows, in a tree */
+    const int r = blk * 256 + tid;
+    red[tid] = r < Q.rows ? Q.lrow[r] : 0.f;
+    __syncthreads();
+    for (int w = 128; w > 0; w >>= 1) {
+      if (tid < w)
+        red[tid] += red[tid + w];
+      __syncthreads();
     }
+    if (tid == 0)
+      C.loss[blk] = red[0] / (float)Q.rows;
+    return;
+  }
+  blk -= C.nb;
+  /* the output gradient's sums over 64 rows */
+  const int slice = blk * 64 + lane, r1 = slice * 64 + 64 < Q.rows ? slice * 64 + 64 : Q.rows;
+  float s = 0.f;
+  for (int r = slice * 64 + wave; r < r1; r += 4)
+    s += Q.dz4[r];
+  red[tid] = s;
+  __syncthreads();
+  if (wave == 0 && slice < C.rs)
+    C.pb[3][slice] = ((red[lane] + red[64 + lane]) + red[128 + lane]) + red[192 + lane];
 }
 
 struct mlp_param {
@@ -588,9 +637,9 @@ struct mlp_param {
 /* where weight (n, k) of layer l lies in the tiled copies */
 static __device__ __forceinline__ void mlp_tiles(const mlp_param &P, int l, int n, int k, float w) {
   const int kc = l == 0 ? P.xc : P.hs / 16;
-  P.wf[l][((size_t)(n / 16) * kc + k / 16) * 256 + 4 * ((n % 16) + 16 * (k % 16 / 4)) + k % 4] = w;
+  P.wf[l][((size_t)(n / 16) * kc + k / 16) * 256 + 4 * ((n % 16) + 16 * (k % 4)) + k % 16 / 4] = w;
   if (l > 0)
-    P.wb[l][((size_t)(k / 16) * (P.hs / 16) + n / 16) * 256 + 4 * ((k % 16) + 16 * (n % 16 / 4)) + n % 4] = w;
+    P.wb[l][((size_t)(k / 16) * (P.hs / 16) + n / 16) * 256 + 4 * ((k % 16) + 16 * (n % 4)) + n % 16 / 4] = w;
 }
 
 static __device__ __forceinline__ float mlp_step(const mlp_param &P, int64_t p, float gi) {
@@ -629,13 +678,29 @@ __global__ void mlp_zero(float *p, int64_t n) {
     p[i] = 0.f;
 }
 
+/* p[0] + p[stride] + ... from zero, in order, n terms */
+static __device__ __forceinline__ float sum_in_order(const float *p, int n, size_t stride) {
+  float s = 0.f;
+  int u = 0;
+  for (; u + 8 <= n; u += 8) {
+    float t[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++)
+      t[e] = p[(size_t)(u + e) * stride];
+#pragma unroll
+    for (int e = 0; e < 8; e++)
+      s += t[e];
+  }
+  for (; u < n; u++)
+    s += p[(size_t)u * stride];
+  return s;
+}
+
 /* The partial gradients summed in order, then Adam (or, with P.g, the
  * gradients themselves): the first nwb workgroups take the weights of the
- * tiled layers, the others 64 entries of the per-workgroup vectors each, in
- * four interleaved sums.  The loss is added to *loss. */
-__global__ void __launch_bounds__(256) mlp_update(mlp_param P, const float *__restrict__ part, int nslice,
-                                                  const float *__restrict__ vec, int nvec, int64_t nw, int nwb,
-                                                  float *loss, float rows) {
+ * tiled layers, the others the rest, 64 entries each so that their chains of
+ * sums run beside each other.  The loss is added to *loss. */
+__global__ void __launch_bounds__(256) mlp_update(mlp_param P, mlp_cut C, int64_t nw, int nwb, float *loss) {
   if ((int)blockIdx.x < nwb) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= nw)
@@ -643,59 +708,36 @@ __global__ void __launch_bounds__(256) mlp_update(mlp_param P, const float *__re
     int n, k;
     const int l = mlp_where(P, i, n, k);
     const int ks = l ? P.hs : P.xs;
-    const size_t all = (size_t)P.hs * P.xs + 2 * (size_t)P.hs * P.hs;
-    const float *q = part + (l ? (size_t)P.hs * P.xs + (size_t)(l - 1) * P.hs * P.hs : 0) + (size_t)n * ks + k;
-    float s = 0.f;
-    int u = 0;
-    for (; u + 8 <= nslice; u += 8) {
-      float t[8];
-#pragma unroll
-      for (int e = 0; e < 8; e++)
-        t[e] = q[(size_t)(u + e) * all];
-#pragma unroll
-      for (int e = 0; e < 8; e++)
-        s += t[e];
-    }
-    for (; u < nslice; u++)
-      s += q[(size_t)u * all];
+    const float g = sum_in_order(C.pw[l] + (size_t)mlp_place(n) * ks + mlp_place(k), C.S[l], (size_t)P.hs * ks);
     const int64_t p = P.woff[l] + (int64_t)n * (l ? P.hidden : P.nin) + k;
     if (P.g)
-      P.g[p] = s;
+      P.g[p] = g;
     else
-      mlp_tiles(P, l, n, k, mlp_step(P, p, s));
+      mlp_tiles(P, l, n, k, mlp_step(P, p, g));
     return;
   }
-  __shared__ float red[4][64];
-  const int V = 4 * P.hs + 2;
-  const int c = ((int)blockIdx.x - nwb) * 64 + (threadIdx.x & 63), q = threadIdx.x >> 6;
-  float s = 0.f;
-  if (c < V) {
-#pragma unroll 8
-    for (int u = q; u < nvec; u += 4)
-      s += vec[(size_t)u * V + c];
-  }
-  red[q][threadIdx.x & 63] = s;
-  __syncthreads();
-  if (q || c >= V)
+  const int c = ((int)blockIdx.x - nwb) * 64 + (int)threadIdx.x, l = c / P.hs, e = c % P.hs;
+  if (threadIdx.x >= 64 || c > 4 * P.hs + 1)
     return;
-  s = ((red[0][threadIdx.x] + red[1][threadIdx.x]) + red[2][threadIdx.x]) + red[3][threadIdx.x];
-  if (c == V - 1) {
-    *loss += s / rows;
+  if (c == 4 * P.hs + 1) {
+    *loss += sum_in_order(C.loss, C.nb, 1);
     return;
   }
+  float g;
   int64_t p;
-  if (c == V - 2)
+  if (c == 4 * P.hs) {
+    g = sum_in_order(C.pb[3], C.rs, 1);
     p = P.boff[3];
-  else {
-    const int l = c / P.hs, e = c % P.hs;
+  } else {
     if (e >= P.hidden)
       return;
+    g = l < 3 ? sum_in_order(C.pb[l] + mlp_place(e), C.rs, P.hs) : sum_in_order(C.pw[3] + mlp_place(e), C.S[3], P.hs);
     p = (l < 3 ? P.boff[l] : P.woff[3]) + e;
   }
   if (P.g)
-    P.g[p] = s;
+    P.g[p] = g;
   else
-    mlp_step(P, p, s);
+    mlp_step(P, p, g);
 }
 
 /* ------------------------------------------------------------ host side */
@@ -725,7 +767,8 @@ struct ehd_mlp {
   float *tiles;          /* wf[0], wf[1], wb[1], wf[2], wb[2] */
   float *fbuf;           /* xb, h[3], dz[3] for fcap rows */
   int64_t fcap;
-  float *fvec, *fpart;   /* per-workgroup vectors, weight-gradient slices */
+  float *fpart;          /* partial gradients and losses */
+  int64_t fpart_cap;
   float *floss;
   float *pin[2], *pout[2]; /* prediction: two chunks of inputs and of probabilities */
   hipStream_t pstream;   /* their copies */
@@ -832,8 +875,7 @@ static int ensure_batch(ehd_mlp *m, int32_t B) {
 
 void ehd_mlp_destroy(ehd_mlp *m);
 
-#define FUSED_WGS 512     /* most workgroups of mlp_rows in training */
-#define FUSED_SLICES 24   /* most batch slices of mlp_wgrad: 36 tiles of a 256-wide net times 24 fill 864 of 1,024 SIMDs */
+#define FUSED_WGS 512 /* most workgroups of mlp_rows in training */
 
 static size_t tiles_len(const ehd_mlp *m) { return (size_t)m->hs * 16 * m->xc + 4 * (size_t)m->hs * m->hs; }
 
@@ -873,10 +915,7 @@ int ehd_mlp_create(ehd_dev *d, int32_t nin, int32_t hidden, const float *init, e
     m->xs = (nin + 63) / 64 * 64;
     m->xc = (nin + 15) / 16;
     m->tiles_stale = 1;
-    const size_t all = (size_t)m->hs * m->xs + 2 * (size_t)m->hs * m->hs;
     if (hipMalloc((void **)&m->tiles, sizeof(float) * tiles_len(m)) != hipSuccess ||
-        hipMalloc((void **)&m->fvec, sizeof(float) * FUSED_WGS * (4 * (size_t)m->hs + 2)) != hipSuccess ||
-        hipMalloc((void **)&m->fpart, sizeof(float) * FUSED_SLICES * all) != hipSuccess ||
         hipMalloc((void **)&m->floss, sizeof(float)) != hipSuccess) {
       ehd_mlp_destroy(m);
       return EH_ERR_NOMEM;
@@ -901,9 +940,9 @@ void ehd_mlp_destroy(ehd_mlp *m) {
   for (int k = 0; k < 4; k++)
     if (m->pev[k])
       (void)hipEventDestroy(m->pev[k]);
-  void *bufs[18] = {m->params, m->grads, m->adam_m, m->adam_v, m->part,   m->Xd,     m->yd,     m->permd,  m->eloss,
-                    m->tiles,  m->fbuf,  m->fvec,   m->fpart,  m->floss,  m->pin[0], m->pin[1], m->pout[0], m->pout[1]};
-  for (int k = 0; k < 18; k++)
+  void *bufs[17] = {m->params, m->grads, m->adam_m, m->adam_v, m->part,   m->Xd,     m->yd,     m->permd,  m->eloss,
+                    m->tiles,  m->fbuf,  m->fpart,  m->floss,  m->pin[0], m->pin[1], m->pout[0], m->pout[1]};
+  for (int k = 0; k < 17; k++)
     if (bufs[k])
       (void)hipFree(bufs[k]);
   for (int l = 0; l <= MLP_LAYERS; l++) {
@@ -925,6 +964,24 @@ static void forward(ehd_mlp *m, int B) {
     launch_gemm(m, 0, 1, m->act[l], m->params + m->woff[l], m->act[l + 1], m->params + m->boff[l], B,
                 m->out_dim[l], m->in_dim[l], m->in_dim[l], m->in_dim[l], m->out_dim[l], last ? 0 : 1, 0);
   }
+}
+
+/* the sum of nb partial losses on the device, which is waited for */
+static int batch_loss(ehd_mlp *m, const float *part, int nb, float *loss) {
+  float *h = (float *)malloc(sizeof(float) * nb);
+  if (!h)
+    return EH_ERR_NOMEM;
+  hipError_t e = hipMemcpyAsync(h, part, sizeof(float) * nb, hipMemcpyDeviceToHost, m->d->stream);
+  const hipError_t w = hipStreamSynchronize(m->d->stream);
+  e = e ? e : w;
+  double s = 0;
+  for (int k = 0; k < nb; k++)
+    s += h[k];
+  free(h);
+  if (e)
+    return mlp_fail(m, e, "reading the loss");
+  *loss = (float)s;
+  return EH_OK;
 }
 
 /* gradient of the mean BCE over the batch into m->grads.  The loss: into
@@ -965,19 +1022,7 @@ static int backward(ehd_mlp *m, int B, float *loss, float *loss_acc) {
                          m->act[l], n);
     }
   }
-  if (loss) {
-    float *h = (float *)malloc(sizeof(float) * nb);
-    if (!h)
-      return EH_ERR_NOMEM;
-    MCHK(hipMemcpyAsync(h, m->loss_part, sizeof(float) * nb, hipMemcpyDeviceToHost, m->d->stream));
-    MCHK(hipStreamSynchronize(m->d->stream));
-    double s = 0;
-    for (int k = 0; k < nb; k++)
-      s += h[k];
-    *loss = (float)s;
-    free(h);
-  }
-  return EH_OK;
+  return loss ? batch_loss(m, m->loss_part, nb, loss) : EH_OK;
 }
 
 static mlp_net fused_net(const ehd_mlp *m) {
@@ -1035,29 +1080,59 @@ static void fused_tiles(ehd_mlp *m) {
   m->tiles_stale = 0;
 }
 
-/* buffers for batches of B rows, and the batch that uses them */
-static int fused_batch(ehd_mlp *m, int32_t B, mlp_batch *Q) {
-  if (B > m->fcap) {
-    if (m->fbuf)
-      MCHK(hipFree(m->fbuf));
-    m->fbuf = NULL;
-    m->fcap = 0;
-    MCHK(hipMalloc((void **)&m->fbuf, sizeof(float) * (size_t)B * (m->xs + 6 * (size_t)m->hs)));
-    m->fcap = B;
-  }
+static int grow_dev(ehd_mlp *m, void **p, int64_t *cap, int64_t count, size_t sz);
+
+/* buffers for batches of B rows, the batch that uses them and how it is cut */
+static int fused_batch(ehd_mlp *m, int32_t B, mlp_batch *Q, mlp_cut *C) {
+  const int64_t hs = m->hs, xs = m->xs;
+  int rc = grow_dev(m, (void **)&m->fbuf, &m->fcap, B * (xs + 6 * hs + 2), sizeof(float));
+  if (rc)
+    return rc;
   memset(Q, 0, sizeof *Q);
   Q->xb = m->fbuf;
   for (int l = 0; l < 3; l++) {
-    Q->h[l] = m->fbuf + (size_t)B * (m->xs + (size_t)l * m->hs);
-    Q->dz[l] = m->fbuf + (size_t)B * (m->xs + (size_t)(3 + l) * m->hs);
+    Q->h[l] = m->fbuf + (size_t)B * (xs + l * hs);
+    Q->dz[l] = m->fbuf + (size_t)B * (xs + (3 + l) * hs);
   }
-  Q->vec = m->fvec;
+  Q->dz4 = m->fbuf + (size_t)B * (xs + 6 * hs);
+  Q->lrow = Q->dz4 + B;
   Q->rows = B;
+  memset(C, 0, sizeof *C);
+  C->hidden = m->hidden;
+  C->nin = m->nin;
+  C->hs = m->hs;
+  C->xs = m->xs;
+  C->rs = (B + 63) / 64;
+  C->nb = (B + 255) / 256;
+  int64_t need = 0, pw[4];
+  for (int l = 0; l < MLP_LAYERS; l++) {
+    C->S[l] = ksplit(m->out_dim[l], m->in_dim[l], B);
+    C->rows[l] = (B + C->S[l] - 1) / C->S[l];
+    C->S[l] = (B + C->rows[l] - 1) / C->rows[l]; /* the slices that have rows */
+    pw[l] = need;
+    need += C->S[l] * (l == 0 ? hs * xs : (l < 3 ? hs * hs : hs));
+  }
+  const int64_t pb = need, loss = pb + C->rs * (3 * hs + 1);
+  rc = grow_dev(m, (void **)&m->fpart, &m->fpart_cap, loss + C->nb, sizeof(float));
+  if (rc)
+    return rc;
+  for (int l = 0; l < MLP_LAYERS; l++) {
+    C->pw[l] = m->fpart + pw[l];
+    C->pb[l] = m->fpart + pb + C->rs * l * hs;
+  }
+  C->loss = m->fpart + loss;
+  for (int l = 2; l >= 0; l--) {
+    const int kn = (m->in_dim[l] + 31) / 32;
+    C->wgs[l] = ((m->hidden + 63) / 64 * kn + 3) / 4;
+    C->first[3 - l] = C->first[2 - l] + 8 * C->wgs[l] * ((C->S[l] + 7) / 8);
+  }
+  C->nbias = C->rs * 3 * (m->hs / 64);
+  C->nlast = C->S[3];
   return EH_OK;
 }
 
 /* one batch: gradients to P.g, or an Adam step; its loss is added to *loss */
-static void fused_step(ehd_mlp *m, const mlp_param &P, const mlp_batch &Q, float *loss) {
+static void fused_step(ehd_mlp *m, const mlp_param &P, const mlp_batch &Q, const mlp_cut &C, float *loss) {
   const mlp_net N = fused_net(m);
   hipStream_t st = m->d->stream;
   int wgs = (Q.rows + 15) / 16;
@@ -1076,23 +1151,14 @@ static void fused_step(ehd_mlp *m, const mlp_param &P, const mlp_batch &Q, float
   default:
     hipLaunchKernelGGL((mlp_rows<4, 1, true>), dim3(wgs), dim3(256), 0, st, N, Q);
   }
-  /* slices of at least 64 rows, a multiple of the step */
-  int ns = (Q.rows + 63) / 64;
-  if (ns > FUSED_SLICES)
-    ns = FUSED_SLICES;
-  const int rows = ((Q.rows + ns - 1) / ns + 4 * WG_D - 1) / (4 * WG_D) * (4 * WG_D);
-  ns = (Q.rows + rows - 1) / rows;
-  const int ht = m->hs / 64, tiles = ht * (m->xs / 64) + 2 * ht * ht, per = (tiles + 3) / 4;
-  hipLaunchKernelGGL(mlp_wgrad, dim3(8 * per * ((ns + 7) / 8)), dim3(256), 0, st, Q, m->hs, m->xs, ns, rows, m->fpart);
+  hipLaunchKernelGGL(mlp_wgrad, dim3(C.first[3] + C.nbias + C.nlast + C.nb + (C.rs + 63) / 64), dim3(256), 0, st, Q, C);
   const int64_t nw = fused_weights(m);
   const int nwb = (int)((nw + 255) / 256), nvb = (4 * m->hs + 2 + 63) / 64;
-  hipLaunchKernelGGL(mlp_update, dim3(nwb + nvb), dim3(256), 0, st, P, m->fpart, ns, m->fvec, wgs, nw, nwb, loss,
-                     (float)Q.rows);
+  hipLaunchKernelGGL(mlp_update, dim3(nwb + nvb), dim3(256), 0, st, P, C, nw, nwb, loss);
 }
 
 static int fused_grad(ehd_mlp *m, const float *X, const float *y, int32_t B, float *grad, float *loss);
 static int fused_predict(ehd_mlp *m, const float *X, int64_t n, float *prob);
-static int grow_dev(ehd_mlp *m, void **p, int64_t *cap, int64_t count, size_t sz);
 
 int ehd_mlp_grad(ehd_mlp *m, const float *X, const float *y, int32_t B, float *grad, float *loss) {
   int rc;
@@ -1127,8 +1193,8 @@ static int grow_dev(ehd_mlp *m, void **p, int64_t *cap, int64_t count, size_t sz
 
 static int fused_grad(ehd_mlp *m, const float *X, const float *y, int32_t B, float *grad, float *loss) {
   mlp_batch Q;
-  float h = 0;
-  int rc = fused_batch(m, B, &Q);
+  mlp_cut C;
+  int rc = fused_batch(m, B, &Q, &C);
   if (!rc)
     rc = grow_dev(m, (void **)&m->Xd, &m->data_cap, (int64_t)B * m->nin, sizeof(float));
   if (!rc)
@@ -1143,13 +1209,12 @@ static int fused_grad(ehd_mlp *m, const float *X, const float *y, int32_t B, flo
   MCHK(hipMemcpyAsync(m->yd, y, sizeof(float) * B, hipMemcpyHostToDevice, m->d->stream));
   fused_tiles(m);
   hipLaunchKernelGGL(mlp_zero, dim3(1), dim3(64), 0, m->d->stream, m->floss, (int64_t)1);
-  fused_step(m, P, Q, m->floss);
+  fused_step(m, P, Q, C, m->floss);
   MCHK(hipGetLastError());
-  MCHK(hipMemcpyAsync(&h, m->floss, sizeof(float), hipMemcpyDeviceToHost, m->d->stream));
   MCHK(hipMemcpyAsync(grad, m->grads, sizeof(float) * m->nparams, hipMemcpyDeviceToHost, m->d->stream));
-  MCHK(hipStreamSynchronize(m->d->stream));
   if (loss)
-    *loss = h;
+    return batch_loss(m, C.loss, C.nb, loss);
+  MCHK(hipStreamSynchronize(m->d->stream));
   return EH_OK;
 }
 
@@ -1228,7 +1293,8 @@ int ehd_mlp_train(ehd_mlp *m, const float *X, const float *y, int64_t n, const i
   if (n > 0x7fffffff)
     return EH_ERR_INVALID;
   mlp_batch Q;
-  if ((rc = m->fused ? fused_batch(m, B, &Q) : ensure_batch(m, B)))
+  mlp_cut C;
+  if ((rc = m->fused ? fused_batch(m, B, &Q, &C) : ensure_batch(m, B)))
     return rc;
   if ((rc = grow_dev(m, (void **)&m->Xd, &m->data_cap, n * m->nin, sizeof(float))) ||
       (rc = grow_dev(m, (void **)&m->yd, &m->y_cap, n, sizeof(float))) ||
@@ -1266,7 +1332,7 @@ int ehd_mlp_train(ehd_mlp *m, const float *X, const float *y, int64_t n, const i
         m->step++;
         P.c1 = 1.f - powf(0.9f, (float)m->step);
         P.c2 = 1.f - powf(0.999f, (float)m->step);
-        fused_step(m, P, Q, m->eloss + ep);
+        fused_step(m, P, Q, C, m->eloss + ep);
       }
   }
   for (int ep = 0; ep < epochs && !m->fused; ep++) {

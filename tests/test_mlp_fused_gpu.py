@@ -90,3 +90,69 @@ def test_training_steps_match_adam(tracker):
     # a step moves each weight by up to 1e-3 whatever its gradient's size, so
     # rounding of the smallest gradients shows: a few 1e-4 of the norm
     assert np.linalg.norm(runs[0][0] - w) < 2e-3 * np.linalg.norm(w)
+
+
+def _embedded(p, n_in, hidden, wide):
+    """the parameters of the same net with inputs that nothing sends"""
+    w = np.zeros((hidden, wide), np.float32)
+    w[:, :n_in] = p[:hidden * n_in].reshape(hidden, n_in)
+    return np.concatenate([w.ravel(), p[hidden * n_in:]])
+
+
+def _without(p, n_in, hidden, wide):
+    w = p[:hidden * wide].reshape(hidden, wide)
+    assert not w[:, n_in:].any()
+    return np.concatenate([w[:, :n_in].ravel(), p[hidden * wide:]])
+
+
+@pytest.mark.parametrize("n_in,hidden,B", [(1, 1, 1), (19, 1, 63), (16, 15, 64), (19, 64, 65), (17, 65, 129),
+                                           (33, 100, 250), (19, 129, 257), (19, 192, 831), (256, 256, 127),
+                                           (19, 256, 831), (19, 100, 1000), (19, 64, 3000)])
+def test_same_bits_as_the_general_path(tracker, n_in, hidden, B):
+    """a net of 257 inputs takes the general path; with the inputs beyond n_in
+    always zero it is the same net, and every sum has the same order wherever
+    both cut the batch into as many slices (B below 64 times the general
+    path's 256 / tiles of the first layer): the gradients, six Adam steps and
+    the probabilities are equal bit for bit"""
+    from elegant_amd import learned
+    wide = 257
+    assert B // 64 <= max(1, 256 // (-(-hidden // 64) * 5))
+    rng = np.random.default_rng(B + hidden)
+    X = rng.normal(size=(3 * B, n_in)).astype(np.float32)
+    y = (rng.random(3 * B) < 0.4).astype(np.float32)
+    XW = np.zeros((3 * B, wide), np.float32)
+    XW[:, :n_in] = X
+    a = learned.MLP(tracker, n_in=n_in, hidden=hidden, seed=3)
+    b = learned.MLP(tracker, n_in=wide, hidden=hidden, seed=3)
+    p = a.params()
+    b.set_params(_embedded(p, n_in, hidden, wide))
+    ga, la = a.gradient(X[:B], y[:B])
+    gb, lb = b.gradient(XW[:B], y[:B])
+    assert la == lb and np.array_equal(ga, _without(gb, n_in, hidden, wide))
+    la = a.train(X, y, epochs=2, batch=B, lr=1e-3, seed=7)
+    lb = b.train(XW, y, epochs=2, batch=B, lr=1e-3, seed=7)
+    assert np.array_equal(la, lb) and np.array_equal(a.params(), _without(b.params(), n_in, hidden, wide))
+    assert np.array_equal(a.predict(X), b.predict(XW))
+    a.close()
+    b.close()
+
+
+@pytest.mark.parametrize("B", [4096, 10007])
+def test_same_bits_beyond_the_first_layer(tracker, B):
+    """larger batches, which the general net's first layer cuts differently:
+    the other layers' gradients"""
+    from elegant_amd import learned
+    n_in, hidden, wide = 19, 256, 257
+    rng = np.random.default_rng(B)
+    X = rng.normal(size=(B, n_in)).astype(np.float32)
+    y = (rng.random(B) < 0.4).astype(np.float32)
+    XW = np.zeros((B, wide), np.float32)
+    XW[:, :n_in] = X
+    a = learned.MLP(tracker, n_in=n_in, hidden=hidden, seed=3)
+    b = learned.MLP(tracker, n_in=wide, hidden=hidden, seed=3)
+    b.set_params(_embedded(a.params(), n_in, hidden, wide))
+    ga, la = a.gradient(X, y)
+    gb, lb = b.gradient(XW, y)
+    assert la == lb and np.array_equal(ga[hidden * n_in:], _without(gb, n_in, hidden, wide)[hidden * n_in:])
+    a.close()
+    b.close()
