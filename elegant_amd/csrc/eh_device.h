@@ -28,7 +28,9 @@ int ehd_get_one(ehd_dev *d, int64_t i, double *s, double *dp, int32_t *loss_pass
 int ehd_get_state(ehd_dev *d, double *x, double *xp, double *y, double *yp, double *s, double *dp,
                   int32_t *loss_pass, int32_t *loss_code, int64_t n);
 int ehd_get_sdp(ehd_dev *d, double *s, double *dp, int32_t *loss_pass, int64_t n);
-int64_t ehd_state_n(const ehd_dev *d);
+/* changes with every upload of particles: who keeps its value can tell whether
+ * the columns still hold that upload's particles */
+int64_t ehd_upload_id(const ehd_dev *d);
 
 /* Rows (AoS, as the caller holds them) moved whole and turned into columns on
  * the device.  ehd_put_rows copies n rows of w columns, sets the loss records

@@ -2017,6 +2017,7 @@ void ehd_destroy(ehd_dev *d) {
 }
 
 int ehd_alloc_state(ehd_dev *d, int64_t n) {
+  d->upload++;
   HIPCHK(d, hipSetDevice(d->device));
   if (n > d->cap) {
     for (int k = 0; k < 6; k++) {
@@ -2046,7 +2047,7 @@ int ehd_alloc_state(ehd_dev *d, int64_t n) {
   return EH_OK;
 }
 
-int64_t ehd_state_n(const ehd_dev *d) { return d->n; }
+int64_t ehd_upload_id(const ehd_dev *d) { return d->upload; }
 
 int ehd_put_state(ehd_dev *d, const double *x, const double *xp, const double *y, const double *yp, const double *s,
                   const double *dp, const int32_t *loss_pass, const int32_t *loss_code, int64_t n) {

@@ -35,6 +35,7 @@ struct ehd_dev {
   int32_t *loss_pass, *loss_code;
   double *ids;         /* particle IDs (column 6 of the rows) */
   int64_t n, cap;
+  int64_t upload;      /* counts the uploads: whose particles the columns hold */
   /* rows as the caller holds them, on their way to or from the columns
    * above: kept between calls, freed with the context */
   double *rows, *rows2;

@@ -35,6 +35,7 @@ struct eh_batch {
   double *ids;
   int64_t n, cap;
   int uploaded;
+  int64_t upload_id; /* ehd_upload_id of that upload */
   int64_t scheduled; /* particles in the current work queue */
   eh_batch_tuning tune;
 };
@@ -42,6 +43,14 @@ struct eh_batch {
 static int bmsg(eh_batch *b, int code, const char *m) {
   snprintf(eh_ctx_msg(b->ctx), 512, "%s", m);
   return code;
+}
+
+/* an uploaded batch whose columns another upload of the context has taken
+ * (an element call, do_tracking, another batch) has lost its particles */
+static int own_columns(eh_batch *b) {
+  return b->upload_id == ehd_upload_id(eh_ctx_dev(b->ctx))
+             ? EH_OK
+             : bmsg(b, EH_ERR_STATE, "the particles on the device are no longer this batch's");
 }
 
 int eh_batch_create(eh_ctx *ctx, eh_batch **out) {
@@ -298,6 +307,7 @@ static int upload(eh_batch *b) {
   int rc;
   if (b->nops > 0x7fffffff || b->n > 0x7fffffff)
     return bmsg(b, EH_ERR_UNSUPPORTED, "batch programs or particle count too large");
+  b->uploaded = 0; /* the host's copies are current: a failed upload can be tried again */
   rc = ehd_alloc_state(d, b->n);
   if (!rc)
     rc = ehd_put_state(d, b->soa[0], b->soa[1], b->soa[2], b->soa[3], b->soa[4], b->soa[5], b->lp, b->lc, b->n);
@@ -308,6 +318,7 @@ static int upload(eh_batch *b) {
   rc = build_queue(b, 0);
   if (rc)
     return rc;
+  b->upload_id = ehd_upload_id(d);
   b->uploaded = 1;
   return EH_OK;
 }
@@ -318,8 +329,10 @@ int eh_batch_set_tuning(eh_batch *b, const eh_batch_tuning *t) {
     return EH_ERR_INVALID;
   if (t->block * t->particles_per_lane != b->tune.block * b->tune.particles_per_lane && b->uploaded) {
     /* the chunk size changed: rebuild the queue from the current device state */
-    int rc;
     ehd_dev *d = eh_ctx_dev(b->ctx);
+    int rc = own_columns(b);
+    if (rc)
+      return rc;
     rc = ehd_get_state(d, b->soa[0], b->soa[1], b->soa[2], b->soa[3], b->soa[4], b->soa[5], b->lp, b->lc, b->n);
     if (rc)
       return bmsg(b, rc, ehd_message(d));
@@ -402,11 +415,9 @@ int eh_batch_track(eh_batch *b, int64_t pass0, int64_t npasses, eh_stats *stats)
   if (!b || npasses < 0 || npasses > 0x7fffffff)
     return EH_ERR_INVALID;
   d = eh_ctx_dev(b->ctx);
-  if (!b->uploaded) {
-    rc = upload(b);
-    if (rc)
-      return rc;
-  }
+  rc = b->uploaded ? own_columns(b) : upload(b);
+  if (rc)
+    return rc;
   ehd_timing_reset(d);
   rc = run_passes(b, pass0, npasses, &ms, &nl);
   if (rc)
@@ -466,7 +477,7 @@ int eh_batch_autotune(eh_batch *b, int64_t sample_passes, eh_batch_tuning *best_
     rc = upload(b);
     if (rc)
       return rc;
-  } else if ((rc = build_queue(b, 0)))
+  } else if ((rc = own_columns(b)) || (rc = build_queue(b, 0)))
     return rc;
   rc = ehd_state_snapshot(d, 0);
   if (rc)
@@ -566,6 +577,9 @@ int eh_batch_loss_passes(eh_batch *b, int32_t variant, int32_t *loss_pass, int64
   if (!b->uploaded)
     memcpy(loss_pass, b->lp + b->var[variant].first, sizeof(int32_t) * n);
   else {
+    rc = own_columns(b);
+    if (rc)
+      return rc;
     rc = ehd_get_state(d, NULL, NULL, NULL, NULL, NULL, NULL, b->lp, b->lc, b->n);
     if (rc)
       return bmsg(b, rc, ehd_message(d));
@@ -600,6 +614,9 @@ int eh_batch_download(eh_batch *b, int32_t variant, double **coord, int64_t n, i
     return EH_ERR_INVALID;
   d = eh_ctx_dev(b->ctx);
   if (b->uploaded) {
+    rc = own_columns(b);
+    if (rc)
+      return rc;
     rc = ehd_get_state(d, b->soa[0], b->soa[1], b->soa[2], b->soa[3], b->soa[4], b->soa[5], b->lp, b->lc, b->n);
     if (rc)
       return bmsg(b, rc, ehd_message(d));

@@ -40,6 +40,7 @@ struct eh_ctx {
   int64_t cap_n;
   int64_t *order, *pos, *scratch;
   int have_order;
+  int64_t upload_id; /* ehd_upload_id of the last upload */
   int64_t n_alive_ref;
   uint8_t *applied;
   int32_t *h_pass, *h_code, *order32;
@@ -388,6 +389,7 @@ static int upload_rows(eh_ctx *c, double **coord, int64_t n, int32_t nprops, int
   if (rc)
     return rc;
   c->bunch_on_device = 0;
+  c->upload_id = -1;
   block = n > 0 ? one_block(coord, n, nprops) : NULL;
   if (n > 0 && !block) {
     block = host_rows(c, n * nprops);
@@ -397,7 +399,17 @@ static int upload_rows(eh_ctx *c, double **coord, int64_t n, int32_t nprops, int
       memcpy(block + nprops * i, coord[i], sizeof(double) * nprops);
   }
   rc = ehd_put_rows(c->dev, block, n, nprops, cull, c->Po);
-  return rc ? devfail(c, rc) : EH_OK;
+  if (rc)
+    return devfail(c, rc);
+  c->upload_id = ehd_upload_id(c->dev);
+  return EH_OK;
+}
+
+/* the device's columns are one upload's: the context's, or that of a batch */
+static int own_columns(eh_ctx *c) {
+  return c->upload_id == ehd_upload_id(c->dev)
+             ? EH_OK
+             : fail(c, EH_ERR_STATE, "the particles on the device are not this context's last upload");
 }
 
 int eh_upload_rows(eh_ctx *c, double **coord, int64_t n, int32_t nprops, int cull) {
@@ -533,7 +545,10 @@ static int replay_until(eh_ctx *c, int64_t pass_lim, int32_t code_lim) {
 }
 
 static int refresh_losses(eh_ctx *c) {
-  int rc = ehd_get_state(c->dev, NULL, NULL, NULL, NULL, NULL, NULL, c->h_pass, c->h_code, c->n);
+  int rc = own_columns(c);
+  if (rc)
+    return rc;
+  rc = ehd_get_state(c->dev, NULL, NULL, NULL, NULL, NULL, NULL, c->h_pass, c->h_code, c->n);
   return rc ? devfail(c, rc) : EH_OK;
 }
 
@@ -543,10 +558,9 @@ static int refresh_losses(eh_ctx *c) {
 static int order_until(eh_ctx *c, int64_t pass_lim, int32_t code_lim) {
   int64_t effort, left;
   int rc;
-  if (ehd_state_n(c->dev) != c->n)
-    return devfail(c, EH_ERR_STATE);
-  if (!c->n)
-    return EH_OK;
+  rc = own_columns(c);
+  if (rc || !c->n)
+    return rc;
   rc = ehd_effort(c->dev, 0, 0, &effort, &left);
   if (rc)
     return devfail(c, rc);
@@ -813,8 +827,9 @@ int eh_track(eh_ctx *c, int64_t pass0, int64_t npasses, double *P_central, eh_st
       memset(stats, 0, sizeof(*stats));
     return EH_OK;
   }
-  if (ehd_state_n(c->dev) != c->n) /* a batch of the context holds the device's columns */
-    return devfail(c, EH_ERR_STATE);
+  rc = own_columns(c);
+  if (rc)
+    return rc;
   ehd_timing_reset(c->dev);
   {
     int64_t pass = pass0, end = pass0 + npasses;

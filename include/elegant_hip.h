@@ -445,7 +445,11 @@ int64_t eh_track_through_wake_noalloc(eh_ctx *ctx, double *const coord[6], int64
  * variant has its own beamline and particles; all are tracked together by a
  * persistent kernel over a queue of (variant, particle run) work items,
  * launched as a captured HIP graph.  Variants may not contain WAKE/ZLONGIT,
- * and RFCA elements need T_REFERENCE or FIDUCIAL=light. */
+ * and RFCA elements need T_REFERENCE or FIDUCIAL=light.
+ * The device holds the particles of the context's last upload, be it a
+ * batch's (its first track or autotune call), eh_upload's, do_tracking's or an
+ * element routine's: calls on particles that a later upload has replaced
+ * return EH_ERR_STATE, whatever their number. */
 typedef struct eh_batch eh_batch;
 typedef struct {
   int32_t particles_per_lane; /* 1 or 2 */

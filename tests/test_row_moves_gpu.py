@@ -104,3 +104,57 @@ def test_columns_taken_by_a_batch(tracker):
         with pytest.raises(native.EHError) as e:
             call()
         assert e.value.code == A.EH_ERR_STATE
+
+
+def refused(call):
+    with pytest.raises(native.EHError) as e:
+        call()
+    assert e.value.code == A.EH_ERR_STATE
+
+
+@pytest.mark.parametrize("sizes", [(300,), (500, 300)])
+def test_columns_taken_by_a_batch_of_the_same_size(tracker, sizes):
+    """the count of particles does not tell whose they are: a batch as large
+    as the upload, also after a larger one for which the columns were
+    allocated anew"""
+    bl = E.Beamline([E.DRIF(L=0.7)])
+    tracker.load(bl, PO)
+    tracker.upload(beam(300, 8))
+    for n in sizes:
+        b = native.Batch(tracker)
+        b.add_variant(bl, PO, beam(n, 9))
+        b.track(0, 1)
+        b.close()
+    for call in (lambda: tracker.track(0, 1), tracker.download, tracker.loss_records):
+        refused(call)
+    r = beam(300, 8)[:, :8]
+    tracker.upload(r)
+    assert tracker.track(0, 1).n_left == 300
+    assert np.array_equal(tracker.download()[0][:, 6], r[:, 6])
+
+
+def test_batch_whose_columns_are_taken(tracker):
+    """an element call, an upload and another batch, each with as many
+    particles as the batch: its own are gone; another context's are not"""
+    bl = E.Beamline([E.MAXAMP(X_MAX=1.0, Y_MAX=1.0), E.DRIF(L=0.7)])
+    r = np.ascontiguousarray(beam(300, 8)[:, :8])
+
+    def batch(t):
+        b = native.Batch(t)
+        b.add_variant(bl, PO, r)
+        b.set_tuning(1, 64, 4)
+        b.track(0, 1)
+        return b
+
+    other = native.Tracker(0)
+    for take in (lambda: tracker.track_particles_drift(r.copy(), E.DRIF(L=0.1).p.drift), lambda: tracker.upload(r),
+                 lambda: batch(tracker).close()):
+        b, o = batch(tracker), batch(other)
+        take()
+        for call in (lambda: b.track(1, 1), lambda: b.download(0), lambda: b.loss_passes(0), b.autotune,
+                     lambda: b.set_tuning(2, 64, 4)):
+            refused(call)
+        assert o.track(1, 1).n_left == 300 and o.download(0)[1] == 300
+        b.close()
+        o.close()
+    other.close()
