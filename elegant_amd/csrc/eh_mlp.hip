@@ -1221,19 +1221,31 @@ static int fused_grad(ehd_mlp *m, const float *X, const float *y, int32_t B, flo
 /* chunks of rows: the copies of the next chunk's inputs and the last one's
  * probabilities run beside a chunk's kernel */
 #define PRED_ROWS 32768
+
+/* each one made where it is missing: a call that failed half way is
+ * completed by the next */
+static int predict_set_up(ehd_mlp *m) {
+  if (!m->pstream)
+    MCHK(hipStreamCreateWithFlags(&m->pstream, hipStreamNonBlocking));
+  for (int k = 0; k < 4; k++)
+    if (!m->pev[k])
+      MCHK(hipEventCreateWithFlags(&m->pev[k], hipEventDisableTiming));
+  for (int k = 0; k < 2; k++) {
+    if (!m->pin[k])
+      MCHK(hipMalloc((void **)&m->pin[k], sizeof(float) * (size_t)PRED_ROWS * m->nin));
+    if (!m->pout[k])
+      MCHK(hipMalloc((void **)&m->pout[k], sizeof(float) * PRED_ROWS));
+  }
+  return EH_OK;
+}
+
 static int fused_predict(ehd_mlp *m, const float *X, int64_t n, float *prob) {
   hipStream_t st = m->d->stream;
   fused_tiles(m);
   const mlp_net N = fused_net(m);
-  if (!m->pstream) {
-    MCHK(hipStreamCreateWithFlags(&m->pstream, hipStreamNonBlocking));
-    for (int k = 0; k < 4; k++)
-      MCHK(hipEventCreateWithFlags(&m->pev[k], hipEventDisableTiming));
-    for (int k = 0; k < 2; k++) {
-      MCHK(hipMalloc((void **)&m->pin[k], sizeof(float) * (size_t)PRED_ROWS * m->nin));
-      MCHK(hipMalloc((void **)&m->pout[k], sizeof(float) * PRED_ROWS));
-    }
-  }
+  int rc = predict_set_up(m);
+  if (rc)
+    return rc;
   int64_t done = 0; /* probabilities copied out */
   int c = 0;
   for (int64_t s0 = 0; s0 < n; s0 += PRED_ROWS, c++) {
