@@ -1107,9 +1107,10 @@ int ehd_put_wake(ehd_dev *d, int32_t slot, const double *W, int64_t npoints) {
     sl->W_cap = npoints;
   }
   int rc = put_table(d, sl->W, W, npoints);
+  const hipError_t e = hipStreamSynchronize(d->stream);
   if (rc)
     return rc;
-  CHK(hipStreamSynchronize(d->stream));
+  CHK(e);
   sl->wpoints = npoints;
   return EH_OK;
 }
@@ -1146,9 +1147,10 @@ int ehd_put_zlongit(ehd_dev *d, int32_t slot, const double *Z, const double *tc,
     if (!rc)
       rc = put_table(d, sl->ts, ts, nb / 2 + 1);
   }
+  const hipError_t e = hipStreamSynchronize(d->stream); /* also after a failure: the tables are the caller's */
   if (rc)
     return rc;
-  CHK(hipStreamSynchronize(d->stream));
+  CHK(e);
   sl->tw_nb = nb;
   sl->nb = nb;
   return EH_OK;

@@ -1191,9 +1191,8 @@ static int grow_dev(ehd_mlp *m, void **p, int64_t *cap, int64_t count, size_t sz
   return EH_OK;
 }
 
-static int fused_grad(ehd_mlp *m, const float *X, const float *y, int32_t B, float *grad, float *loss) {
+static int queue_grad(ehd_mlp *m, const float *X, const float *y, int32_t B, float *grad, mlp_cut &C) {
   mlp_batch Q;
-  mlp_cut C;
   int rc = fused_batch(m, B, &Q, &C);
   if (!rc)
     rc = grow_dev(m, (void **)&m->Xd, &m->data_cap, (int64_t)B * m->nin, sizeof(float));
@@ -1212,10 +1211,16 @@ static int fused_grad(ehd_mlp *m, const float *X, const float *y, int32_t B, flo
   fused_step(m, P, Q, C, m->floss);
   MCHK(hipGetLastError());
   MCHK(hipMemcpyAsync(grad, m->grads, sizeof(float) * m->nparams, hipMemcpyDeviceToHost, m->d->stream));
-  if (loss)
-    return batch_loss(m, C.loss, C.nb, loss);
-  MCHK(hipStreamSynchronize(m->d->stream));
   return EH_OK;
+}
+
+static int fused_grad(ehd_mlp *m, const float *X, const float *y, int32_t B, float *grad, float *loss) {
+  mlp_cut C;
+  const int rc = queue_grad(m, X, y, B, grad, C);
+  if (!rc && loss)
+    return batch_loss(m, C.loss, C.nb, loss);
+  const hipError_t e = hipStreamSynchronize(m->d->stream);
+  return rc || !e ? rc : mlp_fail(m, e, "gradient");
 }
 
 /* chunks of rows: the copies of the next chunk's inputs and the last one's
@@ -1239,7 +1244,7 @@ static int predict_set_up(ehd_mlp *m) {
   return EH_OK;
 }
 
-static int fused_predict(ehd_mlp *m, const float *X, int64_t n, float *prob) {
+static int predict_chunks(ehd_mlp *m, const float *X, int64_t n, float *prob) {
   hipStream_t st = m->d->stream;
   fused_tiles(m);
   const mlp_net N = fused_net(m);
@@ -1287,9 +1292,16 @@ static int fused_predict(ehd_mlp *m, const float *X, int64_t n, float *prob) {
     MCHK(hipMemcpyAsync(prob + done, m->pout[(c - 1) & 1], sizeof(float) * (size_t)(n - done), hipMemcpyDeviceToHost,
                         m->pstream));
   }
-  MCHK(hipStreamSynchronize(m->pstream));
-  MCHK(hipStreamSynchronize(st));
   return EH_OK;
+}
+
+/* also after a failure nothing queued may still use the caller's arrays */
+static int fused_predict(ehd_mlp *m, const float *X, int64_t n, float *prob) {
+  const int rc = predict_chunks(m, X, n, prob);
+  const hipError_t p = m->pstream ? hipStreamSynchronize(m->pstream) : hipSuccess, s = hipStreamSynchronize(m->d->stream);
+  if (rc)
+    return rc;
+  return p || s ? mlp_fail(m, p ? p : s, "prediction") : EH_OK;
 }
 
 /* minibatch Adam over n samples (X row-major [n, nin]) for the given epochs;

@@ -2315,6 +2315,8 @@ static int upload_program(ehd_dev *d) {
     e = hipMemcpyAsync(d->pbuf, d->pstage, bytes, hipMemcpyHostToDevice, d->stream);
     if (!e)
       e = hipEventRecord(d->pev, d->stream);
+    if (e) /* pev cannot tell when pstage is free again */
+      (void)hipStreamSynchronize(d->stream);
   }
   if (!rc && e)
     rc = hip_fail(d, e, "uploading the tracking program");

@@ -83,9 +83,13 @@ static int fail(eh_ctx *c, int code, const char *m) {
   return code;
 }
 
+/* a device call failed; copies queued before it may use rows that are the
+ * caller's again once the error is returned */
 static int devfail(eh_ctx *c, int code) {
-  if (c && code)
+  if (c && code) {
     snprintf(c->msg, sizeof(c->msg), "%s", ehd_message(c->dev));
+    ehd_sync(c->dev);
+  }
   return code;
 }
 
@@ -1118,11 +1122,7 @@ static int track_single(eh_ctx *c, double **rows, int64_t n, int64_t pass) {
   if (rc)
     return rc;
   rc = ehd_track_single(c->dev, pass);
-  if (rc) {
-    devfail(c, rc);
-    ehd_sync(c->dev); /* the rows are the caller's again */
-  }
-  return rc;
+  return rc ? devfail(c, rc) : EH_OK;
 }
 
 /* run a one-element program on host rows and compact them like the

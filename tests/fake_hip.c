@@ -2,7 +2,8 @@
  * memory comes from calloc, kernels do not run, and the calls that may fail
  * fail when told to.  Loaded before the library, its functions take the
  * runtime's place.  It counts what a call left behind: allocations, streams
- * with work nobody waited for, copies through NULL, and bytes moved.
+ * with copies from or to pageable memory (the caller's, mostly) that nobody
+ * waited for, copies through NULL, and bytes moved.
  * Interfaces: the HIP runtime API's public signatures. */
 #include <stddef.h>
 #include <stdlib.h>
@@ -16,6 +17,10 @@ typedef struct {
 static long countdown, failed, live, nulls, h2d, launches, calls;
 static stream_t *streams[64];
 static int nstreams;
+static struct {
+  char *p;
+  size_t n;
+} pinned[256];
 
 static int fails(void) {
   calls++;
@@ -68,7 +73,11 @@ static int copy(void *d, const void *s, size_t n, int kind, stream_t *st) {
   if (kind == 1)
     h2d += (long)n;
   memcpy(d, s, n);
-  if (st)
+  const char *host = kind == 1 ? s : d;
+  for (int k = 0; k < 256; k++)
+    if (pinned[k].p && host >= pinned[k].p && host < pinned[k].p + pinned[k].n)
+      return OK;
+  if (st && (kind == 1 || kind == 2))
     st->queued = 1;
   return OK;
 }
@@ -76,12 +85,28 @@ static int copy(void *d, const void *s, size_t n, int kind, stream_t *st) {
 int hipGetDeviceCount(int *n) { return *n = 1, OK; }
 int hipSetDevice(int d) { return (void)d, OK; }
 int hipDeviceGetAttribute(int *v, int a, int d) { return (void)a, (void)d, *v = 4, OK; }
-int hipGetLastError(void) { return OK; }
+int hipGetLastError(void) { return fails() ? NO_MEMORY : OK; } /* a launch that failed */
 const char *hipGetErrorString(int e) { return e ? "told to fail" : "no error"; }
 int hipMalloc(void **p, size_t n) { return *p = NULL, make(p, n); }
 int hipFree(void *p) { return drop(p); }
-int hipHostMalloc(void **p, size_t n, unsigned f) { return (void)f, *p = NULL, make(p, n); }
-int hipHostFree(void *p) { return drop(p); }
+int hipHostMalloc(void **p, size_t n, unsigned f) {
+  (void)f;
+  *p = NULL;
+  int rc = make(p, n);
+  for (int k = 0; k < 256 && !rc; k++)
+    if (!pinned[k].p) {
+      pinned[k].p = *p;
+      pinned[k].n = n;
+      break;
+    }
+  return rc;
+}
+int hipHostFree(void *p) {
+  for (int k = 0; k < 256; k++)
+    if (p && pinned[k].p == p)
+      pinned[k].p = NULL;
+  return drop(p);
+}
 int hipGetSymbolAddress(void **p, const void *s) {
   static char scratch[1 << 20];
   return (void)s, *p = scratch, OK;

@@ -53,6 +53,7 @@ def each_failure(F, native, fresh, call, after=lambda s: None, most=200):
         hit = bool(F.fake_failed())
         F.fake_fail_at(0)
         assert ok != hit, "call %d failed unnoticed" % k
+        assert F.fake_queued() == 0, "call %d: work left on a stream" % k
         after(s)
         call(s)
         assert F.fake_nulls() == 0, "call %d: NULL used after its failure" % k
@@ -65,19 +66,66 @@ def each_failure(F, native, fresh, call, after=lambda s: None, most=200):
     raise AssertionError("more than %d runtime calls" % most)
 
 
+def net(native):
+    from elegant_amd import learned
+    t = native.Tracker(0)
+    return learned.MLP(t, hidden=16), t
+
+
+def rows(n, w=8):
+    import numpy as np
+    r = np.zeros((n, w))
+    r[:, 6] = np.arange(n)
+    return r
+
+
 def prediction(F, native):
     import numpy as np
-    from elegant_amd import learned
-
-    def fresh():
-        t = native.Tracker(0)
-        return learned.MLP(t, hidden=16), t
-
     X = np.zeros((70000, 19), np.float32)
-    each_failure(F, native, fresh, lambda s: s[0].predict(X))
+    each_failure(F, native, lambda: net(native), lambda s: s[0].predict(X))
 
 
-def test_prediction_set_up(fake):
+def gradient(F, native):
+    import numpy as np
+    X, y = np.zeros((1000, 19), np.float32), np.zeros(1000, np.float32)
+    each_failure(F, native, lambda: net(native), lambda s: s[0].gradient(X, y))
+
+
+def element(F, native):
+    from elegant_amd import elements as E
+    q = E.KQUAD(L=0.3, K1=1.0)
+    for n in (100, 20000):  # the small copy back and the other one
+        each_failure(F, native, lambda: (native.Tracker(0),),
+                     lambda s: s[0].multipole_tracking2(rows(n), q, 1e4, 0.0))
+
+
+def impedance(F, native):
+    from elegant_amd import elements as E
+    z = E.ZLONGIT(BROAD_BAND=1, RS=1e4, Q=1.0, FREQ=20e9, N_BINS=1024, BIN_SIZE=1e-12)
+    each_failure(F, native, lambda: (native.Tracker(0),),
+                 lambda s: s[0].track_through_zlongit(rows(1000), z.p.zlongit, 1e4, 0, 1e-12))
+
+
+def tracking(F, native):
+    from elegant_amd import elements as E
+    from elegant_amd import lattices as Lt
+    bl = E.Beamline([E.CHARGE(TOTAL=1e-9), E.KQUAD(L=0.3, K1=1.0), E.RFCA(L=0.1, VOLT=1e5, FREQ=352e6, PHASE=90.0),
+                     E.WAKE(Lt.resonator_wake(points=200)), E.DRIF(L=0.5)])
+    for n, w in ((300, 8), (300, 11)):
+        def fresh():
+            t = native.Tracker(0)
+            t.set_particle_properties(w)
+            return (t,)
+        each_failure(F, native, fresh, lambda s: s[0].do_tracking(rows(n, w), bl, 1e4, 2), most=1000)
+
+
+def test_prediction(fake):
     """a stream, event or buffer that could not be made is made by the next
     call, not used as if it were there"""
     run(fake, prediction)
+
+
+@pytest.mark.parametrize("call", [gradient, element, impedance, tracking])
+def test_nothing_in_flight(fake, call):
+    """no copy from or to the caller's arrays outlives a failed call"""
+    run(fake, call)
