@@ -363,6 +363,15 @@ static double *one_block(double **rows, int64_t n, int32_t w) {
   return rows[0];
 }
 
+/* the columns of a row that go to the device, which reads seven: all of them,
+ * or of wide rows the first eight, gathered.  Gathering takes the host 4 ns a
+ * row, another column 0.27 ns on its way there and 0.44 on its way back: 3*10^5
+ * rows of 9, 16 and 64 columns through do_tracking take 4.5, 7.4 and 44 ms
+ * whole and 5.7, 8.2 and 42 gathered, through an element routine 3.1, 5.2
+ * and 19 against 4.8, 6.2 and 12 */
+#define EH_WHOLE_COLUMNS 20
+static int32_t device_columns(int32_t nprops) { return nprops <= EH_WHOLE_COLUMNS ? nprops : 8; }
+
 static double *host_rows(eh_ctx *c, int64_t count) {
   if (count > c->hrows_cap) {
     free(c->hrows);
@@ -372,8 +381,8 @@ static double *host_rows(eh_ctx *c, int64_t count) {
   return c->hrows;
 }
 
-/* The rows go to the device whole, as one copy, and are turned into columns
- * there, with do_tracking's initial NaN/Inf cull (do_tracking.c:468-473) when
+/* The rows go to the device as one copy (gathered first where they are wide
+ * or not adjacent) and are turned into columns there, with do_tracking's initial NaN/Inf cull (do_tracking.c:468-473) when
  * cull is set: such rows are recorded as lost on pass 0 before the first
  * element.  The single-element entry points upload without it, as the
  * element routines leave such rows to their caller.  Splitting rows into
@@ -394,15 +403,16 @@ static int upload_rows(eh_ctx *c, double **coord, int64_t n, int32_t nprops, int
     return rc;
   c->bunch_on_device = 0;
   c->upload_id = -1;
-  block = n > 0 ? one_block(coord, n, nprops) : NULL;
+  const int32_t w = device_columns(nprops);
+  block = n > 0 && w == nprops ? one_block(coord, n, w) : NULL;
   if (n > 0 && !block) {
-    block = host_rows(c, n * nprops);
+    block = host_rows(c, n * w);
     if (!block)
       return EH_ERR_NOMEM;
     for (int64_t i = 0; i < n; i++)
-      memcpy(block + nprops * i, coord[i], sizeof(double) * nprops);
+      memcpy(block + w * i, coord[i], sizeof(double) * w);
   }
-  rc = ehd_put_rows(c->dev, block, n, nprops, cull, c->Po);
+  rc = ehd_put_rows(c->dev, block, n, w, cull, c->Po);
   if (rc)
     return devfail(c, rc);
   c->upload_id = ehd_upload_id(c->dev);
@@ -992,14 +1002,15 @@ int eh_download(eh_ctx *c, double **coord, int64_t n, int32_t nprops, int64_t *n
     if (!block)
       return EH_ERR_NOMEM;
   }
+  const int32_t more = nprops - 8 < c->extra_w ? nprops - 8 : c->extra_w;
   rc = ehd_get_rows(c->dev, block, n, order_for_device(c));
   if (rc)
     return devfail(c, rc);
   for (int64_t j = 0; !direct && j < n; j++) {
     double *r = coord[j];
     memcpy(r, block + 8 * j, sizeof(double) * 8);
-    for (int k = 8; k < nprops && k - 8 < c->extra_w; k++)
-      r[k] = c->extra[c->extra_w * slot_at(c, j) + k - 8];
+    if (more > 0)
+      memcpy(r + 8, c->extra + c->extra_w * slot_at(c, j), sizeof(double) * more);
   }
   if (nLeft)
     *nLeft = c->n_alive_ref;
@@ -1049,18 +1060,26 @@ int64_t eh_do_tracking(eh_ctx *c, double **coord, int64_t nOriginal, int64_t *ef
 
 /* ------------------------------------------------ element entry points */
 
+/* columns [a, b) of the rows follow their particles */
+static void follow(const eh_ctx *c, double **rows, int64_t n, int64_t a, int64_t b, double *tmp) {
+  for (int64_t i = 0; i < n; i++)
+    memcpy(tmp + (b - a) * i, rows[i] + a, sizeof(double) * (b - a));
+  for (int64_t j = 0; j < n; j++)
+    memcpy(rows[j] + a, tmp + (b - a) * c->order[j], sizeof(double) * (b - a));
+}
+
 /* The rows of a single-element call back to the caller in the reference's
  * order.  Whole rows move, as swapParticles moves row_props doubles
- * (elegant.c:2663-2670): the element's columns 0..6 come from the device,
- * the other columns keep their values and follow their particle, and the
- * accepted rows, if given, take the same permutation (multipole.c:1075-1076,
- * limit_amplitudes.c:263-264 and 308-309).  Rows were uploaded in their
- * order, so slot i is row i. */
+ * (elegant.c:2663-2670): the element's columns 0..5 come from the device, the
+ * others as they went there or, where they stayed here, following their
+ * particle, and the accepted rows, if given, take the same permutation
+ * (multipole.c:1075-1076, limit_amplitudes.c:263-264 and 308-309).  Rows were
+ * uploaded in their order, so slot i is row i. */
 static int writeback_rows(eh_ctx *c, double **rows, int64_t n, double **accepted, int64_t *nLeft) {
-  const int64_t W = c->row_props;
+  const int64_t W = c->row_props, w = device_columns(c->row_props);
   const double *src = NULL;
   const int32_t *lp = NULL, *lc = NULL;
-  double *block = NULL;
+  double *block = NULL, *rest = NULL;
   int rc = ehd_rows_back(c->dev);
   if (!rc)
     rc = ehd_fetch_small(c->dev, &src, &lp, &lc);
@@ -1075,38 +1094,34 @@ static int writeback_rows(eh_ctx *c, double **rows, int64_t n, double **accepted
       memcpy(c->h_code, lc, sizeof(int32_t) * n);
       rc = replay_until(c, INT64_MAX, INT32_MAX);
     }
-  } else {
+  } else
     rc = order_until(c, INT64_MAX, INT32_MAX);
-    block = one_block(rows, n, (int32_t)W);
-    src = block;
-    if (!rc && !block) {
-      src = block = host_rows(c, n * W);
-      if (!block)
-        rc = EH_ERR_NOMEM;
-    } else
-      src = NULL;
-    if (!rc) {
-      rc = ehd_fetch_rows(c->dev, block, order_for_device(c));
-      if (rc)
-        devfail(c, rc);
-    }
-  }
-  double *acc = NULL;
-  if (!rc && accepted && c->have_order) {
-    acc = (double *)malloc(sizeof(double) * W * n);
-    if (!acc)
+  if (!rc && c->have_order && (W > w || accepted)) {
+    rest = (double *)malloc(sizeof(double) * W * n);
+    if (!rest)
       rc = EH_ERR_NOMEM;
   }
-  if (rc)
+  if (!rc && !src) {
+    block = w == W ? one_block(rows, n, (int32_t)W) : NULL;
+    if (!block)
+      src = block = host_rows(c, n * w);
+    if (!block)
+      rc = EH_ERR_NOMEM;
+    else if ((rc = ehd_fetch_rows(c->dev, block, order_for_device(c))))
+      devfail(c, rc);
+  }
+  if (rc) {
+    free(rest);
     return rc;
+  }
   for (int64_t j = 0; src && j < n; j++)
-    memcpy(rows[j], src + W * (block ? j : slot_at(c, j)), sizeof(double) * W);
-  if (acc) {
-    for (int64_t i = 0; i < n; i++)
-      memcpy(acc + W * i, accepted[i], sizeof(double) * W);
-    for (int64_t j = 0; j < n; j++)
-      memcpy(accepted[j], acc + W * c->order[j], sizeof(double) * W);
-    free(acc);
+    memcpy(rows[j], src + w * (block ? j : slot_at(c, j)), sizeof(double) * w);
+  if (rest) {
+    if (W > w)
+      follow(c, rows, n, w, W, rest);
+    if (accepted)
+      follow(c, accepted, n, 0, W, rest);
+    free(rest);
   }
   *nLeft = c->n_alive_ref;
   return EH_OK;

@@ -129,3 +129,26 @@ def test_prediction(fake):
 def test_nothing_in_flight(fake, call):
     """no copy from or to the caller's arrays outlives a failed call"""
     run(fake, call)
+
+
+def wide_rows(F, native):
+    from elegant_amd import elements as E
+    bl = E.Beamline([E.DRIF(L=0.5)])
+    q = E.KQUAD(L=0.3, K1=1.0)
+    for n in (50, 20000):
+        moved = {}
+        for w in (8, 21, 64):
+            t = native.Tracker(0)
+            t.set_particle_properties(w)
+            before = F.fake_h2d_bytes()
+            t.do_tracking(rows(n, w), bl, 1e4, 1)
+            between = F.fake_h2d_bytes()
+            t.multipole_tracking2(rows(n, w), q, 1e4, 0.0)
+            moved[w] = between - before, F.fake_h2d_bytes() - between
+            t.close()
+        assert moved[21] == moved[64] == moved[8], (n, moved)
+
+
+def test_wide_rows_move_as_eight_columns(fake):
+    """the device reads seven columns of a row: wide rows send eight"""
+    run(fake, wide_rows)

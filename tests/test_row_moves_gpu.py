@@ -158,3 +158,35 @@ def test_batch_whose_columns_are_taken(tracker):
         b.close()
         o.close()
     other.close()
+
+
+@pytest.mark.parametrize("adjacent", [True, False])
+@pytest.mark.parametrize("n,w,loss", [(257, 20, True), (257, 21, True), (256, 33, False), (20011, 20, True),
+                                      (20011, 21, True), (14564, 21, False)])
+def test_element_wide_rows(tracker, n, w, loss, adjacent):
+    """rows of up to 20 columns move whole, wider ones send eight"""
+    test_element_rows(tracker, n, w, loss, adjacent)
+
+
+@pytest.mark.parametrize("w", [9, 20, 21, 40])
+def test_wide_rows_through_do_tracking(tracker, w):
+    """the first eight columns as without the others, which follow their
+    particle, as the accepted rows do"""
+    n = 5003
+    bl = E.Beamline([E.MAXAMP(X_MAX=0.004, Y_MAX=0.003), E.DRIF(L=0.7), E.KQUAD(L=0.3, K1=0.9, N_KICKS=4)])
+    r = np.zeros((n, w))
+    r[:, :8] = beam(n, 6)[:, :8]
+    r[:, 8:] = np.arange(n)[:, None] + np.arange(w - 8) / 64
+    g8, gw = np.ascontiguousarray(r[:, :8]), r.copy()
+    a8, aw = np.zeros_like(g8), np.zeros_like(gw)
+    left8, _ = tracker.do_tracking(g8, bl, PO, 3, accepted=a8)
+    tracker.set_particle_properties(w)
+    try:
+        leftw, _ = tracker.do_tracking(gw, bl, PO, 3, accepted=aw)
+    finally:
+        tracker.set_particle_properties(8)
+    assert left8 == leftw and 0 < left8 < n
+    assert_rows_bitwise(np.ascontiguousarray(gw[:, :8]), g8, "rows")
+    src = gw[:, 6].astype(np.int64) - 1
+    assert_rows_bitwise(np.ascontiguousarray(gw[:, 8:]), np.ascontiguousarray(r[src, 8:]), "other columns")
+    assert_rows_bitwise(aw, np.ascontiguousarray(r[src]), "accepted")
