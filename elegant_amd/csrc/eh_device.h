@@ -33,15 +33,20 @@ int ehd_get_sdp(ehd_dev *d, double *s, double *dp, int32_t *loss_pass, int64_t n
 int64_t ehd_upload_id(const ehd_dev *d);
 
 /* Rows (AoS, as the caller holds them) moved whole and turned into columns on
- * the device.  ehd_put_rows copies n rows of w columns, sets the loss records
+ * the device, at most ehd_stage_rows at a time.  ehd_put_rows copies rows first
+ * .. first + m - 1 (of ehd_alloc_state's n) of w columns, sets the loss records
  * (with cull, rows with a NaN or infinite x or y are lost before the first
- * element, do_tracking.c:468-473) and keeps the rows; the copy may still run
- * when it returns.  ehd_get_rows brings back rows of 8 columns in the given
- * order (NULL: as uploaded) with column 7 = pass of loss.  ehd_rows_back
+ * element, do_tracking.c:468-473) and keeps the rows if they are all n; the
+ * copy may still run when it returns.  ehd_get_rows brings back rows first ..
+ * of 8 columns, their slots given by order[0 .. m) (NULL: as uploaded), with
+ * column 7 = pass of loss.  Where the rows were kept, ehd_rows_back
  * writes columns 0..5 into the kept rows, ehd_fetch_rows copies the kept rows
  * out in the given order. */
-int ehd_put_rows(ehd_dev *d, const double *rows, int64_t n, int32_t w, int cull, double Po);
-int ehd_get_rows(ehd_dev *d, double *out, int64_t n, const int32_t *order);
+int64_t ehd_stage_rows(const ehd_dev *d, int32_t w);
+void ehd_set_stage_rows(ehd_dev *d, int64_t rows);
+int ehd_put_rows(ehd_dev *d, const double *rows, int64_t first, int64_t m, int32_t w, int cull, double Po);
+int ehd_get_rows(ehd_dev *d, double *out, int64_t first, int64_t m, const int32_t *order);
+int ehd_rows_kept(const ehd_dev *d);
 int ehd_rows_back(ehd_dev *d);
 int ehd_fetch_rows(ehd_dev *d, double *out, const int32_t *order);
 /* the same for few rows, with their loss records, in one copy into a pinned

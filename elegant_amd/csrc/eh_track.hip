@@ -1805,12 +1805,12 @@ __global__ void eh_queue_reset(unsigned int *queue) { *queue = 0u; }
 
 /* columns from rows; the loss records start here, and with cull rows with a
  * NaN or infinite x or y are lost before the first element */
-__global__ void __launch_bounds__(256) rows_in(const double *__restrict__ rows, int64_t n, int32_t w, int32_t cull,
-                                               double Po, eh_state st, double *ids) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n)
+__global__ void __launch_bounds__(256) rows_in(const double *__restrict__ rows, int64_t first, int64_t m, int32_t w,
+                                               int32_t cull, double Po, eh_state st, double *ids) {
+  const int64_t j = (int64_t)blockIdx.x * 256 + threadIdx.x, i = first + j;
+  if (j >= m)
     return;
-  const double *r = rows + i * w;
+  const double *r = rows + j * w;
   double v[7];
 #pragma unroll
   for (int k = 0; k < 7; k++)
@@ -1850,13 +1850,14 @@ __global__ void __launch_bounds__(256) rows_back(double *rows, int32_t w, eh_sta
   rec[st.n + i] = st.loss_code[i];
 }
 
-/* rows of 8 columns in the given order, column 7 = pass of loss */
+/* m rows of 8 columns in the given order (NULL: from slot first on), column 7
+ * = pass of loss */
 __global__ void __launch_bounds__(256) rows_out(double *__restrict__ out, eh_state st, const double *__restrict__ ids,
-                                                const int32_t *__restrict__ order) {
+                                                int64_t first, int64_t m, const int32_t *__restrict__ order) {
   const int64_t j = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (j >= st.n)
+  if (j >= m)
     return;
-  const int64_t i = order ? order[j] : j;
+  const int64_t i = order ? order[j] : first + j;
   double *r = out + 8 * j;
   r[0] = st.x[i];
   r[1] = st.xp[i];
@@ -1877,13 +1878,14 @@ __global__ void __launch_bounds__(256) rows_gather(const double *__restrict__ in
   out[e] = in[(int64_t)order[e / w] * w + e % w];
 }
 
-__global__ void __launch_bounds__(256) fiducial_times(eh_state st, double Po, double ahead, double *t) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= st.n)
+__global__ void __launch_bounds__(256) fiducial_times(eh_state st, int64_t first, int64_t m, double Po, double ahead,
+                                                      double *t) {
+  const int64_t j = (int64_t)blockIdx.x * 256 + threadIdx.x, i = first + j;
+  if (j >= m)
     return;
   const double p = Po * (1 + st.dp[i]);
   const double beta = p / __builtin_sqrt(p * p + 1);
-  t[i] = (st.s[i] + ahead) / (EH_C_MKS * beta);
+  t[j] = (st.s[i] + ahead) / (EH_C_MKS * beta);
 }
 
 /* out[0] += passes completed from pass0 on, out[1] += particles alive.  One
@@ -2018,6 +2020,7 @@ void ehd_destroy(ehd_dev *d) {
 
 int ehd_alloc_state(ehd_dev *d, int64_t n) {
   d->upload++;
+  d->rows_kept = 0;
   HIPCHK(d, hipSetDevice(d->device));
   if (n > d->cap) {
     for (int k = 0; k < 6; k++) {
@@ -2127,17 +2130,25 @@ static int grow_rows(ehd_dev *d, double **p, int64_t *cap, int64_t count) {
 
 #define ROW_GRID(n) dim3((unsigned)(((n) + 255) / 256))
 
-int ehd_put_rows(ehd_dev *d, const double *rows, int64_t n, int32_t w, int cull, double Po) {
-  int rc = ehd_alloc_state(d, n);
-  if (rc || n == 0)
-    return rc;
-  rc = grow_rows(d, &d->rows, &d->rows_cap, n * (w + 1)); /* and the loss records behind them */
+void ehd_set_stage_rows(ehd_dev *d, int64_t rows) { d->stage_rows = rows; }
+
+int64_t ehd_stage_rows(const ehd_dev *d, int32_t w) {
+  return d->stage_rows > 0 ? d->stage_rows : EHD_STAGE_BYTES / (int64_t)(sizeof(double) * (size_t)(w + 1));
+}
+
+int ehd_put_rows(ehd_dev *d, const double *rows, int64_t first, int64_t m, int32_t w, int cull, double Po) {
+  d->rows_kept = 0;
+  if (first < 0 || m <= 0 || first + m > d->n)
+    return EH_ERR_INVALID;
+  HIPCHK(d, hipSetDevice(d->device));
+  int rc = grow_rows(d, &d->rows, &d->rows_cap, m * (w + 1)); /* and the loss records behind them */
   if (rc)
     return rc;
-  d->rows_w = w;
-  HIPCHK(d, hipMemcpyAsync(d->rows, rows, sizeof(double) * (size_t)(n * w), hipMemcpyHostToDevice, d->stream));
-  hipLaunchKernelGGL(rows_in, ROW_GRID(n), dim3(256), 0, d->stream, d->rows, n, w, cull, Po, state_of(d), d->ids);
+  HIPCHK(d, hipMemcpyAsync(d->rows, rows, sizeof(double) * (size_t)(m * w), hipMemcpyHostToDevice, d->stream));
+  hipLaunchKernelGGL(rows_in, ROW_GRID(m), dim3(256), 0, d->stream, d->rows, first, m, w, cull, Po, state_of(d), d->ids);
   HIPCHK(d, hipGetLastError());
+  d->rows_w = w;
+  d->rows_kept = m == d->n;
   return EH_OK;
 }
 
@@ -2154,24 +2165,24 @@ static int put_order(ehd_dev *d, const int32_t *order, int64_t n) {
   return EH_OK;
 }
 
-int ehd_get_rows(ehd_dev *d, double *out, int64_t n, const int32_t *order) {
-  if (n != d->n)
-    return EH_ERR_STATE;
-  if (n == 0)
-    return EH_OK;
+int ehd_get_rows(ehd_dev *d, double *out, int64_t first, int64_t m, const int32_t *order) {
+  if (first < 0 || m <= 0 || first + m > d->n)
+    return EH_ERR_INVALID;
   HIPCHK(d, hipSetDevice(d->device));
-  int rc = grow_rows(d, &d->rows2, &d->rows2_cap, 8 * n);
+  int rc = grow_rows(d, &d->rows2, &d->rows2_cap, 8 * m);
   if (!rc && order)
-    rc = put_order(d, order, n);
+    rc = put_order(d, order, m);
   if (rc)
     return rc;
-  hipLaunchKernelGGL(rows_out, ROW_GRID(n), dim3(256), 0, d->stream, d->rows2, state_of(d), d->ids,
+  hipLaunchKernelGGL(rows_out, ROW_GRID(m), dim3(256), 0, d->stream, d->rows2, state_of(d), d->ids, first, m,
                      order ? d->order : (const int32_t *)NULL);
   HIPCHK(d, hipGetLastError());
-  HIPCHK(d, hipMemcpyAsync(out, d->rows2, sizeof(double) * 8 * (size_t)n, hipMemcpyDeviceToHost, d->stream));
+  HIPCHK(d, hipMemcpyAsync(out, d->rows2, sizeof(double) * 8 * (size_t)m, hipMemcpyDeviceToHost, d->stream));
   HIPCHK(d, hipStreamSynchronize(d->stream));
   return EH_OK;
 }
+
+int ehd_rows_kept(const ehd_dev *d) { return d->rows_kept; }
 
 int ehd_rows_back(ehd_dev *d) {
   HIPCHK(d, hipSetDevice(d->device));
@@ -2218,12 +2229,16 @@ int ehd_fetch_small(ehd_dev *d, const double **rows, const int32_t **loss_pass, 
 
 int ehd_fiducial_times(ehd_dev *d, double Po, double ahead, double *t) {
   HIPCHK(d, hipSetDevice(d->device));
-  int rc = grow_rows(d, &d->rows2, &d->rows2_cap, d->n);
-  if (rc)
-    return rc;
-  hipLaunchKernelGGL(fiducial_times, ROW_GRID(d->n), dim3(256), 0, d->stream, state_of(d), Po, ahead, d->rows2);
-  HIPCHK(d, hipGetLastError());
-  HIPCHK(d, hipMemcpyAsync(t, d->rows2, sizeof(double) * (size_t)d->n, hipMemcpyDeviceToHost, d->stream));
+  const int64_t most = ehd_stage_rows(d, 0);
+  for (int64_t first = 0; first < d->n; first += most) {
+    const int64_t m = d->n - first < most ? d->n - first : most;
+    int rc = grow_rows(d, &d->rows2, &d->rows2_cap, m);
+    if (rc)
+      return rc;
+    hipLaunchKernelGGL(fiducial_times, ROW_GRID(m), dim3(256), 0, d->stream, state_of(d), first, m, Po, ahead, d->rows2);
+    HIPCHK(d, hipGetLastError());
+    HIPCHK(d, hipMemcpyAsync(t + first, d->rows2, sizeof(double) * (size_t)m, hipMemcpyDeviceToHost, d->stream));
+  }
   HIPCHK(d, hipStreamSynchronize(d->stream));
   return EH_OK;
 }

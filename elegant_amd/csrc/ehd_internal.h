@@ -14,6 +14,10 @@
  * static scratch (plan 128 B + histogram and voltage for EHD_NOALLOC_BINS + 16
  * bins + 1,025 fixed-point partials, rounded up) */
 #define EHD_ZL_MAX_BINS (1 << 20) /* ZLONGIT bins: the bin optimiser's default cap (ztransverse.c:672-759) */
+/* Rows on their way in or out: 4 million of 8 columns at a time, a copy of 5 ms
+ * against some 20 us of launch and wait, so that they take this much of the
+ * device beside the 64 bytes per particle of the columns, not 140 per particle */
+#define EHD_STAGE_BYTES ((int64_t)256 << 20)
 #define EHD_PIN_BYTES (1 << 20) /* small results come back through pinned memory */
 #define EHD_NOALLOC_BINS 16384
 #define EHD_NOALLOC_BYTES (256 * 1024)
@@ -37,10 +41,13 @@ struct ehd_dev {
   int64_t n, cap;
   int64_t upload;      /* counts the uploads: whose particles the columns hold */
   /* rows as the caller holds them, on their way to or from the columns
-   * above: kept between calls, freed with the context */
+   * above: at most EHD_STAGE_BYTES each, kept between calls, freed with the
+   * context */
   double *rows, *rows2;
   int64_t rows_cap, rows2_cap;   /* doubles */
   int32_t rows_w;                /* columns per row of the last upload */
+  int rows_kept;                 /* rows holds all of it */
+  int64_t stage_rows;            /* tests: rows at a time */
   int32_t *order;
   int64_t order_cap;
   void *pin;           /* pinned host buffer of EHD_PIN_BYTES */

@@ -255,6 +255,13 @@ void eh_set_chunk_passes(eh_ctx *c, int32_t passes) {
     c->chunk_passes = passes;
 }
 
+/* rows moved to or from the device at a time (0: as many as its staging
+ * buffers take; not in the public header) */
+void eh_set_stage_rows(eh_ctx *c, int64_t rows) {
+  if (c)
+    ehd_set_stage_rows(c->dev, rows);
+}
+
 void eh_set_block(eh_ctx *c, int32_t block) {
   if (c)
     ehd_set_block(c->dev, block);
@@ -404,15 +411,25 @@ static int upload_rows(eh_ctx *c, double **coord, int64_t n, int32_t nprops, int
   c->bunch_on_device = 0;
   c->upload_id = -1;
   const int32_t w = device_columns(nprops);
+  const int64_t most = ehd_stage_rows(c->dev, w);
   block = n > 0 && w == nprops ? one_block(coord, n, w) : NULL;
-  if (n > 0 && !block) {
-    block = host_rows(c, n * w);
-    if (!block)
-      return EH_ERR_NOMEM;
-    for (int64_t i = 0; i < n; i++)
-      memcpy(block + w * i, coord[i], sizeof(double) * w);
+  rc = ehd_alloc_state(c->dev, n);
+  for (int64_t first = 0; !rc && first < n; first += most) {
+    const int64_t m = n - first < most ? n - first : most;
+    const double *src = block ? block + w * first : NULL;
+    if (!src) {
+      double *h = host_rows(c, m * w);
+      if (!h)
+        return EH_ERR_NOMEM;
+      if (first)
+        rc = ehd_sync(c->dev); /* the rows before these have left it */
+      for (int64_t i = 0; i < m; i++)
+        memcpy(h + w * i, coord[first + i], sizeof(double) * w);
+      src = h;
+    }
+    if (!rc)
+      rc = ehd_put_rows(c->dev, src, first, m, w, cull, c->Po);
   }
-  rc = ehd_put_rows(c->dev, block, n, w, cull, c->Po);
   if (rc)
     return devfail(c, rc);
   c->upload_id = ehd_upload_id(c->dev);
@@ -996,21 +1013,23 @@ int eh_download(eh_ctx *c, double **coord, int64_t n, int32_t nprops, int64_t *n
   if (rc)
     return rc;
   block = nprops == 8 ? one_block(coord, n, 8) : NULL;
-  const int direct = block != NULL;
-  if (!direct) {
-    block = host_rows(c, 8 * n);
-    if (!block)
-      return EH_ERR_NOMEM;
-  }
   const int32_t more = nprops - 8 < c->extra_w ? nprops - 8 : c->extra_w;
-  rc = ehd_get_rows(c->dev, block, n, order_for_device(c));
-  if (rc)
-    return devfail(c, rc);
-  for (int64_t j = 0; !direct && j < n; j++) {
-    double *r = coord[j];
-    memcpy(r, block + 8 * j, sizeof(double) * 8);
-    if (more > 0)
-      memcpy(r + 8, c->extra + c->extra_w * slot_at(c, j), sizeof(double) * more);
+  const int32_t *order = order_for_device(c);
+  const int64_t most = ehd_stage_rows(c->dev, 8);
+  for (int64_t first = 0; first < n; first += most) {
+    const int64_t m = n - first < most ? n - first : most;
+    double *out = block ? block + 8 * first : host_rows(c, 8 * m);
+    if (!out)
+      return EH_ERR_NOMEM;
+    rc = ehd_get_rows(c->dev, out, first, m, order ? order + first : NULL);
+    if (rc)
+      return devfail(c, rc);
+    for (int64_t j = first; !block && j < first + m; j++) {
+      double *r = coord[j];
+      memcpy(r, out + 8 * (j - first), sizeof(double) * 8);
+      if (more > 0)
+        memcpy(r + 8, c->extra + c->extra_w * slot_at(c, j), sizeof(double) * more);
+    }
   }
   if (nLeft)
     *nLeft = c->n_alive_ref;
@@ -1068,6 +1087,24 @@ static void follow(const eh_ctx *c, double **rows, int64_t n, int64_t a, int64_t
     memcpy(rows[j] + a, tmp + (b - a) * c->order[j], sizeof(double) * (b - a));
 }
 
+/* columns 0..6 of the rows, in their order, a stage at a time */
+static int rows_in_chunks(eh_ctx *c, double **rows, int64_t n) {
+  const int32_t *order = order_for_device(c);
+  const int64_t most = ehd_stage_rows(c->dev, 8);
+  for (int64_t first = 0; first < n; first += most) {
+    const int64_t m = n - first < most ? n - first : most;
+    double *h = host_rows(c, 8 * m);
+    if (!h)
+      return EH_ERR_NOMEM;
+    int rc = ehd_get_rows(c->dev, h, first, m, order ? order + first : NULL);
+    if (rc)
+      return devfail(c, rc);
+    for (int64_t j = 0; j < m; j++)
+      memcpy(rows[first + j], h + 8 * j, sizeof(double) * 7);
+  }
+  return EH_OK;
+}
+
 /* The rows of a single-element call back to the caller in the reference's
  * order.  Whole rows move, as swapParticles moves row_props doubles
  * (elegant.c:2663-2670): the element's columns 0..5 come from the device, the
@@ -1076,12 +1113,16 @@ static void follow(const eh_ctx *c, double **rows, int64_t n, int64_t a, int64_t
  * (multipole.c:1075-1076, limit_amplitudes.c:263-264 and 308-309).  Rows were
  * uploaded in their order, so slot i is row i. */
 static int writeback_rows(eh_ctx *c, double **rows, int64_t n, double **accepted, int64_t *nLeft) {
-  const int64_t W = c->row_props, w = device_columns(c->row_props);
+  const int kept = ehd_rows_kept(c->dev);
+  /* where the device did not keep the rows, its columns are 0..6 */
+  const int64_t W = c->row_props, w = kept ? device_columns(c->row_props) : 7;
   const double *src = NULL;
   const int32_t *lp = NULL, *lc = NULL;
   double *block = NULL, *rest = NULL;
-  int rc = ehd_rows_back(c->dev);
-  if (!rc)
+  int rc = EH_OK;
+  if (kept)
+    rc = ehd_rows_back(c->dev);
+  if (kept && !rc)
     rc = ehd_fetch_small(c->dev, &src, &lp, &lc);
   if (rc)
     return devfail(c, rc);
@@ -1101,7 +1142,9 @@ static int writeback_rows(eh_ctx *c, double **rows, int64_t n, double **accepted
     if (!rest)
       rc = EH_ERR_NOMEM;
   }
-  if (!rc && !src) {
+  if (!rc && !kept)
+    rc = rows_in_chunks(c, rows, n);
+  else if (!rc && !src) {
     block = w == W ? one_block(rows, n, (int32_t)W) : NULL;
     if (!block)
       src = block = host_rows(c, n * w);

@@ -108,6 +108,7 @@ EXTRA = [
     ("eh_test_program_runs", C.c_int32, [P]),
     ("eh_set_chunk_passes", None, [P, C.c_int32]),
     ("eh_set_block", None, [P, C.c_int32]),
+    ("eh_set_stage_rows", None, [P, C.c_int64]),
     ("eh_collective_probe", C.c_int, [P, PP, C.c_int64, PE, C.c_double, C.c_int64, C.c_double, PD, PD,
                                       C.POINTER(C.c_int64), PD]),
 ]
@@ -365,6 +366,9 @@ class Tracker:
 
     def set_chunk_passes(self, k):
         lib().eh_set_chunk_passes(self._ctx, int(k))
+
+    def set_stage_rows(self, n):
+        lib().eh_set_stage_rows(self._ctx, int(n))
 
     def set_block(self, b):
         lib().eh_set_block(self._ctx, int(b))

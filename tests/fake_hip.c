@@ -14,7 +14,7 @@ typedef struct {
   int queued;
 } stream_t;
 
-static long countdown, failed, live, nulls, h2d, launches, calls;
+static long countdown, failed, live, nulls, h2d, launches, calls, bytes;
 static stream_t *streams[64];
 static int nstreams;
 static struct {
@@ -42,6 +42,7 @@ long fake_nulls(void) { return nulls; }
 long fake_launches(void) { return launches; }
 long fake_calls(void) { return calls; }
 long fake_h2d_bytes(void) { return h2d; }
+long fake_device_bytes(void) { return bytes; } /* allocated so far */
 long fake_queued(void) {
   long q = 0;
   for (int k = 0; k < nstreams; k++)
@@ -87,7 +88,7 @@ int hipSetDevice(int d) { return (void)d, OK; }
 int hipDeviceGetAttribute(int *v, int a, int d) { return (void)a, (void)d, *v = 4, OK; }
 int hipGetLastError(void) { return fails() ? NO_MEMORY : OK; } /* a launch that failed */
 const char *hipGetErrorString(int e) { return e ? "told to fail" : "no error"; }
-int hipMalloc(void **p, size_t n) { return *p = NULL, make(p, n); }
+int hipMalloc(void **p, size_t n) { return *p = NULL, bytes += (long)n, make(p, n); }
 int hipFree(void *p) { return drop(p); }
 int hipHostMalloc(void **p, size_t n, unsigned f) {
   (void)f;

@@ -30,7 +30,7 @@ def run(fake, call):
 
 def child(fake, call):
     F = ctypes.CDLL(fake, mode=ctypes.RTLD_GLOBAL)
-    for f in ("failed", "live", "nulls", "launches", "calls", "h2d_bytes", "queued"):
+    for f in ("failed", "live", "nulls", "launches", "calls", "h2d_bytes", "device_bytes", "queued"):
         getattr(F, "fake_" + f).restype = ctypes.c_long
     F.fake_fail_at.argtypes = [ctypes.c_long]
     from elegant_amd import native
@@ -152,3 +152,24 @@ def wide_rows(F, native):
 def test_wide_rows_move_as_eight_columns(fake):
     """the device reads seven columns of a row: wide rows send eight"""
     run(fake, wide_rows)
+
+
+def device_memory(F, native):
+    from elegant_amd import elements as E
+    bl = E.Beamline([E.DRIF(L=0.5), E.RFCA(VOLT=1e5, FREQ=352e6, PHASE=90.0)])
+    q = E.KQUAD(L=0.3, K1=1.0)
+    n, w = 6000011, 8
+    r = rows(n, w)
+    t = native.Tracker(0)
+    before = F.fake_device_bytes()
+    t.do_tracking(r, bl, 1e4, 1)
+    t.multipole_tracking2(r, q, 1e4, 0.0)
+    used = F.fake_device_bytes() - before
+    t.close()
+    assert used <= 64 * n + (2 << 28) + (1 << 26), (used, 64 * n)
+
+
+def test_device_memory_per_particle(fake):
+    """64 bytes per particle in the columns; rows pass through buffers of
+    bounded size (256 MiB each)"""
+    run(fake, device_memory)

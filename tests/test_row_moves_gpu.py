@@ -190,3 +190,48 @@ def test_wide_rows_through_do_tracking(tracker, w):
     src = gw[:, 6].astype(np.int64) - 1
     assert_rows_bitwise(np.ascontiguousarray(gw[:, 8:]), np.ascontiguousarray(r[src, 8:]), "other columns")
     assert_rows_bitwise(aw, np.ascontiguousarray(r[src]), "accepted")
+
+
+@pytest.fixture
+def staged(tracker):
+    """1000 rows at a time to and from the device"""
+    tracker.set_stage_rows(1000)
+    yield tracker
+    tracker.set_stage_rows(0)
+
+
+@pytest.mark.parametrize("adjacent", [True, False])
+@pytest.mark.parametrize("n,w,loss", [(1000, 8, True), (1001, 8, True), (2000, 11, True), (20011, 8, False),
+                                      (20011, 21, True)])
+def test_element_rows_in_stages(staged, n, w, loss, adjacent):
+    test_element_rows(staged, n, w, loss, adjacent)
+
+
+@pytest.mark.parametrize("adjacent", [True, False])
+@pytest.mark.parametrize("n", [1000, 2001, 14565])
+def test_upload_track_download_in_stages(staged, n, adjacent):
+    test_upload_track_download(staged, n, adjacent)
+
+
+@pytest.mark.parametrize("w", [9, 21])
+def test_wide_rows_in_stages(staged, w):
+    test_wide_rows_through_do_tracking(staged, w)
+
+
+def test_cavity_in_stages(staged):
+    """the fiducial mean over arrival times that come back in stages, and an
+    impedance step's rows"""
+    bl = E.Beamline([E.MAXAMP(X_MAX=0.004, Y_MAX=0.003), E.DRIF(L=0.7), E.RFCA(VOLT=1e6, FREQ=352e6, PHASE=90.0)])
+    z = E.ZLONGIT(BROAD_BAND=1, RS=1e4, Q=1.0, FREQ=20e9, N_BINS=1024, BIN_SIZE=1e-12, ALLOW_LONG_BEAM=1)
+    r = np.ascontiguousarray(beam(3500, 6)[:, :8])
+    out = []
+    for stage in (1000, 0):
+        staged.set_stage_rows(stage)
+        a, b = r.copy(), r.copy()
+        left, _ = staged.do_tracking(a, bl, PO, 2)
+        phase = staged.rfca_fiducial(2)
+        staged.track_through_zlongit(b, z.p.zlongit, PO, 0, 1e-12)
+        out.append((left, phase, a, b))
+    assert out[0][:2] == out[1][:2] and 0 < out[0][0] < 3500
+    assert_rows_bitwise(out[0][2], out[1][2], "tracked")
+    assert_rows_bitwise(out[0][3], out[1][3], "impedance")
