@@ -71,6 +71,7 @@
 #define EH_F_CHT_SELF (1 << 26) /* CHANGE_T with each particle as its own beam: the offset from its own time */
 #define EH_F_LEND (1 << 27)    /* KQUAD LEFFECTIVE: exact drifts of EH_D_LEND around the body */
 #define EH_F_WIDE (1 << 29)    /* with EH_F_FAST: a substep angle of 2^-6 or more */
+#define EH_F_SMALL (1 << 30)   /* CSBEND: as EH_F_FAST but for substep angles below 2^-20 */
 #define EH_F_FIRSTPASS (1 << 28) /* before the RECIRC point: tracked on pass 0 only (do_tracking.c:459-465) */
 
 /* Aperture shapes other than the closed rectangle, packed in one int32:
@@ -208,8 +209,8 @@ typedef struct {
 #define EH_D_RRHOA 54     /* 1 / rho_actual rounded to nearest */
 #define EH_D_FIELD 55     /* [<= 28]: field coefficients in the order the sums read them (eh_bend_field.h) */
 #define EH_D_FIELD_MAX 28 /* expansion order 6: K1..K4 and XKICK */
-#define EH_D_ZLIM 44      /* with EH_F_FAST: phi^2 below this keeps every |substep angle + phi| below 2^-5 */
-#define EH_D_TE1 45       /* with EH_F_FAST, unless EH_F_PSI1/2: em_tan of the edge angles */
+#define EH_D_ZLIM 44      /* with EH_F_FAST or EH_F_SMALL: phi^2 below this keeps every |substep angle + phi| below 2^-5 */
+#define EH_D_TE1 45       /* with EH_F_FAST or EH_F_SMALL, unless EH_F_PSI1/2: em_tan of the edge angles */
 #define EH_D_TE2 46
 #define EH_D_ET 83        /* [5]: ETILT exit offsets of x, x', y, y', s (eh_bend_etilt.h) */
 

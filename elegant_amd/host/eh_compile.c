@@ -694,15 +694,18 @@ static int compile_csbend(const eh_element *e, const EH_MAXAMP *maxamp, eh_op *o
    * the shared-reciprocal range, moderate substep angles below 2^-5, and kick
    * lengths that are 0 or moderate; with multipoles (EH_F_FIELD) the one
    * expansion it is written for, order 4 (K1, K2 and XKICK), and the
-   * 4th-order integrator */
+   * 4th-order integrator.  Below 2^-20 (correctors; a dipole's only) it takes
+   * another instance, which watches what the angle no longer guarantees */
   if (rho0 > 0 && rho_actual > 0 && em_recip_ok(rho0) && em_recip_ok(rho_actual) &&
       (!(op->flags & EH_F_FIELD) || (op->nfield == 5 && nsub == 4))) {
-    int fast = 1;
+    int fast = 1, small = 0;
     double amax = 0;
     for (int j = 0; j < nsub; j++) {
       double a = fabs(op->d[EH_D_BDSHR + j]), k = fabs(op->d[EH_D_BDS + j]);
-      if (!(a >= 0x1.0p-20 && a < 0x1.0p-5) || !(k == 0 || em_recip_ok(k)))
+      if (!(a >= 0x1.0p-500 && a < 0x1.0p-5) || !(k == 0 || em_recip_ok(k)))
         fast = 0;
+      if (a < 0x1.0p-20)
+        small = 1;
       amax = a > amax ? a : amax;
     }
     /* the edges' quotients: tan E and the fringe angle 0 or moderate */
@@ -710,6 +713,8 @@ static int compile_csbend(const eh_element *e, const EH_MAXAMP *maxamp, eh_op *o
     for (int j = 0; j < 4; j++)
       if (!(e[j] == 0 || (fabs(e[j]) >= 0x1.0p-500 && fabs(e[j]) <= 0x1.0p+500)))
         fast = 0;
+    if (small && (op->flags & EH_F_FIELD))
+      fast = 0;
     if (fast) {
       if (psi1)
         op->flags |= EH_F_PSI1;
@@ -718,7 +723,7 @@ static int compile_csbend(const eh_element *e, const EH_MAXAMP *maxamp, eh_op *o
       op->d[EH_D_TE1] = em_tan(e1 - psi1);
       op->d[EH_D_TE2] = em_tan(e2 - psi2);
       /* |phi| <= sqrt(zlim) (1 + 2^-52) leaves |a + phi| below 2^-5 after its rounding */
-      op->flags |= EH_F_FAST;
+      op->flags |= small ? EH_F_SMALL : EH_F_FAST;
       op->d[EH_D_ZLIM] = sqr(0x1.0p-5 - amax) * (1 - 0x1.0p-40);
       if (amax >= 0x1.0p-6)
         op->flags |= EH_F_WIDE;

@@ -229,3 +229,75 @@ def test_combined_function_bend(tracker, kw):
         nc = O.lib("emath").or_track_through_csbend(ptr, c.shape[0], C.byref(b), PO, 3.0, C.byref(ap))
         assert_same_survivors(r, g, ng, c, nc)
         assert_rows_bitwise(g[:, :7], c[:, :7], "combined-function bend")
+
+
+# substep angles around 2^-20, where the instance for small bends begins
+# (0.1756 of a slice is the fourth-order integrator's shortest substep, 0.5
+# the second-order one's), and down to the largest radius
+@pytest.mark.parametrize("L,angle,kw", [
+    (0.2, 2.17e-5, {}), (0.2, 2.18e-5, {}), (0.2, 2.1e-7, {}), (0.001, 1.1e-9, {}), (0.1, 7.6e-6, dict(INTEGRATION_ORDER=2)),
+    (0.1, 7.7e-6, dict(INTEGRATION_ORDER=2)), (0.3, 1e-6, dict(INTEGRATION_ORDER=6)), (0.3, -1e-5, dict(TILT=1.5)),
+    (0.2, 1e-6, dict(E1=0.03, E2=-0.02, HGAP=0.02, FSE=0.5, DX=1e-4, DZ=3e-4, ETILT=1e-3)),
+    (0.2, 1e-6, dict(E1=0.2, E2=0.2, EDGE1_KICK_LIMIT=1e-9)), (0.2, 1e-6, dict(K1=0.3)), (0.2, 2.0 ** -22, {}),
+])
+def test_csbend_small_angles(tracker, L, angle, kw):
+    b = E.CSBEND(L=L, ANGLE=angle, N_KICKS=4, **kw).p.csbend
+    r = csbend_edge_rows(3000, 51)
+    h = 2.0 ** -26
+    rng = np.random.default_rng(51)
+    r[600:1200, 1] = rng.choice([-1.0, 1.0], 600) * 10.0 ** rng.uniform(-9.5, -5.5, 600)  # cosines 1 - n 2^-53
+    r[600:1200, [3, 5]] = 0.0
+    r[600:1200:2, 3] = rng.choice([-1.0, 1.0], 300) * 10.0 ** rng.uniform(-9.5, -6.0, 300)
+    r[1200:1300, 1] = rng.choice([0.0, -0.0, h, -h, h / 2, 2 * h, h * (1 + 2.0 ** -52)], 100)
+    r[1200:1300, 3] = rng.choice([0.0, -0.0, h, -h, h / 2], 100)
+    r[1200:1300, 5] = rng.choice([0.0, 1.0, -0.5], 100)
+    r[1200:1300:3, 0] = 0.0
+    r[1300:1350, 1] = -angle * np.linspace(0.0, 1.2, 50)  # c + phi through zero
+    r[1350:1400, 1] = 10.0 ** -np.linspace(150, 320, 50)
+    r[1400:1450, 0] = 10.0 ** -np.linspace(150, 320, 50)
+    r[1450:1500, 5] = np.linspace(-1.0, 1.0, 50)
+    r[1500:1550, 5] = 10.0 ** np.linspace(0, 30, 50)
+    r[1550:1600, 1] = np.linspace(-0.04, 0.04, 50)  # the band's edge
+    r[1600:1650, 0] = np.linspace(-0.0062, 0.0062, 50)
+    for ap in (A.EH_MAXAMP(0.006, 0.004, 0, 2, 2, 0), A.EH_MAXAMP(0.006, 0.004, 1, 2, 4, 0)):
+        g, c = r.copy(), r.copy()
+        ng = tracker.track_through_csbend(g, b, PO, 3.0, ap)
+        ptr, keep = rows_ptr(c)
+        nc = O.lib("emath").or_track_through_csbend(ptr, c.shape[0], C.byref(b), PO, 3.0, C.byref(ap))
+        assert_same_survivors(r, g, ng, c, nc)
+        assert_rows_bitwise(g[:, :7], c[:, :7], "csbend angle %g" % angle)
+
+
+def test_small_bends_take_a_common_path(tracker):
+    """a ring of correctors modelled as bends of 1e-6 rad against one of 1e-3
+    (1.2 times the kernel's time; the general code takes 2.9), tracked alone
+    and in a batch with the same result"""
+    r = np.ascontiguousarray(beam(20000, 53, halo=0.0)[:, :8])
+    r[:, [0, 2]] *= 0.05
+    r[:, [1, 3]] *= 0.05
+    ms, rows = {}, {}
+    for angle in (1e-6, 1e-3):
+        els = [E.MAXAMP(X_MAX=0.02, Y_MAX=0.02)]
+        for i in range(20):
+            els += [E.DRIF(L=0.5), E.CSBEND(L=0.2, ANGLE=angle, N_KICKS=4)]
+        bl = E.Beamline(els)
+        tracker.load(bl, PO)
+        times = []
+        for k in range(5):
+            tracker.upload(r)
+            times.append(tracker.track(0, 20).track_ms)
+        ms[angle], rows[angle] = min(times), tracker.download()[0]
+    assert ms[1e-6] < 2.0 * ms[1e-3], ms
+    els = [E.MAXAMP(X_MAX=0.02, Y_MAX=0.02)]
+    for i in range(20):
+        els += [E.DRIF(L=0.5), E.CSBEND(L=0.2, ANGLE=1e-6, N_KICKS=4)]
+    bl = E.Beamline(els)
+    from elegant_amd import native
+    for ppl in (1, 2):
+        b = native.Batch(tracker)
+        b.add_variant(bl, PO, r)
+        b.set_tuning(ppl, 64, 8)
+        b.track(0, 20)
+        got, _ = b.download(0)
+        b.close()
+        assert_rows_bitwise(got, rows[1e-6], "batch, %d per lane" % ppl)
