@@ -81,8 +81,9 @@ def rows(n, w=8):
 
 def prediction(F, native):
     import numpy as np
-    X = np.zeros((70000, 19), np.float32)
-    each_failure(F, native, lambda: net(native), lambda s: s[0].predict(X))
+    for n in (100, 70000):  # one chunk; three on two streams
+        X = np.zeros((n, 19), np.float32)
+        each_failure(F, native, lambda: net(native), lambda s: s[0].predict(X))
 
 
 def gradient(F, native):
@@ -173,3 +174,22 @@ def test_device_memory_per_particle(fake):
     """64 bytes per particle in the columns; rows pass through buffers of
     bounded size (256 MiB each)"""
     run(fake, device_memory)
+
+
+def few_rows(F, native):
+    import numpy as np
+    n, t = net(native)
+    X = np.zeros((100, 19), np.float32)
+    before = F.fake_calls()
+    n.predict(X)
+    first = F.fake_calls() - before
+    n.predict(X)
+    again = F.fake_calls() - before - first
+    t.close()
+    # in, a launch looked after, out; the first time two buffers more
+    assert (first, again) == (5, 3), (first, again)
+
+
+def test_prediction_of_few_rows(fake):
+    """no second stream and no events where there is one chunk"""
+    run(fake, few_rows)
