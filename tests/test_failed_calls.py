@@ -34,6 +34,7 @@ def child(fake, call):
         getattr(F, "fake_" + f).restype = ctypes.c_long
     F.fake_fail_at.argtypes = [ctypes.c_long]
     from elegant_amd import native
+    native.Tracker(0).close()  # what the first context of a process makes and keeps
     call(F, native)
 
 
@@ -193,3 +194,21 @@ def few_rows(F, native):
 def test_prediction_of_few_rows(fake):
     """no second stream and no events where there is one chunk"""
     run(fake, few_rows)
+
+
+def contexts(F, native):
+    live, calls = F.fake_live(), F.fake_calls()
+    native.Tracker(0).close()
+    each = F.fake_calls() - calls
+    many = [native.Tracker(0) for _ in range(100)]
+    while many:
+        many.pop(len(many) // 2).close()
+    native.Tracker(0).close()
+    assert F.fake_live() == live
+    assert each == 6, each  # a stream and five events, no memory
+
+
+def test_context_makes_no_memory(fake):
+    """creating a context allocates nothing once the process has had one, also
+    after more of them than there are places for"""
+    run(fake, contexts)
