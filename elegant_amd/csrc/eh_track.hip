@@ -2306,13 +2306,17 @@ int ehd_effort(ehd_dev *d, int64_t pass0, int64_t end, int64_t *effort, int64_t 
 }
 
 int ehd_put_ops(ehd_dev *d, const eh_op *ops, int32_t nops) {
+  /* one record more than there are: the batch kernel reads the header of a
+   * variant's first record before it knows that the variant has none */
+  const int64_t room = (int64_t)nops + 1;
   HIPCHK(d, hipSetDevice(d->device));
-  if (nops > d->ops_cap) {
+  if (room > d->ops_cap) {
     if (d->ops)
       HIPCHK(d, hipFree(d->ops));
     d->ops = NULL;
-    HIPCHK(d, hipMalloc((void **)&d->ops, sizeof(eh_op) * (nops > 0 ? nops : 1)));
-    d->ops_cap = nops;
+    d->ops_cap = 0;
+    HIPCHK(d, hipMalloc((void **)&d->ops, sizeof(eh_op) * (size_t)room));
+    d->ops_cap = room;
   }
   if (nops > 0)
     HIPCHK(d, hipMemcpyAsync(d->ops, ops, sizeof(eh_op) * nops, hipMemcpyHostToDevice, d->stream));

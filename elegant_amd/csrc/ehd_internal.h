@@ -52,7 +52,8 @@ struct ehd_dev {
   int64_t order_cap;
   void *pin;           /* pinned host buffer of EHD_PIN_BYTES */
   eh_op *ops;          /* flat records of the batch kernel's programs */
-  int32_t nops, ops_cap;
+  int32_t nops;
+  int64_t ops_cap;
   /* the tracking kernel's program (ehd_put_program) */
   eh_op *host_prog;    /* flat copy on the host: patches refold it */
   int32_t nflat, host_prog_cap;

@@ -171,3 +171,28 @@ def test_batch_many_launches(tracker, compact, graph):
         assert_rows_identical(g, c, "variant %d, %d launches" % (k, passes))
     assert lost > 20
     b.close()
+
+
+def test_variants_without_elements():
+    """a variant of markers alone has no records to track: its rows come back
+    as they went, by itself on a new context, last in a batch and between
+    others"""
+    from elegant_amd import elements as E
+    Po = Lt.momentum(6000.0)
+    rows = np.zeros((70, 8))
+    rows[:, :6] = np.random.default_rng(1).standard_normal((70, 6)) * 1e-4
+    rows[:, 6] = np.arange(1, 71)
+    empty, drift = E.Beamline([E.MARK("M")]), E.Beamline([E.DRIF(L=0.5)])
+    for order in ([empty], [drift, empty], [empty, drift, empty, drift]):
+        t = native.Tracker(0)
+        for ppl in (1, 2):
+            b = native.Batch(t)
+            for bl in order:
+                b.add_variant(bl, Po, rows)
+            b.set_tuning(ppl, 64, 2)
+            assert b.track(0, 5).n_left == 70 * len(order)
+            for v, bl in enumerate(order):
+                got, left = b.download(v)
+                assert left == 70 and (bl is drift or np.array_equal(got[:, :7], rows[:, :7]))
+            b.close()
+        t.close()
