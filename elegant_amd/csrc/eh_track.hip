@@ -68,8 +68,6 @@ struct bend_t { /* around them */
   double dxi, dyi, dzi, ct, st, tane1, te1, po, dxf, dyf, dzf, tane2, te2;
 };
 
-#define PIN4(a, b, c, d) asm volatile("" : "+s"(a), "+s"(b), "+s"(c), "+s"(d))
-
 DEV bounds_t load_bounds(eh_opc &op) {
   bounds_t b = {op.hot[EH_H_CHKX], op.hot[EH_H_CHKY], op.hot[EH_H_INBX], op.hot[EH_H_INBY]};
   return b;

@@ -561,9 +561,6 @@ EM_FN double em_asin_poly_small(double z) {
   return z * p;
 }
 
-/* em_asin(x) for z = x*x < 2^-10 */
-EM_FN double em_asin_small(double x, double z) { return __builtin_fma(x, em_asin_poly5(z), x); }
-
 /* same series, long form for z <= 1/4 (25 terms) */
 EM_FN double em_asin_poly_large(double z) {
   const double a[25] = {0x1.5555555555555p-3, 0x1.3333333333333p-4, 0x1.6db6db6db6db7p-5, 0x1.f1c71c71c71c7p-6,
@@ -793,7 +790,7 @@ EM_FN double em_sqrt_recip_mid(double x, double *y) {
 /* The narrow bands with their coefficients held in registers, for a loop that
  * evaluates them often: em_small_coefs() before the loop takes the scalar
  * instructions that load them (108 of a bend slice's 600) out of it.  Same
- * operations as em_sin_small, em_cos_small and em_asin_small. */
+ * operations as em_sin_small, em_cos_small and, by em_asin_poly5, em_asin. */
 typedef struct {
   double s1, s2, s3, s4, c2, c3, c4, a1, a2, a3, a4, a5, sec;
 } em_small_k;
