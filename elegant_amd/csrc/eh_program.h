@@ -71,6 +71,7 @@
 #define EH_F_CHT_SELF (1 << 26) /* CHANGE_T with each particle as its own beam: the offset from its own time */
 #define EH_F_LEND (1 << 27)    /* KQUAD LEFFECTIVE: exact drifts of EH_D_LEND around the body */
 #define EH_F_WIDE (1 << 29)    /* with EH_F_FAST: a substep angle of 2^-6 or more */
+#define EH_F_INELL INT32_MIN   /* with EH_F_INAP: an ellipse whose reciprocal half-axes are at EH_B_INRX, EH_B_INRY */
 #define EH_F_SMALL (1 << 30)   /* CSBEND: as EH_F_FAST but for substep angles below 2^-20 */
 #define EH_F_FIRSTPASS (1 << 28) /* before the RECIRC point: tracked on pass 0 only (do_tracking.c:459-465) */
 
@@ -143,6 +144,9 @@ typedef struct {
 #define EH_B_DZF 11
 #define EH_B_TANE2 12
 #define EH_B_TE2 13
+/* (and of a MULT) with EH_F_INELL */
+#define EH_B_INRX 14
+#define EH_B_INRY 15
 
 /* ---- MULT ---- */
 #define EH_D_DX 0
@@ -234,7 +238,12 @@ typedef struct {
  * checks after an element remove infinities; nothing is removed in a
  * single-element call), and for a (super-)ellipse the box of 0.7 of its
  * half-axes, as 0.7^2 + 0.7^2 < 1.  Tiny half-axes whose powers leave the
- * normal range get no box. */
+ * normal range get no box.  Inside an element, lanes beyond the box are
+ * tested by the circle that the exponents (even, at least 2) contain, with
+ * the common path once more but out of line: a beam that fills the ellipse
+ * otherwise takes the common path and then the general code (20 sextupoles,
+ * 10^4 particles at 0.75 to 0.95 of the half-axis, 10 turns: 1.88 ms, 1.08
+ * with the circle, 0.39 inside the box). */
 static inline void eh_op_finish(eh_op *op) {
   double *h = op->hot, *b = op->bend;
   const double *d = op->d;
@@ -247,6 +256,13 @@ static inline void eh_op_finish(eh_op *op) {
       h[EH_H_INBX] = c * op->in_xmax;
     if (op->in_ymax > 0)
       h[EH_H_INBY] = c * op->in_ymax;
+    op->flags &= ~EH_F_INELL;
+    if ((op->in_code & EH_AP_ELL) && fmin(op->in_xmax, op->in_ymax) >= 0x1.0p-100 &&
+        fmax(op->in_xmax, op->in_ymax) <= 0x1.0p+100) {
+      op->flags |= EH_F_INELL;
+      b[EH_B_INRX] = 1 / op->in_xmax;
+      b[EH_B_INRY] = 1 / op->in_ymax;
+    }
   }
   if (!(op->flags & EH_F_ALONE)) {
     h[EH_H_CHKX] = h[EH_H_CHKY] = DBL_MAX;

@@ -345,12 +345,18 @@ DEV bool in_aperture(double x, double y, eh_opc &op) {
 }
 
 /* surely inside it (bounds from eh_op_finish): two compares without
- * a branch for the common paths, whose lanes outside take the general code */
-DEV bool in_bounds(double x, double y, const bounds_t &b, int flags, eh_opc &op) {
+ * a branch for the common paths, whose lanes outside take the general code.
+ * ANY: of an ellipse the circle, with a margin for the roundings here and in
+ * the general test */
+template <bool ANY> DEV bool in_bounds(double x, double y, const bounds_t &b, int flags, eh_opc &op) {
   if (flags & EH_F_INTILT) {
     double x0 = x, y0 = y;
     x = x0 * op.in_cs0 + y0 * op.in_cs1;
     y = -x0 * op.in_cs1 + y0 * op.in_cs0;
+  }
+  if (ANY && (flags & EH_F_INELL)) {
+    const double u = x * op.bend[EH_B_INRX], v = y * op.bend[EH_B_INRY];
+    return u * u + v * v <= 1 - 0x1.0p-45;
   }
   return (__builtin_fabs(x) <= b.in_x) & (__builtin_fabs(y) <= b.in_y);
 }
@@ -508,7 +514,7 @@ DEV int multipole_body(double &x, double &xp, double &y, double &yp, double &s, 
  *  - after the kicks qx and qy are 0 or >= 2^-700 in magnitude (binary
  *    exponent >= -699), so every dividend is 0 or within [2^-900, 2^900].
  * Arithmetic is otherwise the general code's, operation for operation. */
-template <int ORD>
+template <int ORD, bool ELL>
 DEV bool multipole_fast(const particle &p, double &x, double &xp, double &y, double &yp, double &s,
                         const opd_recip &o, const hdr_t H, const mult_t &m, eh_opc &op) {
   const int nsub = ORD ? 4 : op.nsub;
@@ -534,7 +540,7 @@ DEV bool multipole_fast(const particle &p, double &x, double &xp, double &y, dou
   yp = em_div_pos(qy, den, r);
   int emin = 0;
   for (int ik = 0; ik < HD_NSLICES(H); ik++) {
-    good &= in_bounds(x + dxa, y + dya, m.b, flags, op);
+    good &= in_bounds<ELL>(x + dxa, y + dya, m.b, flags, op);
 #pragma unroll
     for (int step = 0; step < nsub; step++) {
       if (has_drift) {
@@ -577,7 +583,7 @@ DEV bool multipole_fast(const particle &p, double &x, double &xp, double &y, dou
       yp = em_div_pos(qy, den, r);
     }
   }
-  return good & (emin >= -699) & (dmin >= 0.88 * o2) & in_bounds(x + dxa, y + dya, m.b, flags, op) &
+  return good & (emin >= -699) & (dmin >= 0.88 * o2) & in_bounds<ELL>(x + dxa, y + dya, m.b, flags, op) &
          (__builtin_fabs(x) <= EH_COORD_LIMIT) & (__builtin_fabs(y) <= EH_COORD_LIMIT) &
          (__builtin_fabs(xp) <= EH_SLOPE_LIMIT) & (__builtin_fabs(yp) <= EH_SLOPE_LIMIT);
 }
@@ -685,7 +691,7 @@ DEV int track_multipole(particle &p, eh_opc &op, eh_zc *z) {
 }
 
 /* the same on the common path; false: p is not to be used */
-DEV bool track_multipole_fast(particle &p, const hdr_t H, const mult_t &m, eh_opc &op) {
+template <bool ELL> DEV bool track_multipole_fast(particle &p, const hdr_t H, const mult_t &m, eh_opc &op) {
   const int flags = HD_FLAGS(H);
   if (flags & EH_F_EXPAND)
     return false;
@@ -700,13 +706,13 @@ DEV bool track_multipole_fast(particle &p, const hdr_t H, const mult_t &m, eh_op
   double x, xp, y, yp, s;
   bool done;
   if (body == 1)
-    done = multipole_fast<1>(p, x, xp, y, yp, s, o, H, m, op);
+    done = multipole_fast<1, ELL>(p, x, xp, y, yp, s, o, H, m, op);
   else if (body == 2)
-    done = multipole_fast<2>(p, x, xp, y, yp, s, o, H, m, op);
+    done = multipole_fast<2, ELL>(p, x, xp, y, yp, s, o, H, m, op);
   else if (body == 3)
-    done = multipole_fast<3>(p, x, xp, y, yp, s, o, H, m, op);
+    done = multipole_fast<3, ELL>(p, x, xp, y, yp, s, o, H, m, op);
   else
-    done = multipole_fast<0>(p, x, xp, y, yp, s, o, H, m, op);
+    done = multipole_fast<0, ELL>(p, x, xp, y, yp, s, o, H, m, op);
   p.x = x;
   p.xp = xp;
   p.y = y;
@@ -860,11 +866,12 @@ DEV bool csbend_body(double &X, double &QX, double &Y, double &QY, const double 
  *  - the aperture holds at every slice; dz_lost only matters for a loss.
  * Arithmetic is otherwise csbend_body's, operation for operation.
  *
- * SMALL: substep angles below 2^-20 (EH_F_SMALL; correctors modelled as
- * bends).  A cosine may be 1 - 2^-53 at any substep then, so the cosines'
- * reciprocals are em_recip's, and a running minimum keeps the exponents of
- * c + phi and of QX after a kick at -600 or more, or the values 0. */
-template <int NSUB, bool WIDE, bool SMALL>
+ * ANY: substep angles below 2^-20 too (EH_F_SMALL; correctors modelled as
+ * bends), and ellipses beyond their box.  A cosine may be 1 - 2^-53 at any
+ * substep then, so the cosines' reciprocals are em_recip's, and a running
+ * minimum keeps the exponents of c + phi and of QX after a kick at -600 or
+ * more, or the values 0. */
+template <int NSUB, bool WIDE, bool ANY>
 DEV bool csbend_body_fast(double &X, double &QX, double &Y, double &QY, const double opd, const double r_opd,
                           double &dist, const hdr_t H, const bendc_t &m, eh_opc &op) {
   const double rho0 = m.rho0, rhoa = m.rhoa;
@@ -882,13 +889,13 @@ DEV bool csbend_body_fast(double &X, double &QX, double &Y, double &QY, const do
   const double f1 = em_sqrt_recip_mid(fin1, &r_f1);
   /* sin_phi = 2^-26 exactly over cos_phi = 1 - 2^-53 (em_recip_cos_small): a
    * slope of sqrt(machine epsilon) at the entry, a usual finite-difference step */
-  if (!SMALL)
+  if (!ANY)
     good &= __builtin_fabs(QX) != 0x1.0p-26 * f;
   double acc = 0, zmax = 0;
   int emin = 0;
   const em_small_k K = em_small_coefs();
   for (int i = 0; i < HD_NSLICES(H); i++) {
-    good &= in_bounds(X, Y, m.b, HD_FLAGS(H), op);
+    good &= in_bounds<ANY>(X, Y, m.b, HD_FLAGS(H), op);
     acc += __builtin_fabs(X) + __builtin_fabs(QX);
 #pragma unroll
     for (int j = 0; j < nsub; j++) {
@@ -899,13 +906,13 @@ DEV bool csbend_body_fast(double &X, double &QX, double &Y, double &QY, const do
       zmax = __builtin_fmax(zmax, zp);
       if (WIDE)
         zmax = __builtin_fmax(zmax, za);
-      if (SMALL)
+      if (ANY)
         emin = imin3(emin, __builtin_amdgcn_frexp_exp(ang), 0);
       double sine = em_sin_small_c(ang, za, &K), cosi = em_cos_small_c(za, &K);
-      const double r_c = SMALL ? em_recip(cosi) : em_recip_cos_small(cosi, za, &K);
+      const double r_c = ANY ? em_recip(cosi) : em_recip_cos_small(cosi, za, &K);
       double tang = em_div_pos(sine, cosi, r_c);
       double cos_phi = em_cos_small_c(zp, &K);
-      const double r_p = SMALL ? em_recip(cos_phi) : em_recip_cos_small(cos_phi, zp, &K);
+      const double r_p = ANY ? em_recip(cos_phi) : em_recip_cos_small(cos_phi, zp, &K);
       QX = f * sine;
       double factor = em_div_pos((rho0 + X) * cos_phi, f, r_f) * (tang - em_div_pos(sin_phi, cos_phi, r_p));
       Y += QY * factor;
@@ -918,7 +925,7 @@ DEV bool csbend_body_fast(double &X, double &QX, double &Y, double &QY, const do
       double g = 1 + em_div_pos(X, rho0, m.rrho0);
       /* (-ds) g 1.0 = -(ds g): the general code's bits, one product fewer */
       QX += em_div_pos(-(ds * g), rhoa, m.rrhoa);
-      if (SMALL)
+      if (ANY)
         emin = imin3(emin, __builtin_amdgcn_frexp_exp(QX), 0);
       QX = em_div_pos(QX, opd, r_opd);
       QX *= opd;
@@ -981,7 +988,7 @@ DEV bool csbend_field_fast(double &X, double &QX, double &Y, double &QY, const d
   int emin = 0;
   const em_small_k K = em_small_coefs();
   for (int i = 0; i < HD_NSLICES(H); i++) {
-    good &= in_bounds(X, Y, m.b, HD_FLAGS(H), op);
+    good &= in_bounds<false>(X, Y, m.b, HD_FLAGS(H), op);
     acc += __builtin_fabs(X) + __builtin_fabs(QX);
 #pragma unroll
     for (int j = 0; j < 4; j++) {
@@ -1134,10 +1141,11 @@ static __device__ __attribute__((noinline)) double edge_tan(double a) { return e
  * moderate, and the host has checked the edges (EH_F_FAST).  1 + delta, the
  * edges' radius and the velocity are the same at both ends (nothing changes
  * delta here), so each has one reciprocal. */
-enum bend_kind { DIPOLE, FIELD_BEND, SMALL_DIPOLE };
+enum bend_kind { DIPOLE, FIELD_BEND, ANY_DIPOLE };
 template <bend_kind KIND> DEV bool track_csbend_fast(particle &p, const hdr_t H, hdr_t next, eh_opc &op) {
   const int flags = HD_FLAGS(H);
-  if (!(flags & (KIND == SMALL_DIPOLE ? EH_F_SMALL : EH_F_FAST)) || (KIND == DIPOLE && (flags & EH_F_FIELD)))
+  if (!(flags & (KIND == ANY_DIPOLE ? EH_F_SMALL | EH_F_FAST : EH_F_FAST)) ||
+      (KIND != FIELD_BEND && (flags & EH_F_FIELD)))
     return false;
   const bendc_t m = load_bendc(op, next);
   const bend_t B = load_bend(op);
@@ -1176,15 +1184,15 @@ template <bend_kind KIND> DEV bool track_csbend_fast(particle &p, const hdr_t H,
    * the scheduler overlaps neighbouring substeps */
   if (KIND == FIELD_BEND)
     good &= csbend_field_fast(X, QX, Y, QY, opd, r_opd, dist, H, m, op);
-  else if (KIND == SMALL_DIPOLE && op.nsub == 4)
+  else if (KIND == ANY_DIPOLE && op.nsub == 4 && !(flags & EH_F_WIDE))
     good &= csbend_body_fast<4, false, true>(X, QX, Y, QY, opd, r_opd, dist, H, m, op);
-  else if (KIND == SMALL_DIPOLE)
+  else if (KIND == ANY_DIPOLE)
     good &= csbend_body_fast<0, true, true>(X, QX, Y, QY, opd, r_opd, dist, H, m, op);
   else if (op.nsub == 4 && !(flags & EH_F_WIDE))
     good &= csbend_body_fast<4, false, false>(X, QX, Y, QY, opd, r_opd, dist, H, m, op);
   else
     good &= csbend_body_fast<0, true, false>(X, QX, Y, QY, opd, r_opd, dist, H, m, op);
-  good &= in_bounds(X, Y, m.b, flags, op);
+  good &= in_bounds<KIND == ANY_DIPOLE>(X, Y, m.b, flags, op);
   {
     const double den2 = sq(opd) - sq(QX) - sq(QY);
     good &= den2 >= 0x1.0p-128;
@@ -1491,25 +1499,49 @@ template <class T> DEV T *uniform(T *p) {
                (uint32_t)__builtin_amdgcn_readfirstlane((int)u));
 }
 
-SLOW slow_multipole(particle p, eh_opc *op, eh_zc *z) {
-  step_out o;
-  o.lost = track_multipole(p, *uniform(op), uniform(z));
-  o.p = p;
-  return o;
-}
-
-/* the common path of small bends, out of line behind the general code's entry,
- * so that the others keep their code and registers (as a branch of run_op it
- * took the FODO ring of 10^4 particles from 37 to 44 ms).  A ring of 20
- * correctors of 1e-6 rad, 10^4 particles, 10 turns: 1.82 ms, 4.65 by the
- * general code.  lost < 0: not taken, the row as it came */
-SLOW slow_csbend_small(particle p, eh_opc *op) {
+/* the common path for lanes beyond an ellipse's box but inside the ellipse
+ * (eh_op_finish), part of slow_multipole: called from it, it cost the kernels
+ * scalar registers that they keep across (FODO ring of 10^4 particles 37.2 ms,
+ * 36.4 so).  lost < 0: not taken, the row as it came */
+DEV step_out slow_multipole_ell(particle p, eh_opc *op) {
   step_out o;
   eh_opc &u = *uniform(op);
   const hdr_t H = load_hdr(&u);
   o.p = p;
   o.lost = 0;
-  if (!track_csbend_fast<SMALL_DIPOLE>(o.p, H, H, u)) {
+  if (!track_multipole_fast<true>(o.p, H, load_mult(u, H), u)) {
+    o.p = p;
+    o.lost = -1;
+  }
+  return o;
+}
+
+SLOW slow_multipole(particle p, eh_opc *op, eh_zc *z) {
+  step_out o;
+  eh_opc &u = *uniform(op);
+  if (u.flags & EH_F_INELL) {
+    o = slow_multipole_ell(p, &u);
+    if (!o.lost)
+      return o;
+    p = o.p;
+  }
+  o.lost = track_multipole(p, u, uniform(z));
+  o.p = p;
+  return o;
+}
+
+/* the common path of small bends, and of lanes beyond an ellipse's box, out of
+ * line behind the general code's entry, so that the others keep their code and
+ * registers (as a branch of run_op it took the FODO ring of 10^4 particles from
+ * 37 to 44 ms).  A ring of 20 correctors of 1e-6 rad, 10^4 particles, 10 turns:
+ * 1.86 ms, 4.65 by the general code.  lost < 0: not taken, the row as it came */
+SLOW slow_csbend_any(particle p, eh_opc *op) {
+  step_out o;
+  eh_opc &u = *uniform(op);
+  const hdr_t H = load_hdr(&u);
+  o.p = p;
+  o.lost = 0;
+  if (!track_csbend_fast<ANY_DIPOLE>(o.p, H, H, u)) {
     o.p = p;
     o.lost = -1;
   }
@@ -1519,8 +1551,8 @@ SLOW slow_csbend_small(particle p, eh_opc *op) {
 SLOW slow_csbend(particle p, eh_opc *op, eh_zc *z) {
   step_out o;
   eh_opc &u = *uniform(op);
-  if (u.flags & EH_F_SMALL) {
-    o = slow_csbend_small(p, &u);
+  if (u.flags & (EH_F_SMALL | EH_F_INELL)) {
+    o = slow_csbend_any(p, &u);
     if (!o.lost)
       return o;
     p = o.p;
@@ -1542,8 +1574,8 @@ SLOW slow_csbend_field(particle p, eh_opc *op, eh_zc *z) {
   o.lost = 0;
   if ((HD_FLAGS(H) & EH_F_FIELD) && track_csbend_fast<FIELD_BEND>(o.p, H, H, u))
     return o;
-  if (HD_FLAGS(H) & EH_F_SMALL) {
-    o = slow_csbend_small(p, &u);
+  if (HD_FLAGS(H) & (EH_F_SMALL | EH_F_INELL)) {
+    o = slow_csbend_any(p, &u);
     if (!o.lost)
       return o;
     p = o.p;
@@ -1602,7 +1634,7 @@ template <bool FIELD> DEV int run_op(particle &p, const hdr_t H, hdr_t next, eh_
   if (code == EH_OP_MULT) {
     particle q = p;
     const mult_t m = load_mult(op, next);
-    const bool done = track_multipole_fast(q, H, m, op);
+    const bool done = track_multipole_fast<false>(q, H, m, op);
     if (ALL_LANES(done))
       p = q;
     else if (done)
