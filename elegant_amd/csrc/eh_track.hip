@@ -502,7 +502,7 @@ DEV int multipole_body(double &x, double &xp, double &y, double &yp, double &s, 
  * The slopes at the exit are those after the last kick, as the momenta have
  * not changed since.  A slice of four substeps of a quadrupole takes 182 VALU
  * instructions, 3 of them transcendental (276 with 16 before).  FODO ring, 10^4
- * particles, 64 turns: 84.1 -> 54.9 ms (37.1 with what came after it).
+ * particles, 64 turns: 84.1 -> 54.9 ms (36.4 with what came after it).
  *
  * What makes every step valid:
  *  - the entry and exit limits of the integrator and the aperture at every
@@ -843,7 +843,7 @@ DEV bool csbend_body(double &X, double &QX, double &Y, double &QY, const double 
  * slice of four substeps takes 329 VALU and 36 scalar instructions, where it
  * took 495 (16 of them transcendental, at four times the issue cycles) and
  * 107.  10 turns of 10^6 particles of the storage ring with upload and
- * download: 360 -> 288 ms (206 with what came after it).
+ * download: 360 -> 288 ms (203 with what came after it).
  *
  * What makes every step valid:
  *  - at the entry X, QX, QY are 0 or within [2^-700, 2^600] in magnitude
